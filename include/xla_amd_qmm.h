@@ -231,9 +231,10 @@ int xla_amd_qmm_weight_only_gemm_f32(const float* x, const void* w_tiled, const 
 
 /*
  * Weight-only quantized matmul for any shape, reading the operator's own
- * weight layout (one thread per output element; the slow, always-correct path
- * for shapes the streaming kernel rejects).  Same reference statements and
- * rounding points as xla_amd_qmm_weight_only_skinny.
+ * weight layout: matrix instructions on per-channel weights of any K and
+ * alignment, one thread per output element on blockwise weights (block sizes
+ * the streaming kernel rejects).  Same reference statements and rounding
+ * points as xla_amd_qmm_weight_only_skinny.
  */
 int xla_amd_qmm_weight_only_generic(const void* x, const int8_t* w, const void* scale,
                                     const void* zp, void* out, int64_t M, int64_t N, int64_t K,

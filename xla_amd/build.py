@@ -36,6 +36,7 @@ SOURCES = [
     ("qmm_w8a8_gemm.hip", [], "qmm_w8a8_gemm.o"),
     ("qmm_api.hip", [], "qmm_api.o"),
     ("qmm_generic.hip", [], "qmm_generic.o"),
+    ("qmm_rowmajor.hip", [], "qmm_rowmajor.o"),
     ("qmm_quant_act.hip", [], "qmm_quant_act.o"),
     ("qmm_qdq.hip", [], "qmm_qdq.o"),
     ("qmm_linear.hip", [], "qmm_linear.o"),

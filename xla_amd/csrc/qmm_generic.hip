@@ -1,22 +1,20 @@
-// Always-correct kernels for any shape (one thread per output element) and the
-// one-time weight re-layout.  They define the arithmetic the fast kernels must
-// reproduce: fp32 accumulation inside a reduction, one rounding to the tensor
-// dtype wherever the reference materialises a tensor.
+// The weight-only kernel for blockwise weights of any shape (one thread per output element) and the one-time weight
+// re-layouts.  It defines the arithmetic the fast kernels must reproduce: fp32 accumulation inside a reduction, one
+// rounding to the tensor dtype wherever the reference materialises a tensor.
 #include "qmm_common.h"
+#include "qmm_rowmajor.h"
 
-// out[m,n] for weight-only quantization.
+// out[m,n] for blockwise weights [S,C,N].
 //   p_s   = round_x( sum_c x[m,s,c] * w[s,c,n] )
 //   o     = round_o( sum_s scale[s,n] * p_s )
 //   zpo   = round_z( sum_s round_x(sum_c x[m,s,c]) * zp[s,n] ),  o = round_o(o - zpo)
-// With S == 1 this is the per-channel formula round_o(round_x(dot) * scale[n]).
-// dot_dt replaces x's dtype in the rounding of p_s (f32: the dot product is not rounded);
-// the result is stored as store_dt (out_dt, or a final cast of it).
+// dot_dt replaces x's dtype in the rounding of p_s (f32, one block: the dot product is not rounded); the result is
+// stored as store_dt (out_dt, or a final cast of it).
 __global__ void __launch_bounds__(256)
 qmm_weight_only_generic_kernel(const void* __restrict__ x, const int8_t* __restrict__ w,
                                const void* __restrict__ scale, const void* __restrict__ zp,
                                void* __restrict__ out, int64_t M, int64_t N, int64_t K, int64_t C,
-                               int w_layout, int x_dt, int scale_dt, int zp_dt, int dot_dt, int out_dt,
-                               int store_dt) {
+                               int x_dt, int scale_dt, int zp_dt, int dot_dt, int out_dt, int store_dt) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= M * N) return;
   int64_t m = idx / N, n = idx % N;
@@ -28,8 +26,7 @@ qmm_weight_only_generic_kernel(const void* __restrict__ x, const int8_t* __restr
     for (int64_t c = 0; c < C; ++c) {
       int64_t k = s * C + c;
       float xv = qmm_load(x, m * K + k, x_dt);
-      int8_t wv = (w_layout == XLA_AMD_W_NK) ? w[n * K + k] : w[k * N + n];
-      acc = fmaf(xv, (float)wv, acc);
+      acc = fmaf(xv, (float)w[k * N + n], acc);
       xs += xv;
     }
     float p = qmm_round_dt(acc, dot_dt);
@@ -62,64 +59,21 @@ extern "C" int xla_amd_qmm_weight_only_generic(const void* x, const int8_t* w, c
   if (out_dt != qmm_promote(x_dt, scale_dt))
     return qmm_fail(XLA_AMD_QMM_EINVAL, "weight_only_generic: out dtype must be promote(x, scale)");
   if (M == 0) return XLA_AMD_QMM_OK;
+  if (w_layout == XLA_AMD_W_NK) {
+    QmmRowMajorArgs a = {};
+    a.x = x; a.w = w; a.scale = scale; a.zp = zp; a.out = out;
+    a.M = M; a.N = N; a.K = K;
+    a.scale_dt = scale_dt; a.zp_dt = zp ? zp_dt : x_dt; a.zpo_dt = qmm_promote(x_dt, a.zp_dt); a.out_dt = out_dt;
+    a.dot_dt = dot_dt; a.store_dt = store_dt;
+    return qmm_rowmajor_launch(a, x_dt, (hipStream_t)stream);
+  }
   int64_t total = M * N;
   int64_t blocks = (total + 255) / 256;
   if (blocks > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_generic: too many outputs");
   hipLaunchKernelGGL(qmm_weight_only_generic_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                     (hipStream_t)stream, x, w, scale, zp, out, M, N, K, C, w_layout, x_dt,
-                     scale_dt, zp_dt, dot_dt, out_dt, store_dt);
+                     (hipStream_t)stream, x, w, scale, zp, out, M, N, K, C, x_dt, scale_dt, zp_dt,
+                     dot_dt, out_dt, store_dt);
   return QMM_CHECK_LAUNCH("weight_only_generic launch");
-}
-
-// W8A8 for any K: exact int32 dot, then the epilogue chain documented at
-// xla_amd_qmm_w8a8_gemm.
-__device__ __forceinline__ float qmm_w8a8_epilogue(int acc, int xsum, float ws, float zpv, bool has_zp,
-                                                   float xs, int cvt_dt, int mid_dt, int zpo_dt,
-                                                   int out_dt) {
-  float v = qmm_round_dt((float)acc, cvt_dt);
-  v = qmm_round_dt(v * ws, mid_dt);
-  if (has_zp) {
-    float z = qmm_round_dt(qmm_round_dt((float)xsum, zpo_dt) * zpv, zpo_dt);
-    v = qmm_round_dt(v - z, mid_dt);
-  }
-  return qmm_round_dt(v * xs, out_dt);
-}
-
-__global__ void __launch_bounds__(256)
-qmm_w8a8_generic_kernel(const int8_t* __restrict__ xq, const int8_t* __restrict__ w,
-                        const void* __restrict__ x_scale, const void* __restrict__ w_scale,
-                        const void* __restrict__ zp, const int32_t* __restrict__ x_sum,
-                        void* __restrict__ out, int32_t* __restrict__ acc_out, int64_t M,
-                        int64_t N, int64_t K,
-                        int x_scale_dt, int w_scale_dt, int zp_dt, int cvt_dt, int mid_dt,
-                        int zpo_dt, int out_dt) {
-  int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= M * N) return;
-  int64_t m = idx / N, n = idx % N;
-  int acc = 0;
-  for (int64_t k = 0; k < K; ++k) acc += (int)xq[m * K + k] * (int)w[n * K + k];
-  int xsum = zp ? x_sum[m] : 0;
-  if (acc_out) acc_out[idx] = acc;
-  if (out) {
-    float v = qmm_w8a8_epilogue(acc, xsum, qmm_load(w_scale, n, w_scale_dt),
-                                zp ? qmm_load(zp, n, zp_dt) : 0.f, zp != nullptr,
-                                qmm_load(x_scale, m, x_scale_dt), cvt_dt, mid_dt, zpo_dt, out_dt);
-    qmm_store(out, idx, v, out_dt);
-  }
-}
-
-int qmm_w8a8_generic_launch(const int8_t* xq, const int8_t* w, const void* x_scale,
-                            const void* w_scale, const void* zp, const int32_t* x_sum, void* out,
-                            int32_t* acc_out, int64_t M, int64_t N, int64_t K, int x_scale_dt,
-                            int w_scale_dt,
-                            int zp_dt, int cvt_dt, int mid_dt, int zpo_dt, int out_dt,
-                            hipStream_t stream) {
-  int64_t blocks = (M * N + 255) / 256;
-  if (blocks > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "w8a8 generic: too many outputs");
-  hipLaunchKernelGGL(qmm_w8a8_generic_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, xq, w,
-                     x_scale, w_scale, zp, x_sum, out, acc_out, M, N, K, x_scale_dt, w_scale_dt, zp_dt,
-                     cvt_dt, mid_dt, zpo_dt, out_dt);
-  return QMM_CHECK_LAUNCH("w8a8 generic launch");
 }
 
 // ---- one-time weight re-layout ----------------------------------------------

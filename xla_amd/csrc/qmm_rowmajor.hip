@@ -1,0 +1,249 @@
+// Matmuls against a row-major int8 weight [N, K] for any K and any alignment: the weight-only product of shapes the
+// tiled copy cannot hold (K no multiple of 128) and the int8 product of activations whose K is no multiple of 16.
+//
+// One workgroup of eight waves owns 16 NG NW channels x 16 MT rows of x; NW waves stand side by side along the
+// channels and KW = 8 / NW of them split K.  Nothing goes through LDS but the sums of the K split: a chunk of 64
+// columns is one 16-byte load per lane and 16 channels of weights (lane (r, g) = (lane % 16, lane / 16) takes columns
+// 16 g .. 16 g + 15 of row r) and the same columns of x, which is exactly an operand of the matrix instructions as
+// long as both operands agree on the order of the columns.  Rows start at any byte: the loads are unaligned.
+//
+// What bounds it: memory latency at the sizes it is meant for (a few MB of weight), so a wave has the next chunk's
+// loads in flight during a chunk, and few channels per workgroup put many waves on the chip.  Wide outputs with many
+// rows take more channels per workgroup, since every workgroup reads its rows of x again (out of L2).
+// Per launch, bf16 x against 3000 x 2000: 6.2 us for 1 row, 11.4 for 40 (one thread per output took 1060), 46 for 512.
+#include "qmm_common.h"
+#include "qmm_frag.h"
+#include "qmm_rowmajor.h"
+
+namespace {
+
+using namespace qmm_frag;
+
+constexpr int kWavesAll = 8;
+constexpr int kInt8 = kQmmRowMajorInt8;  // XT of the int8 product (XLA_AMD_DT_* are 0 .. 2)
+
+template <int XT> struct Elem { typedef uint16_t t; };
+template <> struct Elem<XLA_AMD_DT_F32> { typedef float t; };
+template <> struct Elem<kInt8> { typedef int8_t t; };
+
+template <int XT, int MT, int NG, int NW, bool HASZP>
+__global__ void __launch_bounds__(kWavesAll * 64)
+qmm_rowmajor_kernel(QmmRowMajorArgs a) {
+  constexpr int KW = kWavesAll / NW;
+  constexpr bool kInt = XT == kInt8;
+  typedef typename Elem<XT>::t elem_t;
+  constexpr int XV = (int)sizeof(elem_t);  // 16-byte pieces of a lane's 16 elements of x
+  typedef i32x4 acc_t;                     // f32 or int32 sums, by bits
+  __shared__ __attribute__((aligned(16))) int red[KW > 1 ? kWavesAll * (MT * NG + (HASZP ? MT : 0)) * 256 : 1];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = wave % NW, kw = wave / NW;
+  const int r = lane & 15, g = lane >> 4;
+  const int64_t K = a.K;
+  const int64_t n0 = ((int64_t)blockIdx.x * NW + nw) * (16 * NG);
+  const int64_t m0 = (int64_t)blockIdx.y * (16 * MT);
+
+  // rows past the end read the last one again; their sums are dropped
+  const int8_t* wrow[NG];
+  const elem_t* xrow[MT];
+  qmm_static_for<NG>([&](auto gc) { wrow[(int)gc] = a.w + min(n0 + 16 * (int)gc + r, (int64_t)a.N - 1) * K; });
+  qmm_static_for<MT>([&](auto mc) { xrow[(int)mc] = (const elem_t*)a.x + min(m0 + 16 * (int)mc + r, (int64_t)a.M - 1) * K; });
+
+  struct Chunk {
+    i32x4 w[NG];
+    i32x4 x[MT][XV];
+  };
+  auto load = [&](int64_t c, Chunk& d) __attribute__((always_inline)) {
+    const int64_t k = c * 64 + 16 * g;
+    if (c * 64 + 64 <= K) {  // (uniform) whole chunk
+      qmm_static_for<NG>([&](auto gc) { __builtin_memcpy(&d.w[(int)gc], wrow[(int)gc] + k, 16); });
+      qmm_static_for<MT>([&](auto mc) { __builtin_memcpy(&d.x[(int)mc][0], xrow[(int)mc] + k, 16 * XV); });
+    } else {  // the row's end: element by element, zeros after it
+      qmm_static_for<NG>([&](auto gc) {
+        qmm_static_for<4>([&](auto dc) {
+          uint32_t v = 0;
+          qmm_static_for<4>([&](auto bc) {
+            const int64_t at = k + 4 * (int)dc + (int)bc;
+            if (at < K) v |= (uint32_t)(uint8_t)wrow[(int)gc][at] << (8 * (int)bc);
+          });
+          d.w[(int)gc][(int)dc] = (int)v;
+        });
+      });
+      qmm_static_for<MT>([&](auto mc) {
+        constexpr int kPer = 4 / XV;  // elements per dword
+        qmm_static_for<4 * XV>([&](auto dc) {
+          uint32_t v = 0;
+          qmm_static_for<kPer>([&](auto bc) {
+            const int64_t at = k + kPer * (int)dc + (int)bc;
+            if (at < K) {
+              elem_t e = xrow[(int)mc][at];
+              uint32_t bits = 0;
+              __builtin_memcpy(&bits, &e, sizeof(e));
+              v |= bits << (8 * XV * (int)bc);
+            }
+          });
+          d.x[(int)mc][(int)dc / 4][(int)dc % 4] = (int)v;
+        });
+      });
+    }
+  };
+
+  acc_t acc[NG][MT], xs[MT];
+  qmm_static_for<MT>([&](auto mc) {
+    xs[(int)mc] = acc_t{0, 0, 0, 0};
+    qmm_static_for<NG>([&](auto gc) { acc[(int)gc][(int)mc] = acc_t{0, 0, 0, 0}; });
+  });
+  auto multiply = [&](const Chunk& d) __attribute__((always_inline)) {
+    if constexpr (kInt) {
+      qmm_static_for<NG>([&](auto gc) {
+        qmm_static_for<MT>([&](auto mc) {
+          acc[(int)gc][(int)mc] = __builtin_amdgcn_mfma_i32_16x16x64_i8(d.w[(int)gc], d.x[(int)mc][0], acc[(int)gc][(int)mc], 0, 0, 0);
+        });
+      });
+    } else if constexpr (XT == XLA_AMD_DT_F32) {
+      // column 16 g + t of the chunk is k = g of the t-th 16x16x4 instruction
+      qmm_static_for<16>([&](auto tc) {
+        constexpr int t = tc;
+        qmm_static_for<MT>([&](auto mc) {
+          const float xv = __int_as_float(d.x[(int)mc][t / 4][t % 4]);
+          qmm_static_for<NG>([&](auto gc) {
+            const float wv = (float)(int8_t)((uint32_t)d.w[(int)gc][t / 4] >> (8 * (t % 4)));
+            acc[(int)gc][(int)mc] = __builtin_bit_cast(acc_t, __builtin_amdgcn_mfma_f32_16x16x4f32(
+                wv, xv, __builtin_bit_cast(f32x4, acc[(int)gc][(int)mc]), 0, 0, 0));
+          });
+          if constexpr (HASZP)
+            xs[(int)mc] = __builtin_bit_cast(acc_t, __builtin_amdgcn_mfma_f32_16x16x4f32(
+                1.0f, xv, __builtin_bit_cast(f32x4, xs[(int)mc]), 0, 0, 0));
+        });
+      });
+    } else {
+      // columns 16 g + 8 h .. + 7 are the lane's eight of instruction h
+      qmm_static_for<2>([&](auto hc) {
+        constexpr int h = hc;
+        qmm_static_for<NG>([&](auto gc) {
+          const i32x4 wf = cvt_w8<XT>((uint32_t)d.w[(int)gc][2 * h], (uint32_t)d.w[(int)gc][2 * h + 1]);
+          qmm_static_for<MT>([&](auto mc) {
+            acc[(int)gc][(int)mc] = __builtin_bit_cast(acc_t, mfma16<XT>(wf, d.x[(int)mc][h], __builtin_bit_cast(f32x4, acc[(int)gc][(int)mc])));
+          });
+        });
+        if constexpr (HASZP)
+          qmm_static_for<MT>([&](auto mc) {
+            xs[(int)mc] = __builtin_bit_cast(acc_t, mfma16<XT>(ones_frag<XT>(), d.x[(int)mc][h], __builtin_bit_cast(f32x4, xs[(int)mc])));
+          });
+      });
+    }
+  };
+
+  // chunks kw, kw + KW, ...: the next one's loads are in flight during a chunk
+  const int64_t chunks = (K + 63) / 64;
+  Chunk cur;
+  int64_t c = kw;
+  if (c < chunks) load(c, cur);
+  while (c < chunks) {
+    Chunk next;
+    const int64_t cn = c + KW;
+    if (cn < chunks) load(cn, next);
+    multiply(cur);
+    cur = next;
+    c = cn;
+  }
+
+  // one result tile (row set gi, row tile mt): four consecutive channels of one row per lane
+  auto finish = [&](int gi, int mt, acc_t v, acc_t xsum) __attribute__((always_inline)) {
+    const int64_t m = m0 + 16 * mt + r, n = n0 + 16 * gi + 4 * g;
+    if (m >= a.M) return;
+    for (int e = 0; e < 4; ++e) {
+      if (n + e >= a.N) return;
+      const int64_t idx = m * a.N + n + e;
+      if constexpr (kInt) {
+        // the chain documented at xla_amd_qmm_w8a8_gemm
+        if (a.acc_out) a.acc_out[idx] = v[e];
+        if (!a.out) continue;
+        float f = qmm_round_dt((float)v[e], a.cvt_dt);
+        f = qmm_round_dt(f * qmm_load(a.scale, n + e, a.scale_dt), a.mid_dt);
+        if (a.zp) {
+          const float z = qmm_round_dt(qmm_round_dt((float)a.x_sum[m], a.zpo_dt) * qmm_load(a.zp, n + e, a.zp_dt), a.zpo_dt);
+          f = qmm_round_dt(f - z, a.mid_dt);
+        }
+        qmm_store(a.out, idx, qmm_round_dt(f * qmm_load(a.x_scale, m, a.x_scale_dt), a.out_dt), a.out_dt);
+      } else {
+        // p = round_dot(dot); o = round_out(scale p); zero point: o = round_out(o - round_zpo(round_x(sum x) zp))
+        const float p = qmm_round_dt(__int_as_float(v[e]), a.dot_dt);
+        float o = qmm_round_dt(qmm_load(a.scale, n + e, a.scale_dt) * p, a.out_dt);
+        if constexpr (HASZP) {
+          const float z = qmm_round_dt(__int_as_float(xsum[0]), XT) * qmm_load(a.zp, n + e, a.zp_dt);
+          o = qmm_round_dt(o - qmm_round_dt(z, a.zpo_dt), a.out_dt);
+        }
+        qmm_store(a.out, idx, o, a.store_dt);
+      }
+    }
+  };
+  if constexpr (KW == 1) {
+    qmm_static_for<NG>([&](auto gc) {
+      qmm_static_for<MT>([&](auto mc) { finish((int)gc, (int)mc, acc[(int)gc][(int)mc], xs[(int)mc]); });
+    });
+  } else {
+    // every wave leaves its sums; wave kw then adds and finishes the tiles kw, kw + KW, ... of its channels
+    constexpr int T = MT * NG, S = T + (HASZP ? MT : 0);
+    i32x4* const mine = (i32x4*)red + (size_t)wave * S * 64 + lane;
+    qmm_static_for<NG>([&](auto gc) {
+      qmm_static_for<MT>([&](auto mc) { mine[((int)gc * MT + (int)mc) * 64] = acc[(int)gc][(int)mc]; });
+    });
+    if constexpr (HASZP) qmm_static_for<MT>([&](auto mc) { mine[(T + (int)mc) * 64] = xs[(int)mc]; });
+    __syncthreads();
+    for (int t = kw; t < T; t += KW) {
+      acc_t v = {0, 0, 0, 0}, xv = {0, 0, 0, 0};
+      auto add = [&](acc_t& to, int slot) __attribute__((always_inline)) {
+        for (int k2 = 0; k2 < KW; ++k2) {
+          const acc_t o = ((const i32x4*)red)[((size_t)(k2 * NW + nw) * S + slot) * 64 + lane];
+          if constexpr (kInt) to += o;
+          else to = __builtin_bit_cast(acc_t, __builtin_bit_cast(f32x4, to) + __builtin_bit_cast(f32x4, o));
+        }
+      };
+      add(v, t);
+      if constexpr (HASZP) add(xv, T + t % MT);
+      finish(t / MT, t % MT, v, xv);
+    }
+  }
+}
+
+template <int XT, int MT, int NG, int NW>
+int launch(const QmmRowMajorArgs& a, hipStream_t stream) {
+  constexpr int BN = 16 * NG * NW, BM = 16 * MT;
+  const dim3 grid((unsigned)((a.N + BN - 1) / BN), (unsigned)((a.M + BM - 1) / BM)), block(kWavesAll * 64);
+  if (XT != kInt8 && a.zp) hipLaunchKernelGGL((qmm_rowmajor_kernel<XT, MT, NG, NW, XT != kInt8>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((qmm_rowmajor_kernel<XT, MT, NG, NW, false>), grid, block, 0, stream, a);
+  return QMM_CHECK_LAUNCH("row-major matmul launch");
+}
+
+// Channels per workgroup: 256 (every wave its own 32) where that still is two workgroups per compute unit (f32 x, 2048
+// rows against 3000 x 2000, which is 384 of them: 342 us so, 291 with 64 channels), 64 (two waves side by side, four
+// along K) where that fills most of the chip once (512 rows of bf16: 46 us, 52 with 16 channels), else 16 (all eight
+// waves along K: it takes that many waves to have a few MB of weight in flight).
+template <int XT, int MT>
+int launch_width(const QmmRowMajorArgs& a, hipStream_t stream) {
+  const int64_t row_tiles = (a.M + 16 * MT - 1) / (16 * MT);
+  if ((int64_t)((a.N + 255) / 256) * row_tiles >= 512) return launch<XT, MT, 2, 8>(a, stream);
+  if ((int64_t)((a.N + 63) / 64) * row_tiles >= 200) return launch<XT, MT, 2, 2>(a, stream);
+  return launch<XT, MT, 1, 1>(a, stream);
+}
+
+template <int XT>
+int launch_rows(const QmmRowMajorArgs& a, hipStream_t stream) {
+  if (a.M <= 16) return launch_width<XT, 1>(a, stream);
+  if (a.M <= 32) return launch_width<XT, 2>(a, stream);
+  return launch_width<XT, 4>(a, stream);
+}
+
+}  // namespace
+
+int qmm_rowmajor_launch(const QmmRowMajorArgs& a, int x_dt, hipStream_t stream) {
+  if ((a.M + 15) / 16 > 65535) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "row-major matmul: too many rows");
+  switch (x_dt) {
+    case XLA_AMD_DT_F32: return launch_rows<XLA_AMD_DT_F32>(a, stream);
+    case XLA_AMD_DT_BF16: return launch_rows<XLA_AMD_DT_BF16>(a, stream);
+    case XLA_AMD_DT_F16: return launch_rows<XLA_AMD_DT_F16>(a, stream);
+    default: return launch_rows<kInt8>(a, stream);
+  }
+}

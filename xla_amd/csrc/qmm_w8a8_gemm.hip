@@ -16,12 +16,7 @@
 //   result : acc[v] of lane l is D[8*(v/4) + 4*(l/32) + v%4][l%32]  (row = m, col = n)
 // so one result register of a wave is 32 consecutive n of a row: coalesced stores.
 #include "qmm_common.h"
-
-int qmm_w8a8_generic_launch(const int8_t* xq, const int8_t* w, const void* x_scale,
-                            const void* w_scale, const void* zp, const int32_t* x_sum, void* out,
-                            int32_t* acc_out, int64_t M, int64_t N, int64_t K, int x_scale_dt,
-                            int w_scale_dt, int zp_dt, int cvt_dt, int mid_dt, int zpo_dt,
-                            int out_dt, hipStream_t stream);
+#include "qmm_rowmajor.h"
 
 namespace {
 
@@ -602,9 +597,14 @@ extern "C" int xla_amd_qmm_w8a8_gemm(const int8_t* x_q, const int8_t* w, const v
   if (M == 0) return XLA_AMD_QMM_OK;
   hipStream_t s = (hipStream_t)stream;
   const bool fast = (K % 16 == 0) && ((((uintptr_t)x_q | (uintptr_t)w) & 15) == 0);
-  if (!fast)
-    return qmm_w8a8_generic_launch(x_q, w, x_scale, w_scale, zp, x_sum, out, acc_out, M, N, K,
-                                   x_scale_dt, w_scale_dt, zp_dt, cvt_dt, mid_dt, zpo_dt, out_dt, s);
+  if (!fast) {  // K no multiple of 16, or unaligned operands: the kernel for rows that start at any byte
+    QmmRowMajorArgs r = {};
+    r.x = x_q; r.w = w; r.scale = w_scale; r.zp = out ? zp : nullptr; r.out = out; r.acc_out = acc_out;
+    r.M = M; r.N = N; r.K = K;
+    r.scale_dt = w_scale_dt; r.zp_dt = zp_dt; r.zpo_dt = zpo_dt; r.out_dt = out_dt;
+    r.x_scale = x_scale; r.x_sum = x_sum; r.x_scale_dt = x_scale_dt; r.cvt_dt = cvt_dt; r.mid_dt = mid_dt;
+    return qmm_rowmajor_launch(r, kQmmRowMajorInt8, s);
+  }
   GemmArgs g;
   g.a = x_q; g.b = w; g.x_scale = x_scale; g.w_scale = w_scale; g.zp = out ? zp : nullptr;
   g.x_sum = x_sum; g.out = out; g.acc_out = acc_out;
