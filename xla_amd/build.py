@@ -33,6 +33,8 @@ SOURCES = [
     ("qmm_wo_gemm.hip", ["-DQMM_WO_XT=2", "-DQMM_WO_MT=4"], "qmm_wo_gemm_f16_mt4.o"),
     ("qmm_wo_gemm_bw.hip", ["-DQMM_WO_BW_XT=1"], "qmm_wo_gemm_bw_bf16.o"),
     ("qmm_wo_gemm_bw.hip", ["-DQMM_WO_BW_XT=2"], "qmm_wo_gemm_bw_f16.o"),
+    ("qmm_wo_gemm_bw_wide.hip", ["-DQMM_WO_BW_XT=1"], "qmm_wo_gemm_bw_wide_bf16.o"),
+    ("qmm_wo_gemm_bw_wide.hip", ["-DQMM_WO_BW_XT=2"], "qmm_wo_gemm_bw_wide_f16.o"),
     ("qmm_w8a8_gemm.hip", [], "qmm_w8a8_gemm.o"),
     ("qmm_api.hip", [], "qmm_api.o"),
     ("qmm_generic.hip", [], "qmm_generic.o"),

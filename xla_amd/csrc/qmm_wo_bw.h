@@ -16,3 +16,7 @@ struct WoBwArgs {
 // bits = 4 or 8; x's dtype by launcher
 int qmm_wo_bw_launch_bf16(const WoBwArgs& a, int bits, hipStream_t stream);
 int qmm_wo_bw_launch_f16(const WoBwArgs& a, int bits, hipStream_t stream);
+// the same in tiles of 64 x 256 (qmm_wo_gemm_bw_wide.hip), called by the launchers above; cus: compute units to fill;
+// a zero point only with bits = 4 and C = 128
+int qmm_wo_bw_wide_launch_bf16(const WoBwArgs& a, int bits, int cus, hipStream_t stream);
+int qmm_wo_bw_wide_launch_f16(const WoBwArgs& a, int bits, int cus, hipStream_t stream);

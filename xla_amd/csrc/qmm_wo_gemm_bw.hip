@@ -3,7 +3,8 @@
 //
 // The weight-streaming kernel (qmm_skinny.hip) re-reads the whole weight for every 32 rows of
 // x; a prefill-sized M against blockwise int4 weights would take M / 32 passes.  Here a
-// workgroup owns a tile of 64 rows x 128 channels and reads its weights once.
+// workgroup owns a tile of 64 rows x 128 channels and reads its weights once (launches with many
+// tiles take the wider ones of qmm_wo_gemm_bw_wide.hip).
 //
 // Operands, as in qmm_wo_gemm.hip: weights come from the tiled copy (one block per 16 channels x
 // 128 columns, 2 KB int8 / 1 KB int4, in MFMA operand order) straight into registers, one step
@@ -500,10 +501,28 @@ int cu_count() {
   return n;
 }
 
+// The 64 x 256 tiles of qmm_wo_gemm_bw_wide.hip take half as many rounds over the compute units, each 1.45 (int4 with a
+// zero point: 43 against 30 us at K = 4096) to 1.65 times as long (int8: 44 / 27; without a zero point int4 42 / 28,
+// per-channel int4 35 / 23), so they are for launches whose rounds come to that much fewer: from about two rounds of
+// 64 x 128 tiles on (1024 rows against 4096 x 4096, int4: 60 -> 43 us; 512 rows, one round either way: 33 -> 40, kept
+// here).  With a zero point the wide kernel exists for int4 weights in blocks of 128 columns only: 96 accumulator
+// registers leave no room for the second load of int8 weights or for the bookkeeping of longer blocks.
+template <int XT, int BITS>
+bool wide_tiles(const WoBwArgs& a, int64_t items, int cus) {
+  if (a.zp && !(BITS == 4 && a.C == 128)) return false;
+  const int64_t wide = (int64_t)((a.M + BM - 1) / BM) * ((a.N + 255) / 256);
+  const int64_t cost = a.zp ? 145 : BITS == 4 ? 155 : 165;
+  return (wide + cus - 1) / cus * cost < (items + cus - 1) / cus * 100;
+}
+
 template <int XT, int BITS>
 int launch(const WoBwArgs& a, hipStream_t stream) {
   const int64_t items = (int64_t)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
   const int cus = cu_count();
+  if (wide_tiles<XT, BITS>(a, items, cus)) {
+    if constexpr (XT == XLA_AMD_DT_BF16) return qmm_wo_bw_wide_launch_bf16(a, BITS, cus, stream);
+    else return qmm_wo_bw_wide_launch_f16(a, BITS, cus, stream);
+  }
   const dim3 grid((unsigned)(items < cus ? items : cus)), block((kComputeWaves + kCopyWaves) * 64);
   auto go = [&](auto kern) -> int {
     static std::atomic<uint64_t> lds_set{0};
