@@ -391,6 +391,19 @@ int xla_amd_qmm_dequantize_affine(const void* q, void* out, const float* scale, 
                                   int64_t outer, int64_t channels, int64_t inner, int q_dt, int out_dt,
                                   int int_subtract, void* stream);
 
+/*
+ * The per-channel forms with the parameters as quantize_per_channel /
+ * dequantize_per_channel take them: scale f32, bf16 or f16 (scale_dt) and zero
+ * point int64 (zp_int64 != 0) or int32, `channels` entries each; the quantizer
+ * multiplies by 1 / f32(scale[c]).  dequantize: zp may be NULL (zero).
+ */
+int xla_amd_qmm_quantize_channels(const void* x, void* q, const void* scale, const void* zp,
+                                  int64_t outer, int64_t channels, int64_t inner, int x_dt, int q_dt,
+                                  int scale_dt, int zp_int64, int32_t qmin, int32_t qmax, void* stream);
+int xla_amd_qmm_dequantize_channels(const void* q, void* out, const void* scale, const void* zp,
+                                    int64_t outer, int64_t channels, int64_t inner, int q_dt, int out_dt,
+                                    int scale_dt, int zp_int64, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -50,6 +50,8 @@ SIGNATURES = {
     "xla_amd_qmm_w8a8_tile": (_c_int, [_c_i64] * 3 + [ctypes.POINTER(ctypes.c_int32)]),
     "xla_amd_qmm_quantize_affine": (_c_int, [_c_vp] * 4 + [_c_i64] * 3 + [_c_int] * 2 + [ctypes.c_int32] * 2 + [_c_vp]),
     "xla_amd_qmm_dequantize_affine": (_c_int, [_c_vp] * 4 + [_c_i64] * 3 + [_c_int] * 3 + [_c_vp]),
+    "xla_amd_qmm_quantize_channels": (_c_int, [_c_vp] * 4 + [_c_i64] * 3 + [_c_int] * 4 + [ctypes.c_int32] * 2 + [_c_vp]),
+    "xla_amd_qmm_dequantize_channels": (_c_int, [_c_vp] * 4 + [_c_i64] * 3 + [_c_int] * 4 + [_c_vp]),
 }
 
 _lib = None

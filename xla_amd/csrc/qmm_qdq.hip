@@ -34,44 +34,119 @@ __device__ __forceinline__ int quantize_value(float x, float inv_scale, float zp
   return (x != x) ? 0 : (int)r;
 }
 
-// One thread per 8 consecutive elements of a row of `inner` (inner % 8 == 0,
-// 16-byte aligned x, 8-byte aligned q, 1-byte q) or per element otherwise.
-template <int XT, bool VEC>
-__global__ void __launch_bounds__(256)
-qdq_quantize_kernel(const void* __restrict__ x, void* __restrict__ q, const float* __restrict__ inv_scale,
-                    const int32_t* __restrict__ zp, int64_t total, int64_t channels, int64_t inner,
-                    int q_dt, float qmin, float qmax) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if constexpr (VEC) {
-    const int64_t e0 = t * 8;
-    if (e0 >= total) return;
-    const int64_t c = (e0 / inner) % channels;
-    const float is = inv_scale[c], z = (float)zp[c];
-    float f[8];
-    if constexpr (XT == XLA_AMD_DT_F32) {
-      const f32x4 a = ((const f32x4*)((const float*)x + e0))[0], b = ((const f32x4*)((const float*)x + e0))[1];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { f[i] = a[i]; f[4 + i] = b[i]; }
+// The parameters of a call as the caller holds them: scale (or its reciprocal) f32, bf16 or f16, zero point int32 or
+// int64 or none.  Converting them beforehand took four launches of a few microseconds each around a
+// quantize / dequantize pair: 14336 x 4096 bf16 to f32 103.9 us, 75.7 without them and with the streaming stores below
+// (470 MB: 6.2 TB/s).
+struct QdqParams {
+  const void* scale;
+  const void* zp;   // null: 0
+  int scale_dt, zp64, reciprocal;  // reciprocal: what multiplies x is 1 / scale
+};
+__device__ __forceinline__ float qdq_scale(const QdqParams& p, uint32_t c) {
+  const float s = qmm_load(p.scale, c, p.scale_dt);
+  return p.reciprocal ? 1.0f / s : s;
+}
+__device__ __forceinline__ int qdq_zp(const QdqParams& p, uint32_t c) {
+  if (!p.zp) return 0;
+  return p.zp64 ? (int)((const int64_t*)p.zp)[c] : ((const int32_t*)p.zp)[c];
+}
+
+// How the elements of a tensor [outer, channels, inner] find their channel.  A thread of the vector forms handles U
+// runs of consecutive elements: kOne, one channel; kRow, a run lies within a channel (inner a multiple of the run);
+// kAlong, inner == 1, a run lies along the channels (channels a multiple of the run).  kAny: element by element.
+// What bounds the vector forms is memory alone as long as a run's channel costs few instructions: 32-bit divisions by
+// the row length (the 64-bit ones of kAny take over a hundred instructions), none for kOne; in kAlong a thread's runs
+// lie below each other, so that it fetches its channels' parameters (and divides for the quantizer's reciprocals) once
+// for kDown of them (4096 x 4096 along the last axis, a quantize / dequantize pair: 37 us; with two runs side by side 108).
+enum Form { kOne, kRow, kAlong, kAny };
+constexpr int kThreads = 256;
+constexpr int kPerBlock = 4096;  // elements per workgroup of kOne and kRow: several runs in flight per thread
+constexpr int kDown = 8;         // rows per thread of kAlong
+struct QdqShape {
+  int64_t total, outer, channels, inner;
+};
+template <Form F, int RUN> constexpr int runs_per_thread() { return F == kAlong ? kDown : kPerBlock / (kThreads * RUN); }
+// The thread's runs: first + u * stride, u < live (>= 1), and the channel of run u (kAlong: of every one).
+template <Form F, int RUN>
+struct Runs {
+  uint32_t first, stride, live;
+  __device__ __forceinline__ explicit Runs(const QdqShape& sh) {
+    constexpr uint32_t U = runs_per_thread<F, RUN>();
+    if constexpr (F == kAlong) {
+      const uint32_t per_row = (uint32_t)(sh.channels / RUN), rows = (uint32_t)sh.outer;
+      const uint32_t t = blockIdx.x * kThreads + threadIdx.x, down = t / per_row;  // (t < 2^32 / kDown)
+      const uint32_t row = down * U;
+      live = row < rows ? min(U, rows - row) : 0;
+      first = row * per_row + (t - down * per_row);
+      stride = per_row;
     } else {
-      const i32x4 a = *(const i32x4*)((const uint16_t*)x + e0);
+      const uint32_t runs = (uint32_t)(sh.total / RUN);
+      first = blockIdx.x * (kThreads * U) + threadIdx.x;
+      stride = kThreads;
+      live = first < runs ? min(U, (runs - first + kThreads - 1) / kThreads) : 0;
+    }
+  }
+  __device__ __forceinline__ uint32_t run(uint32_t u) const { return first + min(u, live - 1) * stride; }  // (the end repeats the last)
+  __device__ __forceinline__ uint32_t channel(const QdqShape& sh, uint32_t run) const {
+    if constexpr (F == kOne) return 0;
+    if constexpr (F == kRow) return (run / (uint32_t)(sh.inner / RUN)) % (uint32_t)sh.channels;
+    return run % stride * RUN;
+  }
+};
+
+// Quantize; vector forms: runs of 8, 16-byte aligned x, 8-byte aligned q, 1-byte q, total / 8 < 2^32.
+// NT: streaming loads of x.
+template <int XT, Form F, bool NT>
+__global__ void __launch_bounds__(kThreads)
+qdq_quantize_kernel(const void* __restrict__ x, void* __restrict__ q, QdqParams p, QdqShape sh, int q_dt, float qmin,
+                    float qmax) {
+  if constexpr (F != kAny) {
+    constexpr int RUN = 8, U = runs_per_thread<F, RUN>();
+    const Runs<F, RUN> at(sh);
+    if (at.live == 0) return;
+    constexpr int D = XT == XLA_AMD_DT_F32 ? 2 : 1;
+    i32x4 raw[U][D];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t d = (uint32_t)a[i];
-        f[2 * i] = XT == XLA_AMD_DT_BF16 ? __uint_as_float(d << 16) : qmm_f16_to_f32((uint16_t)(d & 0xffffu));
-        f[2 * i + 1] = XT == XLA_AMD_DT_BF16 ? __uint_as_float(d & 0xffff0000u) : qmm_f16_to_f32((uint16_t)(d >> 16));
+    for (int u = 0; u < U; ++u) {
+      const i32x4* const from = (const i32x4*)x + (size_t)at.run(u) * D;
+#pragma unroll
+      for (int d = 0; d < D; ++d) raw[u][d] = NT ? __builtin_nontemporal_load(from + d) : from[d];
+    }
+    float isv[RUN], zv[RUN];
+    if constexpr (F == kAlong) {
+      const uint32_t c = at.channel(sh, at.first);
+#pragma unroll
+      for (int i = 0; i < RUN; ++i) { isv[i] = qdq_scale(p, c + i); zv[i] = (float)qdq_zp(p, c + i); }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t run = at.run(u);
+      float is = 0.f, z = 0.f;
+      if constexpr (F != kAlong) {
+        const uint32_t c = at.channel(sh, run);
+        is = qdq_scale(p, c); z = (float)qdq_zp(p, c);
       }
-    }
-    uint32_t lo = 0, hi = 0;
+      uint32_t out[2] = {0, 0};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      lo |= ((uint32_t)(uint8_t)quantize_value(f[i], is, z, qmin, qmax)) << (8 * i);
-      hi |= ((uint32_t)(uint8_t)quantize_value(f[4 + i], is, z, qmin, qmax)) << (8 * i);
+      for (int i = 0; i < RUN; ++i) {
+        float f;
+        if constexpr (XT == XLA_AMD_DT_F32) {
+          f = __int_as_float(raw[u][i / 4][i % 4]);
+        } else {
+          const uint32_t w = (uint32_t)raw[u][0][i / 2];
+          f = qmm_from_raw((i & 1) ? (w >> 16) : (w & 0xffffu), XT);
+        }
+        if constexpr (F == kAlong) { is = isv[i]; z = zv[i]; }
+        out[i / 4] |= ((uint32_t)(uint8_t)quantize_value(f, is, z, qmin, qmax)) << (8 * (i % 4));
+      }
+      *(i32x2*)((uint8_t*)q + (size_t)run * RUN) = i32x2{(int)out[0], (int)out[1]};
     }
-    *(i32x2*)((uint8_t*)q + e0) = i32x2{(int)lo, (int)hi};
   } else {
-    if (t >= total) return;
-    const int64_t c = (t / inner) % channels;
-    qdq_store_q(q, t, quantize_value(qmm_load(x, t, XT), inv_scale[c], (float)zp[c], qmin, qmax), q_dt);
+    const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (t >= sh.total) return;
+    const uint32_t c = (uint32_t)((t / sh.inner) % sh.channels);
+    qdq_store_q(q, t, quantize_value(qmm_load(x, t, XT), qdq_scale(p, c), (float)qdq_zp(p, c), qmin, qmax), q_dt);
   }
 }
 
@@ -85,105 +160,177 @@ __device__ __forceinline__ float dequantize_value(int qv, int z, float sc, int o
   return d * sc;
 }
 
-// VEC: one thread per 8 consecutive 1-byte elements of a row of `inner`
-// (inner % 8 == 0, 8-byte aligned q, 32-byte aligned out), else one per element.
-template <bool VEC>
-__global__ void __launch_bounds__(256)
-qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, const float* __restrict__ scale,
-                      const int32_t* __restrict__ zp, int64_t total, int64_t channels, int64_t inner,
-                      int q_dt, int out_dt, int int_subtract) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if constexpr (VEC) {
-    const int64_t e0 = t * 8;
-    if (e0 >= total) return;
-    const int64_t c = (e0 / inner) % channels;
-    const int z = zp ? zp[c] : 0;
-    const float sc = scale[c];
-    const i32x2 raw = *(const i32x2*)((const uint8_t*)q + e0);
-    float r[8];
+// Dequantize; vector forms: runs of 4 (f32 out) or 8 (2-byte out), i.e. 16-byte stores, q aligned to a run, out to 16
+// bytes, 1-byte q, total / 4 < 2^32.
+// NT: streaming stores of out.  (A template: a branch around two forms of a store leaves the ordinary one.)
+template <int OT, Form F, bool NT>
+__global__ void __launch_bounds__(kThreads)
+qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, QdqParams p, QdqShape sh, int q_dt,
+                      int int_subtract) {
+  if constexpr (F != kAny) {
+    constexpr int RUN = OT == XLA_AMD_DT_F32 ? 4 : 8, U = runs_per_thread<F, RUN>();
+    const Runs<F, RUN> at(sh);
+    if (at.live == 0) return;
+    uint32_t raw[U][RUN / 4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t b = ((uint32_t)raw[i >> 2] >> (8 * (i & 3))) & 0xffu;
-      const int qv = q_dt == XLA_AMD_QDT_I8 ? (int)(int8_t)b : (int)b;
-      r[i] = dequantize_value(qv, z, sc, out_dt, int_subtract);
-    }
-    if (out_dt == XLA_AMD_DT_F32) {
-      f32x4* o = (f32x4*)((float*)out + e0);
-      o[0] = f32x4{r[0], r[1], r[2], r[3]};
-      o[1] = f32x4{r[4], r[5], r[6], r[7]};
-    } else {
-      i32x4 pk;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t lo = out_dt == XLA_AMD_DT_BF16 ? qmm_f32_to_bf16(r[2 * i]) : qmm_f32_to_f16(r[2 * i]);
-        const uint32_t hi = out_dt == XLA_AMD_DT_BF16 ? qmm_f32_to_bf16(r[2 * i + 1]) : qmm_f32_to_f16(r[2 * i + 1]);
-        pk[i] = (int)(lo | (hi << 16));
+    for (int u = 0; u < U; ++u) {
+      const uint32_t run = at.run(u);
+      if constexpr (RUN == 4) {
+        raw[u][0] = ((const uint32_t*)q)[run];
+      } else {
+        const i32x2 v = ((const i32x2*)q)[run];
+        raw[u][0] = (uint32_t)v[0]; raw[u][1] = (uint32_t)v[1];
       }
-      *(i32x4*)((uint16_t*)out + e0) = pk;
+    }
+    float scv[RUN];
+    int zv[RUN];
+    if constexpr (F == kAlong) {
+      const uint32_t c = at.channel(sh, at.first);
+#pragma unroll
+      for (int i = 0; i < RUN; ++i) { scv[i] = qdq_scale(p, c + i); zv[i] = qdq_zp(p, c + i); }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t run = at.run(u);
+      float sc = 0.f;
+      int z = 0;
+      if constexpr (F != kAlong) {
+        const uint32_t c = at.channel(sh, run);
+        sc = qdq_scale(p, c); z = qdq_zp(p, c);
+      }
+      float r[RUN];
+#pragma unroll
+      for (int i = 0; i < RUN; ++i) {
+        const uint32_t b = (raw[u][i / 4] >> (8 * (i % 4))) & 0xffu;
+        const int qv = q_dt == XLA_AMD_QDT_I8 ? (int)(int8_t)b : (int)b;
+        if constexpr (F == kAlong) { sc = scv[i]; z = zv[i]; }
+        r[i] = dequantize_value(qv, z, sc, OT, int_subtract);
+      }
+      if constexpr (OT == XLA_AMD_DT_F32) {
+        const f32x4 v = {r[0], r[1], r[2], r[3]};
+        if constexpr (NT) __builtin_nontemporal_store(v, (f32x4*)out + run);
+        else ((f32x4*)out)[run] = v;
+      } else {
+        i32x4 pk;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          pk[i] = (int)(OT == XLA_AMD_DT_BF16 ? qmm_f32x2_to_bf16x2(r[2 * i], r[2 * i + 1]) : qmm_f32x2_to_f16x2(r[2 * i], r[2 * i + 1]));
+        if constexpr (NT) __builtin_nontemporal_store(pk, (i32x4*)out + run);
+        else ((i32x4*)out)[run] = pk;
+      }
     }
   } else {
-    if (t >= total) return;
-    const int64_t c = (t / inner) % channels;
-    const int z = zp ? zp[c] : 0;
-    qmm_store(out, t, dequantize_value(qdq_load_q(q, t, q_dt), z, scale[c], out_dt, int_subtract), out_dt);
+    const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (t >= sh.total) return;
+    const uint32_t c = (uint32_t)((t / sh.inner) % sh.channels);
+    qmm_store(out, t, dequantize_value(qdq_load_q(q, t, q_dt), qdq_zp(p, c), qdq_scale(p, c), OT, int_subtract), OT);
   }
 }
 
 bool valid_qdt(int q_dt) { return q_dt >= XLA_AMD_QDT_I8 && q_dt <= XLA_AMD_QDT_I32; }
 
-}  // namespace
+// Tensors that pass through the 256 MB Infinity Cache without staying in it are streamed past it, so that the other
+// side of the call keeps its place: a float input larger than the cache (14336 x 14336 f32, 822 MB, and its f32 result:
+// 355 us a pair with its loads kept, 314 streamed; 117 MB of bf16: 77 kept, 80 streamed), a float result of a quarter of
+// it and more (235 MB of f32: 89 kept, 77 streamed; 117 MB of bf16: 63, 60).
+constexpr int64_t kStreamIn = 256ll << 20, kStreamOut = 64ll << 20;
 
-extern "C" int xla_amd_qmm_quantize_affine(const void* x, void* q, const float* inv_scale,
-                                           const int32_t* zp, int64_t outer, int64_t channels,
-                                           int64_t inner, int x_dt, int q_dt, int32_t qmin,
-                                           int32_t qmax, void* stream) {
-  if (!x || !q || !inv_scale || !zp) return qmm_fail(XLA_AMD_QMM_EINVAL, "quantize_affine: null pointer");
-  if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "quantize_affine: bad sizes");
-  if (!qmm_valid_dt(x_dt) || !valid_qdt(q_dt) || qmin > qmax)
-    return qmm_fail(XLA_AMD_QMM_EINVAL, "quantize_affine: bad dtype enum or bounds");
-  const int64_t total = outer * channels * inner;
-  if (total == 0) return XLA_AMD_QMM_OK;
-  const bool vec = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && inner % 8 == 0 &&
-                   (((uintptr_t)x & 15) == 0) && (((uintptr_t)q & 7) == 0);
-  const int64_t threads = vec ? total / 8 : total;
-  const int64_t blocks = (threads + 255) / 256;
-  if (blocks > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "quantize_affine: tensor too large");
-  hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)blocks), block(256);
-  const float fmin = (float)qmin, fmax = (float)qmax;
-#define QDQ_LAUNCH(XT)                                                                                          \
-  do {                                                                                                          \
-    if (vec) hipLaunchKernelGGL((qdq_quantize_kernel<XT, true>), grid, block, 0, s, x, q, inv_scale, zp, total, \
-                                channels, inner, q_dt, fmin, fmax);                                             \
-    else hipLaunchKernelGGL((qdq_quantize_kernel<XT, false>), grid, block, 0, s, x, q, inv_scale, zp, total,    \
-                            channels, inner, q_dt, fmin, fmax);                                                 \
-  } while (0)
-  if (x_dt == XLA_AMD_DT_BF16) QDQ_LAUNCH(XLA_AMD_DT_BF16);
-  else if (x_dt == XLA_AMD_DT_F16) QDQ_LAUNCH(XLA_AMD_DT_F16);
-  else QDQ_LAUNCH(XLA_AMD_DT_F32);
-#undef QDQ_LAUNCH
-  return QMM_CHECK_LAUNCH("quantize_affine launch");
+// The form for runs of `run` elements, and whether everything is aligned for it.
+Form choose_form(const QdqShape& sh, int run, bool aligned) {
+  if (!aligned || sh.total % run != 0 || sh.total / run > 0xffffffffLL - kPerBlock || sh.channels > 0x7fffffffLL) return kAny;
+  if (sh.channels == 1) return kOne;
+  if (sh.inner % run == 0 && sh.inner / run <= 0x7fffffffLL) return kRow;
+  if (sh.inner == 1 && sh.channels % run == 0 && sh.outer <= 0x7fffffffLL) return kAlong;
+  return kAny;
 }
 
-extern "C" int xla_amd_qmm_dequantize_affine(const void* q, void* out, const float* scale,
-                                             const int32_t* zp, int64_t outer, int64_t channels,
-                                             int64_t inner, int q_dt, int out_dt, int int_subtract,
-                                             void* stream) {
-  if (!q || !out || !scale) return qmm_fail(XLA_AMD_QMM_EINVAL, "dequantize_affine: null pointer");
-  if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "dequantize_affine: bad sizes");
-  if (!qmm_valid_dt(out_dt) || !valid_qdt(q_dt)) return qmm_fail(XLA_AMD_QMM_EINVAL, "dequantize_affine: bad dtype enum");
-  const int64_t total = outer * channels * inner;
-  if (total == 0) return XLA_AMD_QMM_OK;
-  const bool vec = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && inner % 8 == 0 &&
-                   (((uintptr_t)q & 7) == 0) && (((uintptr_t)out & 31) == 0);
-  const int64_t threads = vec ? total / 8 : total;
-  const int64_t blocks = (threads + 255) / 256;
-  if (blocks > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "dequantize_affine: tensor too large");
-  if (vec)
-    hipLaunchKernelGGL(qdq_dequantize_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, q, out,
-                       scale, zp, total, channels, inner, q_dt, out_dt, int_subtract);
-  else
-    hipLaunchKernelGGL(qdq_dequantize_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, q, out,
-                       scale, zp, total, channels, inner, q_dt, out_dt, int_subtract);
-  return QMM_CHECK_LAUNCH("dequantize_affine launch");
+// Calls go(form constant, grid) for runs of `run` elements; returns the launch's status.
+template <class Go>
+int launch_form(Form f, const QdqShape& sh, int run, const char* what, Go&& go) {
+  int64_t threads = sh.total, per = kThreads;
+  if (f == kAlong) threads = (sh.outer + kDown - 1) / kDown * (sh.channels / run);
+  else if (f != kAny) per = kPerBlock;
+  const int64_t blocks = (threads + per - 1) / per;
+  if (blocks > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "%s: tensor too large", what);
+  const dim3 grid((unsigned)blocks);
+  switch (f) {
+    case kOne: go(qmm_const<kOne>{}, grid); break;
+    case kRow: go(qmm_const<kRow>{}, grid); break;
+    case kAlong: go(qmm_const<kAlong>{}, grid); break;
+    default: go(qmm_const<kAny>{}, grid); break;
+  }
+  return QMM_CHECK_LAUNCH(what);
+}
+
+int quantize(const char* what, const void* x, void* q, const QdqParams& p, int64_t outer, int64_t channels,
+             int64_t inner, int x_dt, int q_dt, int32_t qmin, int32_t qmax, void* stream) {
+  if (!x || !q || !p.scale || !p.zp) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: null pointer", what);
+  if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad sizes", what);
+  if (!qmm_valid_dt(x_dt) || !qmm_valid_dt(p.scale_dt) || !valid_qdt(q_dt) || qmin > qmax)
+    return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum or bounds", what);
+  const QdqShape sh = {outer * channels * inner, outer, channels, inner};
+  if (sh.total == 0) return XLA_AMD_QMM_OK;
+  const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)q & 7) == 0);
+  const bool nt = sh.total * qmm_dt_size(x_dt) > kStreamIn;
+  return launch_form(choose_form(sh, 8, aligned), sh, 8, what, [&](auto fc, dim3 grid) {
+    constexpr Form F = (Form)(int)fc;
+    const auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, (hipStream_t)stream, x, q, p, sh, q_dt, (float)qmin, (float)qmax);
+    };
+    if (x_dt == XLA_AMD_DT_BF16) nt ? go(qdq_quantize_kernel<XLA_AMD_DT_BF16, F, F != kAny>) : go(qdq_quantize_kernel<XLA_AMD_DT_BF16, F, false>);
+    else if (x_dt == XLA_AMD_DT_F16) nt ? go(qdq_quantize_kernel<XLA_AMD_DT_F16, F, F != kAny>) : go(qdq_quantize_kernel<XLA_AMD_DT_F16, F, false>);
+    else nt ? go(qdq_quantize_kernel<XLA_AMD_DT_F32, F, F != kAny>) : go(qdq_quantize_kernel<XLA_AMD_DT_F32, F, false>);
+  });
+}
+
+int dequantize(const char* what, const void* q, void* out, const QdqParams& p, int64_t outer, int64_t channels,
+               int64_t inner, int q_dt, int out_dt, int int_subtract, void* stream) {
+  if (!q || !out || !p.scale) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: null pointer", what);
+  if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad sizes", what);
+  if (!qmm_valid_dt(out_dt) || !qmm_valid_dt(p.scale_dt) || !valid_qdt(q_dt))
+    return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum", what);
+  const QdqShape sh = {outer * channels * inner, outer, channels, inner};
+  if (sh.total == 0) return XLA_AMD_QMM_OK;
+  const int run = out_dt == XLA_AMD_DT_F32 ? 4 : 8;
+  const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)q & (run - 1)) == 0) && (((uintptr_t)out & 15) == 0);
+  const bool nt = sh.total * qmm_dt_size(out_dt) > kStreamOut;
+  return launch_form(choose_form(sh, run, aligned), sh, run, what, [&](auto fc, dim3 grid) {
+    constexpr Form F = (Form)(int)fc;
+    const auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, (hipStream_t)stream, q, out, p, sh, q_dt, int_subtract);
+    };
+    if (out_dt == XLA_AMD_DT_BF16) nt ? go(qdq_dequantize_kernel<XLA_AMD_DT_BF16, F, F != kAny>) : go(qdq_dequantize_kernel<XLA_AMD_DT_BF16, F, false>);
+    else if (out_dt == XLA_AMD_DT_F16) nt ? go(qdq_dequantize_kernel<XLA_AMD_DT_F16, F, F != kAny>) : go(qdq_dequantize_kernel<XLA_AMD_DT_F16, F, false>);
+    else nt ? go(qdq_dequantize_kernel<XLA_AMD_DT_F32, F, F != kAny>) : go(qdq_dequantize_kernel<XLA_AMD_DT_F32, F, false>);
+  });
+}
+
+}  // namespace
+
+extern "C" int xla_amd_qmm_quantize_affine(const void* x, void* q, const float* inv_scale, const int32_t* zp,
+                                           int64_t outer, int64_t channels, int64_t inner, int x_dt, int q_dt,
+                                           int32_t qmin, int32_t qmax, void* stream) {
+  return quantize("quantize_affine", x, q, QdqParams{inv_scale, zp, XLA_AMD_DT_F32, 0, 0}, outer, channels, inner, x_dt,
+                  q_dt, qmin, qmax, stream);
+}
+
+extern "C" int xla_amd_qmm_dequantize_affine(const void* q, void* out, const float* scale, const int32_t* zp,
+                                             int64_t outer, int64_t channels, int64_t inner, int q_dt, int out_dt,
+                                             int int_subtract, void* stream) {
+  return dequantize("dequantize_affine", q, out, QdqParams{scale, zp, XLA_AMD_DT_F32, 0, 0}, outer, channels, inner,
+                    q_dt, out_dt, int_subtract, stream);
+}
+
+extern "C" int xla_amd_qmm_quantize_channels(const void* x, void* q, const void* scale, const void* zp, int64_t outer,
+                                             int64_t channels, int64_t inner, int x_dt, int q_dt, int scale_dt,
+                                             int zp_int64, int32_t qmin, int32_t qmax, void* stream) {
+  return quantize("quantize_channels", x, q, QdqParams{scale, zp, scale_dt, zp_int64 != 0, 1}, outer, channels, inner,
+                  x_dt, q_dt, qmin, qmax, stream);
+}
+
+extern "C" int xla_amd_qmm_dequantize_channels(const void* q, void* out, const void* scale, const void* zp,
+                                               int64_t outer, int64_t channels, int64_t inner, int q_dt, int out_dt,
+                                               int scale_dt, int zp_int64, void* stream) {
+  return dequantize("dequantize_channels", q, out, QdqParams{scale, zp, scale_dt, zp_int64 != 0, 0}, outer, channels,
+                    inner, q_dt, out_dt, 1, stream);
 }

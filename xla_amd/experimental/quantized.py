@@ -117,20 +117,30 @@ def _quantize(input, inv_scale, zero_point, quant_min, quant_max, dtype, axis):
   return q
 
 
-def _dequantize(input, scale, zero_point, dtype, out_dtype, axis, int_subtract):
+def _dequantize(input, scale, zero_point, dtype, out_dtype):
   lib = _lib.load()
   assert input.dtype == dtype, f"Expecting input to have dtype: {dtype}, but got {input.dtype}"
   out_dtype = out_dtype or torch.float32
   q = input.contiguous()
-  outer, channels, inner = _geometry(q, axis, scale.numel())
   out = torch.empty(q.shape, dtype=out_dtype, device=q.device)
-  sc = scale.to(device=q.device, dtype=torch.float32).contiguous()
-  zp = None if zero_point is None else zero_point.to(device=q.device, dtype=torch.int32).contiguous()
   _lib.check(
-      lib.xla_amd_qmm_dequantize_affine(q.data_ptr(), out.data_ptr(), sc.data_ptr(), _lib.ptr(zp), outer, channels,
-                                        inner, _QDT[dtype], _lib.dt(out_dtype), int_subtract, _lib.stream_of(q)),
+      lib.xla_amd_qmm_dequantize_affine(q.data_ptr(), out.data_ptr(), scale.data_ptr(), zero_point.data_ptr(), 1, 1,
+                                        q.numel(), _QDT[dtype], _lib.dt(out_dtype), 0, _lib.stream_of(q)),
       "dequantize_affine")
   return out
+
+
+def _kernel_params(scale, zero_point, device):
+  """The parameters of a per-channel call as the kernels read them (contiguous, on the device, scale f32 / bf16 / f16,
+  zero point int64 / int32): the tensors themselves, or converted copies of any others."""
+  if scale.dtype not in _lib._DT:
+    scale = scale.to(torch.float32)
+  scale = scale.to(device).contiguous()
+  if zero_point is not None:
+    if zero_point.dtype not in (torch.int64, torch.int32):
+      zero_point = zero_point.to(torch.int32)
+    zero_point = zero_point.to(device).contiguous()
+  return scale, zero_point, zero_point is not None and zero_point.dtype == torch.int64
 
 
 # per-tensor parameters are host scalars: their one-element device tensors are kept, so that a call
@@ -172,8 +182,18 @@ def rocm_quantize_per_channel(input: torch.Tensor, scales: torch.Tensor, zero_po
   assert axis < input.dim(), f"Expecting axis to be < {input.dim()}"
   _check_scale_zp(input, scales, zero_points, axis, dtype)
   scales, zero_points = _per_channel_params(input, axis, scales, zero_points)
-  inv = 1.0 / scales.to(torch.float32) if scales.dtype != torch.float64 else (1.0 / scales).to(torch.float32)
-  return _quantize(input, inv, zero_points, quant_min, quant_max, dtype, axis)
+  if scales.dtype == torch.float64:  # the reciprocal in double, as torch computes it
+    return _quantize(input, (1.0 / scales).to(torch.float32), zero_points, quant_min, quant_max, dtype, axis)
+  lib = _lib.load()
+  x = input.contiguous()
+  outer, channels, inner = _geometry(x, axis, scales.numel())
+  q = torch.empty(x.shape, dtype=dtype, device=x.device)
+  sc, zp, zp64 = _kernel_params(scales, zero_points, x.device)
+  _lib.check(
+      lib.xla_amd_qmm_quantize_channels(x.data_ptr(), q.data_ptr(), sc.data_ptr(), zp.data_ptr(), outer, channels, inner,
+                                        _lib.dt(x.dtype), _QDT[dtype], _lib.dt(sc.dtype), zp64, quant_min, quant_max,
+                                        _lib.stream_of(x)), "quantize_channels")
+  return q
 
 
 @impl(quantized_decomposed_lib, "dequantize_per_tensor", "CUDA")
@@ -181,7 +201,7 @@ def rocm_dequantize_per_tensor(input: torch.Tensor, scale: float, zero_point: in
                                dtype: torch.dtype, *, out_dtype=None):
   _check_scalar(scale, zero_point, dtype)
   sc, zp = _scalar_params(input.device, scale, zero_point)
-  return _dequantize(input, sc, zp, dtype, out_dtype, -1, 0)
+  return _dequantize(input, sc, zp, dtype, out_dtype)
 
 
 @impl(quantized_decomposed_lib, "dequantize_per_channel", "CUDA")
@@ -191,4 +211,15 @@ def rocm_dequantize_per_channel(input: torch.Tensor, scales: torch.Tensor, zero_
   zp_check = zero_points if zero_points is not None else torch.zeros_like(scales, dtype=torch.int64)
   _check_scale_zp(input, scales, zp_check, axis, dtype)
   scales, zero_points = _per_channel_params(input, axis, scales, zero_points)
-  return _dequantize(input, scales, zero_points, dtype, out_dtype, axis, 1)
+  assert input.dtype == dtype, f"Expecting input to have dtype: {dtype}, but got {input.dtype}"
+  lib = _lib.load()
+  out_dtype = out_dtype or torch.float32
+  q = input.contiguous()
+  outer, channels, inner = _geometry(q, axis, scales.numel())
+  out = torch.empty(q.shape, dtype=out_dtype, device=q.device)
+  sc, zp, zp64 = _kernel_params(scales, zero_points, q.device)
+  _lib.check(
+      lib.xla_amd_qmm_dequantize_channels(q.data_ptr(), out.data_ptr(), sc.data_ptr(), _lib.ptr(zp), outer, channels,
+                                          inner, _QDT[dtype], _lib.dt(out_dtype), _lib.dt(sc.dtype), zp64,
+                                          _lib.stream_of(q)), "dequantize_channels")
+  return out
