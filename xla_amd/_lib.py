@@ -54,6 +54,9 @@ SIGNATURES = {
     "xla_amd_qmm_dequantize_channels": (_c_int, [_c_vp] * 4 + [_c_i64] * 3 + [_c_int] * 4 + [_c_vp]),
 }
 
+# The operators' native implementation (csrc/torch_binding.cpp): linked against the library above and against torch.
+_TORCH_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libxla_amd_torch.so")
+
 _lib = None
 _lock = threading.Lock()
 
@@ -84,6 +87,18 @@ def load():
       raise RuntimeError(f"libxla_amd_qmm.so has ABI version {got}, expected {ABI_VERSION}")
     _lib = lib
   return _lib
+
+
+def load_torch_binding():
+  """Registers the native operator implementations and returns a function (counter index) -> calls, or None when the
+  libraries are not built."""
+  if not (os.path.exists(_LIB_PATH) and os.path.exists(_TORCH_LIB_PATH)):
+    return None
+  load()
+  torch.ops.load_library(_TORCH_LIB_PATH)
+  counter = ctypes.CDLL(_TORCH_LIB_PATH).xla_amd_torch_counter
+  counter.restype, counter.argtypes = _c_i64, [_c_int]
+  return counter
 
 
 def dt(dtype: torch.dtype) -> int:

@@ -1,7 +1,8 @@
-"""Builds libxla_amd_qmm.so (gfx950) in-tree with hipcc.
+"""Builds libxla_amd_qmm.so (gfx950) and libxla_amd_torch.so in-tree with hipcc and the host compiler.
 
 `python -m xla_amd.build` compiles every .hip file of xla_amd/csrc and links
-them into xla_amd/libxla_amd_qmm.so.  hipcc cross-compiles, so no GPU is
+them into xla_amd/libxla_amd_qmm.so; the operators' implementation on torch
+tensors (csrc/torch_binding.cpp) becomes xla_amd/libxla_amd_torch.so.  hipcc cross-compiles, so no GPU is
 needed to build.
 """
 import concurrent.futures
@@ -16,6 +17,8 @@ REPO_DIR = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 OBJ_DIR = os.path.join(PKG_DIR, "csrc", "build")
 LIB_PATH = os.path.join(PKG_DIR, "libxla_amd_qmm.so")
+# the operators' implementation on torch tensors (host code only), linked against the library above
+TORCH_LIB_PATH = os.path.join(PKG_DIR, "libxla_amd_torch.so")
 
 # (source, extra flags, object name); the skinny kernels are built once per
 # activation dtype and the weight-only GEMM once per (dtype, row tile) so that
@@ -130,6 +133,19 @@ def _code_bytes(obj: str):
   return sizes
 
 
+def _build_torch_binding():
+  import torch
+  from torch.utils import cpp_extension
+  lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+  tmp = TORCH_LIB_PATH + ".tmp"
+  _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", os.path.join(REPO_DIR, "include")] +
+       [a for d in cpp_extension.include_paths() + ["/opt/rocm/include"] for a in ("-isystem", d)] +
+       [os.path.join(CSRC, "torch_binding.cpp"), "-o", tmp, "-L", lib, "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+        "-L", PKG_DIR, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN"])
+  os.replace(tmp, TORCH_LIB_PATH)
+
+
 def build(verbose: bool = False, jobs: int = 8) -> str:
   os.makedirs(OBJ_DIR, exist_ok=True)
   objs = []
@@ -182,6 +198,7 @@ def build(verbose: bool = False, jobs: int = 8) -> str:
   _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", "-o", tmp] +
        [timeline_obj if os.path.basename(o) == TIMELINE_REPLACES else o for o in objs] + [diag_obj])
   os.replace(tmp, TIMELINE_LIB_PATH)
+  _build_torch_binding()
   return LIB_PATH
 
 

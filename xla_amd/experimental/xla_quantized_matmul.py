@@ -8,6 +8,7 @@ formulation with the rounding points of the reference's (:139-183), which the
 reference documents as its debugging path; meta tensors only get shapes and
 dtypes.
 """
+import collections.abc
 import os
 import weakref
 
@@ -34,8 +35,36 @@ def _overflow_policy() -> str:
   return p
 
 
+class _Counters(collections.abc.MutableMapping):
+  """Calls counted here plus those the native operators counted."""
+
+  _NAMES = ("skinny_mfma", "wo_gemm", "generic", "w8a8_mfma", "w8a8_generic", "pack", "pack_hit")  # the native order
+
+  def __init__(self):
+    self._here = dict.fromkeys(self._NAMES, 0)
+    self.native = None  # counter index -> calls
+
+  def _there(self, name):
+    return 0 if self.native is None else self.native(self._NAMES.index(name))
+
+  def __getitem__(self, name):
+    return self._here[name] + self._there(name)
+
+  def __setitem__(self, name, value):
+    self._here[name] = value - self._there(name)
+
+  def __delitem__(self, name):
+    raise TypeError("the counters are fixed")
+
+  def __iter__(self):
+    return iter(self._NAMES)
+
+  def __len__(self):
+    return len(self._NAMES)
+
+
 # Dispatch decisions, for tests and profiling (kernel id -> calls).
-counters = {"skinny_mfma": 0, "wo_gemm": 0, "generic": 0, "w8a8_mfma": 0, "w8a8_generic": 0, "pack": 0, "pack_hit": 0}
+counters = _Counters()
 
 
 def _check_per_channel_quant_weight_dtype_shapes(input_dim, output_dim, w, w_scaler, zero_point):
@@ -97,8 +126,14 @@ def _result_dtype(x, scaler, quantize_activation):
 # explicitly (`prepare_weight`, `XlaQuantizedLinear.prepare`) or on the first call
 # that needs it, and kept in `_pack_cache` while the tensor object is alive.
 #
-# key (id(w), kind) -> (version, data_ptr, bits, copy)
+# key (id(w), kind) -> (version, data_ptr, bits, copy, key of the native operators' own record of it or None)
 _pack_cache = {}
+
+
+def _drop_copy(key):
+  entry = _pack_cache.pop(key, None)
+  if entry is not None and entry[4] is not None:
+    torch.ops.xla_amd.forget_tiled(entry[4])
 
 
 def _version_of(w: torch.Tensor) -> int:
@@ -116,11 +151,8 @@ def invalidate_weight_cache(w: torch.Tensor = None):
   call: `w.data.copy_(...)` / `w.data[...] = ...`, anything written into an
   inference-mode tensor, and writes from outside torch to the same memory.
   """
-  if w is None:
-    _pack_cache.clear()
-    return
-  for kind in ("tiled", "packed"):
-    _pack_cache.pop((id(w), kind), None)
+  for key in list(_pack_cache) if w is None else [(id(w), "tiled"), (id(w), "packed")]:
+    _drop_copy(key)
 
 
 def _relayout(w: torch.Tensor, bits: int, layout: int, kind: str) -> torch.Tensor:
@@ -155,8 +187,10 @@ def _relayout(w: torch.Tensor, bits: int, layout: int, kind: str) -> torch.Tenso
   _lib.check(copy_fn(src.data_ptr(), out.data_ptr(), s, c, n, layout, bits, _lib.stream_of(w)), f"{kind} weight")
   counters["pack"] += 1
   if hit is None:
-    weakref.finalize(w, _pack_cache.pop, key, None)
-  _pack_cache[key] = (_version_of(w), w.data_ptr(), bits, out)
+    weakref.finalize(w, _drop_copy, key).atexit = False
+  # (a weight whose record is replaced is the same tensor: the native record is replaced with it)
+  native = torch.ops.xla_amd.remember_tiled(w, bits, out) if kind == "tiled" else None
+  _pack_cache[key] = (_version_of(w), w.data_ptr(), bits, out, native)
   return out
 
 
@@ -365,7 +399,22 @@ def w8a8_linear_gpu(x2, w, w_scale, zero_point, *, x_scale_dtype, cvt_dtype, mid
   return out
 
 
-@impl(XLA_LIB, "quantized_matmul", "CUDA")
+# Not part of the reference's interface: an operator for the tiled form of a weight alone, which a module calls, and
+# what the native implementations of it and of xla::quantized_matmul (csrc/torch_binding.cpp) call in their turn for
+# anything but an ordinary call.
+XLA_AMD_LIB = torch.library.Library("xla_amd", "DEF")
+XLA_AMD_LIB.define(
+    "weight_only_tiled(Tensor x, Tensor w_tiled, Tensor scale, Tensor? zero_point, int out_features, "
+    "int block_size, bool int4_weight) -> Tensor")
+XLA_AMD_LIB.define(
+    "weight_only_tiled_general(Tensor x, Tensor w_tiled, Tensor scale, Tensor? zero_point, int out_features, "
+    "int block_size, bool int4_weight) -> Tensor")
+XLA_AMD_LIB.define(
+    "quantized_matmul_general(Tensor x, Tensor w, Tensor scale, Tensor? zero_point, int block_size, "
+    "bool int4_weight, bool quantize_activation) -> Tensor")
+
+
+@impl(XLA_AMD_LIB, "quantized_matmul_general", "CUDA")
 def quantized_matmul_rocm(x: torch.Tensor,
                           w: torch.Tensor,
                           scaler: torch.Tensor,
@@ -475,15 +524,9 @@ def quantized_matmul_meta(x, w, scaler, zero_point=None, block_size=-1, int4_wei
 
 
 # ---- weight-only matmul on a tiled weight alone ----------------------------------------
-# Not part of the reference's interface: the operator a module calls once it keeps only the
-# tiled form of its weight on the device (XlaQuantizedLinear.prepare(release_weight=True)).
-XLA_AMD_LIB = torch.library.Library("xla_amd", "DEF")
-XLA_AMD_LIB.define(
-    "weight_only_tiled(Tensor x, Tensor w_tiled, Tensor scale, Tensor? zero_point, int out_features, "
-    "int block_size, bool int4_weight) -> Tensor")
-
-
-@impl(XLA_AMD_LIB, "weight_only_tiled", "CUDA")
+# What a module calls once it has the tiled form of its weight on the device (and, after
+# XlaQuantizedLinear.prepare(release_weight=True), nothing else).
+@impl(XLA_AMD_LIB, "weight_only_tiled_general", "CUDA")
 def weight_only_tiled_rocm(x, w_tiled, scaler, zero_point, out_features, block_size, int4_weight):
   if not (x.is_floating_point() and scaler.is_floating_point()):
     raise RuntimeError(f"xla_amd weight_only_tiled: x and scaler must be floating point, got {x.dtype}, {scaler.dtype}")
@@ -504,6 +547,21 @@ def weight_only_tiled_rocm(x, w_tiled, scaler, zero_point, out_features, block_s
 @impl(XLA_AMD_LIB, "weight_only_tiled", "Meta")
 def weight_only_tiled_meta(x, w_tiled, scaler, zero_point, out_features, block_size, int4_weight):
   return torch.empty(*x.shape[:-1], out_features, dtype=_result_dtype(x, scaler, False), device=x.device)
+
+
+counters.native = _lib.load_torch_binding()
+if counters.native is None:
+
+  def _not_built(*args, **kwargs):
+    _lib.load()
+    raise RuntimeError("xla_amd: libxla_amd_torch.so is not built; run `python -m xla_amd.build`. "
+                       "There is no fallback implementation for GPU tensors.")
+
+  XLA_LIB.impl("quantized_matmul", _not_built, "CUDA")
+  XLA_AMD_LIB.impl("weight_only_tiled", _not_built, "CUDA")
+
+_quantized_matmul_op = torch.ops.xla.quantized_matmul.default
+_weight_only_tiled_op = torch.ops.xla_amd.weight_only_tiled.default
 
 
 class XlaQuantizedLinear(torch.nn.Module):
@@ -649,13 +707,7 @@ class XlaQuantizedLinear(torch.nn.Module):
 
   def forward(self, x):
     if x.is_cuda and self._tiled_is_current():
-      return torch.ops.xla_amd.weight_only_tiled(x, self._weight_tiled, self.weight_scaler, self.zero_point,
-                                                 self.output_dim, self.block_size, self.int4_weight)
-    return torch.ops.xla.quantized_matmul(
-        x,
-        self.weight,
-        self.weight_scaler,
-        self.zero_point,
-        block_size=self.block_size,
-        int4_weight=self.int4_weight,
-        quantize_activation=self.quantize_activation)
+      return _weight_only_tiled_op(x, self._weight_tiled, self.weight_scaler, self.zero_point, self.output_dim,
+                                   self.block_size, self.int4_weight)
+    return _quantized_matmul_op(x, self.weight, self.weight_scaler, self.zero_point, self.block_size, self.int4_weight,
+                                self.quantize_activation)
