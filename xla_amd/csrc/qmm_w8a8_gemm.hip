@@ -521,7 +521,7 @@ int launch_tile(const GemmArgs& g, hipStream_t stream) {
 // that is only partly full costs a whole one.
 struct TileCost { double per_round_us, per_k4096_us; };
 static constexpr double kLaunchUs = 4.0;
-static constexpr TileCost kCost256 = {11.0, 52.0}, kCost192 = {8.0, 39.0}, kCost128x256 = {9.0, 27.0},
+static constexpr TileCost kCost256 = {11.0, 52.0}, kCost192 = {8.0, 39.0}, kCost128x256 = {10.0, 22.5},
                           kCost128 = {8.0, 14.0};
 static double rounds_us(const TileCost& c, int64_t tiles, int64_t K) {
   return (double)((tiles + 255) / 256) * (c.per_round_us + c.per_k4096_us * (double)K / 4096.0);
@@ -639,7 +639,9 @@ extern "C" int xla_amd_qmm_w8a8_gemm(const int8_t* x_q, const int8_t* w, const v
     }
     return rc;
   }
-  if (bm == 128 && bn == 256) return launch_tile<128, 256, 2, 4>(g, s);  // 8 waves, wave tile 64 x 64
+  // 8 waves, wave tile 64 x 64, one workgroup per CU with two stages or three: the third keeps two steps' copies in
+  // flight (512 x 14336 x 4096: 45 -> 37 us, two rounds of them, 1024 x 14336 x 4096: 83 -> 70)
+  if (bm == 128 && bn == 256) return launch_tile<128, 256, 2, 4, 3>(g, s);
   if (bm == 128 && bn == 128) {
     // one workgroup per CU at most: LDS is free for a third stage (two fit a CU with two stages)
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
@@ -653,6 +655,10 @@ extern "C" int xla_amd_qmm_w8a8_gemm(const int8_t* x_q, const int8_t* w, const v
     // At most one workgroup per CU and a long K: two K groups halve the K loop.
     const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
     if (tiles <= 256 && K >= 1024) return launch_tile<64, 64, 2, 2, 3, 2>(g, s);
+    // Twice the columns per workgroup while that is at most one per CU: a quarter less to copy and the two K groups as
+    // well (512 x 4096 x 14336: 60 -> 49 us; 256 x 8192 x 8192 40 -> 31, 128 x 14336 x 4096 24 -> 20, 512 x 4096 x 4096 17.3 -> 17.0).
+    // (Up to 32 rows the tile is mostly empty: 16 x 28672 x 4096 28 us as it is, 30 so.)
+    if (M > 32 && ((M + 63) / 64) * ((N + 127) / 128) <= 256 && K >= 4096) return launch_tile<64, 128, 2, 2, 3, 2>(g, s);
     return tiles <= 512 ? launch_tile<64, 64, 2, 2, 3>(g, s) : launch_tile<64, 64, 2, 2, 2>(g, s);
   }
   if (bm == 64 && bn == 32) {  // two waves per K group
