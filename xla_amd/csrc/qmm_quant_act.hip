@@ -15,8 +15,6 @@
 
 namespace {
 
-constexpr int kThreads = 256;
-
 // max that keeps a NaN (fmaxf would drop it): a row that holds a NaN gets a NaN scale, as torch.amax gives
 __device__ __forceinline__ float nan_max(float a, float b) { return (a > b || a != a) ? a : b; }
 __device__ __forceinline__ float wave_max(float v) {
@@ -72,7 +70,7 @@ __device__ __forceinline__ int quantize_one(float xv, const RowDivisor& d, int x
 // VEC = elements per thread per step: 8 (16-byte loads of 2-byte types, two
 // for f32) when K % 8 == 0 and the row starts are 16-byte aligned, else 1.
 // KEEP: vector steps of the row a thread keeps in registers (0 = read twice).
-template <int XT, int VEC, int KEEP>
+template <int XT, int VEC, int KEEP, int kThreads>
 __global__ void __launch_bounds__(kThreads)
 qmm_quantize_kernel(const void* __restrict__ x, int8_t* __restrict__ xq, void* __restrict__ x_scale,
                     int32_t* __restrict__ x_sum, int64_t K, int scale_out_dt, int policy) {
@@ -190,20 +188,25 @@ qmm_quantize_kernel(const void* __restrict__ x, int8_t* __restrict__ xq, void* _
   }
 }
 
+// Threads per row: the launch lasts as long as one row's chain (load, abs-max, quantize) when there are few rows, and
+// rows of many elements per thread make that chain long, so long rows get more threads.  Per launch in a graph, bf16,
+// with 256 / 512 / 1024 threads: 1 x 14336 7.0 / 4.8 / 3.9 us, 512 x 14336 10.2 / 8.1 / 8.1, 4096 x 14336 45 / 39 / 43,
+// 512 x 8192 6.5 / 5.7 / 8.2, 4096 x 8192 24.7 / 23.3 / 47, 512 x 4096 4.1 / 4.9 / 5.6; f32, whose rows take twice the
+// loads: 512 x 4096 4.9 / 4.5 / 4.9, 512 x 2048 3.4 / 3.4 / 4.1.
 template <int XT>
 int launch(const void* x, int8_t* xq, void* x_scale, int32_t* x_sum, int64_t M, int64_t K,
            int scale_out_dt, int policy, bool vec, hipStream_t stream) {
-  const dim3 grid((unsigned)M), block(kThreads);
-  if (!vec)
-    hipLaunchKernelGGL((qmm_quantize_kernel<XT, 1, 0>), grid, block, 0, stream, x, xq, x_scale, x_sum, K, scale_out_dt, policy);
-  else if (K <= 2 * kThreads * 8)
-    hipLaunchKernelGGL((qmm_quantize_kernel<XT, 8, 2>), grid, block, 0, stream, x, xq, x_scale, x_sum, K, scale_out_dt, policy);
-  else if (K <= 4 * kThreads * 8)
-    hipLaunchKernelGGL((qmm_quantize_kernel<XT, 8, 4>), grid, block, 0, stream, x, xq, x_scale, x_sum, K, scale_out_dt, policy);
-  else if (K <= 8 * kThreads * 8)
-    hipLaunchKernelGGL((qmm_quantize_kernel<XT, 8, 8>), grid, block, 0, stream, x, xq, x_scale, x_sum, K, scale_out_dt, policy);
-  else
-    hipLaunchKernelGGL((qmm_quantize_kernel<XT, 8, 0>), grid, block, 0, stream, x, xq, x_scale, x_sum, K, scale_out_dt, policy);
+  auto go = [&](auto kern, int threads) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)M), dim3(threads), 0, stream, x, xq, x_scale, x_sum, K, scale_out_dt, policy);
+  };
+  constexpr int kShort = XT == XLA_AMD_DT_F32 ? 2048 : 4096;
+  if (!vec) go(qmm_quantize_kernel<XT, 1, 0, 256>, 256);
+  else if (K <= kShort) go(qmm_quantize_kernel<XT, 8, kShort / 2048, 256>, 256);
+  else if (K <= 4096) go(qmm_quantize_kernel<XT, 8, 1, 512>, 512);
+  else if (K <= 8192) go(qmm_quantize_kernel<XT, 8, 2, 512>, 512);
+  else if (K <= 16384 && M <= 256) go(qmm_quantize_kernel<XT, 8, 2, 1024>, 1024);
+  else if (K <= 16384) go(qmm_quantize_kernel<XT, 8, 4, 512>, 512);
+  else go(qmm_quantize_kernel<XT, 8, 0, 256>, 256);
   return QMM_CHECK_LAUNCH("quantize_per_token launch");
 }
 
