@@ -521,7 +521,7 @@ int launch_tile(const GemmArgs& g, hipStream_t stream) {
 // that is only partly full costs a whole one.
 struct TileCost { double per_round_us, per_k4096_us; };
 static constexpr double kLaunchUs = 4.0;
-static constexpr TileCost kCost256 = {11.0, 52.0}, kCost192 = {8.0, 39.0}, kCost128x256 = {10.0, 22.5},
+static constexpr TileCost kCost256 = {11.0, 52.0}, kCost192 = {8.0, 39.0}, kCost128x256 = {9.0, 27.0},
                           kCost128 = {8.0, 14.0};
 static double rounds_us(const TileCost& c, int64_t tiles, int64_t K) {
   return (double)((tiles + 255) / 256) * (c.per_round_us + c.per_k4096_us * (double)K / 4096.0);
