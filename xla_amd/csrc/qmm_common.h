@@ -21,6 +21,9 @@ int qmm_check_hip(hipError_t e, const char* what);
 // (one mask per kernel instantiation, shared by all host threads) holds one bit per device
 // ordinal; ordinals from 64 on set the attribute on every launch.
 int qmm_set_max_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done, const char* what);
+// A kernel as a type, for launchers that are handed one of several kernels of the same signature: a static in the
+// launcher then belongs to one kernel (with the kernel as a function pointer all of them would share it).
+template <auto Kernel> struct qmm_kernel { static constexpr auto fn = Kernel; };
 
 static inline bool qmm_valid_dt(int dt) { return dt >= XLA_AMD_DT_F32 && dt <= XLA_AMD_DT_F16; }
 static inline int qmm_dt_size(int dt) { return dt == XLA_AMD_DT_F32 ? 4 : 2; }

@@ -213,14 +213,15 @@ int launch(const SkinnyArgs& a, bool haszp, int workgroups, hipStream_t stream) 
   const int per_wg = ((groups + workgroups - 1) / workgroups + kWaves) * a.G;
   const int scl_bytes = (per_wg * 2 + 255) & ~255;
   const int lds = steps * kXTile + scl_bytes * (haszp ? 2 : 1);
-  auto go = [&](auto kern) -> int {
+  auto go = [&](auto which) -> int {
+    constexpr auto kern = decltype(which)::fn;
     static std::atomic<uint64_t> lds_set{0};
     const int rc = qmm_set_max_lds((const void*)kern, 160 * 1024, lds_set, "weight_only_skinny (resident) hipFuncSetAttribute");
     if (rc != XLA_AMD_QMM_OK) return rc;
     hipLaunchKernelGGL(kern, dim3((unsigned)workgroups), dim3((kWaves + kCopiers) * 64), lds, stream, a);
     return QMM_CHECK_LAUNCH("weight_only_skinny (resident) launch");
   };
-  return haszp ? go(qmm_skinny_resident_kernel<XT, true>) : go(qmm_skinny_resident_kernel<XT, false>);
+  return haszp ? go(qmm_kernel<qmm_skinny_resident_kernel<XT, true>>{}) : go(qmm_kernel<qmm_skinny_resident_kernel<XT, false>>{});
 }
 
 }  // namespace

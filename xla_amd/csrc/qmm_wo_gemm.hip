@@ -641,7 +641,8 @@ int launch(const WoGemmArgs& a, hipStream_t stream) {
   const int cus = cu_count();
   const int64_t rounds = (items + cus - 1) / cus;
   const dim3 grid((unsigned)((items + rounds - 1) / rounds)), block((kComputeWaves + kCopyWaves) * 64);
-  auto go = [&](auto kern) -> int {
+  auto go = [&](auto which) -> int {
+    constexpr auto kern = decltype(which)::fn;
     static std::atomic<uint64_t> lds_set{0};
     const int rc = qmm_set_max_lds((const void*)kern, Cfg::lds_bytes(1 << 20), lds_set, "weight_only_gemm hipFuncSetAttribute");
     if (rc != XLA_AMD_QMM_OK) return rc;
@@ -656,10 +657,10 @@ int launch(const WoGemmArgs& a, hipStream_t stream) {
     // time: the plan never asks for the first, and the second takes the 128 x 128 tile)
     if (a.zp) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_gemm: no 128 x 256 tile with a zero point");
     if (!uni) return launch<XT, MT, 2>(a, stream);
-    return go(qmm_wo_gemm_kernel<XT, MT, NG, false, true>);
+    return go(qmm_kernel<qmm_wo_gemm_kernel<XT, MT, NG, false, true>>{});
   } else {
-    if (uni) return a.zp ? go(qmm_wo_gemm_kernel<XT, MT, NG, true, true>) : go(qmm_wo_gemm_kernel<XT, MT, NG, false, true>);
-    return a.zp ? go(qmm_wo_gemm_kernel<XT, MT, NG, true, false>) : go(qmm_wo_gemm_kernel<XT, MT, NG, false, false>);
+    if (uni) return a.zp ? go(qmm_kernel<qmm_wo_gemm_kernel<XT, MT, NG, true, true>>{}) : go(qmm_kernel<qmm_wo_gemm_kernel<XT, MT, NG, false, true>>{});
+    return a.zp ? go(qmm_kernel<qmm_wo_gemm_kernel<XT, MT, NG, true, false>>{}) : go(qmm_kernel<qmm_wo_gemm_kernel<XT, MT, NG, false, false>>{});
   }
 }
 

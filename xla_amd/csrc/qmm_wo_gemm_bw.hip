@@ -524,7 +524,8 @@ int launch(const WoBwArgs& a, hipStream_t stream) {
     else return qmm_wo_bw_wide_launch_f16(a, BITS, cus, stream);
   }
   const dim3 grid((unsigned)(items < cus ? items : cus)), block((kComputeWaves + kCopyWaves) * 64);
-  auto go = [&](auto kern) -> int {
+  auto go = [&](auto which) -> int {
+    constexpr auto kern = decltype(which)::fn;
     static std::atomic<uint64_t> lds_set{0};
     const int rc = qmm_set_max_lds((const void*)kern, kLdsBytes, lds_set, "weight_only_gemm hipFuncSetAttribute");
     if (rc != XLA_AMD_QMM_OK) return rc;
@@ -534,10 +535,10 @@ int launch(const WoBwArgs& a, hipStream_t stream) {
   // blocks of 128 columns: the kernel with two sets of block sums (int8 weights with a zero point keep the other
   // one: their two 16-byte weight loads per row set leave no registers for the second set)
   if (a.C == 128) {
-    if (!a.zp) return go(qmm_wo_bw_gemm_kernel<XT, BITS, false, true>);
-    if constexpr (BITS == 4) return go(qmm_wo_bw_gemm_kernel<XT, BITS, true, true>);
+    if (!a.zp) return go(qmm_kernel<qmm_wo_bw_gemm_kernel<XT, BITS, false, true>>{});
+    if constexpr (BITS == 4) return go(qmm_kernel<qmm_wo_bw_gemm_kernel<XT, BITS, true, true>>{});
   }
-  return a.zp ? go(qmm_wo_bw_gemm_kernel<XT, BITS, true, false>) : go(qmm_wo_bw_gemm_kernel<XT, BITS, false, false>);
+  return a.zp ? go(qmm_kernel<qmm_wo_bw_gemm_kernel<XT, BITS, true, false>>{}) : go(qmm_kernel<qmm_wo_bw_gemm_kernel<XT, BITS, false, false>>{});
 }
 
 }  // namespace

@@ -433,15 +433,16 @@ template <int XT, int BITS>
 int launch(const WoBwArgs& a, int cus, hipStream_t stream) {
   const int64_t items = (int64_t)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
   const dim3 grid((unsigned)(items < cus ? items : cus)), block((kComputeWaves + kCopyWaves) * 64);
-  auto go = [&](auto kern) -> int {
+  auto go = [&](auto which) -> int {
+    constexpr auto kern = decltype(which)::fn;
     static std::atomic<uint64_t> lds_set{0};
     const int rc = qmm_set_max_lds((const void*)kern, kLdsBytes, lds_set, "weight_only_gemm hipFuncSetAttribute");
     if (rc != XLA_AMD_QMM_OK) return rc;
     hipLaunchKernelGGL(kern, grid, block, kLdsBytes, stream, a);
     return QMM_CHECK_LAUNCH("weight_only_gemm (blockwise, wide tile) launch");
   };
-  if (!a.zp) return a.C == 128 ? go(qmm_wo_bw_wide_kernel<XT, BITS, false, true>) : go(qmm_wo_bw_wide_kernel<XT, BITS, false, false>);
-  if constexpr (BITS == 4) return go(qmm_wo_bw_wide_kernel<XT, BITS, true, true>);
+  if (!a.zp) return a.C == 128 ? go(qmm_kernel<qmm_wo_bw_wide_kernel<XT, BITS, false, true>>{}) : go(qmm_kernel<qmm_wo_bw_wide_kernel<XT, BITS, false, false>>{});
+  if constexpr (BITS == 4) return go(qmm_kernel<qmm_wo_bw_wide_kernel<XT, BITS, true, true>>{});
   return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_gemm (blockwise, wide tile): no such kernel");
 }
 
