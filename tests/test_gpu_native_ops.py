@@ -143,3 +143,77 @@ def test_threads_and_streams(ops):
   for t in threads:
     t.join()
   assert not wrong
+
+
+def _busy(stream, ms=60):
+  with torch.cuda.stream(stream):
+    torch.cuda._sleep(int(ms * 2.4e6))  # (cycles)
+
+
+@pytest.mark.parametrize("call", [native, general])
+def test_copy_made_on_another_stream(ops, call):
+  """A weight's first call on one stream, its second on another: the second waits for the copy the first is making."""
+  x, w, s, _ = cases.per_channel_int8(33, 512, 1024, torch.bfloat16, torch.bfloat16)
+  x, s, w = x.cuda(), s.cuda(), w.cuda()
+  want = call(x, w.clone(), s, None, -1, False, False)
+  first, second = torch.cuda.Stream(), torch.cuda.Stream()
+  torch.cuda.synchronize()
+  _busy(first)
+  with torch.cuda.stream(first):
+    a = call(x, w, s, None, -1, False, False)
+  with torch.cuda.stream(second):
+    b = call(x, w, s, None, -1, False, False)
+  assert not first.query()  # (both calls were made while the copy was still to come)
+  second.synchronize()
+  assert torch.equal(b, want)
+  torch.cuda.synchronize()
+  assert torch.equal(a, want)
+
+
+@pytest.mark.parametrize("call", [native, general])
+def test_copy_replaced_under_another_stream(ops, call):
+  """A copy that is replaced (an in-place write to its weight) while another stream still has to read it keeps its
+  memory until then."""
+  x, w, s, _ = cases.per_channel_int8(33, 512, 1024, torch.bfloat16, torch.bfloat16)
+  x, s, w = x.cuda(), s.cuda(), w.cuda()
+  want = call(x, w, s, None, -1, False, False)
+  size = ops._pack_cache[(id(w), "tiled")][3].numel()
+  other = torch.cuda.Stream()
+  with torch.cuda.stream(other):
+    call(x, w, s, None, -1, False, False)
+  # (memory the calls below take without going to the driver, which may wait for the whole device)
+  del [torch.empty(size, dtype=torch.uint8, device="cuda") for _ in range(16)][:]
+  torch.cuda.synchronize()
+  _busy(other)
+  with torch.cuda.stream(other):
+    a = call(x, w, s, None, -1, False, False)
+  w.neg_()
+  call(x, w, s, None, -1, False, False)  # makes the new copy, lets go of the old one
+  taken = [torch.full((size,), 99, dtype=torch.uint8, device="cuda") for _ in range(8)]
+  assert not other.query()  # (all of this was launched before the read; where the streams share a hardware queue it also runs in that order)
+  torch.cuda.synchronize()
+  assert torch.equal(a, want)
+  del taken
+
+
+@pytest.mark.parametrize("call", [native, general])
+def test_copy_still_being_made_at_a_capture(ops, call):
+  """A capture on another stream than the one that is making the copy: the graph finds it complete."""
+  x, w, s, _ = cases.per_channel_int8(33, 512, 1024, torch.bfloat16, torch.bfloat16)
+  x, s, w = x.cuda(), s.cuda(), w.cuda()
+  want = call(x, w.clone(), s, None, -1, False, False)
+  first, second = torch.cuda.Stream(), torch.cuda.Stream()
+  torch.cuda.synchronize()
+  _busy(first)
+  with torch.cuda.stream(first):
+    call(x, w, s, None, -1, False, False)
+  g = torch.cuda.CUDAGraph()
+  with torch.cuda.stream(second):
+    g.capture_begin()
+    out = call(x, w, s, None, -1, False, False)
+    g.capture_end()
+    for _ in range(3):
+      out.zero_()
+      g.replay()
+      second.synchronize()
+      assert torch.equal(out, want)

@@ -11,14 +11,18 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <optional>
 #include <unordered_map>
+#include <vector>
 
 #include "xla_amd_qmm.h"
 
@@ -53,12 +57,18 @@ void check(int rc, const char* what) {
 // A mirror of the Python module's cache, which makes the copies and says when they are to be dropped.  An entry holds
 // its weight weakly: the address of its TensorImpl cannot be taken by another tensor while the entry exists.  It
 // stands as long as the weight is unmodified (version counter, storage address).
+// The copy is made by a kernel on the stream of whichever call came first and read on the stream of any later one, so
+// an entry keeps that stream and an event behind the kernel.
 struct Copy {
   c10::weak_intrusive_ptr<c10::TensorImpl> weight;
   int64_t version;
   const void* data;
   int64_t bits;
   Tensor tiled;
+  c10::Stream made_on;
+  c10::Event made;                   // recorded behind the kernel that makes the copy
+  bool complete;                     // that kernel has been seen to be done
+  std::vector<c10::Stream> used_on;  // other streams the allocator knows to read the copy
 };
 struct Cache {
   std::mutex mu;
@@ -68,31 +78,72 @@ Cache& cache() {
   static Cache* c = new Cache;  // (never destroyed: its tensors would outlive the allocator)
   return *c;
 }
+c10::Stream current_stream(const Tensor& t) {
+  return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).unwrap();
+}
 int64_t version_of(const Tensor& w) { return w.is_inference() ? -1 : (int64_t)w._version(); }
 
 int64_t remember_tiled(const Tensor& w, int64_t bits, const Tensor& tiled) {
   c10::TensorImpl* const key = w.unsafeGetTensorImpl();
-  Copy copy{c10::weak_intrusive_ptr<c10::TensorImpl>(w.getIntrusivePtr()), version_of(w), w.data_ptr(), bits, tiled};
+  const c10::Stream made_on = current_stream(tiled);
+  Copy copy{c10::weak_intrusive_ptr<c10::TensorImpl>(w.getIntrusivePtr()), version_of(w), w.data_ptr(), bits, tiled, made_on,
+            c10::Event(made_on.device_type()), false, {}};
+  copy.made.record(made_on);
   std::lock_guard<std::mutex> lock(cache().mu);
   cache().of.insert_or_assign(key, std::move(copy));
   return (int64_t)(uintptr_t)key;
 }
 void forget_tiled(int64_t key) {
-  Copy gone{c10::weak_intrusive_ptr<c10::TensorImpl>(c10::intrusive_ptr<c10::TensorImpl>()), 0, nullptr, 0, Tensor()};
+  std::optional<Copy> gone;  // (destroyed after the lock is released)
   std::lock_guard<std::mutex> lock(cache().mu);
   auto it = cache().of.find((const c10::TensorImpl*)(uintptr_t)key);
   if (it == cache().of.end()) return;
-  gone = std::move(it->second);
+  gone.emplace(std::move(it->second));
   cache().of.erase(it);
+}
+// Makes the copy safe to read by work that is launched on the current stream from here on, and keeps its memory from
+// being handed out again before that work is done.  (The lock is held.)
+void use_on_current_stream(Copy& c) {
+  const c10::Stream now = current_stream(c.tiled);
+  if (!c.complete) {
+    // (event queries and waits are refused while any thread captures, unless this thread's capture mode is relaxed)
+    c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (c.made.query()) {
+      c.complete = true;
+    } else {
+      C10_HIP_CHECK(hipStreamIsCapturing(c10::hip::getCurrentHIPStream(now.device_index()), &capturing));
+      if (capturing != hipStreamCaptureStatusNone) {
+        // the graph may be replayed on any stream, and cannot wait for work outside of it: wait for it here
+        c.made.synchronize();
+        c.complete = true;
+      } else if (now != c.made_on) {
+        c.made.block(now);
+      }
+    }
+  }
+  if (now != c.made_on && std::find(c.used_on.begin(), c.used_on.end(), now) == c.used_on.end()) {
+    c.tiled.record_stream(now);
+    c.used_on.push_back(now);
+  }
 }
 Tensor find_tiled(const Tensor& w, int64_t bits) {
   std::lock_guard<std::mutex> lock(cache().mu);
   auto it = cache().of.find(w.unsafeGetTensorImpl());
   if (it == cache().of.end()) return Tensor();
-  const Copy& c = it->second;
+  Copy& c = it->second;
   if (c.bits != bits || c.data != w.data_ptr() || c.version != version_of(w)) return Tensor();
+  use_on_current_stream(c);
   count(kPackHit);
   return c.tiled;
+}
+// The same for a copy that Python has found in its own cache; false if it is no longer the one recorded under its key.
+bool use_tiled(int64_t key, const Tensor& tiled) {
+  std::lock_guard<std::mutex> lock(cache().mu);
+  auto it = cache().of.find((const c10::TensorImpl*)(uintptr_t)key);
+  if (it == cache().of.end() || !it->second.tiled.is_same(tiled)) return false;
+  use_on_current_stream(it->second);
+  return true;
 }
 
 // ---- one call ---------------------------------------------------------------------------------------------------
@@ -245,6 +296,7 @@ TORCH_LIBRARY_IMPL(xla_amd, CUDA, m) { m.impl("weight_only_tiled", weight_only_t
 TORCH_LIBRARY_FRAGMENT(xla_amd, m) {
   m.def("remember_tiled(Tensor w, int bits, Tensor tiled) -> int", remember_tiled);
   m.def("forget_tiled(int key) -> ()", forget_tiled);
+  m.def("use_tiled(int key, Tensor tiled) -> bool", use_tiled);
 }
 
 extern "C" int64_t xla_amd_torch_counter(int i) {

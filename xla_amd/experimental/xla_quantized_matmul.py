@@ -155,10 +155,21 @@ def invalidate_weight_cache(w: torch.Tensor = None):
     _drop_copy(key)
 
 
+def _usable_here(entry) -> bool:
+  """Orders the current stream behind the kernel that makes the entry's copy, and keeps the copy's memory from being
+  reused under work on this stream (the copy was made on the stream of whichever call came first).  False if the
+  entry's copy has just been replaced or dropped."""
+  _, _, _, copy, native = entry
+  if native is not None:
+    return torch.ops.xla_amd.use_tiled(native, copy)
+  copy.record_stream(torch.cuda.current_stream(copy.device))
+  return True
+
+
 def _relayout(w: torch.Tensor, bits: int, layout: int, kind: str) -> torch.Tensor:
   key = (id(w), kind)
   hit = _pack_cache.get(key)
-  if hit is not None and hit[0] == _version_of(w) and hit[1] == w.data_ptr() and hit[2] == bits:
+  if hit is not None and hit[0] == _version_of(w) and hit[1] == w.data_ptr() and hit[2] == bits and _usable_here(hit):
     counters["pack_hit"] += 1
     return hit[3]
   if torch.cuda.is_current_stream_capturing():
@@ -189,7 +200,11 @@ def _relayout(w: torch.Tensor, bits: int, layout: int, kind: str) -> torch.Tenso
   if hit is None:
     weakref.finalize(w, _drop_copy, key).atexit = False
   # (a weight whose record is replaced is the same tensor: the native record is replaced with it)
-  native = torch.ops.xla_amd.remember_tiled(w, bits, out) if kind == "tiled" else None
+  native = None
+  if kind == "tiled":
+    native = torch.ops.xla_amd.remember_tiled(w, bits, out)
+  else:
+    torch.cuda.current_stream(w.device).synchronize()  # (any stream may read it from here on)
   _pack_cache[key] = (_version_of(w), w.data_ptr(), bits, out, native)
   return out
 
