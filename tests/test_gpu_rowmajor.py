@@ -52,3 +52,27 @@ def test_int8_product_any_k_exact(ops, m, n, k):
   assert torch.equal(acc.cpu().double(), ref)
   exp = (ref.float() * ws - xsum.float()[:, None] * zp) * xs
   torch.testing.assert_close(out.cpu(), exp, rtol=1e-6, atol=1e-2 * float(exp.abs().max()) * 1e-4)
+
+
+# one row more than 65535 tiles of 16 rows, and than the 65535 tiles of 64 that one launch covers
+@pytest.mark.parametrize("m", [65535 * 16 + 1, 65535 * 64 + 1])
+def test_rows_past_one_grid(ops, m):
+  k, n, last = 20, 3, 200
+  g = cases.gen(m)
+  x = torch.randn(last, k, generator=g).to(torch.bfloat16)
+  w = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int32).to(torch.int8)
+  s, z = torch.rand(n, generator=g).to(torch.bfloat16), torch.randn(n, generator=g).to(torch.bfloat16)
+  xd = torch.zeros(m, k, dtype=torch.bfloat16, device="cuda")
+  xd[-last:] = x.cuda()
+  out = torch.ops.xla.quantized_matmul(xd, w.cuda(), s.cuda(), z.cuda())
+  exp = oracle.quantized_matmul(x, w, s, z)
+  assert cases.within_tolerance(out[-last:].cpu(), exp) and not out[:-last].any()
+  # the int8 product: exact sums
+  xq = torch.zeros(m, k, dtype=torch.int8, device="cuda")
+  xq[-last:] = torch.randint(-128, 128, (last, k), generator=g, dtype=torch.int32).to(torch.int8).cuda()
+  f32 = dict(cvt_dtype=torch.float32, mid_dtype=torch.float32, out_dtype=torch.float32)
+  xs = torch.rand(m, 1, generator=g).cuda()
+  out, acc = ops.w8a8_gemm_gpu(xq, w.cuda(), xs, s.float().cuda(), None, None, want_acc=True, **f32)
+  want = xq[-last:].cpu().int() @ w.int().t()
+  assert torch.equal(acc[-last:].cpu(), want) and not acc[:-last].any()
+  assert torch.equal(out[-last:].cpu(), want.float() * s.float() * xs[-last:].cpu())

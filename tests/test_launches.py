@@ -33,3 +33,34 @@ def test_every_kernel_gets_its_lds(tmp_path):
       assert l.lds <= l.lds_limit, (l.name, l.lds, l.lds_limit)
   for kernel in ("qmm_wo_bw_wide_kernel", "qmm_wo_bw_gemm_kernel", "qmm_wo_gemm_kernel", "qmm_skinny_resident_kernel", "qmm_w8a8_gemm_kernel"):
     assert sum(kernel in s for s in seen) > 1, kernel
+
+
+@pytest.mark.parametrize("zp", [False, True])
+def test_row_major_rows_of_any_number(tmp_path, zp):
+  """Rows past what one launch's grid can hold: pieces that follow each other and cover them all, within the limits of a
+  grid (65535 in y, 2^32 threads in x)."""
+  max_rows = 65535 * 64
+  sizes = [(1 << 20, 8, 100), ((1 << 20) + 1, 8, 100), (max_rows, 3, 20), (max_rows + 1, 3, 20), (3 * max_rows - 5, 1, 9),
+           (1, 1 << 31, 1), (5, (1 << 31) + 300, 1)]
+  calls = [rec.generic(m, n, k, zp=zp) for m, n, k in sizes]
+  calls += [rec.w8a8(m, n, k) for m, n, k in sizes if n <= 1 << 30]
+  sizes += [s for s in sizes if s[1] <= 1 << 30]
+  for (m, n, k), call, (rc, text, launches) in zip(sizes, calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0, (m, n, k, text)
+    x_size = 2 if "generic" in call[0] else 1
+    covered = {}
+    for l in launches:
+      assert l.grid[1] <= 65535 and l.grid[2] == 1 and l.grid[0] * l.block[0] < 1 << 32, l
+      x, w, scale, _, out, lm, ln, lk = l.args
+      row, col = (x - rec.PTR) // (k * x_size), (w - rec.PTR) // k
+      assert lk == k and (scale - rec.PTR) == col * (2 if "generic" in call[0] else 4) and (out - rec.PTR) == (row * n + col) * 2
+      # tiles of 16, 32 or 64 rows and of 16, 64 or 256 channels
+      assert any(l.grid[1] == -(-lm // t) for t in (16, 32, 64)) and any(l.grid[0] == -(-ln // t) for t in (16, 64, 256))
+      covered.setdefault((col, ln), []).append((row, lm))
+    assert sum(ln for _, ln in covered) == n and sorted(covered)[0][0] == 0
+    for rows in covered.values():
+      at = 0
+      for row, lm in rows:
+        assert row == at
+        at += lm
+      assert at == m

@@ -10,6 +10,7 @@ struct QmmRowMajorArgs {
   const void* zp;      // [N] or null
   void* out;           // [M, N]
   int64_t M, N, K;
+  int64_t ldo;         // elements between rows of out (and acc_out): N, or more in a piece of the channels
   int scale_dt, zp_dt, zpo_dt, out_dt;
   int dot_dt, store_dt;               // weight-only
   const void* x_scale;                // int8 activations: [M]

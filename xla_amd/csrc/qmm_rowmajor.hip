@@ -155,7 +155,7 @@ qmm_rowmajor_kernel(QmmRowMajorArgs a) {
     if (m >= a.M) return;
     for (int e = 0; e < 4; ++e) {
       if (n + e >= a.N) return;
-      const int64_t idx = m * a.N + n + e;
+      const int64_t idx = m * a.ldo + n + e;
       if constexpr (kInt) {
         // the chain documented at xla_amd_qmm_w8a8_gemm
         if (a.acc_out) a.acc_out[idx] = v[e];
@@ -238,12 +238,40 @@ int launch_rows(const QmmRowMajorArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-int qmm_rowmajor_launch(const QmmRowMajorArgs& a, int x_dt, hipStream_t stream) {
-  if ((a.M + 15) / 16 > 65535) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "row-major matmul: too many rows");
+static int launch_piece(const QmmRowMajorArgs& a, int x_dt, hipStream_t stream) {
   switch (x_dt) {
     case XLA_AMD_DT_F32: return launch_rows<XLA_AMD_DT_F32>(a, stream);
     case XLA_AMD_DT_BF16: return launch_rows<XLA_AMD_DT_BF16>(a, stream);
     case XLA_AMD_DT_F16: return launch_rows<XLA_AMD_DT_F16>(a, stream);
     default: return launch_rows<kInt8>(a, stream);
   }
+}
+
+// What one grid cannot hold goes in pieces: 65535 tiles of 64 rows, and channels whose tiles come to less than 2^32
+// threads.
+int qmm_rowmajor_launch(const QmmRowMajorArgs& whole, int x_dt, hipStream_t stream) {
+  constexpr int64_t kRows = 65535ll * 64, kChannels = 1ll << 30;
+  if ((whole.M * whole.N + 255) / 256 > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "row-major matmul: too many outputs");
+  const bool int8 = x_dt == kInt8;
+  const size_t x_size = int8 ? 1 : qmm_dt_size(x_dt), out_size = qmm_dt_size(int8 ? whole.out_dt : whole.store_dt);
+  auto at = [](const void* p, int64_t elements, size_t size) { return p ? (void*)((char*)p + elements * size) : nullptr; };
+  for (int64_t n = 0; n < whole.N; n += kChannels) {
+    for (int64_t m = 0; m < whole.M; m += kRows) {
+      QmmRowMajorArgs a = whole;
+      a.ldo = whole.N;
+      a.M = whole.M - m < kRows ? whole.M - m : kRows;
+      a.N = whole.N - n < kChannels ? whole.N - n : kChannels;
+      a.x = at(whole.x, m * whole.K, x_size);
+      a.w = whole.w + n * whole.K;
+      a.scale = at(whole.scale, n, qmm_dt_size(whole.scale_dt));
+      a.zp = at(whole.zp, n, qmm_dt_size(whole.zp_dt));
+      a.out = at(whole.out, m * whole.N + n, out_size);
+      a.x_scale = at(whole.x_scale, m, qmm_dt_size(whole.x_scale_dt));
+      a.x_sum = (const int32_t*)at(whole.x_sum, m, 4);
+      a.acc_out = (int32_t*)at(whole.acc_out, m * whole.N + n, 4);
+      const int rc = launch_piece(a, x_dt, stream);
+      if (rc != XLA_AMD_QMM_OK) return rc;
+    }
+  }
+  return XLA_AMD_QMM_OK;
 }
