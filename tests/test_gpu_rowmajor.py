@@ -76,3 +76,29 @@ def test_rows_past_one_grid(ops, m):
   want = xq[-last:].cpu().int() @ w.int().t()
   assert torch.equal(acc[-last:].cpu(), want) and not acc[:-last].any()
   assert torch.equal(out[-last:].cpu(), want.float() * s.float() * xs[-last:].cpu())
+
+
+# one thread per output on either side of where it begins: by columns, by outputs (512 x 512), few rows against many
+# channels; more outputs than the threads of its grid
+SHORT = [(1, 1, 1), (7, 300, 16), (7, 300, 17), (7, 301, 47), (7, 301, 49), (301, 801, 31), (301, 801, 33), (512, 512, 15), (513, 512, 8), (513, 512, 9),
+         (4, 32768, 40), (4, 32769, 41), (5, 32768, 9), (2100, 8200, 3)]
+
+
+@pytest.mark.parametrize("m,n,k", SHORT)
+def test_short_rows(ops, m, n, k):
+  g = cases.gen(m + n + k)
+  for xdt in (torch.bfloat16, torch.float16, torch.float32):
+    x, w, s, _ = cases.per_channel_int8(m, n, k, xdt, xdt, seed=m + n + k)
+    for z in (None, (torch.randn(n, generator=g) * 0.01).to(xdt)):
+      exp = oracle.quantized_matmul(x, w, s, z)
+      out = torch.ops.xla.quantized_matmul(x.cuda(), w.cuda(), s.cuda(), None if z is None else z.cuda()).cpu()
+      assert out.dtype == exp.dtype and cases.within_tolerance(out, exp), (xdt, z is None)
+  xq = torch.randint(-128, 128, (m, k), generator=g, dtype=torch.int32).to(torch.int8)
+  xs, ws, zp = torch.rand(m, 1, generator=g), torch.rand(n, generator=g), torch.randn(n, generator=g)
+  xsum = xq.to(torch.int32).sum(-1).to(torch.int32)
+  f32 = dict(cvt_dtype=torch.float32, mid_dtype=torch.float32, out_dtype=torch.float32)
+  out, acc = ops.w8a8_gemm_gpu(xq.cuda(), w.cuda(), xs.cuda(), ws.cuda(), zp.cuda(), xsum.cuda(), want_acc=True, **f32)
+  ref = (xq.double() @ w.double().t()).float()  # (exact)
+  assert torch.equal(acc.cpu().float(), ref)
+  exp = (ref * ws - xsum.float()[:, None] * zp) * xs
+  torch.testing.assert_close(out.cpu(), exp, rtol=1e-6, atol=1e-6 * float(exp.abs().max()))

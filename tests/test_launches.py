@@ -41,7 +41,7 @@ def test_row_major_rows_of_any_number(tmp_path, zp):
   grid (65535 in y, 2^32 threads in x)."""
   max_rows = 65535 * 64
   sizes = [(1 << 20, 8, 100), ((1 << 20) + 1, 8, 100), (max_rows, 3, 20), (max_rows + 1, 3, 20), (3 * max_rows - 5, 1, 9),
-           (1, 1 << 31, 1), (5, (1 << 31) + 300, 1)]
+           (1, 1 << 31, 41), (5, (1 << 31) + 300, 41)]
   calls = [rec.generic(m, n, k, zp=zp) for m, n, k in sizes]
   calls += [rec.w8a8(m, n, k) for m, n, k in sizes if n <= 1 << 30]
   sizes += [s for s in sizes if s[1] <= 1 << 30]
@@ -64,3 +64,19 @@ def test_row_major_rows_of_any_number(tmp_path, zp):
         assert row == at
         at += lm
       assert at == m
+
+
+def test_row_major_short_rows(tmp_path):
+  """One thread per output up to a number of columns that depends on the outputs; its grid may be smaller than they are
+  (the kernel strides) but not empty."""
+  short = [(1, 1, 1), (300, 800, 16), (512, 512, 16), (513, 512, 8), (1, 32768, 40), (4, 1 << 20, 40), (1 << 20, 64, 8)]
+  tiled = [(300, 800, 33), (513, 512, 9), (1, 32768, 41), (5, 65536, 9), (1, 32767, 49), (40, 3000, 2000)]
+  calls = [f(*s) for f in (rec.generic, rec.w8a8) for s in short + tiled]
+  calls += [rec.generic(300, 800, 17), rec.w8a8(300, 800, 31), rec.w8a8(100, 800, 47), rec.w8a8(100, 800, 49)]
+  want = ([True] * len(short) + [False] * len(tiled)) * 2 + [False, True, True, False]
+  for call, one_thread, (rc, text, launches) in zip(calls, want, rec.record(calls, str(tmp_path))):
+    if "w8a8" in call[0] and call[2][10] % 16 == 0:
+      continue  # (aligned operands take the LDS-tiled kernel)
+    assert rc == 0 and len(launches) == 1, text
+    assert ("qmm_rowmajor_short_kernel" in launches[0].name) == one_thread, call
+    assert 0 < launches[0].grid[0] * launches[0].block[0] < 1 << 32

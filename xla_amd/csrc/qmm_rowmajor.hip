@@ -26,6 +26,59 @@ template <int XT> struct Elem { typedef uint16_t t; };
 template <> struct Elem<XLA_AMD_DT_F32> { typedef float t; };
 template <> struct Elem<kInt8> { typedef int8_t t; };
 
+// Result (m, n) from its sum v (f32 by bits, or int32) and, with a zero point, the row's sum of x.
+template <int XT, bool HASZP>
+__device__ __forceinline__ void finish_one(const QmmRowMajorArgs& a, int64_t m, int64_t n, int v, float xsum) {
+  const int64_t idx = m * a.ldo + n;
+  if constexpr (XT == kInt8) {
+    // the chain documented at xla_amd_qmm_w8a8_gemm
+    if (a.acc_out) a.acc_out[idx] = v;
+    if (!a.out) return;
+    float f = qmm_round_dt((float)v, a.cvt_dt);
+    f = qmm_round_dt(f * qmm_load(a.scale, n, a.scale_dt), a.mid_dt);
+    if (a.zp) {
+      const float z = qmm_round_dt(qmm_round_dt((float)a.x_sum[m], a.zpo_dt) * qmm_load(a.zp, n, a.zp_dt), a.zpo_dt);
+      f = qmm_round_dt(f - z, a.mid_dt);
+    }
+    qmm_store(a.out, idx, qmm_round_dt(f * qmm_load(a.x_scale, m, a.x_scale_dt), a.out_dt), a.out_dt);
+  } else {
+    // p = round_dot(dot); o = round_out(scale p); zero point: o = round_out(o - round_zpo(round_x(sum x) zp))
+    const float p = qmm_round_dt(__int_as_float(v), a.dot_dt);
+    float o = qmm_round_dt(qmm_load(a.scale, n, a.scale_dt) * p, a.out_dt);
+    if constexpr (HASZP) {
+      const float z = qmm_round_dt(xsum, XT) * qmm_load(a.zp, n, a.zp_dt);
+      o = qmm_round_dt(o - qmm_round_dt(z, a.zpo_dt), a.out_dt);
+    }
+    qmm_store(a.out, idx, o, a.store_dt);
+  }
+}
+
+// Rows of a few columns: one thread per output.  The tiles below load a row's end element by element under a condition
+// each, and 16 rows of x whatever M is.
+template <int XT, bool HASZP>
+__global__ void __launch_bounds__(256)
+qmm_rowmajor_short_kernel(QmmRowMajorArgs a) {
+  typedef typename Elem<XT>::t elem_t;
+  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < a.M * a.N; idx += (int64_t)gridDim.x * 256) {
+    const int64_t m = idx / a.N, n = idx - m * a.N;
+    const elem_t* const x = (const elem_t*)a.x + m * a.K;
+    const int8_t* const w = a.w + n * a.K;
+    if constexpr (XT == kInt8) {
+      int sum = 0;
+      for (int k = 0; k < (int)a.K; ++k) sum += (int)x[k] * (int)w[k];
+      finish_one<XT, HASZP>(a, m, n, sum, 0.f);
+    } else {
+      float sum = 0.f, xsum = 0.f;
+      for (int k = 0; k < (int)a.K; ++k) {
+        const float xv = qmm_load(x, k, XT);
+        sum = fmaf(xv, (float)w[k], sum);
+        if constexpr (HASZP) xsum += xv;
+      }
+      finish_one<XT, HASZP>(a, m, n, __float_as_int(sum), xsum);
+    }
+  }
+}
+
 template <int XT, int MT, int NG, int NW, bool HASZP>
 __global__ void __launch_bounds__(kWavesAll * 64)
 qmm_rowmajor_kernel(QmmRowMajorArgs a) {
@@ -155,28 +208,7 @@ qmm_rowmajor_kernel(QmmRowMajorArgs a) {
     if (m >= a.M) return;
     for (int e = 0; e < 4; ++e) {
       if (n + e >= a.N) return;
-      const int64_t idx = m * a.ldo + n + e;
-      if constexpr (kInt) {
-        // the chain documented at xla_amd_qmm_w8a8_gemm
-        if (a.acc_out) a.acc_out[idx] = v[e];
-        if (!a.out) continue;
-        float f = qmm_round_dt((float)v[e], a.cvt_dt);
-        f = qmm_round_dt(f * qmm_load(a.scale, n + e, a.scale_dt), a.mid_dt);
-        if (a.zp) {
-          const float z = qmm_round_dt(qmm_round_dt((float)a.x_sum[m], a.zpo_dt) * qmm_load(a.zp, n + e, a.zp_dt), a.zpo_dt);
-          f = qmm_round_dt(f - z, a.mid_dt);
-        }
-        qmm_store(a.out, idx, qmm_round_dt(f * qmm_load(a.x_scale, m, a.x_scale_dt), a.out_dt), a.out_dt);
-      } else {
-        // p = round_dot(dot); o = round_out(scale p); zero point: o = round_out(o - round_zpo(round_x(sum x) zp))
-        const float p = qmm_round_dt(__int_as_float(v[e]), a.dot_dt);
-        float o = qmm_round_dt(qmm_load(a.scale, n + e, a.scale_dt) * p, a.out_dt);
-        if constexpr (HASZP) {
-          const float z = qmm_round_dt(__int_as_float(xsum[0]), XT) * qmm_load(a.zp, n + e, a.zp_dt);
-          o = qmm_round_dt(o - qmm_round_dt(z, a.zpo_dt), a.out_dt);
-        }
-        qmm_store(a.out, idx, o, a.store_dt);
-      }
+      finish_one<XT, HASZP>(a, m, n + e, v[e], __int_as_float(xsum[0]));
     }
   };
   if constexpr (KW == 1) {
@@ -229,8 +261,27 @@ int launch_width(const QmmRowMajorArgs& a, hipStream_t stream) {
   return launch<XT, MT, 1, 1>(a, stream);
 }
 
+// Columns up to which one thread per output is faster (bf16 x / int8 x, us, one thread per output against tiles): the
+// latency of its loop decides for few outputs (512 x 512: K = 12 6.0 / 4.7 against 7.3 / 8.6, K = 25 9.1 / 8.3 against
+// 7.9 / 9.5, K = 33 12.1 / 11.1 against 8.0 / 9.7; 40 x 3000: K = 12 5.3 / 3.9 against 7.0 / 8.4, K = 40 11.7 / 7.5
+// against 7.7 / 9.4, K = 50 14.3 / 9.0 against 7.8 / 9.5), its many loads for many (2048 x 2048: K = 4 24 / 17 against
+// 32 / 24, K = 8 33 / 23 against 35 / 25, K = 12 42 / 32 against 38 / 27), and the tiles' empty rows for one row against
+// many channels (1 x 1 048 576: K = 8 11 / 8 against 40 / 56, K = 40 62 / 61 against 65 / 79).
+inline int64_t short_columns(const QmmRowMajorArgs& a, bool int8) {
+  if (a.M <= 4 && a.N >= 32768) return 40;
+  if (a.M * a.N > (1 << 18)) return 8;
+  return !int8 ? 16 : a.M * a.N > (1 << 17) ? 32 : 48;
+}
+
 template <int XT>
 int launch_rows(const QmmRowMajorArgs& a, hipStream_t stream) {
+  if (a.K <= short_columns(a, XT == kInt8)) {
+    const int64_t blocks = (a.M * a.N + 255) / 256;
+    const dim3 grid((unsigned)(blocks < 65536 ? blocks : 65536)), block(256);
+    if (XT != kInt8 && a.zp) hipLaunchKernelGGL((qmm_rowmajor_short_kernel<XT, XT != kInt8>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((qmm_rowmajor_short_kernel<XT, false>), grid, block, 0, stream, a);
+    return QMM_CHECK_LAUNCH("row-major matmul launch");
+  }
   if (a.M <= 16) return launch_width<XT, 1>(a, stream);
   if (a.M <= 32) return launch_width<XT, 2>(a, stream);
   return launch_width<XT, 4>(a, stream);
