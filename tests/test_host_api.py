@@ -4,6 +4,8 @@ checks with the reference's messages, the module and the quantizer utilities."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -376,3 +378,22 @@ def test_headline_kernels_keep_their_code_budget():
   for name, budget in build.CODE_BUDGET_BYTES.items():
     assert name in by_name, name
     assert by_name[name]["code_bytes"] <= budget, (name, by_name[name]["code_bytes"], budget)
+
+
+def test_a_replaced_library_replaces_the_operators_kernels():
+  """A program that names another build of the library (the diagnostic one) gets that build's kernels from the operators
+  too: the native operators, which are linked against the ordinary build, stay out of the process."""
+  code = """
+import os, torch
+from xla_amd import _lib
+_lib._LIB_PATH = os.path.join(os.path.dirname(_lib._LIB_PATH), "libxla_amd_qmm_timeline.so")
+import xla_amd.experimental.xla_quantized_matmul as q
+maps = open("/proc/self/maps").read()
+_lib.load()
+assert "libxla_amd_qmm_timeline.so" in open("/proc/self/maps").read()
+assert "libxla_amd_qmm.so" not in maps and "libxla_amd_torch.so" not in maps
+for op in ("xla::quantized_matmul", "xla_amd::weight_only_tiled"):
+  assert torch._C._dispatch_has_kernel_for_dispatch_key(op, "CUDA")
+assert q.counters.native is None and q.counters["pack"] == 0
+"""
+  subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT, timeout=120)

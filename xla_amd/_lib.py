@@ -9,7 +9,8 @@ import threading
 
 import torch
 
-_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libxla_amd_qmm.so")
+_OWN_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libxla_amd_qmm.so")
+_LIB_PATH = _OWN_LIB_PATH  # (a program may name another build of the library here, such as the diagnostic one, before it is loaded)
 
 OK, EINVAL, EUNSUPPORTED, EHIP = 0, -1, -2, -3
 DT_F32, DT_BF16, DT_F16 = 0, 1, 2
@@ -89,10 +90,15 @@ def load():
   return _lib
 
 
+def replaced() -> bool:
+  """Another build of the library stands in the place of the one the native operators are linked against."""
+  return _LIB_PATH != _OWN_LIB_PATH
+
+
 def load_torch_binding():
   """Registers the native operator implementations and returns a function (counter index) -> calls, or None when the
-  libraries are not built."""
-  if not (os.path.exists(_LIB_PATH) and os.path.exists(_TORCH_LIB_PATH)):
+  libraries are not built or the library is replaced (the native operators would run the one they are linked against)."""
+  if replaced() or not (os.path.exists(_LIB_PATH) and os.path.exists(_TORCH_LIB_PATH)):
     return None
   load()
   torch.ops.load_library(_TORCH_LIB_PATH)

@@ -201,7 +201,7 @@ def _relayout(w: torch.Tensor, bits: int, layout: int, kind: str) -> torch.Tenso
     weakref.finalize(w, _drop_copy, key).atexit = False
   # (a weight whose record is replaced is the same tensor: the native record is replaced with it)
   native = None
-  if kind == "tiled":
+  if kind == "tiled" and counters.native is not None:
     native = torch.ops.xla_amd.remember_tiled(w, bits, out)
   else:
     torch.cuda.current_stream(w.device).synchronize()  # (any stream may read it from here on)
@@ -565,7 +565,11 @@ def weight_only_tiled_meta(x, w_tiled, scaler, zero_point, out_features, block_s
 
 
 counters.native = _lib.load_torch_binding()
-if counters.native is None:
+if counters.native is None and _lib.replaced():
+  # another build of the library: its kernels through the Python formulation
+  XLA_LIB.impl("quantized_matmul", quantized_matmul_rocm, "CUDA")
+  XLA_AMD_LIB.impl("weight_only_tiled", weight_only_tiled_rocm, "CUDA")
+elif counters.native is None:
 
   def _not_built(*args, **kwargs):
     _lib.load()
