@@ -275,8 +275,9 @@ int xla_amd_qmm_quantize_per_token(const void* x, int8_t* x_q, void* x_scale, in
  * multiplies, hence cvt_dt and the inner round of x_sum.)
  * If acc_out != NULL the raw int32 accumulators are also stored to
  * acc_out [M,N] (parity/debug).  If out == NULL only acc_out is written.
- * The MFMA kernel needs K % 16 == 0 and 16-byte aligned x_q and w; other
- * shapes run a one-thread-per-output kernel.
+ * The LDS-tiled kernel needs K % 16 == 0 and 16-byte aligned x_q and w; other
+ * operands run a kernel that reads rows from any byte (matrix instructions too,
+ * or one thread per output up to a few dozen columns).
  * block_m/block_n select the workgroup tile (the role of batch_block_size /
  * out_block_size, custom_kernel.py:1088-1100): 0,0 = choose by shape;
  * otherwise one of the pairs xla_amd_qmm_w8a8_tile can return, else
@@ -358,8 +359,9 @@ int xla_amd_qmm_dispatch(int64_t M, int64_t N, int64_t K, int64_t C, int bits, i
                          int quantize_activation);
 
 /*
- * Tile configuration the W8A8 GEMM would use for a shape: fills
- * tile_mnk[3] = {block_M, block_N, block_K}; the analogue of
+ * Tile configuration the W8A8 GEMM uses for a shape: fills
+ * tile_mnk[3] = {block_M, block_N, block_K} (a shape that takes 256 x 256 may
+ * have its last columns covered by tiles of 256 x 192); the analogue of
  * get_tuned_block_sizes (pallas_kernels/quantized_matmul_kernel.py:537-555).
  */
 int xla_amd_qmm_w8a8_tile(int64_t M, int64_t N, int64_t K, int32_t* tile_mnk /* host */);

@@ -1,6 +1,10 @@
 """W8A8: the tiles with three stages and two K groups, and the quantizer's thread counts, at their edges."""
+import ctypes
+
 import pytest
 import torch
+
+from xla_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -37,10 +41,19 @@ def test_128x256(ops, m, n, k):
   _check(ops, m, n, k, block_m=128, block_n=256)
 
 
-# more than 256 tiles of 64 x 64, at most 256 of 64 x 128, K from 4096: an even and an odd number of steps, a partial one
-@pytest.mark.parametrize("m,n,k", [(130, 5512, 4096), (130, 5511, 4112), (200, 4228, 4224), (33, 16500, 4096)])
+# more than 256 tiles of 64 x 64, at most 256 of 64 x 128, K from 4096, more than two row tiles (else 64 x 64): an even and an odd number of steps, a partial one
+@pytest.mark.parametrize("m,n,k", [(130, 5512, 4096), (130, 5511, 4112), (200, 4228, 4224), (33, 16500, 4096),
+                                   (129, 5500, 4096)])
 def test_64x128_two_k_groups(ops, m, n, k):
+  tile = (ctypes.c_int32 * 3)()
+  assert _lib.load().xla_amd_qmm_w8a8_tile(m, n, k, tile) == 0 and tuple(tile)[:2] == (64, 128 if m > 128 else 64)
   _check(ops, m, n, k)
+
+
+# asked for at any size: fewer steps of K than the two groups, one each, more; row and column tails
+@pytest.mark.parametrize("m,n,k", [(64, 128, 16), (65, 129, 128), (30, 100, 144), (100, 300, 256), (1, 1, 1040)])
+def test_64x128_asked_for(ops, m, n, k):
+  _check(ops, m, n, k, block_m=64, block_n=128)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])

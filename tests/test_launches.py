@@ -1,7 +1,11 @@
 """What the library's entry points launch, recorded without a GPU."""
+import ctypes
+import re
+
 import pytest
 
 from tests import launch_recorder as rec
+from xla_amd import _lib
 
 
 def test_every_kernel_gets_its_lds(tmp_path):
@@ -80,3 +84,31 @@ def test_row_major_short_rows(tmp_path):
     assert rc == 0 and len(launches) == 1, text
     assert ("qmm_rowmajor_short_kernel" in launches[0].name) == one_thread, call
     assert 0 < launches[0].grid[0] * launches[0].block[0] < 1 << 32
+
+
+TILES = [(32, 32), (64, 32), (64, 64), (64, 128), (128, 128), (128, 256), (256, 256)]
+
+
+def _tile(launch):
+  return tuple(int(v) for v in re.search(r"qmm_w8a8_gemm_kernelILi(\d+)ELi(\d+)E", launch.name).groups())
+
+
+def test_w8a8_tile_reported_is_the_tile_launched(tmp_path):
+  lib, tile = _lib.load(), (ctypes.c_int32 * 3)()
+  shapes = [(m, n, k) for m in (1, 32, 33, 64, 65, 128, 200, 256, 512, 1024, 2048)
+            for n, k in ((1024, 4096), (4096, 4096), (4096, 14336), (14336, 4096), (28672, 4096), (8192, 1024), (5511, 4112))]
+  calls = [rec.w8a8(*s) for s in shapes]
+  chosen = set()
+  for (m, n, k), (rc, text, launches) in zip(shapes, rec.record(calls, str(tmp_path))):
+    assert rc == 0, text
+    assert lib.xla_amd_qmm_w8a8_tile(m, n, k, tile) == 0
+    chosen.add(tuple(tile)[:2])
+    # (256 x 256 covers the last columns with tiles of 192)
+    assert {_tile(l) for l in launches} <= ({(256, 256), (256, 192)} if tile[0] == 256 else {tuple(tile)[:2]}), (m, n, k)
+  assert chosen == set(TILES)
+  from xla_amd.experimental.hip_kernels.quantized_matmul_kernel import _SUPPORTED_TILES
+  assert sorted(_SUPPORTED_TILES) == TILES
+  # ... and a tile that is asked for is the one launched, at any size
+  calls = [rec.w8a8(m, n, k, bm, bn) for bm, bn in TILES[:-1] for m, n, k in ((512, 4096, 4096), (10, 100, 128), (200, 4096, 14336))]
+  for call, (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0 and [_tile(l) for l in launches] == [tuple(call[2][-3:-1])], call

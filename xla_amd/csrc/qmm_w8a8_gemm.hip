@@ -558,6 +558,12 @@ static void choose_tile(int64_t M, int64_t N, int64_t K, int* bm, int* bn) {
   // fetched per tile as well) and while that is at most one tile per CU (64 rows against 4096
   // channels: 8.1 against 8.7 us; 128 rows against 1280 x 8192: 10.6 against 12.7 us), else 64 x 32.
   if (tiles(64, 64) <= 128) { *bm = (M <= 32 || tiles(32, 32) <= 256) ? 32 : 64; *bn = 32; return; }
+  // Twice the columns per workgroup and two K groups while that is at most one workgroup per CU: a quarter less to copy
+  // (us, 64 x 64 / 64 x 128, weights out of HBM; out of the Infinity Cache: 512 x 4096 x 14336 68 / 53; 49 / 45,
+  // 256 x 8192 x 8192 45 / 36; 30 / 28, 160 x 6144 x 4096 21.1 / 20.2; 15.3 / 16.1).  From three row tiles on: one row tile
+  // reads every weight once either way (48 x 28672 x 4096 41.7 / 43.2; 23.9 / 23.7), with two it depends on where the
+  // weights come from (96 x 11008 x 4096 24.6 / 24.4; 16.2 / 17.1, 128 x 14336 x 4096 28.8 / 26.8; 16.9 / 16.5).
+  if (M > 128 && tiles(64, 64) > 256 && tiles(64, 128) <= 256 && K >= 4096) { *bm = 64; *bn = 128; return; }
   if (M <= 64 || tiles(64, 64) <= 768) { *bm = 64; *bn = 64; return; }
   int64_t n1;
   const double c256 = M > 128 && N > 128 ? best_column_split(M, N, K, &n1) : 1e30;
@@ -655,12 +661,9 @@ extern "C" int xla_amd_qmm_w8a8_gemm(const int8_t* x_q, const int8_t* w, const v
     // At most one workgroup per CU and a long K: two K groups halve the K loop.
     const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
     if (tiles <= 256 && K >= 1024) return launch_tile<64, 64, 2, 2, 3, 2>(g, s);
-    // Twice the columns per workgroup while that is at most one per CU: a quarter less to copy and the two K groups as
-    // well (512 x 4096 x 14336: 60 -> 49 us; 256 x 8192 x 8192 40 -> 31, 128 x 14336 x 4096 24 -> 20, 512 x 4096 x 4096 17.3 -> 17.0).
-    // (Up to 32 rows the tile is mostly empty: 16 x 28672 x 4096 28 us as it is, 30 so.)
-    if (M > 32 && ((M + 63) / 64) * ((N + 127) / 128) <= 256 && K >= 4096) return launch_tile<64, 128, 2, 2, 3, 2>(g, s);
     return tiles <= 512 ? launch_tile<64, 64, 2, 2, 3>(g, s) : launch_tile<64, 64, 2, 2, 2>(g, s);
   }
+  if (bm == 64 && bn == 128) return launch_tile<64, 128, 2, 2, 3, 2>(g, s);  // (chosen for K >= 4096; right for any)
   if (bm == 64 && bn == 32) {  // two waves per K group
     return K >= 1024 ? launch_tile<64, 32, 2, 1, 3, 4>(g, s) : launch_tile<64, 32, 2, 1, 3, 1>(g, s);
   }
