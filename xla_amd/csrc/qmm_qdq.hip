@@ -43,14 +43,42 @@ struct QdqParams {
   const void* zp;   // null: 0
   int scale_dt, zp64, reciprocal;  // reciprocal: what multiplies x is 1 / scale
 };
-__device__ __forceinline__ float qdq_scale(const QdqParams& p, uint32_t c) {
-  const float s = qmm_load(p.scale, c, p.scale_dt);
-  return p.reciprocal ? 1.0f / s : s;
+// A channel's parameters.  They are requested without a conversion, and converted when they are needed: a conversion
+// inside the branch on a type waits for its load, and each load would wait for the one before (a bf16 pair over 4096 x 64
+// elements 5.8 us, 5.1 so).
+struct RawParams {
+  uint32_t scale;
+  int zp;
+};
+__device__ __forceinline__ RawParams qdq_request(const QdqParams& p, uint32_t c) {
+  RawParams r = {qmm_load_raw(p.scale, c, p.scale_dt), 0};
+  if (p.zp) r.zp = ((const int32_t*)p.zp)[(size_t)c << p.zp64];  // (the low half of an int64)
+  return r;
 }
-__device__ __forceinline__ int qdq_zp(const QdqParams& p, uint32_t c) {
-  if (!p.zp) return 0;
-  return p.zp64 ? (int)((const int64_t*)p.zp)[c] : ((const int32_t*)p.zp)[c];
+__device__ __forceinline__ float qdq_factor(const QdqParams& p, float s) { return p.reciprocal ? 1.0f / s : s; }
+__device__ __forceinline__ float qdq_scale(const QdqParams& p, const RawParams& r) {
+  return qdq_factor(p, qmm_from_raw(r.scale, p.scale_dt));
 }
+// ... and those of RUN consecutive channels, in 16-byte pieces (at any element's address).
+template <int RUN>
+struct RawAlong {
+  i32x4 scale[RUN / 4], zp[RUN / 2];
+  __device__ __forceinline__ void request(const QdqParams& p, uint32_t c) {
+    if (p.scale_dt == XLA_AMD_DT_F32) __builtin_memcpy(scale, (const float*)p.scale + c, RUN * 4);
+    else __builtin_memcpy(scale, (const uint16_t*)p.scale + c, RUN * 2);
+    if (!p.zp) return;
+    if (p.zp64) __builtin_memcpy(zp, (const int64_t*)p.zp + c, RUN * 8);
+    else __builtin_memcpy(zp, (const int32_t*)p.zp + c, RUN * 4);
+  }
+  __device__ __forceinline__ float scale_of(const QdqParams& p, int i) const {
+    const uint32_t pair = (uint32_t)scale[i / 8][i / 2 % 4];
+    return qdq_factor(p, p.scale_dt == XLA_AMD_DT_F32 ? __int_as_float(scale[i / 4][i % 4])
+                                                      : qmm_from_raw(i & 1 ? pair >> 16 : pair & 0xffffu, p.scale_dt));
+  }
+  __device__ __forceinline__ int zp_of(const QdqParams& p, int i) const {
+    return !p.zp ? 0 : p.zp64 ? zp[i / 2][i % 2 * 2] : zp[i / 4][i % 4];
+  }
+};
 
 // How the elements of a tensor [outer, channels, inner] find their channel.  A thread of the vector forms handles U
 // runs of consecutive elements: kOne, one channel; kRow, a run lies within a channel (inner a multiple of the run);
@@ -58,33 +86,39 @@ __device__ __forceinline__ int qdq_zp(const QdqParams& p, uint32_t c) {
 // What bounds the vector forms is memory alone as long as a run's channel costs few instructions: 32-bit divisions by
 // the row length (the 64-bit ones of kAny take over a hundred instructions), none for kOne; in kAlong a thread's runs
 // lie below each other, so that it fetches its channels' parameters (and divides for the quantizer's reciprocals) once
-// for kDown of them (4096 x 4096 along the last axis, a quantize / dequantize pair: 37 us; with two runs side by side 108).
+// for kDown of them (4096 x 4096 along the last axis, a bf16 pair: 22 us; element by element 66).
 enum Form { kOne, kRow, kAlong, kAny };
 constexpr int kThreads = 256;
 constexpr int kPerBlock = 4096;  // elements per workgroup of kOne and kRow: several runs in flight per thread
 constexpr int kDown = 8;         // rows per thread of kAlong
+// Threads that keep the chip busy: fewer runs per thread rather than fewer threads than that (kAlong: parameters fetched
+// for fewer rows at a time).
+constexpr int kFill = 1 << 20, kFillAlong = 1 << 18;
 struct QdqShape {
   int64_t total, outer, channels, inner;
+  uint32_t per;  // runs per thread of this launch, at most runs_per_thread: fewer where the tensor would leave the chip idle
 };
 template <Form F, int RUN> constexpr int runs_per_thread() { return F == kAlong ? kDown : kPerBlock / (kThreads * RUN); }
-// The thread's runs: first + u * stride, u < live (>= 1), and the channel of run u (kAlong: of every one).
+// The thread's runs, if it has any: first + u * stride, u < live (1 .. per), and the channel of run u (kAlong: of every one).
 template <Form F, int RUN>
 struct Runs {
   uint32_t first, stride, live;
+  bool any;
   __device__ __forceinline__ explicit Runs(const QdqShape& sh) {
-    constexpr uint32_t U = runs_per_thread<F, RUN>();
     if constexpr (F == kAlong) {
       const uint32_t per_row = (uint32_t)(sh.channels / RUN), rows = (uint32_t)sh.outer;
-      const uint32_t t = blockIdx.x * kThreads + threadIdx.x, down = t / per_row;  // (t < 2^32 / kDown)
-      const uint32_t row = down * U;
-      live = row < rows ? min(U, rows - row) : 0;
+      const uint32_t t = blockIdx.x * kThreads + threadIdx.x, down = t / per_row;
+      const uint32_t row = down * sh.per;
+      any = row < rows;
+      live = min(sh.per, rows - row);
       first = row * per_row + (t - down * per_row);
       stride = per_row;
     } else {
       const uint32_t runs = (uint32_t)(sh.total / RUN);
-      first = blockIdx.x * (kThreads * U) + threadIdx.x;
+      first = blockIdx.x * (kThreads * sh.per) + threadIdx.x;
       stride = kThreads;
-      live = first < runs ? min(U, (runs - first + kThreads - 1) / kThreads) : 0;
+      any = first < runs;
+      live = min(sh.per, (runs - first + kThreads - 1) / kThreads);
     }
   }
   __device__ __forceinline__ uint32_t run(uint32_t u) const { return first + min(u, live - 1) * stride; }  // (the end repeats the last)
@@ -95,6 +129,35 @@ struct Runs {
   }
 };
 
+// The parameters of a thread's runs: one channel's per run, or (kAlong) those of the channels of all of them.
+template <Form F, int RUN, int U>
+struct RunParams {
+  RawParams of[F == kAlong ? 1 : U];
+  RawAlong<RUN> along;
+  __device__ __forceinline__ RunParams(const QdqParams& p, const QdqShape& sh, const Runs<F, RUN>& at) {
+    if constexpr (F == kAlong) {
+      along.request(p, at.channel(sh, at.first));
+    } else {
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        if (u >= sh.per) break;
+        of[u] = qdq_request(p, at.channel(sh, at.run(u)));
+      }
+    }
+  }
+};
+
+// kAny: an element's channel (64-bit divisions, over a hundred instructions, only for tensors that need them) and its
+// zero point.
+__device__ __forceinline__ uint32_t element_channel(const QdqShape& sh, int64_t t) {
+  if (sh.total <= 0xffffffffLL) return (uint32_t)t / (uint32_t)sh.inner % (uint32_t)sh.channels;
+  return (uint32_t)((t / sh.inner) % sh.channels);
+}
+__device__ __forceinline__ int element_zp(const QdqParams& p, uint32_t c) {
+  if (!p.zp) return 0;
+  return ((const int32_t*)p.zp)[(size_t)c << p.zp64];
+}
+
 // Quantize; vector forms: runs of 8, 16-byte aligned x, 8-byte aligned q, 1-byte q, total / 8 < 2^32.
 // NT: streaming loads of x.
 template <int XT, Form F, bool NT>
@@ -104,29 +167,28 @@ qdq_quantize_kernel(const void* __restrict__ x, void* __restrict__ q, QdqParams 
   if constexpr (F != kAny) {
     constexpr int RUN = 8, U = runs_per_thread<F, RUN>();
     const Runs<F, RUN> at(sh);
-    if (at.live == 0) return;
+    if (!at.any) return;
     constexpr int D = XT == XLA_AMD_DT_F32 ? 2 : 1;
+    const RunParams<F, RUN, U> par(p, sh, at);
     i32x4 raw[U][D];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (uint32_t u = 0; u < U; ++u) {
+      if (u >= sh.per) break;
       const i32x4* const from = (const i32x4*)x + (size_t)at.run(u) * D;
 #pragma unroll
       for (int d = 0; d < D; ++d) raw[u][d] = NT ? __builtin_nontemporal_load(from + d) : from[d];
     }
     float isv[RUN], zv[RUN];
     if constexpr (F == kAlong) {
-      const uint32_t c = at.channel(sh, at.first);
 #pragma unroll
-      for (int i = 0; i < RUN; ++i) { isv[i] = qdq_scale(p, c + i); zv[i] = (float)qdq_zp(p, c + i); }
+      for (int i = 0; i < RUN; ++i) { isv[i] = par.along.scale_of(p, i); zv[i] = (float)par.along.zp_of(p, i); }
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (uint32_t u = 0; u < U; ++u) {
+      if (u >= sh.per) break;
       const uint32_t run = at.run(u);
       float is = 0.f, z = 0.f;
-      if constexpr (F != kAlong) {
-        const uint32_t c = at.channel(sh, run);
-        is = qdq_scale(p, c); z = (float)qdq_zp(p, c);
-      }
+      if constexpr (F != kAlong) { is = qdq_scale(p, par.of[u]); z = (float)par.of[u].zp; }
       uint32_t out[2] = {0, 0};
 #pragma unroll
       for (int i = 0; i < RUN; ++i) {
@@ -145,8 +207,8 @@ qdq_quantize_kernel(const void* __restrict__ x, void* __restrict__ q, QdqParams 
   } else {
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (t >= sh.total) return;
-    const uint32_t c = (uint32_t)((t / sh.inner) % sh.channels);
-    qdq_store_q(q, t, quantize_value(qmm_load(x, t, XT), qdq_scale(p, c), (float)qdq_zp(p, c), qmin, qmax), q_dt);
+    const uint32_t c = element_channel(sh, t);
+    qdq_store_q(q, t, quantize_value(qmm_load(x, t, XT), qdq_factor(p, qmm_load(p.scale, c, p.scale_dt)), (float)element_zp(p, c), qmin, qmax), q_dt);
   }
 }
 
@@ -170,10 +232,12 @@ qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, QdqPar
   if constexpr (F != kAny) {
     constexpr int RUN = OT == XLA_AMD_DT_F32 ? 4 : 8, U = runs_per_thread<F, RUN>();
     const Runs<F, RUN> at(sh);
-    if (at.live == 0) return;
+    if (!at.any) return;
+    const RunParams<F, RUN, U> par(p, sh, at);
     uint32_t raw[U][RUN / 4];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (uint32_t u = 0; u < U; ++u) {
+      if (u >= sh.per) break;
       const uint32_t run = at.run(u);
       if constexpr (RUN == 4) {
         raw[u][0] = ((const uint32_t*)q)[run];
@@ -185,19 +249,16 @@ qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, QdqPar
     float scv[RUN];
     int zv[RUN];
     if constexpr (F == kAlong) {
-      const uint32_t c = at.channel(sh, at.first);
 #pragma unroll
-      for (int i = 0; i < RUN; ++i) { scv[i] = qdq_scale(p, c + i); zv[i] = qdq_zp(p, c + i); }
+      for (int i = 0; i < RUN; ++i) { scv[i] = par.along.scale_of(p, i); zv[i] = par.along.zp_of(p, i); }
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (uint32_t u = 0; u < U; ++u) {
+      if (u >= sh.per) break;
       const uint32_t run = at.run(u);
       float sc = 0.f;
       int z = 0;
-      if constexpr (F != kAlong) {
-        const uint32_t c = at.channel(sh, run);
-        sc = qdq_scale(p, c); z = qdq_zp(p, c);
-      }
+      if constexpr (F != kAlong) { sc = qdq_scale(p, par.of[u]); z = par.of[u].zp; }
       float r[RUN];
 #pragma unroll
       for (int i = 0; i < RUN; ++i) {
@@ -222,8 +283,8 @@ qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, QdqPar
   } else {
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (t >= sh.total) return;
-    const uint32_t c = (uint32_t)((t / sh.inner) % sh.channels);
-    qmm_store(out, t, dequantize_value(qdq_load_q(q, t, q_dt), qdq_zp(p, c), qdq_scale(p, c), OT, int_subtract), OT);
+    const uint32_t c = element_channel(sh, t);
+    qmm_store(out, t, dequantize_value(qdq_load_q(q, t, q_dt), element_zp(p, c), qdq_factor(p, qmm_load(p.scale, c, p.scale_dt)), OT, int_subtract), OT);
   }
 }
 
@@ -240,17 +301,24 @@ Form choose_form(const QdqShape& sh, int run, bool aligned) {
   if (!aligned || sh.total % run != 0 || sh.total / run > 0xffffffffLL - kPerBlock || sh.channels > 0x7fffffffLL) return kAny;
   if (sh.channels == 1) return kOne;
   if (sh.inner % run == 0 && sh.inner / run <= 0x7fffffffLL) return kRow;
-  if (sh.inner == 1 && sh.channels % run == 0 && sh.outer <= 0x7fffffffLL) return kAlong;
+  // (one row has nothing to share, and below 256 K elements a thread's eight channels take longer than eight threads:
+  // a bf16 pair over 1 x 16.8 M 77 us element by element, 94 so, over 8 x 14336 4.8, 5.8)
+  if (sh.inner == 1 && sh.channels % run == 0 && sh.outer > 1 && sh.outer <= 0x7fffffffLL && sh.total >= (1 << 18)) return kAlong;
   return kAny;
 }
 
-// Calls go(form constant, grid) for runs of `run` elements; returns the launch's status.
+// Calls go(form constant, grid) for runs of `run` elements; returns the launch's status.  Sets sh.per.
 template <class Go>
-int launch_form(Form f, const QdqShape& sh, int run, const char* what, Go&& go) {
-  int64_t threads = sh.total, per = kThreads;
-  if (f == kAlong) threads = (sh.outer + kDown - 1) / kDown * (sh.channels / run);
-  else if (f != kAny) per = kPerBlock;
-  const int64_t blocks = (threads + per - 1) / per;
+int launch_form(Form f, QdqShape& sh, int run, const char* what, Go&& go) {
+  auto threads = [&](int64_t per) -> int64_t {
+    if (f == kAny) return sh.total;
+    return f == kAlong ? (sh.outer + per - 1) / per * (sh.channels / run) : (sh.total / run + per - 1) / per;
+  };
+  sh.per = f == kAny ? 1 : f == kAlong ? kDown : kPerBlock / (kThreads * run);
+  while (sh.per > 1 && threads(sh.per) < (f == kAlong ? kFillAlong : kFill)) sh.per /= 2;
+  // (a workgroup of kOne and kRow covers 256 per runs side by side)
+  const int64_t blocks = f == kOne || f == kRow ? (sh.total / run + kThreads * sh.per - 1) / (kThreads * sh.per)
+                                                : (threads(sh.per) + kThreads - 1) / kThreads;
   if (blocks > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "%s: tensor too large", what);
   const dim3 grid((unsigned)blocks);
   switch (f) {
@@ -268,7 +336,7 @@ int quantize(const char* what, const void* x, void* q, const QdqParams& p, int64
   if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad sizes", what);
   if (!qmm_valid_dt(x_dt) || !qmm_valid_dt(p.scale_dt) || !valid_qdt(q_dt) || qmin > qmax)
     return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum or bounds", what);
-  const QdqShape sh = {outer * channels * inner, outer, channels, inner};
+  QdqShape sh = {outer * channels * inner, outer, channels, inner, 1};
   if (sh.total == 0) return XLA_AMD_QMM_OK;
   const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)q & 7) == 0);
   const bool nt = sh.total * qmm_dt_size(x_dt) > kStreamIn;
@@ -289,7 +357,7 @@ int dequantize(const char* what, const void* q, void* out, const QdqParams& p, i
   if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad sizes", what);
   if (!qmm_valid_dt(out_dt) || !qmm_valid_dt(p.scale_dt) || !valid_qdt(q_dt))
     return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum", what);
-  const QdqShape sh = {outer * channels * inner, outer, channels, inner};
+  QdqShape sh = {outer * channels * inner, outer, channels, inner, 1};
   if (sh.total == 0) return XLA_AMD_QMM_OK;
   const int run = out_dt == XLA_AMD_DT_F32 ? 4 : 8;
   const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)q & (run - 1)) == 0) && (((uintptr_t)out & 15) == 0);
