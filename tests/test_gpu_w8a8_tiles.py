@@ -66,3 +66,16 @@ def test_quantizer_thread_counts(ops, dtype):
       qw, sw = ops._quantize_tensor(x)
       assert torch.equal(q.cpu(), qw) and torch.equal(s.cpu(), sw), (dtype, m, k)
       assert torch.equal(xsum.cpu(), qw.int().sum(-1, dtype=torch.int32))
+
+
+# many rows of up to 6144 (f32: 4096) elements take 256 threads: either side of where
+@pytest.mark.parametrize("dtype,k,rows", [(torch.bfloat16, 4104, (767, 768)), (torch.float16, 6144, (768,)), (torch.bfloat16, 6152, (768,)),
+                                          (torch.float32, 2056, (1535, 1536)), (torch.float32, 4096, (1536,))])
+def test_quantizer_many_rows(ops, dtype, k, rows):
+  for m in rows:
+    x = (torch.randn(m, k, generator=torch.Generator().manual_seed(k + m)) * 3).to(dtype)
+    x[0, k - 1], x[m - 1, 0] = 50.0, -60.0
+    q, s, xsum = ops.quantize_per_token_gpu(x.cuda(), want_sum=True)
+    qw, sw = ops._quantize_tensor(x)
+    assert torch.equal(q.cpu(), qw) and torch.equal(s.cpu(), sw)
+    assert torch.equal(xsum.cpu(), qw.int().sum(-1, dtype=torch.int32))

@@ -189,10 +189,14 @@ qmm_quantize_kernel(const void* __restrict__ x, int8_t* __restrict__ xq, void* _
 }
 
 // Threads per row: the launch lasts as long as one row's chain (load, abs-max, quantize) when there are few rows, and
-// rows of many elements per thread make that chain long, so long rows get more threads.  Per launch in a graph, bf16,
-// with 256 / 512 / 1024 threads: 1 x 14336 7.0 / 4.8 / 3.9 us, 512 x 14336 10.2 / 8.1 / 8.1, 4096 x 14336 45 / 39 / 43,
-// 512 x 8192 6.5 / 5.7 / 8.2, 4096 x 8192 24.7 / 23.3 / 47, 512 x 4096 4.1 / 4.9 / 5.6; f32, whose rows take twice the
-// loads: 512 x 4096 4.9 / 4.5 / 4.9, 512 x 2048 3.4 / 3.4 / 4.1.
+// rows of many elements per thread make that chain long, so rows of up to 16384 elements get more threads the longer they
+// are.  Per launch in a graph, bf16, with 256 / 512 / 1024 threads: 1 x 14336 7.0 / 4.8 / 3.9 us, 512 x 14336
+// 10.2 / 8.1 / 8.1, 4096 x 14336 45 / 39 / 43, 512 x 8192 6.5 / 5.7 / 8.2, 4096 x 8192 24.7 / 23.3 / 47, 512 x 4096
+// 4.1 / 4.9 / 5.6; f32, whose rows take twice the loads: 512 x 4096 4.9 / 4.5 / 4.9, 512 x 2048 3.4 / 3.4 / 4.1.
+// With many rows the chip is full anyway and 256 threads with more elements each are faster, bf16 up to 6144 elements from
+// 768 rows on (256 / 512: 1024 x 5120 6.1 / 6.5, 2048 x 4104 8.6 / 9.5, 4096 x 6144 18.3 / 18.9, but 512 x 5120 5.2 / 4.7
+// and 4096 x 8192 above), f32 up to 4096 from 1536 on (2048 x 3072 7.9 / 8.7, 2048 x 4096 10.1 / 10.6; 1024 x 3072 5.3 / 5.3).
+// Longer rows (18944: 11 us for one, 13.7 for 512) are read twice by 256 threads.
 template <int XT>
 int launch(const void* x, int8_t* xq, void* x_scale, int32_t* x_sum, int64_t M, int64_t K,
            int scale_out_dt, int policy, bool vec, hipStream_t stream) {
@@ -202,8 +206,11 @@ int launch(const void* x, int8_t* xq, void* x_scale, int32_t* x_sum, int64_t M, 
   constexpr int kShort = XT == XLA_AMD_DT_F32 ? 2048 : 4096;
   if (!vec) go(qmm_quantize_kernel<XT, 1, 0, 256>, 256);
   else if (K <= kShort) go(qmm_quantize_kernel<XT, 8, kShort / 2048, 256>, 256);
-  else if (K <= 4096) go(qmm_quantize_kernel<XT, 8, 1, 512>, 512);
-  else if (K <= 8192) go(qmm_quantize_kernel<XT, 8, 2, 512>, 512);
+  else if (K <= 4096) {
+    if constexpr (XT == XLA_AMD_DT_F32) M < 1536 ? go(qmm_quantize_kernel<XT, 8, 1, 512>, 512) : go(qmm_quantize_kernel<XT, 8, 2, 256>, 256);
+  } else if (XT != XLA_AMD_DT_F32 && M >= 768 && K <= 6144) {
+    if constexpr (XT != XLA_AMD_DT_F32) go(qmm_quantize_kernel<XT, 8, 4, 256>, 256);
+  } else if (K <= 8192) go(qmm_quantize_kernel<XT, 8, 2, 512>, 512);
   else if (K <= 16384 && M <= 256) go(qmm_quantize_kernel<XT, 8, 2, 1024>, 1024);
   else if (K <= 16384) go(qmm_quantize_kernel<XT, 8, 4, 512>, 512);
   else go(qmm_quantize_kernel<XT, 8, 0, 256>, 256);
