@@ -112,3 +112,13 @@ def test_w8a8_tile_reported_is_the_tile_launched(tmp_path):
   calls = [rec.w8a8(m, n, k, bm, bn) for bm, bn in TILES[:-1] for m, n, k in ((512, 4096, 4096), (10, 100, 128), (200, 4096, 14336))]
   for call, (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
     assert rc == 0 and [_tile(l) for l in launches] == [tuple(call[2][-3:-1])], call
+
+
+def test_quantizer_rows_of_any_number(tmp_path):
+  """A grid holds fewer than 2^32 threads, whatever number of them a row gets."""
+  sizes = [(m, k) for m in ((1 << 23) - 1, 1 << 23, (1 << 24) - 1) for k in (2056, 4096, 4104, 8192, 8200, 16384, 16392, 4099)]
+  calls = [("xla_amd_qmm_quantize_per_token", "pppp" + "qq" + "iii" + "p", [rec.PTR, rec.PTR, rec.PTR, 0, m, k, dt, dt, 0, 0])
+           for m, k in sizes for dt in (0, 1, 2)]
+  for call, (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0 and len(launches) == 1, (call, text)
+    assert launches[0].grid[0] * launches[0].block[0] < 1 << 32, (call, launches[0])

@@ -196,7 +196,8 @@ qmm_quantize_kernel(const void* __restrict__ x, int8_t* __restrict__ xq, void* _
 // With many rows the chip is full anyway and 256 threads with more elements each are faster, bf16 up to 6144 elements from
 // 768 rows on (256 / 512: 1024 x 5120 6.1 / 6.5, 2048 x 4104 8.6 / 9.5, 4096 x 6144 18.3 / 18.9, but 512 x 5120 5.2 / 4.7
 // and 4096 x 8192 above), f32 up to 4096 from 1536 on (2048 x 3072 7.9 / 8.7, 2048 x 4096 10.1 / 10.6; 1024 x 3072 5.3 / 5.3).
-// Longer rows (18944: 11 us for one, 13.7 for 512) are read twice by 256 threads.
+// Longer rows (18944: 11 us for one, 13.7 for 512) are read twice by 256 threads, and so are rows too many for a grid of
+// 512 threads each (2^32 threads at most).
 template <int XT>
 int launch(const void* x, int8_t* xq, void* x_scale, int32_t* x_sum, int64_t M, int64_t K,
            int scale_out_dt, int policy, bool vec, hipStream_t stream) {
@@ -206,6 +207,7 @@ int launch(const void* x, int8_t* xq, void* x_scale, int32_t* x_sum, int64_t M, 
   constexpr int kShort = XT == XLA_AMD_DT_F32 ? 2048 : 4096;
   if (!vec) go(qmm_quantize_kernel<XT, 1, 0, 256>, 256);
   else if (K <= kShort) go(qmm_quantize_kernel<XT, 8, kShort / 2048, 256>, 256);
+  else if (M >= (1 << 23)) go(qmm_quantize_kernel<XT, 8, 0, 256>, 256);
   else if (K <= 4096) {
     if constexpr (XT == XLA_AMD_DT_F32) M < 1536 ? go(qmm_quantize_kernel<XT, 8, 1, 512>, 512) : go(qmm_quantize_kernel<XT, 8, 2, 256>, 256);
   } else if (XT != XLA_AMD_DT_F32 && M >= 768 && K <= 6144) {
