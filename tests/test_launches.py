@@ -122,3 +122,25 @@ def test_quantizer_rows_of_any_number(tmp_path):
   for call, (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
     assert rc == 0 and len(launches) == 1, (call, text)
     assert launches[0].grid[0] * launches[0].block[0] < 1 << 32, (call, launches[0])
+
+
+@pytest.mark.parametrize("name,out_size", [("quantize", 1), ("dequantize", 4)])
+def test_quantize_tensors_of_any_size(tmp_path, name, out_size):
+  """More elements than 32-bit runs and one grid reach (an f32 result of more than 2^34 elements): pieces that follow
+  each other, whichever dimension they are cut along."""
+  sizes = [(1, 1, (1 << 34) + 8), (3, 1, 3 << 33), (1, 5, 7 << 32), (5, 3, (1 << 31) + 64), (1, (1 << 20) + 3, 32768)]
+  calls = []
+  for o, c, i in sizes:
+    if name == "quantize":
+      calls.append(("xla_amd_qmm_quantize_affine", "pppp" + "qqq" + "iiii" + "p", [rec.PTR, rec.PTR, rec.PTR, rec.PTR, o, c, i, 0, 0, -128, 127, 0]))
+    else:
+      calls.append(("xla_amd_qmm_dequantize_affine", "pppp" + "qqq" + "iii" + "p", [rec.PTR, rec.PTR, rec.PTR, rec.PTR, o, c, i, 0, 0, 1, 0]))
+  in_size = 4 if name == "quantize" else 1
+  for (o, c, i), (rc, text, launches) in zip(sizes, rec.record(calls, str(tmp_path))):
+    assert rc == 0 and launches, text
+    starts = [(l.args[0] - rec.PTR) // in_size for l in launches]
+    assert starts[0] == 0 and starts == sorted(starts)
+    for l, at, end in zip(launches, starts, starts[1:] + [o * c * i]):
+      # a vector form, whose workgroups cover 4096 elements, or 2048 or 1024 of a short last piece
+      assert "FormE3" not in l.name and l.grid[0] * l.block[0] < 1 << 32
+      assert any(l.grid[0] == -(-(end - at) // n) for n in (4096, 2048, 1024)), (l, at, end)

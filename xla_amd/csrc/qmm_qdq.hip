@@ -288,6 +288,7 @@ qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, QdqPar
   }
 }
 
+int qdt_size(int q_dt) { return q_dt == XLA_AMD_QDT_I16 ? 2 : q_dt == XLA_AMD_QDT_I32 ? 4 : 1; }
 bool valid_qdt(int q_dt) { return q_dt >= XLA_AMD_QDT_I8 && q_dt <= XLA_AMD_QDT_I32; }
 
 // Tensors that pass through the 256 MB Infinity Cache without staying in it are streamed past it, so that the other
@@ -330,6 +331,30 @@ int launch_form(Form f, QdqShape& sh, int run, const char* what, Go&& go) {
   return QMM_CHECK_LAUNCH(what);
 }
 
+// Tensors of more elements than this go in pieces, which keeps runs and grids within 32 bits (and far from their cost).
+constexpr int64_t kPiece = 1ll << 33;
+
+// Calls piece(outer, channels, inner, parameters, first element) for a tensor of more than kPiece elements, cut along its
+// first dimension of more than one entry; a piece may still be too large, along the next one.
+template <class Piece>
+int in_pieces(const QdqParams& p, int64_t outer, int64_t channels, int64_t inner, Piece&& piece) {
+  if (channels == 1) { inner *= outer; outer = 1; }
+  int64_t& cut = outer > 1 ? outer : channels > 1 ? channels : inner;
+  const int64_t all = cut, rest = outer * channels * inner / all, most = kPiece / rest > 0 ? kPiece / rest : 1;
+  const bool along = &cut == &channels;
+  for (int64_t at = 0; at < all; at += most) {
+    cut = all - at < most ? all - at : most;
+    QdqParams pp = p;
+    if (along) {
+      pp.scale = (const char*)p.scale + at * qmm_dt_size(p.scale_dt);
+      if (p.zp) pp.zp = (const char*)p.zp + at * (p.zp64 ? 8 : 4);
+    }
+    const int rc = piece(outer, channels, inner, pp, at * rest);
+    if (rc != XLA_AMD_QMM_OK) return rc;
+  }
+  return XLA_AMD_QMM_OK;
+}
+
 int quantize(const char* what, const void* x, void* q, const QdqParams& p, int64_t outer, int64_t channels,
              int64_t inner, int x_dt, int q_dt, int32_t qmin, int32_t qmax, void* stream) {
   if (!x || !q || !p.scale || !p.zp) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: null pointer", what);
@@ -338,6 +363,10 @@ int quantize(const char* what, const void* x, void* q, const QdqParams& p, int64
     return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum or bounds", what);
   QdqShape sh = {outer * channels * inner, outer, channels, inner, 1};
   if (sh.total == 0) return XLA_AMD_QMM_OK;
+  if (sh.total > kPiece)
+    return in_pieces(p, outer, channels, inner, [&](int64_t o, int64_t c, int64_t i, const QdqParams& pp, int64_t first) {
+      return quantize(what, (const char*)x + first * qmm_dt_size(x_dt), (char*)q + first * qdt_size(q_dt), pp, o, c, i, x_dt, q_dt, qmin, qmax, stream);
+    });
   const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)q & 7) == 0);
   const bool nt = sh.total * qmm_dt_size(x_dt) > kStreamIn;
   return launch_form(choose_form(sh, 8, aligned), sh, 8, what, [&](auto fc, dim3 grid) {
@@ -359,6 +388,10 @@ int dequantize(const char* what, const void* q, void* out, const QdqParams& p, i
     return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum", what);
   QdqShape sh = {outer * channels * inner, outer, channels, inner, 1};
   if (sh.total == 0) return XLA_AMD_QMM_OK;
+  if (sh.total > kPiece)
+    return in_pieces(p, outer, channels, inner, [&](int64_t o, int64_t c, int64_t i, const QdqParams& pp, int64_t first) {
+      return dequantize(what, (const char*)q + first * qdt_size(q_dt), (char*)out + first * qmm_dt_size(out_dt), pp, o, c, i, q_dt, out_dt, int_subtract, stream);
+    });
   const int run = out_dt == XLA_AMD_DT_F32 ? 4 : 8;
   const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)q & (run - 1)) == 0) && (((uintptr_t)out & 15) == 0);
   const bool nt = sh.total * qmm_dt_size(out_dt) > kStreamOut;
