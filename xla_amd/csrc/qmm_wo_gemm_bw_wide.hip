@@ -53,10 +53,11 @@ struct BwItem {
   int m0, n0, rows;
 };
 
-// BLK1: quantization blocks of 128 columns, one per step.
+// BLK1: quantization blocks of 128 columns, one per step.  With a zero point there is no other form.
 template <int XT, int BITS, bool HASZP, bool BLK1>
 __global__ void __launch_bounds__((kComputeWaves + kCopyWaves) * 64)
 qmm_wo_bw_wide_kernel(WoBwArgs a) {
+  static_assert(BLK1 || !HASZP, "zero points: one block per step");
   constexpr bool NEEDXS = HASZP || BITS == 4;        // sums of x: zero point, int4 affine map
   constexpr int BLK = BITS == 8 ? 2048 : 1024;       // bytes of one weight block (16 channels x 128 columns)
   constexpr int WL = BITS == 8 ? 2 : 1;              // 16-byte loads per lane and block
@@ -87,8 +88,7 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
     // ---- copying waves: chunk after chunk of x (and its scales, zero points and sums) into the two slots in turn.
     // Wave cw copies the rows 16 cw .. 16 cw + 15 and sums what it has copied itself.
     const int cw = wave - kComputeWaves;
-    float blk_xs = 0.f;  // sum of x of row 16 cw + r over the current quantization block so far
-    int blk = 0, left = sub;  // that block, and its steps that are still to come
+    int blk = 0;  // current step of the item, which with a zero point is a quantization block
     // one entry (the workgroup's channels of row `at` of a [K/C, N] tensor): 4 bytes (two channels) per lane
     auto copy_entry = [&](const void* from, int at, int n0, char* to) __attribute__((always_inline)) {
 #pragma unroll
@@ -101,14 +101,13 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
     auto chunk_load = [&](const BwItem& w, int c, int slot_i, int zg0) __attribute__((always_inline)) {
       const int s0 = c * CS;
       const int nst = min(CS, steps - s0);
-      // step s0 + cw: its scales, and the zero points of the block that begins with it
+      // step s0 + cw: its scales, and zero points
       static_assert(CS == kCopyWaves, "one step's entries per copying wave");
       if (cw < nst) {
         const int at = (s0 + cw) / sub;
         copy_entry(a.scale, at, w.n0, smem + (slot_i * CS + cw) * kEntry);
         if constexpr (HASZP)
-          if (at * sub == s0 + cw)
-            copy_entry(a.zp, at, w.n0, smem + kZent + (((zg0 + at / kZBlocks) & 1) * kZBlocks + at % kZBlocks) * kEntry);
+          copy_entry(a.zp, at, w.n0, smem + kZent + (((zg0 + at / kZBlocks) & 1) * kZBlocks + at % kZBlocks) * kEntry);
       }
       char* const slot = xsm + slot_i * (CS * X_TILE);
       const char* const xb = (const char*)a.x + (size_t)w.m0 * K * 2;
@@ -128,7 +127,7 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if constexpr (NEEDXS) {
-        if (c == 0) { blk = 0; left = sub; blk_xs = 0.f; }
+        if (c == 0) blk = 0;
         for (int t = 0; t < nst; ++t) {
           const char* xrow = slot + t * X_TILE + (16 * cw + r) * 256;
           f32x4 xs = {0, 0, 0, 0};
@@ -141,15 +140,10 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
             if (g == 0) *(f32x4*)(smem + kXsq + ((slot_i * CS + t) * BM + 16 * cw + r) * 16) = f32x4{q, q, q, q};
           }
           if constexpr (HASZP) {
-            blk_xs = BLK1 ? s : blk_xs + s;
-            if (--left == 0) {
-              const uint16_t v = XT == XLA_AMD_DT_BF16 ? qmm_f32_to_bf16(blk_xs) : qmm_f32_to_f16(blk_xs);
-              if (g == 0)
-                *(uint16_t*)(smem + kZx + ((((zg0 + blk / kZBlocks) & 1) * BM + 16 * cw + r) * kZBlocks + blk % kZBlocks) * 2) = v;
-              ++blk;
-              left = sub;
-              blk_xs = 0.f;
-            }
+            const uint16_t v = XT == XLA_AMD_DT_BF16 ? qmm_f32_to_bf16(s) : qmm_f32_to_f16(s);
+            if (g == 0)
+              *(uint16_t*)(smem + kZx + ((((zg0 + blk / kZBlocks) & 1) * BM + 16 * cw + r) * kZBlocks + blk % kZBlocks) * 2) = v;
+            ++blk;
           }
         }
       }

@@ -31,8 +31,9 @@ namespace {
 using at::Tensor;
 typedef std::optional<Tensor> OptTensor;
 
-// Dispatch decisions since the library was loaded, in the order of the Python module's `counters`.
-enum Counter { kSkinny, kWoGemm, kGeneric, kW8a8, kW8a8Generic, kPack, kPackHit, kCounters };
+// Dispatch decisions since the library was loaded, in the order of the Python module's `counters` (whose last, the copies
+// made, happen in Python only).
+enum Counter { kSkinny, kWoGemm, kGeneric, kW8a8, kW8a8Generic, kPackHit, kCounters };
 std::atomic<int64_t> g_counters[kCounters];
 void count(Counter c) { g_counters[c].fetch_add(1, std::memory_order_relaxed); }
 

@@ -38,7 +38,7 @@ def _overflow_policy() -> str:
 class _Counters(collections.abc.MutableMapping):
   """Calls counted here plus those the native operators counted."""
 
-  _NAMES = ("skinny_mfma", "wo_gemm", "generic", "w8a8_mfma", "w8a8_generic", "pack", "pack_hit")  # the native order
+  _NAMES = ("skinny_mfma", "wo_gemm", "generic", "w8a8_mfma", "w8a8_generic", "pack_hit", "pack")  # the native order
 
   def __init__(self):
     self._here = dict.fromkeys(self._NAMES, 0)
