@@ -86,21 +86,21 @@ struct RawAlong {
 // What bounds the vector forms is memory alone as long as a run's channel costs few instructions: 32-bit divisions by
 // the row length (the 64-bit ones of kAny take over a hundred instructions), none for kOne; in kAlong a thread's runs
 // lie below each other, so that it fetches its channels' parameters (and divides for the quantizer's reciprocals) once
-// for kDown of them (4096 x 4096 along the last axis, a bf16 pair: 22 us; element by element 66).
+// for kDown of them (4096 x 4096 along the last axis, a bf16 pair: 20 us; element by element 67).
 enum Form { kOne, kRow, kAlong, kAny };
 constexpr int kThreads = 256;
 constexpr int kPerBlock = 4096;  // elements per workgroup of kOne and kRow: several runs in flight per thread
 constexpr int kDown = 8;         // rows per thread of kAlong
-// Threads that keep the chip busy: fewer runs per thread rather than fewer threads than that (kAlong: parameters fetched
-// for fewer rows at a time).
-constexpr int kFill = 1 << 20, kFillAlong = 1 << 18;
+// Workgroups that keep the chip busy: one run per thread rather than fewer workgroups than that (kAlong, where a run then
+// fetches its channels' parameters by itself, a few less).
+constexpr int kFill = 4096, kFillAlong = 512;
 struct QdqShape {
   int64_t total, outer, channels, inner;
-  uint32_t per;  // runs per thread of this launch, at most runs_per_thread: fewer where the tensor would leave the chip idle
 };
-template <Form F, int RUN> constexpr int runs_per_thread() { return F == kAlong ? kDown : kPerBlock / (kThreads * RUN); }
-// The thread's runs, if it has any: first + u * stride, u < live (1 .. per), and the channel of run u (kAlong: of every one).
-template <Form F, int RUN>
+// Runs per thread: one where more would leave the chip idle (FEW).
+template <Form F, int RUN, bool FEW> constexpr int runs_per_thread() { return FEW ? 1 : F == kAlong ? kDown : kPerBlock / (kThreads * RUN); }
+// The thread's runs, if it has any: first + u * stride, u < live (1 .. U), and the channel of run u (kAlong: of every one).
+template <Form F, int RUN, uint32_t U>
 struct Runs {
   uint32_t first, stride, live;
   bool any;
@@ -108,17 +108,17 @@ struct Runs {
     if constexpr (F == kAlong) {
       const uint32_t per_row = (uint32_t)(sh.channels / RUN), rows = (uint32_t)sh.outer;
       const uint32_t t = blockIdx.x * kThreads + threadIdx.x, down = t / per_row;
-      const uint32_t row = down * sh.per;
+      const uint32_t row = down * U;
       any = row < rows;
-      live = min(sh.per, rows - row);
+      live = min(U, rows - row);
       first = row * per_row + (t - down * per_row);
       stride = per_row;
     } else {
       const uint32_t runs = (uint32_t)(sh.total / RUN);
-      first = blockIdx.x * (kThreads * sh.per) + threadIdx.x;
+      first = blockIdx.x * (kThreads * U) + threadIdx.x;
       stride = kThreads;
       any = first < runs;
-      live = min(sh.per, (runs - first + kThreads - 1) / kThreads);
+      live = min(U, (runs - first + kThreads - 1) / kThreads);
     }
   }
   __device__ __forceinline__ uint32_t run(uint32_t u) const { return first + min(u, live - 1) * stride; }  // (the end repeats the last)
@@ -134,15 +134,12 @@ template <Form F, int RUN, int U>
 struct RunParams {
   RawParams of[F == kAlong ? 1 : U];
   RawAlong<RUN> along;
-  __device__ __forceinline__ RunParams(const QdqParams& p, const QdqShape& sh, const Runs<F, RUN>& at) {
+  __device__ __forceinline__ RunParams(const QdqParams& p, const QdqShape& sh, const Runs<F, RUN, U>& at) {
     if constexpr (F == kAlong) {
       along.request(p, at.channel(sh, at.first));
     } else {
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u) {
-        if (u >= sh.per) break;
-        of[u] = qdq_request(p, at.channel(sh, at.run(u)));
-      }
+      for (int u = 0; u < U; ++u) of[u] = qdq_request(p, at.channel(sh, at.run(u)));
     }
   }
 };
@@ -160,20 +157,19 @@ __device__ __forceinline__ int element_zp(const QdqParams& p, uint32_t c) {
 
 // Quantize; vector forms: runs of 8, 16-byte aligned x, 8-byte aligned q, 1-byte q, total / 8 < 2^32.
 // NT: streaming loads of x.
-template <int XT, Form F, bool NT>
+template <int XT, Form F, bool NT, bool FEW>
 __global__ void __launch_bounds__(kThreads)
 qdq_quantize_kernel(const void* __restrict__ x, void* __restrict__ q, QdqParams p, QdqShape sh, int q_dt, float qmin,
                     float qmax) {
   if constexpr (F != kAny) {
-    constexpr int RUN = 8, U = runs_per_thread<F, RUN>();
-    const Runs<F, RUN> at(sh);
+    constexpr int RUN = 8, U = runs_per_thread<F, RUN, FEW>();
+    const Runs<F, RUN, U> at(sh);
     if (!at.any) return;
     constexpr int D = XT == XLA_AMD_DT_F32 ? 2 : 1;
     const RunParams<F, RUN, U> par(p, sh, at);
     i32x4 raw[U][D];
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-      if (u >= sh.per) break;
+    for (int u = 0; u < U; ++u) {
       const i32x4* const from = (const i32x4*)x + (size_t)at.run(u) * D;
 #pragma unroll
       for (int d = 0; d < D; ++d) raw[u][d] = NT ? __builtin_nontemporal_load(from + d) : from[d];
@@ -184,8 +180,7 @@ qdq_quantize_kernel(const void* __restrict__ x, void* __restrict__ q, QdqParams 
       for (int i = 0; i < RUN; ++i) { isv[i] = par.along.scale_of(p, i); zv[i] = (float)par.along.zp_of(p, i); }
     }
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-      if (u >= sh.per) break;
+    for (int u = 0; u < U; ++u) {
       const uint32_t run = at.run(u);
       float is = 0.f, z = 0.f;
       if constexpr (F != kAlong) { is = qdq_scale(p, par.of[u]); z = (float)par.of[u].zp; }
@@ -225,19 +220,18 @@ __device__ __forceinline__ float dequantize_value(int qv, int z, float sc, int o
 // Dequantize; vector forms: runs of 4 (f32 out) or 8 (2-byte out), i.e. 16-byte stores, q aligned to a run, out to 16
 // bytes, 1-byte q, total / 4 < 2^32.
 // NT: streaming stores of out.  (A template: a branch around two forms of a store leaves the ordinary one.)
-template <int OT, Form F, bool NT>
+template <int OT, Form F, bool NT, bool FEW>
 __global__ void __launch_bounds__(kThreads)
 qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, QdqParams p, QdqShape sh, int q_dt,
                       int int_subtract) {
   if constexpr (F != kAny) {
-    constexpr int RUN = OT == XLA_AMD_DT_F32 ? 4 : 8, U = runs_per_thread<F, RUN>();
-    const Runs<F, RUN> at(sh);
+    constexpr int RUN = OT == XLA_AMD_DT_F32 ? 4 : 8, U = runs_per_thread<F, RUN, FEW>();
+    const Runs<F, RUN, U> at(sh);
     if (!at.any) return;
     const RunParams<F, RUN, U> par(p, sh, at);
     uint32_t raw[U][RUN / 4];
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-      if (u >= sh.per) break;
+    for (int u = 0; u < U; ++u) {
       const uint32_t run = at.run(u);
       if constexpr (RUN == 4) {
         raw[u][0] = ((const uint32_t*)q)[run];
@@ -253,8 +247,7 @@ qdq_dequantize_kernel(const void* __restrict__ q, void* __restrict__ out, QdqPar
       for (int i = 0; i < RUN; ++i) { scv[i] = par.along.scale_of(p, i); zv[i] = par.along.zp_of(p, i); }
     }
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-      if (u >= sh.per) break;
+    for (int u = 0; u < U; ++u) {
       const uint32_t run = at.run(u);
       float sc = 0.f;
       int z = 0;
@@ -308,25 +301,24 @@ Form choose_form(const QdqShape& sh, int run, bool aligned) {
   return kAny;
 }
 
-// Calls go(form constant, grid) for runs of `run` elements; returns the launch's status.  Sets sh.per.
+// Calls go(form constant, whether one run per thread, grid) for runs of `run` elements; returns the launch's status.
 template <class Go>
-int launch_form(Form f, QdqShape& sh, int run, const char* what, Go&& go) {
-  auto threads = [&](int64_t per) -> int64_t {
-    if (f == kAny) return sh.total;
-    return f == kAlong ? (sh.outer + per - 1) / per * (sh.channels / run) : (sh.total / run + per - 1) / per;
+int launch_form(Form f, const QdqShape& sh, int run, const char* what, Go&& go) {
+  auto blocks_of = [&](int64_t u) -> int64_t {  // ... with u runs per thread
+    if (f == kAny) return (sh.total + kThreads - 1) / kThreads;
+    if (f == kAlong) return ((sh.outer + u - 1) / u * (sh.channels / run) + kThreads - 1) / kThreads;
+    return (sh.total / run + kThreads * u - 1) / (kThreads * u);
   };
-  sh.per = f == kAny ? 1 : f == kAlong ? kDown : kPerBlock / (kThreads * run);
-  while (sh.per > 1 && threads(sh.per) < (f == kAlong ? kFillAlong : kFill)) sh.per /= 2;
-  // (a workgroup of kOne and kRow covers 256 per runs side by side)
-  const int64_t blocks = f == kOne || f == kRow ? (sh.total / run + kThreads * sh.per - 1) / (kThreads * sh.per)
-                                                : (threads(sh.per) + kThreads - 1) / kThreads;
+  const int64_t many = f == kAlong ? kDown : kPerBlock / (kThreads * run);
+  const bool few = blocks_of(many) < (f == kAlong ? kFillAlong : kFill);
+  const int64_t blocks = blocks_of(few ? 1 : many);
   if (blocks > 0x7fffffffLL) return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "%s: tensor too large", what);
   const dim3 grid((unsigned)blocks);
   switch (f) {
-    case kOne: go(qmm_const<kOne>{}, grid); break;
-    case kRow: go(qmm_const<kRow>{}, grid); break;
-    case kAlong: go(qmm_const<kAlong>{}, grid); break;
-    default: go(qmm_const<kAny>{}, grid); break;
+    case kOne: go(qmm_const<kOne>{}, few, grid); break;
+    case kRow: go(qmm_const<kRow>{}, few, grid); break;
+    case kAlong: go(qmm_const<kAlong>{}, few, grid); break;
+    default: go(qmm_const<kAny>{}, few, grid); break;
   }
   return QMM_CHECK_LAUNCH(what);
 }
@@ -361,7 +353,7 @@ int quantize(const char* what, const void* x, void* q, const QdqParams& p, int64
   if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad sizes", what);
   if (!qmm_valid_dt(x_dt) || !qmm_valid_dt(p.scale_dt) || !valid_qdt(q_dt) || qmin > qmax)
     return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum or bounds", what);
-  QdqShape sh = {outer * channels * inner, outer, channels, inner, 1};
+  const QdqShape sh = {outer * channels * inner, outer, channels, inner};
   if (sh.total == 0) return XLA_AMD_QMM_OK;
   if (sh.total > kPiece)
     return in_pieces(p, outer, channels, inner, [&](int64_t o, int64_t c, int64_t i, const QdqParams& pp, int64_t first) {
@@ -369,14 +361,21 @@ int quantize(const char* what, const void* x, void* q, const QdqParams& p, int64
     });
   const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)q & 7) == 0);
   const bool nt = sh.total * qmm_dt_size(x_dt) > kStreamIn;
-  return launch_form(choose_form(sh, 8, aligned), sh, 8, what, [&](auto fc, dim3 grid) {
+  return launch_form(choose_form(sh, 8, aligned), sh, 8, what, [&](auto fc, bool few, dim3 grid) {
     constexpr Form F = (Form)(int)fc;
+    constexpr bool V = F != kAny;  // (element by element there is one kernel)
     const auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, (hipStream_t)stream, x, q, p, sh, q_dt, (float)qmin, (float)qmax);
     };
-    if (x_dt == XLA_AMD_DT_BF16) nt ? go(qdq_quantize_kernel<XLA_AMD_DT_BF16, F, F != kAny>) : go(qdq_quantize_kernel<XLA_AMD_DT_BF16, F, false>);
-    else if (x_dt == XLA_AMD_DT_F16) nt ? go(qdq_quantize_kernel<XLA_AMD_DT_F16, F, F != kAny>) : go(qdq_quantize_kernel<XLA_AMD_DT_F16, F, false>);
-    else nt ? go(qdq_quantize_kernel<XLA_AMD_DT_F32, F, F != kAny>) : go(qdq_quantize_kernel<XLA_AMD_DT_F32, F, false>);
+    // (a tensor large enough to be streamed has many runs)
+    const auto pick = [&](auto dc) {
+      if (V && few) go(qdq_quantize_kernel<(int)dc, F, false, V>);
+      else if (nt) go(qdq_quantize_kernel<(int)dc, F, V, false>);
+      else go(qdq_quantize_kernel<(int)dc, F, false, false>);
+    };
+    if (x_dt == XLA_AMD_DT_BF16) pick(qmm_const<XLA_AMD_DT_BF16>{});
+    else if (x_dt == XLA_AMD_DT_F16) pick(qmm_const<XLA_AMD_DT_F16>{});
+    else pick(qmm_const<XLA_AMD_DT_F32>{});
   });
 }
 
@@ -386,7 +385,7 @@ int dequantize(const char* what, const void* q, void* out, const QdqParams& p, i
   if (outer < 0 || channels <= 0 || inner < 0) return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad sizes", what);
   if (!qmm_valid_dt(out_dt) || !qmm_valid_dt(p.scale_dt) || !valid_qdt(q_dt))
     return qmm_fail(XLA_AMD_QMM_EINVAL, "%s: bad dtype enum", what);
-  QdqShape sh = {outer * channels * inner, outer, channels, inner, 1};
+  const QdqShape sh = {outer * channels * inner, outer, channels, inner};
   if (sh.total == 0) return XLA_AMD_QMM_OK;
   if (sh.total > kPiece)
     return in_pieces(p, outer, channels, inner, [&](int64_t o, int64_t c, int64_t i, const QdqParams& pp, int64_t first) {
@@ -395,14 +394,20 @@ int dequantize(const char* what, const void* q, void* out, const QdqParams& p, i
   const int run = out_dt == XLA_AMD_DT_F32 ? 4 : 8;
   const bool aligned = (q_dt == XLA_AMD_QDT_I8 || q_dt == XLA_AMD_QDT_U8) && (((uintptr_t)q & (run - 1)) == 0) && (((uintptr_t)out & 15) == 0);
   const bool nt = sh.total * qmm_dt_size(out_dt) > kStreamOut;
-  return launch_form(choose_form(sh, run, aligned), sh, run, what, [&](auto fc, dim3 grid) {
+  return launch_form(choose_form(sh, run, aligned), sh, run, what, [&](auto fc, bool few, dim3 grid) {
     constexpr Form F = (Form)(int)fc;
+    constexpr bool V = F != kAny;  // (element by element there is one kernel)
     const auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, (hipStream_t)stream, q, out, p, sh, q_dt, int_subtract);
     };
-    if (out_dt == XLA_AMD_DT_BF16) nt ? go(qdq_dequantize_kernel<XLA_AMD_DT_BF16, F, F != kAny>) : go(qdq_dequantize_kernel<XLA_AMD_DT_BF16, F, false>);
-    else if (out_dt == XLA_AMD_DT_F16) nt ? go(qdq_dequantize_kernel<XLA_AMD_DT_F16, F, F != kAny>) : go(qdq_dequantize_kernel<XLA_AMD_DT_F16, F, false>);
-    else nt ? go(qdq_dequantize_kernel<XLA_AMD_DT_F32, F, F != kAny>) : go(qdq_dequantize_kernel<XLA_AMD_DT_F32, F, false>);
+    const auto pick = [&](auto dc) {
+      if (V && few) go(qdq_dequantize_kernel<(int)dc, F, false, V>);
+      else if (nt) go(qdq_dequantize_kernel<(int)dc, F, V, false>);
+      else go(qdq_dequantize_kernel<(int)dc, F, false, false>);
+    };
+    if (out_dt == XLA_AMD_DT_BF16) pick(qmm_const<XLA_AMD_DT_BF16>{});
+    else if (out_dt == XLA_AMD_DT_F16) pick(qmm_const<XLA_AMD_DT_F16>{});
+    else pick(qmm_const<XLA_AMD_DT_F32>{});
   });
 }
 
