@@ -144,3 +144,17 @@ def test_quantize_tensors_of_any_size(tmp_path, name, out_size):
       # a vector form, whose workgroups cover 4096 elements, or 2048 or 1024 of a short last piece
       assert "FormE3" not in l.name and l.grid[0] * l.block[0] < 1 << 32
       assert any(l.grid[0] == -(-(end - at) // n) for n in (4096, 2048, 1024)), (l, at, end)
+
+
+def test_wide_tile_tests_run_the_wide_kernel(tmp_path):
+  """The sizes tests/test_gpu_wo_bw_wide.py checks take the 64 x 256 tiles (the operator's counter does not tell them from
+  the 64 x 128 ones), and launches of few tiles, and zero points in any other form, do not."""
+  from tests.test_gpu_wo_bw_wide import test_wide_tiles
+  (_, sizes), = (m.args for m in test_wide_tiles.pytestmark if m.name == "parametrize" and m.args[0].startswith("m,n,k"))
+  wide = [(m, n, k, k if c == -1 else c, bits, asym) for m, n, k, c, bits, asym in sizes]
+  assert len(wide) >= 9
+  narrow = [(512, 4096, 4096, 128, 4, True), (100, 4096, 4096, 128, 4, False), (2048, 4096, 4096, 256, 4, True), (2048, 4096, 4096, 128, 8, True)]
+  calls = [rec.blockwise(*s, x_dt) for x_dt in (1, 2) for s in wide + narrow]
+  want = ["qmm_wo_bw_wide_kernel"] * len(wide) + ["qmm_wo_bw_gemm_kernel"] * len(narrow)
+  for call, kernel, (rc, text, launches) in zip(calls, want * 2, rec.record(calls, str(tmp_path))):
+    assert rc == 0 and len(launches) == 1 and kernel in launches[0].name, (call, text, launches)
