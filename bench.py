@@ -442,7 +442,7 @@ def main():
         "us": round(ev * 1e3, 2),
         "roofline": {"bound": "mfma", "achieved": round(f3 / ev / 1e9, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(f3 / ev / 1e9 / BF16_PEAK_TFLOPS, 4), "traffic": None,
-                     "kernel": "qmm_wo_bw_gemm_kernel<bf16, int4, zero point> (64 x 128 tiles)"}}
+                     "kernel": "qmm_wo_bw_wide_kernel<bf16, int4, zero point> (64 x 256 tiles)"}}
     del w3s, fns, x3p, w3d
 
     # W8A8 prefill GEMM (config 4)
@@ -573,7 +573,7 @@ def main():
                                                        mid_dtype=torch.float32, out_dtype=torch.bfloat16)],
                             20, 5, use_graph)
       small[f"M{m}_us"] = round(ev * 1e3, 2)
-    small["note"] = "GEMM alone, bf16 output, weights (59 MB) cache-warm; M=32: 32x32 tiles, M=128: 64x32, M=512: 64x64"
+    small["note"] = "GEMM alone, bf16 output, weights (59 MB) cache-warm; M=32: 32x32 tiles, M=128: 64x32, M=512: 64x128"
     extra["w8a8_gemm_4096x14336_small_M"] = small
     # quantized_decomposed quantize / dequantize of a weight-sized tensor (HBM-bound elementwise)
     import xla_amd.experimental.quantized  # noqa: F401

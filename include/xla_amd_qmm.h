@@ -61,10 +61,10 @@ extern "C" {
 #define XLA_AMD_W_SCN 1 /* blockwise:   [K/C, C, N]            (xla_quantized_matmul.py:89) */
 
 /* kernels the dispatcher can choose (xla_amd_qmm_dispatch) */
-#define XLA_AMD_KERNEL_GENERIC 0    /* one thread per output, any shape          */
+#define XLA_AMD_KERNEL_GENERIC 0    /* the operator's own weight layout, any shape */
 #define XLA_AMD_KERNEL_SKINNY_MFMA 1 /* weight-streaming GEMV / skinny GEMM       */
 #define XLA_AMD_KERNEL_W8A8_MFMA 2  /* LDS-tiled int8 MFMA GEMM                   */
-#define XLA_AMD_KERNEL_W8A8_GENERIC 3
+#define XLA_AMD_KERNEL_W8A8_GENERIC 3 /* int8 products the dispatcher keeps from it: K no multiple of 64, few outputs */
 #define XLA_AMD_KERNEL_WEIGHT_ONLY_GEMM 4 /* tiled bf16/f16 MFMA GEMM on int8 weights */
 
 int xla_amd_qmm_abi_version(void);
@@ -232,8 +232,9 @@ int xla_amd_qmm_weight_only_gemm_f32(const float* x, const void* w_tiled, const 
 /*
  * Weight-only quantized matmul for any shape, reading the operator's own
  * weight layout: matrix instructions on per-channel weights of any K and
- * alignment, one thread per output element on blockwise weights (block sizes
- * the streaming kernel rejects).  Same reference statements and rounding
+ * alignment (one thread per output element up to 8 - 40 columns), one thread
+ * per output element on blockwise weights (block sizes the streaming kernel
+ * rejects).  Same reference statements and rounding
  * points as xla_amd_qmm_weight_only_skinny.
  */
 int xla_amd_qmm_weight_only_generic(const void* x, const int8_t* w, const void* scale,

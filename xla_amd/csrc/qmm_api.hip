@@ -121,7 +121,7 @@ int qmm_skinny_k_slices(int64_t M, int64_t N, int64_t K, int64_t C, int bits, in
 //    ~630 int8 ops/byte (or ~310 bf16 flops/byte) the chip can do per HBM
 //    byte, so the weight is streamed exactly once by the skinny kernel;
 //  * many rows with int8 activations (prefill): LDS-tiled int8 MFMA GEMM.
-// Shapes neither fast kernel accepts run the one-thread-per-output kernels.
+// Shapes neither accepts run the kernels that read the operator's own weight layout.
 extern "C" int xla_amd_qmm_dispatch(int64_t M, int64_t N, int64_t K, int64_t C, int bits,
                                     int x_dt, int quantize_activation) {
   if (quantize_activation) {

@@ -505,7 +505,9 @@ int cu_count() {
 // zero point: 43 against 30 us at K = 4096) to 1.65 times as long (int8: 44 / 27; without a zero point int4 42 / 28,
 // per-channel int4 35 / 23), so they are for launches whose rounds come to that much fewer: from about two rounds of
 // 64 x 128 tiles on (1024 rows against 4096 x 4096, int4: 60 -> 43 us; 512 rows, one round either way: 33 -> 40, kept
-// here).  With a zero point the wide kernel exists for int4 weights in blocks of 128 columns only: 96 accumulator
+// here).  The ratios hold for other K: of 239 launches the rule gives to the wide tiles, K = 256 ... 14336, one is 3 %
+// slower so (3000 x 2048 x 512 int4 with a zero point, 18.7 / 19.3) and the rest at most 2, the least gain being at K = 256.
+// With a zero point the wide kernel exists for int4 weights in blocks of 128 columns only: 96 accumulator
 // registers leave no room for the second load of int8 weights or for the bookkeeping of longer blocks.
 template <int XT, int BITS>
 bool wide_tiles(const WoBwArgs& a, int64_t items, int cus) {

@@ -13,9 +13,9 @@
 //  * the zero points' term is a matrix product over the blocks: the copying waves leave round_x(sum x) of 16 blocks
 //    in LDS, next to the zero points of the 16 blocks, and the computing waves add them with one MFMA per result tile.
 // The second wave per SIMD covers the waits of the first, and twice the channels per workgroup halve the copies of x.
-// 2048 rows against 4096 x 4096, bf16, blocks of 128, per launch in a graph (this kernel / the 64 x 128 tile): int4
-// with zero point 86 / 121 us, without 84 / 110, int8 89 / 107; per-channel int4 70 / 91.  Everything but the MFMAs,
-// expansion and rounding switched off it takes 65 us.
+// 2048 rows against 4096 x 4096, bf16, blocks of 128, per launch in a graph (this kernel / the 64 x 128 tile, one box; from
+// box to box 75 - 86 / 108 - 121): int4 with zero point 81 / 114 us, without 77 / 105, int8 84 / 97; per-channel int4
+// 69 / 90.  Everything but the MFMAs, expansion and rounding switched off it takes 65 us.
 #include "qmm_common.h"
 #include "qmm_frag.h"
 #include "qmm_wo_bw.h"

@@ -75,11 +75,11 @@ def _add(batches, n_out, n_in, blocks):
       TUNED_BLOCK_SIZES[(_ARCH, bs, n_out, n_in, dtype, True)] = blocks
 
 
-# Fastest measured tile per shape (MI355X, one sweep over the workgroup tiles but 64 x 128, quantized Gaussian operands,
-# graph replays; a tile within 3 % of the fastest goes to what the library would pick by itself, which leaves four
-# entries that differ from the shape rule: (5120, 640) at 2048 / 4096 rows and (5120, 1280) at 2048 rows, where a
-# short K favours 128 x 128, and (37888, 3584) at 128 rows).  64 x 128, which came later, stands where the shape rule has
-# it and at 128 rows of two more (all 5 - 22 % faster than 64 x 64 with weights out of HBM).  Shapes: the (out, in) pairs of the reference's table
+# Fastest measured tile per shape (MI355X, sweeps over the workgroup tiles, quantized Gaussian operands, graph replays
+# with the weights in the Infinity Cache; a tile within 4 % of the fastest goes to what the library would pick by itself,
+# which leaves five entries that differ from the shape rule: (5120, 640) at 2048 ... 8192 rows, where a short K favours
+# 128-row tiles, (13824, 5120) at 128 rows, and (14336, 4096) at 128 rows for its weights out of HBM, where 64 x 128 is
+# 7 - 10 % faster than the rule's 64 x 64).  Shapes: the (out, in) pairs of the reference's table
 # (Llama-3-8B; Llama-3-70B, Qwen2.5-7B and a 5120-wide model sharded over devices) plus the single projections
 # and two square ones; batches as in the reference's table, 16 ... 16384 (where the result fits 700 M elements).
 # (n_out, n_in): {batch: (batch_block, out_block)}
@@ -112,16 +112,16 @@ _MEASURED = {
                    1024: (128, 256), 2048: (256, 256), 4096: (256, 256), 8192: (256, 256), 16384: (256, 256)},
     (3584, 3584): {16: (32, 32), 32: (32, 32), 64: (32, 32), 128: (64, 32), 256: (64, 64), 512: (64, 64),
                    1024: (128, 128), 2048: (128, 256), 4096: (256, 256), 8192: (256, 256), 16384: (256, 256)},
-    (37888, 3584): {16: (64, 64), 32: (64, 64), 64: (64, 64), 128: (128, 128), 256: (256, 256), 512: (256, 256),
+    (37888, 3584): {16: (64, 64), 32: (64, 64), 64: (64, 64), 128: (128, 256), 256: (256, 256), 512: (256, 256),
                     1024: (256, 256), 2048: (256, 256), 4096: (256, 256), 8192: (256, 256), 16384: (256, 256)},
     (3584, 18944): {16: (32, 32), 32: (32, 32), 64: (32, 32), 128: (64, 32), 256: (64, 64), 512: (64, 128),
                     1024: (128, 128), 2048: (128, 256), 4096: (256, 256), 8192: (256, 256), 16384: (256, 256)},
     (896, 5120): {16: (32, 32), 32: (32, 32), 64: (32, 32), 128: (32, 32), 256: (32, 32), 512: (64, 32),
                   1024: (64, 64), 2048: (64, 128), 4096: (128, 128), 8192: (128, 256), 16384: (256, 256)},
     (5120, 640): {16: (32, 32), 32: (32, 32), 64: (64, 32), 128: (64, 64), 256: (64, 64), 512: (64, 64),
-                  1024: (128, 256), 2048: (128, 128), 4096: (128, 128), 8192: (256, 256), 16384: (256, 256)},
+                  1024: (128, 256), 2048: (128, 128), 4096: (128, 128), 8192: (128, 256), 16384: (256, 256)},
     (5120, 1280): {16: (32, 32), 32: (32, 32), 64: (64, 32), 128: (64, 64), 256: (64, 64), 512: (64, 64),
-                   1024: (128, 256), 2048: (128, 128), 4096: (256, 256), 8192: (256, 256), 16384: (256, 256)},
+                   1024: (128, 256), 2048: (256, 256), 4096: (256, 256), 8192: (256, 256), 16384: (256, 256)},
     (1792, 5120): {16: (32, 32), 32: (32, 32), 64: (32, 32), 128: (32, 32), 256: (64, 32), 512: (64, 64),
                    1024: (64, 128), 2048: (128, 128), 4096: (128, 256), 8192: (256, 256), 16384: (256, 256)},
     (13824, 5120): {16: (64, 64), 32: (64, 64), 64: (64, 64), 128: (64, 128), 256: (128, 128), 512: (128, 256),
