@@ -105,6 +105,7 @@ void forget_tiled(int64_t key) {
 // Makes the copy safe to read by work that is launched on the current stream from here on, and keeps its memory from
 // being handed out again before that work is done.  (The lock is held.)
 void use_on_current_stream(Copy& c) {
+  if (c.complete && c10::hip::getCurrentHIPStream(c.made_on.device_index()).id() == c.made_on.id()) return;  // the usual case
   const c10::Stream now = current_stream(c.tiled);
   if (!c.complete) {
     // (event queries and waits are refused while any thread captures, unless this thread's capture mode is relaxed)
