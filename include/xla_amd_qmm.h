@@ -170,6 +170,12 @@ int xla_amd_qmm_weight_only_skinny(const void* x, const void* w_tiled, const voi
                                    int dot_dt, int out_dt, int store_dt, void* stream);
 
 /*
+ * Between the two kernels above and below lies a third (qmm_wo_ksplit.hip, per-channel int8 weights, bf16 or f16 x): a
+ * tile of 16 - 64 rows x 16 - 128 channels per workgroup whose waves split K.  Both entry points run it where a
+ * measured rule on M, N and K says so (more than 16 rows); it needs no workspace.
+ */
+
+/*
  * Bytes of workspace xla_amd_qmm_weight_only_gemm needs for a shape (0 when it
  * needs none, or for arguments it rejects).
  */

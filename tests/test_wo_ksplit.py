@@ -1,0 +1,97 @@
+"""Batches of rows against per-channel int8 weights: K split over the waves of a workgroup, one shape or more per tile."""
+import re
+
+import pytest
+import torch
+
+from oracle import quantized_matmul_oracle as oracle
+from tests import cases
+from tests import launch_recorder as rec
+
+# (m, n, k, rows and channels of the tile): row tiles of unequal length, a last tile of few rows and of few channels, n
+# that is and is not a multiple of 4 (channel groups of 10, 12, 14 and 16), k of less than a slot, of one, and of several
+# with a last one that not every wave has a share of
+SHAPES = [
+    (17, 16, 128, 16, 16), (31, 30, 2176, 16, 16), (129, 17, 1152, 16, 16),
+    (17, 2049, 640, 16, 32), (128, 520, 2176, 16, 32),
+    (17, 2049, 128, 32, 32), (32, 6146, 384, 32, 32), (193, 1030, 512, 32, 32),
+    (97, 2049, 128, 32, 64), (64, 7165, 384, 32, 64), (511, 1000, 640, 32, 64),
+    (33, 4100, 128, 48, 32), (97, 2049, 1152, 48, 32),
+    (129, 4100, 128, 48, 64), (100, 4100, 2176, 48, 64),
+    (65, 6146, 128, 64, 64), (385, 2049, 640, 64, 64),
+    (129, 7165, 128, 64, 96), (250, 5000, 640, 64, 96),
+    (193, 6146, 128, 64, 128), (300, 6146, 1152, 64, 128), (2048, 1000, 640, 64, 128),
+]
+
+
+def test_tiles_of_the_shapes(tmp_path):
+  calls = [rec.blockwise(m, n, k, k, 8, zp, dt) for m, n, k, _, _ in SHAPES for zp in (False, True) for dt in (1, 2)]
+  calls += [rec.skinny(m, n, k, k, 8, zp, 1) for m, n, k, _, _ in SHAPES if m <= 32 for zp in (False, True)]
+  want = {(m, n, k): (bm, bn) for m, n, k, bm, bn in SHAPES}
+  seen = set()
+  for (_, sig, args), (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0, text
+    m, n, k = args[7:10] if len(args) > 18 else args[5:8]
+    (l,) = launches
+    mt, ng, kw, cw = (int(v) for v in re.search(r"qmm_wo_ksplit_kernelILi\dELi(\d)ELi(\d)ELi(\d)ELi(\d)E", l.name).groups())
+    assert (16 * mt, 16 * ng * cw) == want[m, n, k], (m, n, k, l.name)
+    tiles = -(-m // (16 * mt)) * -(-n // (16 * ng * cw))
+    assert l.lds <= l.lds_limit and l.block[0] == 64 * (kw * cw + 4) and tiles <= l.grid[0] < tiles + 8, l
+    seen.add(want[m, n, k])
+  assert len(seen) == 9
+  # 16 rows or fewer, and wide outputs of up to 32, keep the streaming kernel; what fills the chip keeps the tiled GEMM
+  calls = [rec.skinny(16, 4096, 4096, 4096, 8, False), rec.skinny(32, 14336, 4096, 4096, 8, False),
+           rec.blockwise(2048, 14336, 4096, 4096, 8, False)]
+  for rc, text, launches in rec.record(calls, str(tmp_path)):
+    assert rc == 0 and not any("ksplit" in l.name for l in launches), text
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,bm,bn", SHAPES)
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_against_the_oracle(m, n, k, bm, bn, xdt):
+  import xla_amd.experimental.custom_kernel  # noqa: F401
+  op = torch.ops.xla.quantized_matmul
+  for zp, sdt in ((False, xdt), (True, xdt), (True, torch.float32)):
+    x, w, s, _ = cases.per_channel_int8(m, n, k, xdt, sdt, seed=m + n)
+    z = (torch.randn(n, generator=cases.gen(5)) * 0.01).to(sdt) if zp else None
+    exp = oracle.quantized_matmul(x, w, s, z)
+    wd, sd, zd = w.cuda(), s.cuda(), None if z is None else z.cuda()
+    out = op(x.cuda(), wd, sd, zd).cpu()
+    # f32 sums in another order: a dot product rounds to its other neighbour now and then
+    assert out.dtype == exp.dtype and cases.within_tolerance(out, exp), (zp, sdt)
+    assert cases.rel_l2(out, exp) < 1e-3, (zp, sdt)
+  # an infinity stays in its row: the other rows of the tile, and of the row quad copied with it, are untouched
+  row = m - 1
+  x[row, 3] = float("inf")
+  bad = op(x.cuda(), wd, sd, zd).cpu()
+  assert torch.equal(bad[:row], out[:row])
+  assert not torch.isfinite(bad[row]).any()
+
+
+@pytest.mark.gpu
+def test_replays_and_streams():
+  """No workspace, no state: replays of a captured launch and launches on two streams at once give the same results."""
+  import xla_amd.experimental.custom_kernel  # noqa: F401
+  op = torch.ops.xla.quantized_matmul
+  x, w, s, _ = cases.per_channel_int8(100, 2049, 1152, torch.bfloat16, torch.bfloat16, seed=1)
+  x, w, s = x.cuda(), w.cuda(), s.cuda()
+  ref = op(x, w, s)
+  torch.cuda.synchronize()
+  graph = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(graph):
+    out = op(x, w, s)
+  for _ in range(4):
+    out.zero_()
+    graph.replay()
+    assert torch.equal(op(x, w, s), ref)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
+  streams = [torch.cuda.Stream() for _ in range(2)]
+  outs = []
+  for _ in range(8):
+    for st in streams:
+      with torch.cuda.stream(st):
+        outs.append(op(x, w, s))
+  torch.cuda.synchronize()
+  assert all(torch.equal(o, ref) for o in outs)

@@ -44,6 +44,7 @@
 
 #include "qmm_frag.h"
 #include "qmm_skinny.h"
+#include "qmm_wo_gemm.h"
 
 // Diagnostic build (-DQMM_SKINNY_TIMELINE, a library of its own; see xla_amd/build.py): every wave
 // notes the time (the chip-wide 100 MHz counter) at fixed points of the kernel - entry, first
@@ -945,6 +946,9 @@ extern "C" int xla_amd_qmm_weight_only_skinny(const void* x, const void* w_tiled
   if (((uintptr_t)out & 15) && (N & 3) == 0)
     return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_skinny: out must be 16-byte aligned");
   if (M == 0) return XLA_AMD_QMM_OK;
+  // a batch of 17 - 32 rows against a per-channel int8 weight: K split over the waves of a workgroup where that is faster
+  if (M <= 32 && C == K && bits == 8 && x_dt != XLA_AMD_DT_F32 && qmm_wo_ksplit_tile(M, N, K) >= 0)
+    return qmm_wo_ksplit_run(x, w_tiled, scale, zp, out, M, N, K, x_dt, scale_dt, zp_dt, dot_dt, out_dt, store_dt, (hipStream_t)stream);
   const int xsz = qmm_dt_size(x_dt), osz = qmm_dt_size(store_dt);
   const int pass = x_dt == XLA_AMD_DT_F32 ? 16 : 32;  // rows of x per pass over the weight
   for (int64_t m0 = 0; m0 < M; m0 += pass) {

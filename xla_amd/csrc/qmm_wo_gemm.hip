@@ -39,28 +39,11 @@
 #include "qmm_frag.h"
 #include "qmm_skinny.h"
 #include "qmm_wo_bw.h"
+#include "qmm_wo_gemm.h"
 
 #if !defined(QMM_WO_XT) || !defined(QMM_WO_MT)
 #error "compile with -DQMM_WO_XT=<XLA_AMD_DT_BF16|XLA_AMD_DT_F16 value> -DQMM_WO_MT=<4|8>"
 #endif
-
-struct WoGemmArgs {
-  const void* x;       // [M, K]
-  const uint8_t* w;    // tiled weight, 8 bits
-  const void* scale;   // [N]
-  const void* zp;      // [N] or null
-  void* out;           // [M, N] of store_dt (split == 1)
-  float* part;         // [split][M][N] partial dot products (split > 1)
-  float* part_xs;      // [split][M] partial row sums of x (split > 1, zero point)
-  int M, N, K;
-  int G;               // channels per group of the tiled weight (xla_amd_qmm_tile_group)
-  int k_per_split;     // columns per K slice (a multiple of 128)
-  int split;
-  int scale_dt, zp_dt, dot_dt, out_dt, store_dt;
-  int Kw;    // columns of the weight: K, or K / 3 when x is an f32 matrix split into three bf16 parts side by side
-  int x_dt;  // the caller's x dtype (the row sums of x are rounded to it): the kernel's, or f32 for split f32 rows
-  int stage_out;  // 128 x 256 tile: results leave through LDS, written out by the copying waves during the next item
-};
 
 // one launcher per unit: row tile of 16 * MT rows, ng = 2 or 4 channel groups per computing wave
 int qmm_wo_launch_bf16_mt4(const WoGemmArgs& a, int ng, hipStream_t stream);
@@ -98,102 +81,6 @@ template <int MT, int NG> struct WoCfg {
   static_assert(R >= 3, "the x ring needs room to run ahead");
   static constexpr int lds_bytes(int steps) { return kStage + (steps < R ? steps : R) * X_TILE; }
 };
-
-// The dtypes of the epilogue: those of the call, or (UNI) all equal to x's dtype and known at
-// compile time, which is the common case and removes every branch on a dtype.
-template <int XT, bool UNI> struct WoDts {
-  int scale_dt, zp_dt, dot_dt, out_dt, store_dt, x_dt;
-  __device__ __forceinline__ explicit WoDts(const WoGemmArgs& a)
-      : scale_dt(UNI ? XT : a.scale_dt), zp_dt(UNI ? XT : a.zp_dt), dot_dt(UNI ? XT : a.dot_dt),
-        out_dt(UNI ? XT : a.out_dt), store_dt(UNI ? XT : a.store_dt), x_dt(UNI ? XT : a.x_dt) {}
-};
-
-// Scale (or zero point) of four consecutive channels as raw bits; channels past N repeat the last one.
-__device__ __forceinline__ void wo_load4_raw(const void* p, int n, int N, int dt, uint32_t raw[4]) {
-#pragma unroll
-  for (int v = 0; v < 4; ++v) raw[v] = qmm_load_raw(p, min(n + v, N - 1), dt);
-}
-
-// The reference's epilogue for four consecutive channels of one row:
-//   p = round_dot(dot); r = round_out(scale * p); with a zero point r = round_out(r - round_zpo(round_x(xsum) * zp)).
-template <class Dts>
-__device__ __forceinline__ void wo_finish4(const Dts& d, const uint32_t sraw[4], const uint32_t zraw[4], bool has_zp,
-                                           f32x4 dot, float xsum, int x_dt, float o[4]) {
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const float p = qmm_round_dt(dot[v], d.dot_dt);
-    float r = qmm_round_dt(qmm_from_raw(sraw[v], d.scale_dt) * p, d.out_dt);
-    if (has_zp) {
-      const int zpo_dt = qmm_promote(x_dt, d.zp_dt);
-      const float z = qmm_round_dt(qmm_round_dt(xsum, x_dt) * qmm_from_raw(zraw[v], d.zp_dt), zpo_dt);
-      r = qmm_round_dt(r - z, d.out_dt);
-    }
-    o[v] = r;
-  }
-}
-
-// Stores four consecutive channels of row m starting at channel n (n % 4 == 0).  VEC: N is a
-// multiple of 4, so the four channels exist and their address is aligned for one store.
-template <bool VEC>
-__device__ __forceinline__ void wo_store4(void* out, int m, int n, int N, const float o[4], int store_dt) {
-  const size_t idx = (size_t)m * N + n;
-  if constexpr (VEC) {
-    if (store_dt == XLA_AMD_DT_F32) {
-      *(f32x4*)((float*)out + idx) = f32x4{o[0], o[1], o[2], o[3]};
-    } else {
-      const bool bf = store_dt == XLA_AMD_DT_BF16;
-      const uint32_t lo = bf ? qmm_f32x2_to_bf16x2(o[0], o[1]) : qmm_f32x2_to_f16x2(o[0], o[1]);
-      const uint32_t hi = bf ? qmm_f32x2_to_bf16x2(o[2], o[3]) : qmm_f32x2_to_f16x2(o[2], o[3]);
-      *(i32x2*)((uint16_t*)out + idx) = i32x2{(int)lo, (int)hi};
-    }
-  } else {
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (n + v < N) qmm_store(out, idx + v, o[v], store_dt);
-  }
-}
-
-// Stores the first cnt (1 .. 4) of four consecutive channels of row m starting at channel n, n even: in
-// pairs where the row length allows it (rows whose length is no multiple of 4).
-__device__ __forceinline__ void wo_store_some(void* out, int m, int n, int N, int cnt, const float o[4], int store_dt) {
-  const size_t idx = (size_t)m * N + n;
-  if ((N & 1) == 0) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (cnt >= 2 * h + 2) {
-        if (store_dt == XLA_AMD_DT_F32) {
-          typedef float f32x2_t __attribute__((ext_vector_type(2)));
-          *(f32x2_t*)((float*)out + idx + 2 * h) = f32x2_t{o[2 * h], o[2 * h + 1]};
-        } else {
-          *(uint32_t*)((uint16_t*)out + idx + 2 * h) = store_dt == XLA_AMD_DT_BF16 ? qmm_f32x2_to_bf16x2(o[2 * h], o[2 * h + 1])
-                                                                                  : qmm_f32x2_to_f16x2(o[2 * h], o[2 * h + 1]);
-        }
-      } else if (cnt == 2 * h + 1) {
-        qmm_store(out, idx + 2 * h, o[2 * h], store_dt);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (v < cnt) qmm_store(out, idx + v, o[v], store_dt);
-  }
-}
-
-// The same epilogue and store when every dtype is bf16 and there is no zero point: two
-// values per conversion, and the rounded product is already the stored bit pattern.
-__device__ __forceinline__ void wo_finish_pack_bf16(const uint32_t sraw[4], f32x4 dot, uint32_t res[2]) {
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint32_t p = qmm_f32x2_to_bf16x2(dot[2 * h], dot[2 * h + 1]);
-    const float p0 = __uint_as_float(p << 16), p1 = __uint_as_float(p & 0xffff0000u);
-    res[h] = qmm_f32x2_to_bf16x2(__uint_as_float(sraw[2 * h] << 16) * p0, __uint_as_float(sraw[2 * h + 1] << 16) * p1);
-  }
-}
-__device__ __forceinline__ void wo_finish_store_bf16(void* out, int m, int n, int N, const uint32_t sraw[4], f32x4 dot) {
-  uint32_t res[2];
-  wo_finish_pack_bf16(sraw, dot, res);
-  *(i32x2*)((uint16_t*)out + (size_t)m * N + n) = i32x2{(int)res[0], (int)res[1]};
-}
 
 // One unit of work: a tile of rows x channels over one K slice.
 struct WoItem {
@@ -790,7 +677,64 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, bool has_zp) {
   return p;
 }
 
+// Time of a launch of the tiled GEMM by its plan, us: fitted to 299 of the same shapes as the tiles of the K split
+// over waves (root mean square error 4 - 5 %).
+double plan_us(const Plan& p, int64_t M, int64_t N, int64_t K) {
+  const int64_t bm = 16 * p.mt, bn = 64 * p.ng;
+  const int64_t items = (M + bm - 1) / bm * ((N + bn - 1) / bn) * p.split;
+  const double rounds = (double)((items + 255) / 256), steps = p.k_per_split / 128;
+  const double finish = p.split > 1 ? 1e-6 * (double)p.split * (double)M * (double)N * 4 : 0, weight = 1e-6 * (double)N * (double)K;
+  if (p.mt == 4) return 2.29 + 2.29 * rounds + 0.598 * rounds * steps + (p.split > 1 ? 1.85 + 0.626 * finish : 0) + 0.027 * weight;
+  if (p.ng == 2) return 3.22 + 3.22 * rounds + 0.796 * rounds * steps + (p.split > 1 ? 1.16 + 0.551 * finish : 0) + 0.019 * weight;
+  return 4.03 + 6.49 * rounds + 1.14 * rounds * steps + 0.006 * weight;
+}
+
 }  // namespace
+
+// Up to 16 rows the streaming kernel is as fast.  17 - 32 rows: against up to 8192 channels (0.72 - 0.99 of the
+// streaming kernel's time; wider outputs 0.99 - 1.06), except where that runs K slices of a long K (4096 x 14336: 1.01
+// - 1.03, 512 x 14336: 1.1).  More rows: the shorter of the two estimates.  Over 297 measured shapes that is on
+// average 0.4 % off the better of the two, and 0.68 of the time of the tiled GEMM with its K slices; the worst choice
+// took 5 % longer than the tiled GEMM.
+int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
+  if (M <= 16 || K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14)) return -1;
+  if (M <= 32) {
+    int per;
+    if (N > 8192 || (K > 8192 && qmm_skinny_k_slices(M, N, K, K, 8, &per) > 1)) return -1;
+  }
+  int best = -1;
+  double best_us = 0;
+  if (M > 32) {
+    const Plan p = make_plan(M, N, K, false);
+    if (p.mt == 4 && p.ng == 4) return -1;  // more than 49152 channels: the tiled GEMM's rounds are full
+    best_us = plan_us(p, M, N, K);
+  }
+  for (int i = 0; i < (int)(sizeof(kKsTiles) / sizeof(kKsTiles[0])); ++i) {
+    const KsTile& t = kKsTiles[i];
+    const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn);
+    if (tiles > 4096) continue;
+    const double rounds = (double)((tiles + 255) / 256), steps = (double)((K / 128 + t.kw - 1) / t.kw);
+    const double us = t.fixed + t.round * rounds + (t.step * rounds + t.load * (double)tiles / 256) * steps + t.weight * 1e-6 * (double)N * (double)K;
+    if ((best < 0 && M <= 32) || us < best_us) { best = i; best_us = us; }
+  }
+  return best;
+}
+
+int qmm_wo_ksplit_run(const void* x, const void* w_tiled, const void* scale, const void* zp, void* out, int64_t M, int64_t N,
+                      int64_t K, int x_dt, int scale_dt, int zp_dt, int dot_dt, int out_dt, int store_dt, hipStream_t s) {
+  const int tile = qmm_wo_ksplit_tile(M, N, K);
+  WoGemmArgs a;
+  a.x = x; a.w = (const uint8_t*)w_tiled; a.scale = scale; a.zp = zp; a.out = out;
+  a.part = nullptr; a.part_xs = nullptr;
+  a.M = (int)M; a.N = (int)N; a.K = (int)K;
+  a.Kw = (int)K; a.x_dt = x_dt; a.stage_out = 0;
+  a.G = xla_amd_qmm_tile_group(N, K, K, 8);
+  a.k_per_split = (int)K; a.split = 1;
+  a.scale_dt = scale_dt; a.zp_dt = zp ? zp_dt : x_dt; a.dot_dt = dot_dt; a.out_dt = out_dt; a.store_dt = store_dt;
+  if (x_dt == XLA_AMD_DT_BF16)
+    return tile < 4 ? qmm_wo_ksplit_launch_bf16_0(a, tile, s) : tile < 7 ? qmm_wo_ksplit_launch_bf16_1(a, tile, s) : qmm_wo_ksplit_launch_bf16_2(a, tile, s);
+  return tile < 4 ? qmm_wo_ksplit_launch_f16_0(a, tile, s) : tile < 7 ? qmm_wo_ksplit_launch_f16_1(a, tile, s) : qmm_wo_ksplit_launch_f16_2(a, tile, s);
+}
 
 namespace {
 
@@ -867,6 +811,7 @@ extern "C" size_t xla_amd_qmm_weight_only_gemm_workspace_bytes(int64_t M, int64_
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0) return 0;
   if (C <= 0) C = K;
   if (K % C != 0) return 0;
+  if (C == K && bits == 8 && qmm_wo_ksplit_tile(M, N, K) >= 0) return 0;
   if (M <= 32) {  // the weight-streaming kernel over K slices
     int per;
     const int slices = qmm_skinny_k_slices(M, N, K, C, bits, &per);
@@ -910,6 +855,8 @@ extern "C" int xla_amd_qmm_weight_only_gemm(const void* x, const void* w_tiled, 
     return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_gemm: out must be 16-byte aligned");
   if (M == 0) return XLA_AMD_QMM_OK;
   const bool blockwise = C != K;
+  if (!blockwise && bits == 8 && qmm_wo_ksplit_tile(M, N, K) >= 0)
+    return qmm_wo_ksplit_run(x, w_tiled, scale, zp, out, M, N, K, x_dt, scale_dt, zp_dt, dot_dt, out_dt, store_dt, (hipStream_t)stream);
   // (blockwise weights in the weight-streaming kernel: every dtype but the stored one is x's, at least 8 scales)
   const bool bw_ok = !blockwise || (scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt && (K / C) * N >= 8 &&
                                     (((uintptr_t)scale | (uintptr_t)zp) & 3) == 0);
