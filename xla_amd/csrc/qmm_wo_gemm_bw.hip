@@ -273,10 +273,10 @@ qmm_wo_bw_gemm_kernel(WoBwArgs a) {
   f32x4 acc2[2][NG][MT], xs2[2][MT];
   i32x2 ent_s[2][NG], ent_z[2][NG];  // scales and zero points of this lane's channels for the block in set P
   // The rounding sequence of the block in set Q for the results (gi, v, mt) and (gi, v, mt + 1), in kPhases parts
-  // (one after each of kPhases consecutive MFMAs): the dot products rounded and packed; unpacked and added to the
-  // scaled sums; the zero-point sums.
+  // (one after each of kPhases consecutive MFMAs): the dot products rounded; added to the scaled sums; the
+  // zero-point sums.
   float xs_r[MT];
-  uint32_t packed = 0;  // the pair's rounded dot products between the first and the second part
+  float p0 = 0.f, p1 = 0.f;  // the pair's rounded dot products between the first and the second part
   constexpr int kPairs = NG * 4 * (MT / 2);                 // pairs of results per block and lane
   constexpr int kSlots = 4 * (NG * MT + (NEEDXS ? MT : 0));  // MFMAs per step
   constexpr int kPhases = kSlots / kPairs;                  // MFMAs per pair
@@ -290,12 +290,11 @@ qmm_wo_bw_gemm_kernel(WoBwArgs a) {
         d0 = fmaf(-1.5f, xs2[Q][mt][0], d0);
         d1 = fmaf(-1.5f, xs2[Q][mt + 1][0], d1);
       }
-      packed = XT == XLA_AMD_DT_BF16 ? qmm_f32x2_to_bf16x2(d0, d1) : qmm_f32x2_to_f16x2(d0, d1);
+      wo_bw_round2<XT>(d0, d1, p0, p1);
     }
     if constexpr (ph == 1) {
       const uint32_t sw = (uint32_t)ent_s[Q][gi][v >> 1];
       const float sc = qmm_from_raw((v & 1) ? (sw >> 16) : (sw & 0xffffu), XT);
-      const float p0 = qmm_from_raw(packed & 0xffffu, XT), p1 = qmm_from_raw(packed >> 16, XT);
       sacc[gi][mt][v] = fmaf(sc, p0, sacc[gi][mt][v]);
       sacc[gi][mt + 1][v] = fmaf(sc, p1, sacc[gi][mt + 1][v]);
     }

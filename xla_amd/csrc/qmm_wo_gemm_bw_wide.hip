@@ -3,7 +3,8 @@
 // channels, with eight computing waves instead of four.
 //
 // What bounds it: instruction issue.  A step of a wave (64 rows x 32 channels x 128 columns) is 32 MFMAs, and beside
-// them the expansion of the weights (64 instructions for int4) and the block's rounding sequence (86).  On a SIMD an
+// them the expansion of the weights (64 instructions for int4) and the block's rounding sequence (72 in
+// bf16, see wo_bw_round2; 88 in f16).  On a SIMD an
 // MFMA takes about 13 cycles of issue and every other vector instruction 4, whichever of its waves they come from, so
 // what counts is how few instructions a step has:
 //  * the sums of x per step come from the copying waves, once per row (four MFMAs against ones for their 16 rows)
@@ -219,9 +220,10 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
         qmm_static_for<MT / 2>([&](auto mc) {
           constexpr int mt = 2 * (int)mc;
           const float d0 = acc[gi][mt][v], d1 = acc[gi][mt + 1][v];
-          const uint32_t p = XT == XLA_AMD_DT_BF16 ? qmm_f32x2_to_bf16x2(d0, d1) : qmm_f32x2_to_f16x2(d0, d1);
-          sacc[gi][mt][v] = fmaf(sc, qmm_from_raw(p & 0xffffu, XT), sacc[gi][mt][v]);
-          sacc[gi][mt + 1][v] = fmaf(sc, qmm_from_raw(p >> 16, XT), sacc[gi][mt + 1][v]);
+          float p0, p1;
+          wo_bw_round2<XT>(d0, d1, p0, p1);
+          sacc[gi][mt][v] = fmaf(sc, p0, sacc[gi][mt][v]);
+          sacc[gi][mt + 1][v] = fmaf(sc, p1, sacc[gi][mt + 1][v]);
         });
       });
       // (here: the compiler would sink it behind the zero points' product, with the accumulators live meanwhile)
