@@ -24,6 +24,36 @@ SHAPES = [
 ]
 
 
+# f32 rows: from one; a tile of 16 x 16 with four and with eight K groups
+F32_SHAPES = [
+    (1, 5, 128, 16, 16), (17, 333, 384, 16, 16), (1, 5, 640, 16, 16), (127, 333, 2176, 16, 16),
+    (1, 4100, 640, 16, 32), (100, 4100, 640, 16, 32),
+    (33, 4100, 2176, 16, 64), (100, 2049, 640, 16, 64),
+    (17, 4100, 384, 32, 32), (127, 1030, 128, 32, 32),
+    (33, 7165, 128, 32, 64), (127, 7165, 1152, 32, 64),
+    (300, 520, 640, 32, 32),  # more rows than the streaming kernel gets
+]
+
+
+def test_tiles_of_the_f32_shapes(tmp_path):
+  calls = [rec.skinny(m, n, k, k, 8, zp, 0) for m, n, k, _, _ in F32_SHAPES for zp in (False, True)]
+  seen = set()
+  for (_, _, args), (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0, text
+    m, n, k = args[5:8]
+    (l,) = launches
+    xt, mt, ng, kw, cw = (int(v) for v in re.search(r"qmm_wo_ksplit_kernelILi(\d)ELi(\d)ELi(\d)ELi(\d)ELi(\d)E", l.name).groups())
+    assert xt == 0 and (m, n, k, 16 * mt, 16 * ng * cw) in F32_SHAPES, (m, n, k, l.name)
+    assert l.lds <= l.lds_limit and l.block[0] == 64 * (kw * cw + 4)
+    seen.add((mt, ng, kw, cw))
+  assert len(seen) == 6
+  # rows that fill the chip keep the split into three bf16 parts, sizes past the kernel's range the streaming kernel
+  calls = [rec.skinny(4, 64, 131072, 131072, 8, False, 0),
+           ("xla_amd_qmm_weight_only_gemm_f32", "pppppp" + "z" + "qqq" + "iip", [rec.PTR] * 3 + [0, rec.PTR, rec.PTR, 1 << 40, 2048, 4096, 4096, 0, 0, 0])]
+  for rc, text, launches in rec.record(calls, str(tmp_path)):
+    assert rc == 0 and launches and not any("ksplit" in l.name for l in launches), text
+
+
 def test_tiles_of_the_shapes(tmp_path):
   calls = [rec.blockwise(m, n, k, k, 8, zp, dt) for m, n, k, _, _ in SHAPES for zp in (False, True) for dt in (1, 2)]
   calls += [rec.skinny(m, n, k, k, 8, zp, 1) for m, n, k, _, _ in SHAPES if m <= 32 for zp in (False, True)]
@@ -62,6 +92,31 @@ def test_against_the_oracle(m, n, k, bm, bn, xdt):
     assert out.dtype == exp.dtype and cases.within_tolerance(out, exp), (zp, sdt)
     assert cases.rel_l2(out, exp) < 1e-3, (zp, sdt)
   # an infinity stays in its row: the other rows of the tile, and of the row quad copied with it, are untouched
+  row = m - 1
+  x[row, 3] = float("inf")
+  bad = op(x.cuda(), wd, sd, zd).cpu()
+  assert torch.equal(bad[:row], out[:row])
+  assert not torch.isfinite(bad[row]).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,bm,bn", F32_SHAPES)
+def test_f32_against_f64(m, n, k, bm, bn):
+  import xla_amd.experimental.custom_kernel  # noqa: F401
+  op = torch.ops.xla.quantized_matmul
+  for zp, sdt in ((False, torch.float32), (True, torch.float32), (True, torch.bfloat16)):
+    x, w, s, _ = cases.per_channel_int8(m, n, k, torch.float32, sdt, seed=m + n)
+    z = (torch.randn(n, generator=cases.gen(5)) * 0.01).to(sdt) if zp else None
+    exp = (x.double() @ w.double().T) * s.double()
+    mag = (x.double().abs() @ w.double().abs().T) * s.double().abs()
+    if zp:
+      exp -= x.double().sum(1, keepdim=True) * z.double()
+      mag += x.double().abs().sum(1, keepdim=True) * z.double().abs()
+    wd, sd, zd = w.cuda(), s.cuda(), None if z is None else z.cuda()
+    out = op(x.cuda(), wd, sd, zd).cpu()
+    # products, sums and the few operations behind them, each within half an ulp of what it handles
+    assert out.dtype == torch.float32 and ((out.double() - exp).abs() <= (k / 2 + 8) * 2.0**-24 * mag).all(), (zp, sdt)
+    assert cases.rel_l2(out, exp) < 1e-5, (zp, sdt)
   row = m - 1
   x[row, 3] = float("inf")
   bad = op(x.cuda(), wd, sd, zd).cpu()

@@ -946,9 +946,11 @@ extern "C" int xla_amd_qmm_weight_only_skinny(const void* x, const void* w_tiled
   if (((uintptr_t)out & 15) && (N & 3) == 0)
     return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_skinny: out must be 16-byte aligned");
   if (M == 0) return XLA_AMD_QMM_OK;
-  // a batch of 17 - 32 rows against a per-channel int8 weight: K split over the waves of a workgroup where that is faster
-  if (M <= 32 && C == K && bits == 8 && x_dt != XLA_AMD_DT_F32 && qmm_wo_ksplit_tile(M, N, K) >= 0)
-    return qmm_wo_ksplit_run(x, w_tiled, scale, zp, out, M, N, K, x_dt, scale_dt, zp_dt, dot_dt, out_dt, store_dt, (hipStream_t)stream);
+  // per-channel int8 weights against 17 - 32 rows of 2-byte x or any number of f32: K split over the waves of a workgroup
+  // where that is faster
+  const int ks_tile = C != K || bits != 8 ? -1 : x_dt == XLA_AMD_DT_F32 ? qmm_wo_ksplit_f32_tile(M, N, K) : M <= 32 ? qmm_wo_ksplit_tile(M, N, K) : -1;
+  if (ks_tile >= 0)
+    return qmm_wo_ksplit_run(ks_tile, x, w_tiled, scale, zp, out, M, N, K, x_dt, scale_dt, zp_dt, dot_dt, out_dt, store_dt, (hipStream_t)stream);
   const int xsz = qmm_dt_size(x_dt), osz = qmm_dt_size(store_dt);
   const int pass = x_dt == XLA_AMD_DT_F32 ? 16 : 32;  // rows of x per pass over the weight
   for (int64_t m0 = 0; m0 < M; m0 += pass) {

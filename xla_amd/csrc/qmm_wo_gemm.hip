@@ -689,6 +689,26 @@ double plan_us(const Plan& p, int64_t M, int64_t N, int64_t K) {
   return 4.03 + 6.49 * rounds + 1.14 * rounds * steps + 0.006 * weight;
 }
 
+// The tile of least estimated time, below `limit` if there is one; -1: none.
+template <size_t n>
+int ks_best(const KsTile (&of)[n], int64_t M, int64_t N, int64_t K, bool limited, double limit) {
+  int best = -1;
+  // (32-bit divisions: this runs on every call)
+  const uint32_t m = (uint32_t)M, nn = (uint32_t)N, k128 = (uint32_t)K / 128;
+  const float weight = 1e-6f * (float)N * (float)K;
+  float least = (float)limit;
+  for (size_t i = 0; i < n; ++i) {
+    const KsTile& t = of[i];
+    const uint32_t tm = (m + t.bm - 1) / t.bm, tn = (nn + t.bn - 1) / t.bn;
+    if ((uint64_t)tm * tn > 65535) continue;
+    const uint32_t tiles = tm * tn;
+    const float rounds = (float)((tiles + 255) / 256), steps = (float)((k128 + t.kw - 1) / t.kw);
+    const float us = t.fixed + t.round * rounds + (t.step * rounds + t.load * (float)tiles / 256) * steps + t.weight * weight;
+    if ((best < 0 && !limited) || us < least) { best = (int)i; least = us; }
+  }
+  return best;
+}
+
 }  // namespace
 
 // Up to 16 rows the streaming kernel is as fast.  17 - 32 rows: against up to 8192 channels (0.72 - 0.99 of the
@@ -702,27 +722,27 @@ int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
     int per;
     if (N > 8192 || (K > 8192 && qmm_skinny_k_slices(M, N, K, K, 8, &per) > 1)) return -1;
   }
-  int best = -1;
-  double best_us = 0;
+  double limit = 0;
   if (M > 32) {
     const Plan p = make_plan(M, N, K, false);
     if (p.mt == 4 && p.ng == 4) return -1;  // more than 49152 channels: the tiled GEMM's rounds are full
-    best_us = plan_us(p, M, N, K);
+    limit = plan_us(p, M, N, K);
   }
-  for (int i = 0; i < (int)(sizeof(kKsTiles) / sizeof(kKsTiles[0])); ++i) {
-    const KsTile& t = kKsTiles[i];
-    const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn);
-    if (tiles > 4096) continue;
-    const double rounds = (double)((tiles + 255) / 256), steps = (double)((K / 128 + t.kw - 1) / t.kw);
-    const double us = t.fixed + t.round * rounds + (t.step * rounds + t.load * (double)tiles / 256) * steps + t.weight * 1e-6 * (double)N * (double)K;
-    if ((best < 0 && M <= 32) || us < best_us) { best = i; best_us = us; }
-  }
-  return best;
+  return ks_best(kKsTiles, M, N, K, M > 32, limit);
 }
 
-int qmm_wo_ksplit_run(const void* x, const void* w_tiled, const void* scale, const void* zp, void* out, int64_t M, int64_t N,
+// Fewer than 128 rows: always (0.93 of the streaming kernel's time at most, see qmm_wo_ksplit.hip).  More: while that is
+// the shorter of the two estimates; the other is x split into three bf16 parts, 11 us and per round of 128 x 128 tiles
+// 3.2 + 0.78 per 128 of 3 K columns (measured at 128 - 700 rows: 512 x 1024 x 4096 92 -> 39 us, 200 x 4096 x 4096 90 ->
+// 69; 256 x 6144 x 4096 would be 90 -> 112).
+int qmm_wo_ksplit_f32_tile(int64_t M, int64_t N, int64_t K) {
+  if (K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14)) return -1;
+  const double rounds = (double)(((M + 127) / 128 * ((N + 127) / 128) + 255) / 256);
+  return ks_best(kKsTilesF32, M, N, K, M >= 128, 11 + rounds * (3.2 + 0.78 * (double)(3 * K / 128)));
+}
+
+int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* scale, const void* zp, void* out, int64_t M, int64_t N,
                       int64_t K, int x_dt, int scale_dt, int zp_dt, int dot_dt, int out_dt, int store_dt, hipStream_t s) {
-  const int tile = qmm_wo_ksplit_tile(M, N, K);
   WoGemmArgs a;
   a.x = x; a.w = (const uint8_t*)w_tiled; a.scale = scale; a.zp = zp; a.out = out;
   a.part = nullptr; a.part_xs = nullptr;
@@ -731,6 +751,7 @@ int qmm_wo_ksplit_run(const void* x, const void* w_tiled, const void* scale, con
   a.G = xla_amd_qmm_tile_group(N, K, K, 8);
   a.k_per_split = (int)K; a.split = 1;
   a.scale_dt = scale_dt; a.zp_dt = zp ? zp_dt : x_dt; a.dot_dt = dot_dt; a.out_dt = out_dt; a.store_dt = store_dt;
+  if (x_dt == XLA_AMD_DT_F32) return tile < 3 ? qmm_wo_ksplit_launch_f32_0(a, tile, s) : qmm_wo_ksplit_launch_f32_1(a, tile, s);
   if (x_dt == XLA_AMD_DT_BF16)
     return tile < 4 ? qmm_wo_ksplit_launch_bf16_0(a, tile, s) : tile < 7 ? qmm_wo_ksplit_launch_bf16_1(a, tile, s) : qmm_wo_ksplit_launch_bf16_2(a, tile, s);
   return tile < 4 ? qmm_wo_ksplit_launch_f16_0(a, tile, s) : tile < 7 ? qmm_wo_ksplit_launch_f16_1(a, tile, s) : qmm_wo_ksplit_launch_f16_2(a, tile, s);
@@ -789,6 +810,9 @@ extern "C" int xla_amd_qmm_weight_only_gemm_f32(const float* x, const void* w_ti
   if (!workspace || workspace_bytes < need)
     return qmm_fail(XLA_AMD_QMM_EINVAL, "weight_only_gemm_f32: workspace of %zu bytes, need %zu", workspace ? workspace_bytes : (size_t)0, need);
   hipStream_t s = (hipStream_t)stream;
+  const int ks_tile = qmm_wo_ksplit_f32_tile(M, N, K);
+  if (ks_tile >= 0)
+    return qmm_wo_ksplit_run(ks_tile, x, w_tiled, scale, zp, out, M, N, K, XLA_AMD_DT_F32, scale_dt, zp_dt, XLA_AMD_DT_F32, XLA_AMD_DT_F32, XLA_AMD_DT_F32, s);
   const int64_t quads = M * (K / 4);
   hipLaunchKernelGGL(qmm_split3_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, x, (uint16_t*)workspace, quads, (int)K);
   int rc = QMM_CHECK_LAUNCH("weight_only_gemm_f32 split launch");
@@ -855,8 +879,9 @@ extern "C" int xla_amd_qmm_weight_only_gemm(const void* x, const void* w_tiled, 
     return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_gemm: out must be 16-byte aligned");
   if (M == 0) return XLA_AMD_QMM_OK;
   const bool blockwise = C != K;
-  if (!blockwise && bits == 8 && qmm_wo_ksplit_tile(M, N, K) >= 0)
-    return qmm_wo_ksplit_run(x, w_tiled, scale, zp, out, M, N, K, x_dt, scale_dt, zp_dt, dot_dt, out_dt, store_dt, (hipStream_t)stream);
+  const int ks_tile = !blockwise && bits == 8 ? qmm_wo_ksplit_tile(M, N, K) : -1;
+  if (ks_tile >= 0)
+    return qmm_wo_ksplit_run(ks_tile, x, w_tiled, scale, zp, out, M, N, K, x_dt, scale_dt, zp_dt, dot_dt, out_dt, store_dt, (hipStream_t)stream);
   // (blockwise weights in the weight-streaming kernel: every dtype but the stored one is x's, at least 8 scales)
   const bool bw_ok = !blockwise || (scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt && (K / C) * N >= 8 &&
                                     (((uintptr_t)scale | (uintptr_t)zp) & 3) == 0);

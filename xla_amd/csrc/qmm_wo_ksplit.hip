@@ -1,5 +1,5 @@
-// Weight-only quantized matmul for a batch of rows (a decode batch of more than 16 sequences up to short prompts):
-// per-channel int8 weights against bf16 / f16 rows, K split over the waves of a workgroup.
+// Weight-only quantized matmul for a batch of rows (a decode batch of more than 16 sequences up to short prompts) and for
+// f32 rows: per-channel int8 weights, K split over the waves of a workgroup.
 //
 // Between the weight-streaming kernel (qmm_skinny.hip) and the tiled GEMM (qmm_wo_gemm.hip) lie the launches whose
 // time is what every compute unit has to fetch: BM rows of x and BN channels of weights over all of K,
@@ -25,10 +25,14 @@
 // ring where ragged rows leave room for it; conversions placed by hand between the MFMAs (12.1 -> 12.8: the wave needs
 // its weights a quarter of a step earlier); workgroups that start at different columns (within 3 % either way).
 //
-// This file is compiled per activation dtype and set of tiles (-DQMM_WO_XT=1|2 for bf16 | f16, -DQMM_KS_PART=0|1|2).
-#include "qmm_common.h"
-#include "qmm_frag.h"
-#include "qmm_wo_gemm.h"
+// f32 rows (any number of them below 128, and more where the launch has few tiles) run the same kernel on 16x16x4 f32
+// MFMAs, one column per lane and instruction: true f32 products, an eighth of the bf16 rate, so the matrix cores bound
+// all but the smallest launches (64 x 4096 x 4096: 22 us, 14 of them MFMAs).  The streaming kernel before it made a pass
+// over the weight per 16 rows and split K over two waves at most, 512 columns each: 8 x 1024 x 1024 6.6 -> 4.6 us, 32 x
+// 4096 x 4096 25.6 -> 14.4, 100 x 1024 x 1024 43 -> 6.5; over 300 shapes of 1 - 127 rows 0.49 of the time, 0.93 at most.
+//
+// This file is compiled per activation dtype and set of tiles (-DQMM_WO_XT=0|1|2 for f32 | bf16 | f16, -DQMM_KS_PART=0|1|2).
+#include "qmm_wo_ksplit.h"
 
 #if !defined(QMM_WO_XT) || !defined(QMM_KS_PART)
 #error "compile with -DQMM_WO_XT=<XLA_AMD_DT_BF16|XLA_AMD_DT_F16 value> -DQMM_KS_PART=<0|1|2>"
@@ -36,120 +40,51 @@
 
 namespace {
 
-using namespace qmm_frag;
-
-constexpr int kCopyWaves = 4;
-constexpr int kLds = 160 * 1024;
-
-// The launch's tiles: rows per tile (M spread evenly over the row tiles), row tiles, all tiles.
-struct KsTiles {
-  int rows, tiles_m, tiles;
-  uint64_t tiles_m_magic;  // ceil(2^32 / tiles_m)
-};
-
-template <int MT, int NG, int KW, int CW> struct KsCfg {
-  static constexpr int NW = KW * CW;             // computing waves
-  static constexpr int BM = 16 * MT, BN = 16 * NG * CW;
-  static constexpr int TILE = BM * 256;          // bytes of the x columns of one tile (128 columns, 2-byte x)
-  static constexpr int SLOT = KW * TILE;
-  static constexpr int PITCH = BN + 4;           // floats per row of the partial sums (4 more: rows start on other banks)
-  static constexpr int kSums = KW * BM * (PITCH + 1) * 4;  // partial sums, and partial row sums of x
-  static constexpr int kTail = 2 * BN * 4;       // scales and zero points as f32
-  static constexpr int kFit = (kLds - kTail) / SLOT;
-  static constexpr int R = kFit < 8 ? kFit : 8;  // slots of the ring
-  static_assert(R >= 2, "the ring needs room to run ahead");
-  static constexpr int lds_bytes(int steps) {
-    const int ring = (steps < R ? steps : R) * SLOT;
-    return kTail + (ring > kSums ? ring : kSums);
-  }
-  static_assert(kTail + kSums <= kLds, "the partial sums fit");
-};
+// scales and zero points of the tile as f32
+template <int NG, int CW> constexpr int ks_tail() { return 2 * 16 * NG * CW * 4; }
 
 template <int XT, int MT, int NG, int KW, int CW, int P, bool HASZP, bool UNI>
 __global__ void __launch_bounds__((KW * CW + kCopyWaves) * 64)
 qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
-  using Cfg = KsCfg<MT, NG, KW, CW>;
-  constexpr int NW = Cfg::NW, BM = Cfg::BM, BN = Cfg::BN, TILE = Cfg::TILE, SLOT = Cfg::SLOT, R = Cfg::R, D = R - 1;
+  using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, ks_tail<NG, CW>()>;
+  constexpr bool kF32 = XT == XLA_AMD_DT_F32;
+  constexpr int NW = Cfg::NW, BM = Cfg::BM, BN = Cfg::BN, TILE = Cfg::TILE, SLOT = Cfg::SLOT, R = Cfg::R;
   constexpr int kThreads = (NW + kCopyWaves) * 64;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* const scl = (float*)smem;          // [BN] scales, [BN] zero points
-  char* const ring = smem + Cfg::kTail;     // x slots; afterwards the partial sums
-  float* const red = (float*)ring;          // [KW][BM][PITCH]
+  float* const scl = (float*)smem;             // [BN] scales, [BN] zero points
+  char* const ring = smem + ks_tail<NG, CW>(); // x slots; afterwards the partial sums
+  float* const red = (float*)ring;             // [KW][BM][PITCH]
   float* const xsr = red + KW * BM * Cfg::PITCH;  // [KW][BM] partial row sums of x
-  typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int M = a.M, N = a.N, K = a.K;
-  // Workgroups are dealt round-robin to the 8 XCDs: each XCD gets a contiguous run of the tiles, row tiles fastest, so
-  // that the row tiles of a column share its weights in that L2 (tile / tiles_m by multiply-shift: tile < 2^16).
-  const int tile = ((int)blockIdx.x & 7) * (int)(gridDim.x >> 3) + ((int)blockIdx.x >> 3);
-  if (tile >= t.tiles) return;
-  const int col = (int)(((uint64_t)(uint32_t)tile * t.tiles_m_magic) >> 32);
-  const int n0 = col * BN;
-  const int m0 = (tile - col * t.tiles_m) * t.rows;
-  const int rows = min(t.rows, M - m0);
+  int n0, m0, rows;
+  if (!ks_tile_of(t, M, BN, n0, m0, rows)) return;
   const int n_tiles = K / 128;
   const int steps = (n_tiles + KW - 1) / KW;
   const WoDts<XT, UNI> dts(a);
 
-  f32x4 acc[NG][MT], xs[MT];
-  uint32_t s_raw = 0, z_raw = 0;
   if (__builtin_expect(wave >= NW, 0)) {
-    // ---- copying waves ----
+    // ---- copying waves: x, and the scales of the tile's channels, which are used at the very end ----
     const int cw = wave - NW;
-    const int quads = (rows + 3) >> 2;                         // an instruction copies four rows of 256 bytes
-    const int nq = quads > cw ? (quads - cw + 3) >> 2 : 0;     // of this wave: cw, cw + 4, ...
-    const char* const xb = (const char*)a.x + (size_t)m0 * K * 2;
-    uint32_t x_off[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int row = min((cw + i * kCopyWaves) * 4 + (lane >> 4), rows - 1);
-      x_off[i] = (uint32_t)row * ((uint32_t)K * 2u) + (uint32_t)(((lane & 15) ^ (row & 15)) * 16);
-    }
-    int issued = 0, slot = 0;
-    auto issue = [&]() __attribute__((always_inline)) {
-      char* const dst = ring + slot * SLOT;
-#pragma unroll
-      for (int k = 0; k < KW; ++k) {
-        const char* const src = xb + (size_t)min(issued * KW + k, n_tiles - 1) * 256;
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-          if (i < nq)
-            __builtin_amdgcn_global_load_lds((const void*)(src + (size_t)x_off[i]), (lds_ptr_t)(dst + k * TILE + (cw + i * kCopyWaves) * 1024), 16, 0, 0);
-      }
-      ++issued;
-      slot = slot + 1 == R ? 0 : slot + 1;
-    };
-    while (issued < min(D, steps)) issue();
-    // the scales of the tile's channels: used at the very end
-    if (cw * 64 + lane < BN) {
-      const int n = min(n0 + cw * 64 + lane, N - 1);
-      s_raw = qmm_load_raw(a.scale, n, dts.scale_dt);
-      if constexpr (HASZP) z_raw = qmm_load_raw(a.zp, n, dts.zp_dt);
-    }
-    for (int n = 0; n < steps; ++n) {
-      // the loads of the slots after n may be in flight (a wave's loads complete in order)
-      const int ahead = issued - 1 - n;
-      bool done = false;
-      qmm_static_for<D>([&](auto dc) {
-        qmm_static_for<MT + 1>([&](auto qc) {
-          constexpr int c = (int)dc * KW * (int)qc;
-          if (!done && ahead == (int)dc && nq == (int)qc) {
-            qmm_wait_vmcnt<(c < 63 ? c : 63)>();
-            done = true;
+    uint32_t s_raw = 0, z_raw = 0;
+    ks_copy_x<Cfg, MT, KW>(
+        a.x, K, m0, rows, steps, cw, lane, ring, [&](int n, int k) { return min(n * KW + k, n_tiles - 1); },
+        [&]() {
+          if (cw * 64 + lane < BN) {
+            const int n = min(n0 + cw * 64 + lane, N - 1);
+            s_raw = qmm_load_raw(a.scale, n, dts.scale_dt);
+            if constexpr (HASZP) z_raw = qmm_load_raw(a.zp, n, dts.zp_dt);
+          }
+        },
+        [&]() {
+          if (cw * 64 + lane < BN) {
+            scl[cw * 64 + lane] = qmm_from_raw(s_raw, dts.scale_dt);
+            if constexpr (HASZP) scl[BN + cw * 64 + lane] = qmm_from_raw(z_raw, dts.zp_dt);
           }
         });
-      });
-      qmm_bare_barrier();  // slot n is there; the computing waves have read slot n - 1
-      if (issued < steps) issue();
-    }
-    if (cw * 64 + lane < BN) {
-      scl[cw * 64 + lane] = qmm_from_raw(s_raw, dts.scale_dt);
-      if constexpr (HASZP) scl[BN + cw * 64 + lane] = qmm_from_raw(z_raw, dts.zp_dt);
-    }
-    qmm_bare_barrier();  // the computing waves have read the last slot
   } else {
     // ---- computing waves: wave (kw, cw) multiplies the tiles kw, kw + KW, ... against its NG row sets of 16 channels ----
     const int kw = wave / CW, cw = wave % CW;
@@ -180,6 +115,7 @@ qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
       request((int)pc, pc, qmm_const<1>{});
     });
     __builtin_amdgcn_sched_barrier(0);
+    f32x4 acc[NG][MT], xs[MT];
     qmm_static_for<MT>([&](auto mc) {
       xs[(int)mc] = f32x4{0, 0, 0, 0};
       qmm_static_for<NG>([&](auto gc) { acc[(int)gc][(int)mc] = f32x4{0, 0, 0, 0}; });
@@ -187,30 +123,46 @@ qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
     auto step = [&](int s, int slot, auto pc) __attribute__((always_inline)) {
       constexpr int p = pc;
       qmm_bare_barrier();
-      const char* const xrow = ring + slot * SLOT + kw * TILE + r * 256;
+      const char* const xrow = ring + slot * SLOT + kw * TILE + r * Cfg::ROW;
       const bool live = s * KW + kw < n_tiles;  // (the last slot may hold fewer than KW tiles)
+      constexpr int J = Cfg::ROW / 64;  // 16-byte pieces of a row of the tile per lane
       i32x4 xq[2][MT];
       auto read = [&](auto jc) __attribute__((always_inline)) {
         constexpr int j = jc;
-        qmm_static_for<MT>([&](auto mc) { xq[j & 1][(int)mc] = *(const i32x4*)(xrow + (int)mc * (16 * 256) + (((4 * g + j) ^ r) * 16)); });
+        qmm_static_for<MT>([&](auto mc) { xq[j & 1][(int)mc] = *(const i32x4*)(xrow + (int)mc * (16 * Cfg::ROW) + (((J * g + j) ^ r) * 16)); });
       };
       read(qmm_const<0>{});
-      qmm_static_for<4>([&](auto jc) {
+      qmm_static_for<J>([&](auto jc) {
         constexpr int j = jc;
-        if constexpr (j < 3) read(qmm_const<j + 1>{});
+        if constexpr (j + 1 < J) read(qmm_const<j + 1>{});
         __builtin_amdgcn_sched_barrier(0);
         if (live) {
-          qmm_static_for<NG>([&](auto gc) {
-            constexpr int gi = gc;
-            const i32x4 src = wreg[p][j >> 1][gi];
-            const i32x4 af = cvt_w8<XT>((uint32_t)src[(j & 1) * 2], (uint32_t)src[(j & 1) * 2 + 1]);
-            qmm_static_for<MT>([&](auto mc) { acc[gi][(int)mc] = mfma16<XT>(af, xq[j & 1][(int)mc], acc[gi][(int)mc]); });
-          });
-          if constexpr (HASZP) {
-            qmm_static_for<MT>([&](auto mc) { xs[(int)mc] = mfma16<XT>(ones_frag<XT>(), xq[j & 1][(int)mc], xs[(int)mc]); });
+          if constexpr (kF32) {
+            // columns 32 g + 4 j .. + 3, one per instruction (true f32 products); their sum by vector instructions: an
+            // MFMA against ones takes as long as one against weights
+            qmm_static_for<4>([&](auto ec) {
+              constexpr int e = ec;
+              qmm_static_for<NG>([&](auto gc) {
+                const float wf = (float)(int8_t)((uint32_t)wreg[p][j >> 2][(int)gc][j & 3] >> (8 * e));
+                qmm_static_for<MT>([&](auto mc) {
+                  acc[(int)gc][(int)mc] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf, __builtin_bit_cast(f32x4, xq[j & 1][(int)mc])[e], acc[(int)gc][(int)mc], 0, 0, 0);
+                });
+              });
+              if constexpr (HASZP) qmm_static_for<MT>([&](auto mc) { xs[(int)mc][e] += __builtin_bit_cast(f32x4, xq[j & 1][(int)mc])[e]; });
+            });
+          } else {
+            qmm_static_for<NG>([&](auto gc) {
+              constexpr int gi = gc;
+              const i32x4 src = wreg[p][j >> 1][gi];
+              const i32x4 af = cvt_w8<XT>((uint32_t)src[(j & 1) * 2], (uint32_t)src[(j & 1) * 2 + 1]);
+              qmm_static_for<MT>([&](auto mc) { acc[gi][(int)mc] = mfma16<XT>(af, xq[j & 1][(int)mc], acc[gi][(int)mc]); });
+            });
+            if constexpr (HASZP) {
+              qmm_static_for<MT>([&](auto mc) { xs[(int)mc] = mfma16<XT>(ones_frag<XT>(), xq[j & 1][(int)mc], xs[(int)mc]); });
+            }
           }
         }
-        if constexpr ((j & 1) == 1) request(s + P, pc, qmm_const<(j >> 1)>{});
+        if constexpr (j % (J / 2) == J / 2 - 1) request(s + P, pc, qmm_const<j / (J / 2)>{});
         __builtin_amdgcn_sched_barrier(0);
       });
     };
@@ -235,7 +187,13 @@ qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
         *(f32x4*)(red + ((size_t)kw * BM + row) * Cfg::PITCH + (cw * NG + gi) * 16 + 4 * g) = acc[gi][mt];
       });
       if constexpr (HASZP) {
-        if (cw == 0 && g == 0) xsr[kw * BM + row] = xs[mt][0];
+        float sum = xs[mt][0];
+        if constexpr (kF32) {  // four of the lane's columns each, and a quarter of the row per lane
+          sum = (xs[mt][0] + xs[mt][1]) + (xs[mt][2] + xs[mt][3]);
+          sum += __shfl_xor(sum, 16);
+          sum += __shfl_xor(sum, 32);
+        }
+        if (cw == 0 && g == 0) xsr[kw * BM + row] = sum;
       }
     });
   }
@@ -263,12 +221,8 @@ qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
 
 template <int XT, int MT, int NG, int KW, int CW, int P>
 int launch(const WoGemmArgs& a, hipStream_t stream) {
-  using Cfg = KsCfg<MT, NG, KW, CW>;
-  KsTiles t;
-  t.tiles_m = (a.M + Cfg::BM - 1) / Cfg::BM;
-  t.rows = (a.M + t.tiles_m - 1) / t.tiles_m;
-  t.tiles = t.tiles_m * ((a.N + Cfg::BN - 1) / Cfg::BN);
-  t.tiles_m_magic = (((uint64_t)1 << 32) + t.tiles_m - 1) / t.tiles_m;
+  using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, ks_tail<NG, CW>()>;
+  const KsTiles t = ks_tiles(a.M, a.N, Cfg::BM, Cfg::BN);
   const dim3 grid(8u * (unsigned)((t.tiles + 7) / 8)), block((Cfg::NW + kCopyWaves) * 64);
   const int steps = (a.K / 128 + KW - 1) / KW;
   auto go = [&](auto which) -> int {
@@ -292,13 +246,25 @@ int launch(const WoGemmArgs& a, hipStream_t stream) {
 #define QMM_KS_CAT(a, b) QMM_KS_CAT2(a, b)
 #if QMM_WO_XT == XLA_AMD_DT_BF16
 #define QMM_KS_NAME QMM_KS_CAT(qmm_wo_ksplit_launch_bf16_, QMM_KS_PART)
-#else
+#elif QMM_WO_XT == XLA_AMD_DT_F16
 #define QMM_KS_NAME QMM_KS_CAT(qmm_wo_ksplit_launch_f16_, QMM_KS_PART)
+#else
+#define QMM_KS_NAME QMM_KS_CAT(qmm_wo_ksplit_launch_f32_, QMM_KS_PART)
 #endif
-// tile: index into kKsTiles (qmm_wo_gemm.h)
+// tile: index into kKsTiles, or kKsTilesF32 (qmm_wo_gemm.h)
 int QMM_KS_NAME(const WoGemmArgs& a, int tile, hipStream_t stream) {
   switch (tile) {
+#if QMM_WO_XT == XLA_AMD_DT_F32
 #if QMM_KS_PART == 0
+    case 0: return launch<QMM_WO_XT, 1, 1, 8, 1, 2>(a, stream);
+    case 1: return launch<QMM_WO_XT, 1, 2, 8, 1, 2>(a, stream);
+    case 2: return launch<QMM_WO_XT, 1, 4, 8, 1, 1>(a, stream);
+#elif QMM_KS_PART == 1
+    case 3: return launch<QMM_WO_XT, 1, 1, 4, 1, 2>(a, stream);
+    case 4: return launch<QMM_WO_XT, 2, 1, 4, 2, 2>(a, stream);
+    case 5: return launch<QMM_WO_XT, 2, 2, 4, 2, 1>(a, stream);
+#endif
+#elif QMM_KS_PART == 0
     case 0: return launch<QMM_WO_XT, 1, 1, 8, 1, 2>(a, stream);
     case 1: return launch<QMM_WO_XT, 1, 2, 8, 1, 2>(a, stream);
     case 2: return launch<QMM_WO_XT, 2, 1, 4, 2, 2>(a, stream);
@@ -307,7 +273,7 @@ int QMM_KS_NAME(const WoGemmArgs& a, int tile, hipStream_t stream) {
     case 4: return launch<QMM_WO_XT, 3, 2, 4, 1, 2>(a, stream);
     case 5: return launch<QMM_WO_XT, 3, 2, 4, 2, 1>(a, stream);
     case 6: return launch<QMM_WO_XT, 4, 2, 4, 2, 1>(a, stream);
-#else
+#elif QMM_KS_PART == 2
     case 7: return launch<QMM_WO_XT, 4, 3, 4, 2, 1>(a, stream);
     case 8: return launch<QMM_WO_XT, 4, 4, 4, 2, 1>(a, stream);
 #endif
