@@ -725,6 +725,19 @@ class XlaQuantizedLinear(torch.nn.Module):
     return self._tiled_from == (_version_of(self.weight), self.weight.data_ptr())
 
   def forward(self, x):
+    # (an eager call on the GPU is bound by what happens here: tensors out of `_buffers` cost a tenth of Module's
+    # __getattr__, five of which took 1.6 of the 8.1 us of a call; what is no plain buffer any more - a Parameter, a
+    # parametrization - takes the attributes below, and so does a graph that is being traced)
+    buffers = self._buffers
+    scaler, weight = buffers.get('weight_scaler'), buffers.get('weight')
+    if scaler is not None and weight is not None and not torch.compiler.is_compiling():
+      zero_point = buffers['zero_point'] if 'zero_point' in buffers else self.zero_point
+      tiled = buffers.get('_weight_tiled')
+      if tiled is not None and x.is_cuda and (self._released_shape is not None or
+                                              self._tiled_from == (_version_of(weight), weight.data_ptr())):
+        return _weight_only_tiled_op(x, tiled, scaler, zero_point, self.output_dim, self.block_size, self.int4_weight)
+      return _quantized_matmul_op(x, weight, scaler, zero_point, self.block_size, self.int4_weight,
+                                  self.quantize_activation)
     if x.is_cuda and self._tiled_is_current():
       return _weight_only_tiled_op(x, self._weight_tiled, self.weight_scaler, self.zero_point, self.output_dim,
                                    self.block_size, self.int4_weight)
