@@ -35,6 +35,40 @@ F32_SHAPES = [
 ]
 
 
+# blockwise and int4 weights (m, n, k, c, bits, zero point, rows and channels of the tile): c = -1 is per-channel; blocks of
+# one, two, three and five tiles of 128 columns; fewer blocks than K groups, and a last round that not every group has
+BW_SHAPES = [
+    (17, 20, 256, 128, 4, True, 16, 16), (64, 132, 2176, 128, 8, True, 16, 16), (33, 100, 1920, 640, 4, False, 16, 16),
+    (17, 2300, 2304, 256, 4, False, 16, 32), (100, 1024, 1152, 128, 4, True, 16, 32),
+    (32, 5000, 384, 384, 4, True, 32, 32), (64, 4096, 1152, 128, 8, False, 32, 32), (40, 4100, 2560, 256, 8, True, 48, 32),
+    (65, 4096, 1280, 128, 4, True, 48, 32), (48, 6144, 640, -1, 4, True, 48, 32),
+    (48, 12000, 1152, 128, 4, True, 48, 64), (96, 6000, 768, 256, 8, False, 48, 64),
+    (128, 4096, 640, 128, 4, True, 64, 32), (200, 2048, 1152, -1, 4, False, 64, 32),
+    (200, 4096, 1152, 128, 4, False, 64, 64), (250, 4000, 1536, 512, 8, False, 64, 64),
+]
+
+
+def test_tiles_of_the_blockwise_shapes(tmp_path):
+  calls = [rec.blockwise(m, n, k, k if c == -1 else c, bits, zp, dt) for m, n, k, c, bits, zp, _, _ in BW_SHAPES for dt in (1, 2)]
+  calls += [rec.skinny(m, n, k, k if c == -1 else c, bits, zp, 1) for m, n, k, c, bits, zp, _, _ in BW_SHAPES if m <= 64]
+  want = {(m, n, k): (bm, bn) for m, n, k, _, _, _, bm, bn in BW_SHAPES}
+  got = {}
+  for (_, _, args), (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0, text
+    m, n, k = args[7:10] if len(args) > 18 else args[5:8]
+    (l,) = launches
+    mt, ng, kw, cw = (int(v) for v in re.search(r"_ksplitILi\dELi\dELi(\d)ELi(\d)ELi(\d)ELi(\d)E", l.name).groups())
+    assert l.lds <= l.lds_limit and l.block[0] == 64 * (kw * cw + 4)
+    got[m, n, k] = (16 * mt, 16 * ng * cw)
+  assert got == want
+  assert len(set(want.values())) == 7
+  # scales of another dtype, 16 rows or fewer and wide outputs of up to 64 keep the streaming kernel
+  name, sig, args = rec.skinny(40, 64, 256, 256, 4, False, 1)
+  calls = [(name, sig, args[:11] + [0, 1, 1, 0, 0] + args[-1:]), rec.skinny(16, 2048, 2048, 128, 4, True), rec.skinny(64, 32768, 1024, 128, 4, True)]
+  for rc, text, launches in rec.record(calls, str(tmp_path)):
+    assert rc == 0 and launches and not any("ksplit" in l.name for l in launches), text
+
+
 def test_tiles_of_the_f32_shapes(tmp_path):
   calls = [rec.skinny(m, n, k, k, 8, zp, 0) for m, n, k, _, _ in F32_SHAPES for zp in (False, True)]
   seen = set()
@@ -122,6 +156,30 @@ def test_f32_against_f64(m, n, k, bm, bn):
   bad = op(x.cuda(), wd, sd, zd).cpu()
   assert torch.equal(bad[:row], out[:row])
   assert not torch.isfinite(bad[row]).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,c,bits,zp,bm,bn", BW_SHAPES)
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_blockwise_against_the_oracle(m, n, k, c, bits, zp, bm, bn, xdt):
+  import xla_amd.experimental.custom_kernel  # noqa: F401
+  op = torch.ops.xla.quantized_matmul
+  if c == -1:
+    x, w, s, _ = cases.per_channel_int8(m, n, k, xdt, xdt, seed=m)
+    w, z = w.clamp(-8, 7), (torch.randn(n, generator=cases.gen(5)) * 0.01).to(xdt)
+  else:
+    x, w, s, z, _ = cases.blockwise(m, n, k, c, bits, xdt, symmetric=not zp, seed=m + k)
+  z = z if zp else None
+  exp = oracle.quantized_matmul(x, w, s, z, block_size=c, int4_weight=bits == 4)
+  wd, sd, zd = w.cuda(), s.cuda(), None if z is None else z.cuda()
+  out = op(x.cuda(), wd, sd, zd, c, bits == 4).cpu()
+  # f32 sums in another order: a dot product rounds to its other neighbour now and then (the bound of the tiled GEMM)
+  assert out.dtype == exp.dtype and cases.within_tolerance(out, exp)
+  assert cases.rel_l2(out, exp) < 1e-3
+  x[m - 1, 3] = float("inf")
+  bad = op(x.cuda(), wd, sd, zd, c, bits == 4).cpu()
+  assert torch.equal(bad[:m - 1], out[:m - 1])
+  assert not torch.isfinite(bad[m - 1]).any()
 
 
 @pytest.mark.gpu

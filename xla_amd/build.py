@@ -36,6 +36,8 @@ SOURCES = [
     ("qmm_wo_gemm.hip", ["-DQMM_WO_XT=2", "-DQMM_WO_MT=4"], "qmm_wo_gemm_f16_mt4.o"),
     *[("qmm_wo_ksplit.hip", ["-DQMM_WO_XT=%d" % xt, "-DQMM_KS_PART=%d" % part], "qmm_wo_ksplit_%s_%d.o" % (name, part))
       for xt, name, parts in ((1, "bf16", 3), (2, "f16", 3), (0, "f32", 2)) for part in range(parts)],
+    *[("qmm_wo_ksplit_bw.hip", ["-DQMM_WO_XT=%d" % xt, "-DQMM_KS_BITS=%d" % bits], "qmm_wo_ksplit_bw_%s_%d.o" % (name, bits))
+      for xt, name in ((1, "bf16"), (2, "f16")) for bits in (4, 8)],
     ("qmm_wo_gemm_bw.hip", ["-DQMM_WO_BW_XT=1"], "qmm_wo_gemm_bw_bf16.o"),
     ("qmm_wo_gemm_bw.hip", ["-DQMM_WO_BW_XT=2"], "qmm_wo_gemm_bw_f16.o"),
     ("qmm_wo_gemm_bw_wide.hip", ["-DQMM_WO_BW_XT=1"], "qmm_wo_gemm_bw_wide_bf16.o"),

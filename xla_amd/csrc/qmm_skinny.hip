@@ -44,6 +44,7 @@
 
 #include "qmm_frag.h"
 #include "qmm_skinny.h"
+#include "qmm_wo_bw.h"
 #include "qmm_wo_gemm.h"
 
 // Diagnostic build (-DQMM_SKINNY_TIMELINE, a library of its own; see xla_amd/build.py): every wave
@@ -951,6 +952,15 @@ extern "C" int xla_amd_qmm_weight_only_skinny(const void* x, const void* w_tiled
   const int ks_tile = C != K || bits != 8 ? -1 : x_dt == XLA_AMD_DT_F32 ? qmm_wo_ksplit_f32_tile(M, N, K) : M <= 32 ? qmm_wo_ksplit_tile(M, N, K) : -1;
   if (ks_tile >= 0)
     return qmm_wo_ksplit_run(ks_tile, x, w_tiled, scale, zp, out, M, N, K, x_dt, scale_dt, zp_dt, dot_dt, out_dt, store_dt, (hipStream_t)stream);
+  // the same for blockwise and int4 weights against 17 - 64 rows of 2-byte x, every dtype x's
+  if ((C != K || bits == 4) && M <= 64 && x_dt != XLA_AMD_DT_F32 && scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt &&
+      store_dt == x_dt && (((uintptr_t)scale | (uintptr_t)zp) & 3) == 0) {
+    const int tile = qmm_wo_ksplit_bw_tile(M, N, K, C, bits, zp != nullptr);
+    if (tile >= 0) {
+      const WoBwArgs b{x, (const uint8_t*)w_tiled, scale, zp, out, (int)M, (int)N, (int)K, (int)C};
+      return qmm_wo_ksplit_bw_run(tile, b, bits, x_dt, (hipStream_t)stream);
+    }
+  }
   const int xsz = qmm_dt_size(x_dt), osz = qmm_dt_size(store_dt);
   const int pass = x_dt == XLA_AMD_DT_F32 ? 16 : 32;  // rows of x per pass over the weight
   for (int64_t m0 = 0; m0 < M; m0 += pass) {

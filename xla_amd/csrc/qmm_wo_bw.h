@@ -23,6 +23,36 @@ int qmm_wo_bw_launch_f16(const WoBwArgs& a, int bits, hipStream_t stream);
 int qmm_wo_bw_wide_launch_bf16(const WoBwArgs& a, int bits, int cus, hipStream_t stream);
 int qmm_wo_bw_wide_launch_f16(const WoBwArgs& a, int bits, int cus, hipStream_t stream);
 
+// ---- K split over the waves of a workgroup (qmm_wo_ksplit_bw.hip) ----
+// Tiles of that kernel: rows, channels, K groups of waves, whether it takes a zero point, and the time of a launch, us,
+// as fitted to 78 - 185 measured launches per tile (8 - 1000 rows, 18 weights of N 512 - 14336, K 1024 - 14336, 4 and 8
+// bits; root mean square error 7 - 11 %):
+//   fixed + round * rounds + (step + zp (with a zero point) + int8 (8 bits)) * rounds * steps + load * tiles / 256 * steps
+//     + weight * (bytes of the weight) / 10^6
+// rounds of 256 tiles, steps of 128 columns per wave (whole blocks).
+struct KsBwTile {
+  uint32_t bm, bn, kw;
+  bool with_zp;
+  float fixed, round, step, load, weight, zp, int8;
+};
+constexpr KsBwTile kKsBwTiles[] = {
+    {16, 16, 8, true, 2.46f, 0.10f, 0.681f, 0.252f, 0.032f, 0.185f, 0.197f},
+    {16, 32, 8, true, 1.72f, 1.08f, 0.906f, 0.130f, 0.080f, 0.282f, 0.231f},
+    {32, 32, 4, true, 1.62f, 1.67f, 0.648f, 0.116f, 0.061f, 0.189f, -0.036f},
+    {48, 32, 4, true, 1.46f, 1.87f, 0.748f, 0.091f, 0.103f, 0.267f, 0.008f},
+    {48, 64, 4, true, 0.95f, 2.90f, 1.034f, 0.085f, 0.083f, 0.351f, -0.026f},
+    {64, 32, 4, true, 1.43f, 2.12f, 0.819f, 0.188f, 0.069f, 0.258f, -0.054f},
+    {64, 64, 4, false, 0.64f, 3.27f, 1.200f, 0.167f, 0.074f, 0.000f, -0.077f},
+};
+// The tile a launch of M rows runs with (-1: not one for this kernel): bf16 or f16 x and every other dtype x's, blockwise
+// (C < K, C % 128 == 0) or int4 weights, N % 4 == 0.
+int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, bool zp);
+int qmm_wo_ksplit_bw_run(int tile, const WoBwArgs& a, int bits, int x_dt, hipStream_t stream);
+int qmm_wo_ksplit_bw_launch_bf16_4(const WoBwArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_bw_launch_bf16_8(const WoBwArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_bw_launch_f16_4(const WoBwArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_bw_launch_f16_8(const WoBwArgs& a, int tile, hipStream_t stream);
+
 // Two dot products rounded to x's dtype, as f32.  bf16: one at a time, beside a zero, which leaves the value in f32 (as a
 // pair and unpacked again it is three instructions for two; 2048 x 4096 x 4096 int4 in blocks of 128 with zero points:
 // 80.5 -> 77.0 us).  f16: as a pair (one at a time 77.1 -> 81.4).

@@ -757,6 +757,42 @@ int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* 
   return tile < 4 ? qmm_wo_ksplit_launch_f16_0(a, tile, s) : tile < 7 ? qmm_wo_ksplit_launch_f16_1(a, tile, s) : qmm_wo_ksplit_launch_f16_2(a, tile, s);
 }
 
+// Up to 16 rows the streaming kernel is as fast (0.8 - 1.2 of its time here).  17 - 32 rows: against up to 8192 channels
+// (0.57 - 0.91 of the streaming kernel's time; 11008 and 14336 channels 0.8 - 1.2).  33 - 64 rows, two passes of the
+// streaming kernel: against up to 16384 channels (0.34 - 0.71).  More: the shorter of the two estimates, the other being
+// the tiled GEMM's with its two tiles, fitted to 129 launches (root mean square error 4 - 6 %).
+int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, bool zp) {
+  if (M <= 16 || M > (1 << 14) || N > (1 << 20) || N % 4 != 0 || K > 65536 || K % 128 != 0 || C % 128 != 0) return -1;
+  if (bits == 8 && C == K) return -1;
+  if (N > (M <= 32 ? 8192 : 16384) && M <= 64) return -1;
+  const uint32_t m = (uint32_t)M, n = (uint32_t)N, k128 = (uint32_t)K / 128, sub = C == K ? 1 : (uint32_t)C / 128;
+  const float mb = 1e-6f * (float)N * (float)K * (float)bits / 8;
+  float least = 0;
+  if (M > 64) {
+    const uint32_t tm = (m + 63) / 64, narrow = (tm * ((n + 127) / 128) + 255) / 256, wide = (tm * ((n + 255) / 256) + 255) / 256;
+    const bool use_wide = (!zp || (bits == 4 && C == 128)) && wide * (zp ? 145u : bits == 4 ? 155u : 165u) < narrow * 100u;  // (wide_tiles)
+    least = use_wide ? 2.13f + (float)wide * (2.13f + (zp ? 1.232f : 1.092f) * (float)k128) + 0.054f * mb
+                     : 1.02f + (float)narrow * (2.85f + (zp ? 0.757f : 0.667f) * (float)k128) + 0.085f * mb;
+  }
+  int best = -1;
+  for (int i = 0; i < (int)(sizeof(kKsBwTiles) / sizeof(kKsBwTiles[0])); ++i) {
+    const KsBwTile& t = kKsBwTiles[i];
+    if (zp && !t.with_zp) continue;
+    const uint32_t tm = (m + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
+    if ((uint64_t)tm * tn > 65535) continue;
+    const float rounds = (float)((tm * tn + 255) / 256), steps = (float)((k128 / sub + t.kw - 1) / t.kw * sub);
+    const float us = t.fixed + t.round * rounds + (t.step + (zp ? t.zp : 0.f) + (bits == 8 ? t.int8 : 0.f)) * rounds * steps +
+                     t.load * (float)(tm * tn) / 256 * steps + t.weight * mb;
+    if ((best < 0 && M <= 64) || us < least) { best = i; least = us; }
+  }
+  return best;
+}
+
+int qmm_wo_ksplit_bw_run(int tile, const WoBwArgs& a, int bits, int x_dt, hipStream_t stream) {
+  if (x_dt == XLA_AMD_DT_BF16) return bits == 4 ? qmm_wo_ksplit_bw_launch_bf16_4(a, tile, stream) : qmm_wo_ksplit_bw_launch_bf16_8(a, tile, stream);
+  return bits == 4 ? qmm_wo_ksplit_bw_launch_f16_4(a, tile, stream) : qmm_wo_ksplit_bw_launch_f16_8(a, tile, stream);
+}
+
 namespace {
 
 // x f32 [M, K] -> [M, 3 K] bf16: hi | mid | lo side by side, hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid)
@@ -885,6 +921,14 @@ extern "C" int xla_amd_qmm_weight_only_gemm(const void* x, const void* w_tiled, 
   // (blockwise weights in the weight-streaming kernel: every dtype but the stored one is x's, at least 8 scales)
   const bool bw_ok = !blockwise || (scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt && (K / C) * N >= 8 &&
                                     (((uintptr_t)scale | (uintptr_t)zp) & 3) == 0);
+  if ((blockwise || bits == 4) && scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt && store_dt == x_dt &&
+      ((((uintptr_t)scale | (uintptr_t)zp) & 3) | ((uintptr_t)out & 7)) == 0) {
+    const int tile = qmm_wo_ksplit_bw_tile(M, N, K, C, bits, zp != nullptr);
+    if (tile >= 0) {
+      const WoBwArgs b{x, (const uint8_t*)w_tiled, scale, zp, out, (int)M, (int)N, (int)K, (int)C};
+      return qmm_wo_ksplit_bw_run(tile, b, bits, x_dt, (hipStream_t)stream);
+    }
+  }
   if (M <= 32 && bw_ok) {
     // few rows: the weight-streaming kernel over K slices, when that is what its plan says and the workspace is there
     int per;
