@@ -82,7 +82,7 @@ def test_tiles_of_the_f32_shapes(tmp_path):
     seen.add((mt, ng, kw, cw))
   assert len(seen) == 6
   # rows that fill the chip keep the split into three bf16 parts, sizes past the kernel's range the streaming kernel
-  calls = [rec.skinny(4, 64, 131072, 131072, 8, False, 0),
+  calls = [rec.skinny(4, 64, 131072, 131072, 8, False, 0), rec.skinny(16, 16384, 640, 640, 8, False, 0),
            ("xla_amd_qmm_weight_only_gemm_f32", "pppppp" + "z" + "qqq" + "iip", [rec.PTR] * 3 + [0, rec.PTR, rec.PTR, 1 << 40, 2048, 4096, 4096, 0, 0, 0])]
   for rc, text, launches in rec.record(calls, str(tmp_path)):
     assert rc == 0 and launches and not any("ksplit" in l.name for l in launches), text

@@ -700,7 +700,8 @@ int ks_best(const KsTile (&of)[n], int64_t M, int64_t N, int64_t K, bool limited
   for (size_t i = 0; i < n; ++i) {
     const KsTile& t = of[i];
     const uint32_t tm = (m + t.bm - 1) / t.bm, tn = (nn + t.bn - 1) / t.bn;
-    if ((uint64_t)tm * tn > 65535) continue;
+    // (more than four rounds lie outside of what the estimates were fitted to)
+    if ((uint64_t)tm * tn > (limited ? 1024 : 65535)) continue;
     const uint32_t tiles = tm * tn;
     const float rounds = (float)((tiles + 255) / 256), steps = (float)((k128 + t.kw - 1) / t.kw);
     const float us = t.fixed + t.round * rounds + (t.step * rounds + t.load * (float)tiles / 256) * steps + t.weight * weight;
@@ -731,12 +732,13 @@ int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
   return ks_best(kKsTiles, M, N, K, M > 32, limit);
 }
 
-// Fewer than 128 rows: always (0.93 of the streaming kernel's time at most, see qmm_wo_ksplit.hip).  More: while that is
+// Up to 16 rows, one pass of the streaming kernel: against up to 8192 channels (0.66 - 0.97 of its time; 0.88 - 1.23 at 11700
+// - 32768).  Up to 127: always (a second pass makes it 0.7 at most).  More: while that is
 // the shorter of the two estimates; the other is x split into three bf16 parts, 11 us and per round of 128 x 128 tiles
 // 3.2 + 0.78 per 128 of 3 K columns (measured at 128 - 700 rows: 512 x 1024 x 4096 92 -> 39 us, 200 x 4096 x 4096 90 ->
 // 69; 256 x 6144 x 4096 would be 90 -> 112).
 int qmm_wo_ksplit_f32_tile(int64_t M, int64_t N, int64_t K) {
-  if (K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14)) return -1;
+  if (K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14) || (M <= 16 && N > 8192)) return -1;
   const double rounds = (double)(((M + 127) / 128 * ((N + 127) / 128) + 255) / 256);
   return ks_best(kKsTilesF32, M, N, K, M >= 128, 11 + rounds * (3.2 + 0.78 * (double)(3 * K / 128)));
 }
@@ -779,7 +781,7 @@ int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, 
     const KsBwTile& t = kKsBwTiles[i];
     if (zp && !t.with_zp) continue;
     const uint32_t tm = (m + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
-    if ((uint64_t)tm * tn > 65535) continue;
+    if ((uint64_t)tm * tn > 1024) continue;  // (as in ks_best)
     const float rounds = (float)((tm * tn + 255) / 256), steps = (float)((k128 / sub + t.kw - 1) / t.kw * sub);
     const float us = t.fixed + t.round * rounds + (t.step + (zp ? t.zp : 0.f) + (bits == 8 ? t.int8 : 0.f)) * rounds * steps +
                      t.load * (float)(tm * tn) / 256 * steps + t.weight * mb;

@@ -25,11 +25,11 @@
 // ring where ragged rows leave room for it; conversions placed by hand between the MFMAs (12.1 -> 12.8: the wave needs
 // its weights a quarter of a step earlier); workgroups that start at different columns (within 3 % either way).
 //
-// f32 rows (any number of them below 128, and more where the launch has few tiles) run the same kernel on 16x16x4 f32
+// f32 rows (below 128, and more where the launch has few tiles) run the same kernel on 16x16x4 f32
 // MFMAs, one column per lane and instruction: true f32 products, an eighth of the bf16 rate, so the matrix cores bound
 // all but the smallest launches (64 x 4096 x 4096: 22 us, 14 of them MFMAs).  The streaming kernel before it made a pass
 // over the weight per 16 rows and split K over two waves at most, 512 columns each: 8 x 1024 x 1024 6.6 -> 4.6 us, 32 x
-// 4096 x 4096 25.6 -> 14.4, 100 x 1024 x 1024 43 -> 6.5; over 300 shapes of 1 - 127 rows 0.49 of the time, 0.93 at most.
+// 4096 x 4096 25.6 -> 14.4, 100 x 1024 x 1024 43 -> 6.5; over 300 shapes of 1 - 127 rows 0.49 of the time.
 //
 // This file is compiled per activation dtype and set of tiles (-DQMM_WO_XT=0|1|2 for f32 | bf16 | f16, -DQMM_KS_PART=0|1|2).
 #include "qmm_wo_ksplit.h"
