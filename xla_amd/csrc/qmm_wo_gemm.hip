@@ -35,6 +35,8 @@
 // This file is compiled once per (activation dtype, row tile) pair (-DQMM_WO_XT=1|2 for bf16 | f16,
 // -DQMM_WO_MT=4|8) so that the units build in parallel; the unit of bf16 with MT = 8 also
 // holds the second kernel of a K split and the C entry points.
+#include <utility>
+
 #include "qmm_common.h"
 #include "qmm_frag.h"
 #include "qmm_skinny.h"
@@ -689,26 +691,34 @@ double plan_us(const Plan& p, int64_t M, int64_t N, int64_t K) {
   return 4.03 + 6.49 * rounds + 1.14 * rounds * steps + 0.006 * weight;
 }
 
-// The tile of least estimated time, below `limit` if there is one; -1: none.
-template <size_t n>
-int ks_best(const KsTile (&of)[n], int64_t M, int64_t N, int64_t K, bool limited, double limit) {
+// What the estimates of all tiles of a launch have in common, and the least of them so far.
+struct KsLaunch {
+  uint32_t m, n, k128;
+  float weight;        // 10^-6 of the weight's bytes
+  bool limited;        // only a tile below `least` at the start
+  float least;
   int best = -1;
-  // (32-bit divisions: this runs on every call)
-  const uint32_t m = (uint32_t)M, nn = (uint32_t)N, k128 = (uint32_t)K / 128;
-  const float weight = 1e-6f * (float)N * (float)K;
-  float least = (float)limit;
-  for (size_t i = 0; i < n; ++i) {
-    const KsTile& t = of[i];
-    const uint32_t tm = (m + t.bm - 1) / t.bm, tn = (nn + t.bn - 1) / t.bn;
-    // (more than four rounds lie outside of what the estimates were fitted to)
-    if ((uint64_t)tm * tn > (limited ? 1024 : 65535)) continue;
-    const uint32_t tiles = tm * tn;
-    const float rounds = (float)((tiles + 255) / 256), steps = (float)((k128 + t.kw - 1) / t.kw);
-    const float us = t.fixed + t.round * rounds + (t.step * rounds + t.load * (float)tiles / 256) * steps + t.weight * weight;
-    if ((best < 0 && !limited) || us < least) { best = (int)i; least = us; }
+  void offer(int i, float us) {
+    if ((best < 0 && !limited) || us < least) { best = i; least = us; }
   }
-  return best;
+};
+// (The tables' numbers are constants here: with divisions by variables the choice took 0.2 us of a 5 us call.)
+template <const auto& tiles, size_t i>
+inline void ks_offer(KsLaunch& l) {
+  constexpr KsTile t = tiles[i];
+  const uint32_t tm = (l.m + t.bm - 1) / t.bm, tn = (l.n + t.bn - 1) / t.bn;
+  // (more than four rounds lie outside of what the estimates were fitted to)
+  if ((uint64_t)tm * tn > (l.limited ? 1024 : 65535)) return;
+  const uint32_t all = tm * tn;
+  const float rounds = (float)((all + 255) / 256), steps = (float)((l.k128 + t.kw - 1) / t.kw);
+  l.offer((int)i, t.fixed + t.round * rounds + (t.step * rounds + t.load * (float)all / 256) * steps + t.weight * l.weight);
 }
+template <const auto& tiles, size_t... i>
+inline int ks_best(KsLaunch l, std::index_sequence<i...>) {
+  (ks_offer<tiles, i>(l), ...);
+  return l.best;
+}
+template <const auto& tiles> constexpr auto ks_indices() { return std::make_index_sequence<sizeof(tiles) / sizeof(tiles[0])>(); }
 
 }  // namespace
 
@@ -729,7 +739,7 @@ int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
     if (p.mt == 4 && p.ng == 4) return -1;  // more than 49152 channels: the tiled GEMM's rounds are full
     limit = plan_us(p, M, N, K);
   }
-  return ks_best(kKsTiles, M, N, K, M > 32, limit);
+  return ks_best<kKsTiles>({(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, M > 32, (float)limit}, ks_indices<kKsTiles>());
 }
 
 // Up to 16 rows, one pass of the streaming kernel: against up to 8192 channels (0.66 - 0.97 of its time; 0.88 - 1.23 at 11700
@@ -740,7 +750,8 @@ int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
 int qmm_wo_ksplit_f32_tile(int64_t M, int64_t N, int64_t K) {
   if (K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14) || (M <= 16 && N > 8192)) return -1;
   const double rounds = (double)(((M + 127) / 128 * ((N + 127) / 128) + 255) / 256);
-  return ks_best(kKsTilesF32, M, N, K, M >= 128, 11 + rounds * (3.2 + 0.78 * (double)(3 * K / 128)));
+  return ks_best<kKsTilesF32>({(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, M >= 128,
+                               (float)(11 + rounds * (3.2 + 0.78 * (double)(3 * K / 128)))}, ks_indices<kKsTilesF32>());
 }
 
 int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* scale, const void* zp, void* out, int64_t M, int64_t N,
@@ -759,6 +770,27 @@ int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* 
   return tile < 4 ? qmm_wo_ksplit_launch_f16_0(a, tile, s) : tile < 7 ? qmm_wo_ksplit_launch_f16_1(a, tile, s) : qmm_wo_ksplit_launch_f16_2(a, tile, s);
 }
 
+namespace {
+
+template <size_t i>
+inline void ks_bw_offer(KsLaunch& l, uint32_t sub, bool int8, bool zp) {
+  constexpr KsBwTile t = kKsBwTiles[i];
+  if (zp && !t.with_zp) return;
+  const uint32_t tm = (l.m + t.bm - 1) / t.bm, tn = (l.n + t.bn - 1) / t.bn;
+  if ((uint64_t)tm * tn > 1024) return;  // (as in ks_offer)
+  const uint32_t all = tm * tn, blocks = sub == 1 ? l.k128 : l.k128 / sub;
+  const float rounds = (float)((all + 255) / 256), steps = (float)((blocks + t.kw - 1) / t.kw * sub);
+  l.offer((int)i, t.fixed + t.round * rounds + (t.step + (zp ? t.zp : 0.f) + (int8 ? t.int8 : 0.f)) * rounds * steps +
+                      t.load * (float)all / 256 * steps + t.weight * l.weight);
+}
+template <size_t... i>
+inline int ks_bw_best(KsLaunch l, uint32_t sub, bool int8, bool zp, std::index_sequence<i...>) {
+  (ks_bw_offer<i>(l, sub, int8, zp), ...);
+  return l.best;
+}
+
+}  // namespace
+
 // Up to 16 rows the streaming kernel is as fast (0.8 - 1.2 of its time here).  17 - 32 rows: against up to 8192 channels
 // (0.57 - 0.91 of the streaming kernel's time; 11008 and 14336 channels 0.8 - 1.2).  33 - 64 rows, two passes of the
 // streaming kernel: against up to 16384 channels (0.34 - 0.71).  More: the shorter of the two estimates, the other being
@@ -776,18 +808,7 @@ int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, 
     least = use_wide ? 2.13f + (float)wide * (2.13f + (zp ? 1.232f : 1.092f) * (float)k128) + 0.054f * mb
                      : 1.02f + (float)narrow * (2.85f + (zp ? 0.757f : 0.667f) * (float)k128) + 0.085f * mb;
   }
-  int best = -1;
-  for (int i = 0; i < (int)(sizeof(kKsBwTiles) / sizeof(kKsBwTiles[0])); ++i) {
-    const KsBwTile& t = kKsBwTiles[i];
-    if (zp && !t.with_zp) continue;
-    const uint32_t tm = (m + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
-    if ((uint64_t)tm * tn > 1024) continue;  // (as in ks_best)
-    const float rounds = (float)((tm * tn + 255) / 256), steps = (float)((k128 / sub + t.kw - 1) / t.kw * sub);
-    const float us = t.fixed + t.round * rounds + (t.step + (zp ? t.zp : 0.f) + (bits == 8 ? t.int8 : 0.f)) * rounds * steps +
-                     t.load * (float)(tm * tn) / 256 * steps + t.weight * mb;
-    if ((best < 0 && M <= 64) || us < least) { best = i; least = us; }
-  }
-  return best;
+  return ks_bw_best({m, n, k128, mb, M > 64, least}, sub, bits == 8, zp, ks_indices<kKsBwTiles>());
 }
 
 int qmm_wo_ksplit_bw_run(int tile, const WoBwArgs& a, int bits, int x_dt, hipStream_t stream) {
