@@ -3,14 +3,18 @@
 //
 // One workgroup of eight waves owns 16 NG NW channels x 16 MT rows of x; NW waves stand side by side along the
 // channels and KW = 8 / NW of them split K.  Nothing goes through LDS but the sums of the K split: a chunk of 64
-// columns is one 16-byte load per lane and 16 channels of weights (lane (r, g) = (lane % 16, lane / 16) takes columns
-// 16 g .. 16 g + 15 of row r) and the same columns of x, which is exactly an operand of the matrix instructions as
-// long as both operands agree on the order of the columns.  Rows start at any byte: the loads are unaligned.
+// columns is 16 bytes per lane and 16 channels of weights (lane (r, g) = (lane % 16, lane / 16) takes 16 columns of row
+// r) and the same columns of x, which is exactly an operand of the matrix instructions as long as both operands agree
+// on the order of the columns.  Rows start at any byte: the loads are unaligned.
 //
 // What bounds it: memory latency at the sizes it is meant for (a few MB of weight), so a wave has the next chunk's
 // loads in flight during a chunk, and few channels per workgroup put many waves on the chip.  Wide outputs with many
 // rows take more channels per workgroup, since every workgroup reads its rows of x again (out of L2).
-// Per launch, bf16 x against 3000 x 2000: 6.2 us for 1 row, 11.4 for 40 (one thread per output took 1060), 46 for 512.
+// Per launch, bf16 x against 3000 x 2000: 6.2 us for 1 row, 8.1 for 40 (one thread per output took 1060), 46 for 512.
+// Then it is the loads' addresses: 40 rows took 11.0 us with 16 columns of x side by side per lane (32 bytes at a stride
+// of 32, where the four lanes of a row now cover 64 consecutive bytes per load), the row's end element by element (now
+// the row's last 64 columns, less those of the chunk before) and 64 rows of x loaded for 40 (now 48).  Loads two
+// chunks ahead, without a branch around those past the end, made rows at odd addresses 1.5 - 3.3 times slower.
 #include "qmm_common.h"
 #include "qmm_frag.h"
 #include "qmm_rowmajor.h"
@@ -107,39 +111,76 @@ qmm_rowmajor_kernel(QmmRowMajorArgs a) {
     i32x4 w[NG];
     i32x4 x[MT][XV];
   };
+  // First column, within the chunk, of dword i of this lane's weights and of its x.  2-byte x takes columns 8 g .. 8 g + 7
+  // of either half of the chunk, so that the four lanes of a row load 64 consecutive bytes of x; the others columns
+  // 16 g .. 16 g + 15.
+  constexpr bool kHalves = XV == 2;
+  const int lane_col = (kHalves ? 8 : 16) * g;
+  auto w_at = [](int i) constexpr { return kHalves ? 32 * (i / 2) + 4 * (i % 2) : 4 * i; };       // from there
+  auto x_at = [](int i) constexpr { return kHalves ? 32 * (i / 4) + 2 * (i % 4) : 4 / XV * i; };
+  constexpr bool kElements = XT == XLA_AMD_DT_F32;
+  // Chunk c.  The last one ends with the row, whatever the row's length: its first columns are the chunk's before it,
+  // which drop_overlap takes out.
+  const int64_t last_k = K - 64;
   auto load = [&](int64_t c, Chunk& d) __attribute__((always_inline)) {
-    const int64_t k = c * 64 + 16 * g;
-    if (c * 64 + 64 <= K) {  // (uniform) whole chunk
-      qmm_static_for<NG>([&](auto gc) { __builtin_memcpy(&d.w[(int)gc], wrow[(int)gc] + k, 16); });
-      qmm_static_for<MT>([&](auto mc) { __builtin_memcpy(&d.x[(int)mc][0], xrow[(int)mc] + k, 16 * XV); });
-    } else {  // the row's end: element by element, zeros after it
-      qmm_static_for<NG>([&](auto gc) {
-        qmm_static_for<4>([&](auto dc) {
-          uint32_t v = 0;
-          qmm_static_for<4>([&](auto bc) {
-            const int64_t at = k + 4 * (int)dc + (int)bc;
-            if (at < K) v |= (uint32_t)(uint8_t)wrow[(int)gc][at] << (8 * (int)bc);
-          });
-          d.w[(int)gc][(int)dc] = (int)v;
+    const int64_t k = (kElements ? c * 64 : min(c * 64, last_k)) + lane_col;
+    qmm_static_for<NG>([&](auto gc) {
+      constexpr int gi = gc;
+      if constexpr (kHalves) {
+        i32x2 half[2];
+        qmm_static_for<2>([&](auto hc) { __builtin_memcpy(&half[(int)hc], wrow[gi] + k + w_at(2 * (int)hc), 8); });
+        d.w[gi] = i32x4{half[0][0], half[0][1], half[1][0], half[1][1]};
+      } else {
+        __builtin_memcpy(&d.w[gi], wrow[gi] + k, 16);
+      }
+    });
+    qmm_static_for<MT>([&](auto mc) {
+      qmm_static_for<XV>([&](auto qc) { __builtin_memcpy(&d.x[(int)mc][(int)qc], xrow[(int)mc] + k + x_at(4 * (int)qc), 16); });
+    });
+  };
+  const int64_t chunks = (K + 63) / 64;
+  const int overlap = (int)(chunks * 64 - K);
+  // zeros for the columns of x in the last chunk that the one before it holds (the weights are finite)
+  auto drop_overlap = [&](Chunk& d) __attribute__((always_inline)) {
+    auto mask = [&](int first, int per) __attribute__((always_inline)) {  // of a dword that holds columns first .. first + per - 1
+      const int k = min(max(overlap - first, 0), per);
+      return k == per ? 0 : (int)(~0u << (32 / per * k));
+    };
+    qmm_static_for<4 * XV>([&](auto dc) {
+      const int m = mask(lane_col + x_at((int)dc), 4 / XV);
+      qmm_static_for<MT>([&](auto mc) { d.x[(int)mc][(int)dc / 4][(int)dc % 4] &= m; });
+    });
+  };
+  // a chunk that the row ends in, element by element, zeros after it: the only chunk of a short row, and f32's last one
+  // (there are no registers for the masks above beside f32's chunks)
+  auto load_elements = [&](int64_t c, Chunk& d) __attribute__((always_inline)) {
+    const int64_t k = c * 64 + lane_col;
+    qmm_static_for<NG>([&](auto gc) {
+      qmm_static_for<4>([&](auto dc) {
+        uint32_t v = 0;
+        qmm_static_for<4>([&](auto bc) {
+          const int64_t at = k + w_at((int)dc) + (int)bc;
+          if (at < K) v |= (uint32_t)(uint8_t)wrow[(int)gc][at] << (8 * (int)bc);
         });
+        d.w[(int)gc][(int)dc] = (int)v;
       });
-      qmm_static_for<MT>([&](auto mc) {
-        constexpr int kPer = 4 / XV;  // elements per dword
-        qmm_static_for<4 * XV>([&](auto dc) {
-          uint32_t v = 0;
-          qmm_static_for<kPer>([&](auto bc) {
-            const int64_t at = k + kPer * (int)dc + (int)bc;
-            if (at < K) {
-              elem_t e = xrow[(int)mc][at];
-              uint32_t bits = 0;
-              __builtin_memcpy(&bits, &e, sizeof(e));
-              v |= bits << (8 * XV * (int)bc);
-            }
-          });
-          d.x[(int)mc][(int)dc / 4][(int)dc % 4] = (int)v;
+    });
+    qmm_static_for<MT>([&](auto mc) {
+      constexpr int kPer = 4 / XV;  // elements per dword
+      qmm_static_for<4 * XV>([&](auto dc) {
+        uint32_t v = 0;
+        qmm_static_for<kPer>([&](auto bc) {
+          const int64_t at = k + x_at((int)dc) + (int)bc;
+          if (at < K) {
+            elem_t e = xrow[(int)mc][at];
+            uint32_t bits = 0;
+            __builtin_memcpy(&bits, &e, sizeof(e));
+            v |= bits << (8 * XV * (int)bc);
+          }
         });
+        d.x[(int)mc][(int)dc / 4][(int)dc % 4] = (int)v;
       });
-    }
+    });
   };
 
   acc_t acc[NG][MT], xs[MT];
@@ -171,7 +212,7 @@ qmm_rowmajor_kernel(QmmRowMajorArgs a) {
         });
       });
     } else {
-      // columns 16 g + 8 h .. + 7 are the lane's eight of instruction h
+      // columns 32 h + 8 g .. + 7 are the lane's eight of instruction h
       qmm_static_for<2>([&](auto hc) {
         constexpr int h = hc;
         qmm_static_for<NG>([&](auto gc) {
@@ -188,15 +229,22 @@ qmm_rowmajor_kernel(QmmRowMajorArgs a) {
     }
   };
 
-  // chunks kw, kw + KW, ...: the next one's loads are in flight during a chunk
-  const int64_t chunks = (K + 63) / 64;
+  auto fetch = [&](int64_t c, Chunk& d) __attribute__((always_inline)) {
+    if (kElements ? c * 64 + 64 <= K : K >= 64) load(c, d);
+    else load_elements(c, d);
+  };
+  // chunks kw, kw + KW, ...: the next one's loads are in flight during a chunk (none past the end: the loads' addresses
+  // are what takes time here)
   Chunk cur;
   int64_t c = kw;
-  if (c < chunks) load(c, cur);
+  if (c < chunks) fetch(c, cur);
   while (c < chunks) {
     Chunk next;
     const int64_t cn = c + KW;
-    if (cn < chunks) load(cn, next);
+    if (cn < chunks) fetch(cn, next);
+    if constexpr (!kElements) {
+      if (c == chunks - 1 && overlap > 0 && K >= 64) drop_overlap(cur);
+    }
     multiply(cur);
     cur = next;
     c = cn;
@@ -284,6 +332,7 @@ int launch_rows(const QmmRowMajorArgs& a, hipStream_t stream) {
   }
   if (a.M <= 16) return launch_width<XT, 1>(a, stream);
   if (a.M <= 32) return launch_width<XT, 2>(a, stream);
+  if (a.M <= 48) return launch_width<XT, 3>(a, stream);
   return launch_width<XT, 4>(a, stream);
 }
 
