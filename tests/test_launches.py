@@ -1,11 +1,12 @@
 """What the library's entry points launch, recorded without a GPU."""
 import ctypes
+import json
 import re
 
 import pytest
 
 from tests import launch_recorder as rec
-from xla_amd import _lib
+from xla_amd import _lib, build
 
 
 def test_every_kernel_gets_its_lds(tmp_path):
@@ -158,3 +159,13 @@ def test_wide_tile_tests_run_the_wide_kernel(tmp_path):
   want = ["qmm_wo_bw_wide_kernel"] * len(wide) + ["qmm_wo_bw_gemm_kernel"] * len(narrow)
   for call, kernel, (rc, text, launches) in zip(calls, want * 2, rec.record(calls, str(tmp_path))):
     assert rc == 0 and len(launches) == 1 and kernel in launches[0].name, (call, text, launches)
+
+
+def test_arguments_of_the_k_split_kernels():
+  """The runtime writes a kernel's arguments out at every launch.  A kernel that asks for the size of its grid gets 256
+  bytes of hidden ones, which made the eager call of a small launch slower than with the kernel before it."""
+  with open(build.RESOURCES_PATH) as f:
+    kernels = [k for k in json.load(f) if "ksplit" in k["kernel"]]
+  assert len(kernels) > 50
+  for k in kernels:
+    assert k["kernarg_bytes"] <= 120, (k["kernel"], k["kernarg_bytes"])

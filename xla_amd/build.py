@@ -117,14 +117,16 @@ CODE_BUDGET_BYTES = {
 }
 
 
-def _code_bytes(obj: str):
-  """{kernel symbol: bytes} of the gfx950 code object bundled in `obj`."""
+def _code_object(obj: str):
+  """({kernel symbol: bytes of code}, {kernel symbol: bytes of arguments, hidden ones included}) of the gfx950 code
+  object bundled in `obj`."""
   fat, dev = obj + ".fatbin", obj + ".gfx950.co"
   try:
     _run(["objcopy", "-O", "binary", "--only-section=.hip_fatbin", obj, fat])
     _run([os.path.join(LLVM_BIN, "clang-offload-bundler"), "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950",
           "--input=" + fat, "--output=" + dev, "--unbundle"])
     table = _run([os.path.join(LLVM_BIN, "llvm-readelf"), "-sW", dev])
+    notes = _run([os.path.join(LLVM_BIN, "llvm-readelf"), "--notes", dev])
   finally:
     for f in (fat, dev):
       if os.path.exists(f):
@@ -134,7 +136,10 @@ def _code_bytes(obj: str):
     f = line.split()
     if len(f) >= 8 and f[3] == "FUNC" and f[6] != "UND":
       sizes[f[7]] = int(f[2])
-  return sizes
+  # (one entry per kernel, its keys in alphabetical order)
+  args = {name: int(n) for n, name in re.findall(r"\.kernarg_segment_size: +(\d+)(?:(?!\.kernarg_segment_size).)*?\.symbol: +'?(\S+?)\.kd",
+                                                 notes, re.S)}
+  return sizes, args
 
 
 def _build_torch_binding():
@@ -160,10 +165,12 @@ def build(verbose: bool = False, jobs: int = 8) -> str:
     out = _run([HIPCC] + FLAGS + ["-Rpass-analysis=kernel-resource-usage"] + extra +
                ["-c", os.path.join(CSRC, src), "-o", obj])
     kernels = _kernel_resources(out, name)
-    sizes = _code_bytes(obj) if kernels else {}  # (a unit without kernels carries no device code object)
+    sizes, args = _code_object(obj) if kernels else ({}, {})  # (a unit without kernels carries no device code object)
     for k in kernels:
       if k["kernel"] in sizes:
         k["code_bytes"] = sizes[k["kernel"]]
+      if k["kernel"] in args:
+        k["kernarg_bytes"] = args[k["kernel"]]
     if verbose:
       # (a remark is followed by the source line it points at and a caret line)
       rest = "\n".join(l for l in out.splitlines() if "kernel-resource-usage" not in l and

@@ -24,7 +24,8 @@ struct WoGemmArgs {
 // compile time, which is the common case and removes every branch on a dtype.
 template <int XT, bool UNI> struct WoDts {
   int scale_dt, zp_dt, dot_dt, out_dt, store_dt, x_dt;
-  __device__ __forceinline__ explicit WoDts(const WoGemmArgs& a)
+  template <class Args>
+  __device__ __forceinline__ explicit WoDts(const Args& a)
       : scale_dt(UNI ? XT : a.scale_dt), zp_dt(UNI ? XT : a.zp_dt), dot_dt(UNI ? XT : a.dot_dt),
         out_dt(UNI ? XT : a.out_dt), store_dt(UNI ? XT : a.store_dt), x_dt(UNI ? XT : a.x_dt) {}
 };
@@ -151,6 +152,24 @@ constexpr KsTile kKsTilesF32[] = {
     {16, 64, 8, 2.16f, 4.711f, 0.129f, 1.077f, 0.078f}, {16, 16, 4, 2.93f, 0.935f, 0.138f, 0.000f, 0.000f},
     {32, 32, 4, 2.46f, 2.119f, 0.207f, 0.919f, 0.022f}, {32, 64, 4, 2.58f, 4.150f, 0.132f, 0.960f, 0.046f},
 };
+// Arguments of the kernel, tiles included: one struct of no more bytes than the kernel reads.  (A launch's arguments are
+// written out by the host each time; with WoGemmArgs, the tiles beside it and the 256 bytes of hidden arguments that
+// reading gridDim brings, 392 bytes in all, an eager call of 8 x 1024 x 1024 f32 took 0.1 - 0.15 us longer, of 7.6.)
+struct KsTiles {
+  int rows, tiles_m, tiles, per_xcd;  // rows per tile (M spread evenly over the row tiles), row tiles, all tiles, tiles per XCD
+  uint64_t tiles_m_magic;             // ceil(2^32 / tiles_m)
+};
+struct KsArgs {
+  const void* x;       // [M, K]
+  const uint8_t* w;    // tiled weight, 8 bits
+  const void* scale;   // [N]
+  const void* zp;      // [N] or null
+  void* out;           // [M, N] of store_dt
+  int M, N, K;
+  int G;               // channels per group of the tiled weight (xla_amd_qmm_tile_group)
+  int scale_dt, zp_dt, dot_dt, out_dt, store_dt, x_dt;
+  KsTiles t;
+};
 // The tile a launch of M rows of 2-byte x against a per-channel int8 weight runs with (-1: not one for this kernel).
 int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K);
 // ... of f32 x
@@ -158,11 +177,11 @@ int qmm_wo_ksplit_f32_tile(int64_t M, int64_t N, int64_t K);
 // Runs a launch with the tile that one of them gave (arguments checked by the entry points: per-channel int8 weight, a tile for it).
 int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* scale, const void* zp, void* out, int64_t M, int64_t N,
                       int64_t K, int x_dt, int scale_dt, int zp_dt, int dot_dt, int out_dt, int store_dt, hipStream_t s);
-int qmm_wo_ksplit_launch_bf16_0(const WoGemmArgs& a, int tile, hipStream_t stream);
-int qmm_wo_ksplit_launch_bf16_1(const WoGemmArgs& a, int tile, hipStream_t stream);
-int qmm_wo_ksplit_launch_bf16_2(const WoGemmArgs& a, int tile, hipStream_t stream);
-int qmm_wo_ksplit_launch_f16_0(const WoGemmArgs& a, int tile, hipStream_t stream);
-int qmm_wo_ksplit_launch_f16_1(const WoGemmArgs& a, int tile, hipStream_t stream);
-int qmm_wo_ksplit_launch_f16_2(const WoGemmArgs& a, int tile, hipStream_t stream);
-int qmm_wo_ksplit_launch_f32_0(const WoGemmArgs& a, int tile, hipStream_t stream);
-int qmm_wo_ksplit_launch_f32_1(const WoGemmArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_bf16_0(KsArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_bf16_1(KsArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_bf16_2(KsArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_f16_0(KsArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_f16_1(KsArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_f16_2(KsArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_f32_0(KsArgs& a, int tile, hipStream_t stream);
+int qmm_wo_ksplit_launch_f32_1(KsArgs& a, int tile, hipStream_t stream);

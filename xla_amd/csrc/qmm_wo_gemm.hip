@@ -749,21 +749,25 @@ int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
 // 69; 256 x 6144 x 4096 would be 90 -> 112).
 int qmm_wo_ksplit_f32_tile(int64_t M, int64_t N, int64_t K) {
   if (K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14) || (M <= 16 && N > 8192)) return -1;
-  const double rounds = (double)(((M + 127) / 128 * ((N + 127) / 128) + 255) / 256);
-  return ks_best<kKsTilesF32>({(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, M >= 128,
-                               (float)(11 + rounds * (3.2 + 0.78 * (double)(3 * K / 128)))}, ks_indices<kKsTilesF32>());
+  KsLaunch l{(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, false, 0};
+  // (up to 16 rows none of the other tiles is the least at any N and K; the choice is part of a call of some 5 us)
+  if (M <= 16) return ks_best<kKsTilesF32>(l, std::index_sequence<0, 1, 3>());
+  if (M >= 128) {
+    const double rounds = (double)(((M + 127) / 128 * ((N + 127) / 128) + 255) / 256);
+    l.limited = true;
+    l.least = (float)(11 + rounds * (3.2 + 0.78 * (double)(3 * K / 128)));
+  }
+  return ks_best<kKsTilesF32>(l, ks_indices<kKsTilesF32>());
 }
 
 int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* scale, const void* zp, void* out, int64_t M, int64_t N,
                       int64_t K, int x_dt, int scale_dt, int zp_dt, int dot_dt, int out_dt, int store_dt, hipStream_t s) {
-  WoGemmArgs a;
+  KsArgs a;
   a.x = x; a.w = (const uint8_t*)w_tiled; a.scale = scale; a.zp = zp; a.out = out;
-  a.part = nullptr; a.part_xs = nullptr;
   a.M = (int)M; a.N = (int)N; a.K = (int)K;
-  a.Kw = (int)K; a.x_dt = x_dt; a.stage_out = 0;
   a.G = xla_amd_qmm_tile_group(N, K, K, 8);
-  a.k_per_split = (int)K; a.split = 1;
   a.scale_dt = scale_dt; a.zp_dt = zp ? zp_dt : x_dt; a.dot_dt = dot_dt; a.out_dt = out_dt; a.store_dt = store_dt;
+  a.x_dt = x_dt;
   if (x_dt == XLA_AMD_DT_F32) return tile < 3 ? qmm_wo_ksplit_launch_f32_0(a, tile, s) : qmm_wo_ksplit_launch_f32_1(a, tile, s);
   if (x_dt == XLA_AMD_DT_BF16)
     return tile < 4 ? qmm_wo_ksplit_launch_bf16_0(a, tile, s) : tile < 7 ? qmm_wo_ksplit_launch_bf16_1(a, tile, s) : qmm_wo_ksplit_launch_bf16_2(a, tile, s);

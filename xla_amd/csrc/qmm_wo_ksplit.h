@@ -12,16 +12,13 @@ using namespace qmm_frag;
 constexpr int kCopyWaves = 4;
 constexpr int kLds = 160 * 1024;
 
-// The launch's tiles: rows per tile (M spread evenly over the row tiles), row tiles, all tiles.
-struct KsTiles {
-  int rows, tiles_m, tiles;
-  uint64_t tiles_m_magic;  // ceil(2^32 / tiles_m)
-};
+// The launch's tiles.  (All that a kernel needs to know of its grid, see KsArgs.)
 inline KsTiles ks_tiles(int M, int N, int bm, int bn) {
   KsTiles t;
   t.tiles_m = (M + bm - 1) / bm;
   t.rows = (M + t.tiles_m - 1) / t.tiles_m;
   t.tiles = t.tiles_m * ((N + bn - 1) / bn);
+  t.per_xcd = (t.tiles + 7) / 8;
   t.tiles_m_magic = (((uint64_t)1 << 32) + t.tiles_m - 1) / t.tiles_m;
   return t;
 }
@@ -49,7 +46,7 @@ template <int XT, int MT, int NG, int KW, int CW, int SUMS, int TAIL> struct KsC
 // to the 8 XCDs: each XCD gets a contiguous run of the tiles, row tiles fastest, so that the row tiles of a column share
 // its weights in that L2 (tile / tiles_m by multiply-shift: tile < 2^16).
 __device__ __forceinline__ bool ks_tile_of(const KsTiles& t, int M, int bn, int& n0, int& m0, int& rows) {
-  const int tile = ((int)blockIdx.x & 7) * (int)(gridDim.x >> 3) + ((int)blockIdx.x >> 3);
+  const int tile = ((int)blockIdx.x & 7) * t.per_xcd + ((int)blockIdx.x >> 3);
   if (tile >= t.tiles) return false;
   const int col = (int)(((uint64_t)(uint32_t)tile * t.tiles_m_magic) >> 32);
   n0 = col * bn;

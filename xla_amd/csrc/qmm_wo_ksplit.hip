@@ -45,7 +45,7 @@ template <int NG, int CW> constexpr int ks_tail() { return 2 * 16 * NG * CW * 4;
 
 template <int XT, int MT, int NG, int KW, int CW, int P, bool HASZP, bool UNI>
 __global__ void __launch_bounds__((KW * CW + kCopyWaves) * 64)
-qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
+qmm_wo_ksplit_kernel(KsArgs a) {
   using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, ks_tail<NG, CW>()>;
   constexpr bool kF32 = XT == XLA_AMD_DT_F32;
   constexpr int NW = Cfg::NW, BM = Cfg::BM, BN = Cfg::BN, TILE = Cfg::TILE, SLOT = Cfg::SLOT, R = Cfg::R;
@@ -61,7 +61,7 @@ qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
   const int r = lane & 15, g = lane >> 4;
   const int M = a.M, N = a.N, K = a.K;
   int n0, m0, rows;
-  if (!ks_tile_of(t, M, BN, n0, m0, rows)) return;
+  if (!ks_tile_of(a.t, M, BN, n0, m0, rows)) return;
   const int n_tiles = K / 128;
   const int steps = (n_tiles + KW - 1) / KW;
   const WoDts<XT, UNI> dts(a);
@@ -220,17 +220,17 @@ qmm_wo_ksplit_kernel(WoGemmArgs a, KsTiles t) {
 }
 
 template <int XT, int MT, int NG, int KW, int CW, int P>
-int launch(const WoGemmArgs& a, hipStream_t stream) {
+int launch(KsArgs& a, hipStream_t stream) {
   using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, ks_tail<NG, CW>()>;
-  const KsTiles t = ks_tiles(a.M, a.N, Cfg::BM, Cfg::BN);
-  const dim3 grid(8u * (unsigned)((t.tiles + 7) / 8)), block((Cfg::NW + kCopyWaves) * 64);
+  a.t = ks_tiles(a.M, a.N, Cfg::BM, Cfg::BN);
+  const dim3 grid(8u * (unsigned)a.t.per_xcd), block((Cfg::NW + kCopyWaves) * 64);
   const int steps = (a.K / 128 + KW - 1) / KW;
   auto go = [&](auto which) -> int {
     constexpr auto kern = decltype(which)::fn;
     static std::atomic<uint64_t> lds_set{0};
     const int rc = qmm_set_max_lds((const void*)kern, Cfg::lds_bytes(1 << 20), lds_set, "weight_only_gemm hipFuncSetAttribute");
     if (rc != XLA_AMD_QMM_OK) return rc;
-    hipLaunchKernelGGL(kern, grid, block, Cfg::lds_bytes(steps), stream, a, t);
+    hipLaunchKernelGGL(kern, grid, block, Cfg::lds_bytes(steps), stream, a);
     return QMM_CHECK_LAUNCH("weight_only_gemm launch");
   };
   const bool uni = a.scale_dt == XT && a.zp_dt == XT && a.dot_dt == XT && a.out_dt == XT && a.store_dt == XT;
@@ -252,7 +252,7 @@ int launch(const WoGemmArgs& a, hipStream_t stream) {
 #define QMM_KS_NAME QMM_KS_CAT(qmm_wo_ksplit_launch_f32_, QMM_KS_PART)
 #endif
 // tile: index into kKsTiles, or kKsTilesF32 (qmm_wo_gemm.h)
-int QMM_KS_NAME(const WoGemmArgs& a, int tile, hipStream_t stream) {
+int QMM_KS_NAME(KsArgs& a, int tile, hipStream_t stream) {
   switch (tile) {
 #if QMM_WO_XT == XLA_AMD_DT_F32
 #if QMM_KS_PART == 0

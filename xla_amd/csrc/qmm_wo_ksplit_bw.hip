@@ -257,7 +257,7 @@ template <int XT, int BITS, int MT, int NG, int KW, int CW, int P, bool ZP = tru
 int launch(const WoBwArgs& a, hipStream_t stream) {
   using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, 0>;
   const KsTiles t = ks_tiles(a.M, a.N, Cfg::BM, Cfg::BN);
-  const dim3 grid(8u * (unsigned)((t.tiles + 7) / 8)), block((Cfg::NW + kCopyWaves) * 64);
+  const dim3 grid(8u * (unsigned)t.per_xcd), block((Cfg::NW + kCopyWaves) * 64);
   const bool perch = a.C == a.K;
   const int sub = perch ? 1 : a.C / 128, blocks = a.K / 128 / sub;
   const int steps = (blocks + KW - 1) / KW * sub;
