@@ -88,6 +88,22 @@ def test_tiles_of_the_f32_shapes(tmp_path):
     assert rc == 0 and launches and not any("ksplit" in l.name for l in launches), text
 
 
+def test_f32_rows_against_wide_outputs(tmp_path):
+  """17 - 127 rows against many channels and a short K: a pass of the streaming kernel per 16 rows where a third, fifth or
+  seventh one is shorter than a row tile of 32 for the last of them, K split over waves otherwise."""
+  stream = [(33, 128256, 384), (48, 65536, 128), (33, 32768, 640), (65, 128256, 768), (97, 128256, 640), (17, 262144, 640)]
+  split = [(33, 16384, 384), (49, 128256, 384), (33, 32768, 512), (64, 128256, 768), (127, 128256, 640), (32, 128256, 512),
+           (33, 128256, 1152), (100, 128256, 4096), (127, 1 << 19, 2048)]
+  calls = [rec.skinny(m, n, k, k, 8, zp, 0) for m, n, k in stream + split for zp in (False, True)]
+  for (_, _, args), (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0, text
+    m, n, k = args[5:8]
+    if (m, n, k) in stream:
+      assert len(launches) == -(-m // 16) and all("qmm_skinny_kernel" in l.name for l in launches), (m, n, k, launches)
+    else:
+      assert len(launches) == 1 and "qmm_wo_ksplit_kernel" in launches[0].name, (m, n, k, launches)
+
+
 def test_tiles_of_the_shapes(tmp_path):
   calls = [rec.blockwise(m, n, k, k, 8, zp, dt) for m, n, k, _, _ in SHAPES for zp in (False, True) for dt in (1, 2)]
   calls += [rec.skinny(m, n, k, k, 8, zp, 1) for m, n, k, _, _ in SHAPES if m <= 32 for zp in (False, True)]
@@ -134,7 +150,7 @@ def test_against_the_oracle(m, n, k, bm, bn, xdt):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k,bm,bn", F32_SHAPES)
+@pytest.mark.parametrize("m,n,k,bm,bn", F32_SHAPES + [(33, 32768, 640, 16, 64)])  # (the last: three passes of the streaming kernel)
 def test_f32_against_f64(m, n, k, bm, bn):
   import xla_amd.experimental.custom_kernel  # noqa: F401
   op = torch.ops.xla.quantized_matmul

@@ -694,27 +694,28 @@ double plan_us(const Plan& p, int64_t M, int64_t N, int64_t K) {
 // What the estimates of all tiles of a launch have in common, and the least of them so far.
 struct KsLaunch {
   uint32_t m, n, k128;
-  float weight;        // 10^-6 of the weight's bytes
-  bool limited;        // only a tile below `least` at the start
-  float least;
+  float weight;         // 10^-6 of the weight's bytes
+  uint32_t most_tiles;  // tiles of a launch at most: 1024 (four rounds), as many as the estimates were fitted to, or more
+                        // where more has been measured too
+  float least;          // at the start what the launch would take without this kernel: only a tile below it is taken
   int best = -1;
   void offer(int i, float us) {
-    if ((best < 0 && !limited) || us < least) { best = i; least = us; }
+    if (us < least) { best = i; least = us; }
   }
 };
+constexpr float kNoLimit = 1e30f;
 // (The tables' numbers are constants here: with divisions by variables the choice took 0.2 us of a 5 us call.)
 template <const auto& tiles, size_t i>
 inline void ks_offer(KsLaunch& l) {
   constexpr KsTile t = tiles[i];
   const uint32_t tm = (l.m + t.bm - 1) / t.bm, tn = (l.n + t.bn - 1) / t.bn;
-  // (more than four rounds lie outside of what the estimates were fitted to)
-  if ((uint64_t)tm * tn > (l.limited ? 1024 : 65535)) return;
+  if ((uint64_t)tm * tn > l.most_tiles) return;
   const uint32_t all = tm * tn;
   const float rounds = (float)((all + 255) / 256), steps = (float)((l.k128 + t.kw - 1) / t.kw);
   l.offer((int)i, t.fixed + t.round * rounds + (t.step * rounds + t.load * (float)all / 256) * steps + t.weight * l.weight);
 }
 template <const auto& tiles, size_t... i>
-inline int ks_best(KsLaunch l, std::index_sequence<i...>) {
+inline int ks_best(KsLaunch& l, std::index_sequence<i...>) {
   (ks_offer<tiles, i>(l), ...);
   return l.best;
 }
@@ -733,31 +734,46 @@ int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
     int per;
     if (N > 8192 || (K > 8192 && qmm_skinny_k_slices(M, N, K, K, 8, &per) > 1)) return -1;
   }
-  double limit = 0;
+  KsLaunch l{(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, 1024, kNoLimit};
   if (M > 32) {
     const Plan p = make_plan(M, N, K, false);
     if (p.mt == 4 && p.ng == 4) return -1;  // more than 49152 channels: the tiled GEMM's rounds are full
-    limit = plan_us(p, M, N, K);
+    l.least = (float)plan_us(p, M, N, K);
   }
-  return ks_best<kKsTiles>({(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, M > 32, (float)limit}, ks_indices<kKsTiles>());
+  return ks_best<kKsTiles>(l, ks_indices<kKsTiles>());
 }
 
 // Up to 16 rows, one pass of the streaming kernel: against up to 8192 channels (0.66 - 0.97 of its time; 0.88 - 1.23 at 11700
-// - 32768).  Up to 127: always (a second pass makes it 0.7 at most).  More: while that is
-// the shorter of the two estimates; the other is x split into three bf16 parts, 11 us and per round of 128 x 128 tiles
-// 3.2 + 0.78 per 128 of 3 K columns (measured at 128 - 700 rows: 512 x 1024 x 4096 92 -> 39 us, 200 x 4096 x 4096 90 ->
-// 69; 256 x 6144 x 4096 would be 90 -> 112).
+// - 32768).  Up to 127, where that makes a pass per 16 rows: always against up to 16384 channels (0.3 - 0.87) and from
+// K = 1152 on (0.28 - 0.98), and otherwise where the estimate is shorter than the streaming kernel's (fitted to 400
+// launches against 24576 - 262144 channels, K 128 - 1024: within 13 %).  The estimates here hold far past
+// four rounds of tiles (within 12 % at 262144 channels and 127 rows), except for a short K, where the last step may leave
+// K groups without a share (kShortK).  What makes the streaming kernel the shorter one is a row tile of 32 rows with 16 of
+// them dead: 33 x 128256 x 384 would take 80 us for its 67, 49 x 128256 x 384 takes 81 for 89.
+// More rows: while this is the shorter of the two estimates; the other is x split into three bf16 parts, 11 us and per
+// round of 128 x 128 tiles 3.2 + 0.78 per 128 of 3 K columns (measured at 128 - 700 rows: 512 x 1024 x 4096 92 -> 39 us,
+// 200 x 4096 x 4096 90 -> 69; 256 x 6144 x 4096 would be 90 -> 112).
 int qmm_wo_ksplit_f32_tile(int64_t M, int64_t N, int64_t K) {
   if (K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14) || (M <= 16 && N > 8192)) return -1;
-  KsLaunch l{(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, false, 0};
+  KsLaunch l{(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, 65535, kNoLimit};
   // (up to 16 rows none of the other tiles is the least at any N and K; the choice is part of a call of some 5 us)
   if (M <= 16) return ks_best<kKsTilesF32>(l, std::index_sequence<0, 1, 3>());
   if (M >= 128) {
     const double rounds = (double)(((M + 127) / 128 * ((N + 127) / 128) + 255) / 256);
-    l.limited = true;
+    l.most_tiles = 1024;
     l.least = (float)(11 + rounds * (3.2 + 0.78 * (double)(3 * K / 128)));
   }
-  return ks_best<kKsTilesF32>(l, ks_indices<kKsTilesF32>());
+  const int tile = ks_best<kKsTilesF32>(l, ks_indices<kKsTilesF32>());
+  if (M < 128 && N > 16384 && K <= 1024) {
+    // time over estimate, by tiles of K: of the 16 x 32 tile (eight K groups, taken from five tiles of K on), and of 32 x 64 (four)
+    constexpr float kShortK[2][8] = {{1, 1, 1, 1, 1, 1.03f, 1.06f, 1.07f}, {0.62f, 0.62f, 0.92f, 1, 0.95f, 0.95f, 1.1f, 1.11f}};
+    const float passes = (float)((M + 15) / 16), rounds = (float)((N + 32767) / 32768), k = (float)K;
+    const float stream = K <= 512 ? 1.3f + 0.0062f * k + rounds * (2.3f + 0.006f * k) : 3.5f + rounds * (2.6f + 0.0088f * k);
+    // (2 % for the errors of both: over 800 launches none takes more than 1.03 of the streaming kernel's time, and none
+    // that is left to that takes more than 1.05 of the time here)
+    if (1.02f * passes * stream < kShortK[tile == 1 ? 0 : 1][l.k128 - 1] * l.least) return -1;
+  }
+  return tile;
 }
 
 int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* scale, const void* zp, void* out, int64_t M, int64_t N,
@@ -781,14 +797,14 @@ inline void ks_bw_offer(KsLaunch& l, uint32_t sub, bool int8, bool zp) {
   constexpr KsBwTile t = kKsBwTiles[i];
   if (zp && !t.with_zp) return;
   const uint32_t tm = (l.m + t.bm - 1) / t.bm, tn = (l.n + t.bn - 1) / t.bn;
-  if ((uint64_t)tm * tn > 1024) return;  // (as in ks_offer)
+  if ((uint64_t)tm * tn > l.most_tiles) return;
   const uint32_t all = tm * tn, blocks = sub == 1 ? l.k128 : l.k128 / sub;
   const float rounds = (float)((all + 255) / 256), steps = (float)((blocks + t.kw - 1) / t.kw * sub);
   l.offer((int)i, t.fixed + t.round * rounds + (t.step + (zp ? t.zp : 0.f) + (int8 ? t.int8 : 0.f)) * rounds * steps +
                       t.load * (float)all / 256 * steps + t.weight * l.weight);
 }
 template <size_t... i>
-inline int ks_bw_best(KsLaunch l, uint32_t sub, bool int8, bool zp, std::index_sequence<i...>) {
+inline int ks_bw_best(KsLaunch& l, uint32_t sub, bool int8, bool zp, std::index_sequence<i...>) {
   (ks_bw_offer<i>(l, sub, int8, zp), ...);
   return l.best;
 }
@@ -805,14 +821,14 @@ int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, 
   if (N > (M <= 32 ? 8192 : 16384) && M <= 64) return -1;
   const uint32_t m = (uint32_t)M, n = (uint32_t)N, k128 = (uint32_t)K / 128, sub = C == K ? 1 : (uint32_t)C / 128;
   const float mb = 1e-6f * (float)N * (float)K * (float)bits / 8;
-  float least = 0;
+  KsLaunch l{m, n, k128, mb, 1024, kNoLimit};
   if (M > 64) {
     const uint32_t tm = (m + 63) / 64, narrow = (tm * ((n + 127) / 128) + 255) / 256, wide = (tm * ((n + 255) / 256) + 255) / 256;
     const bool use_wide = (!zp || (bits == 4 && C == 128)) && wide * (zp ? 145u : bits == 4 ? 155u : 165u) < narrow * 100u;  // (wide_tiles)
-    least = use_wide ? 2.13f + (float)wide * (2.13f + (zp ? 1.232f : 1.092f) * (float)k128) + 0.054f * mb
-                     : 1.02f + (float)narrow * (2.85f + (zp ? 0.757f : 0.667f) * (float)k128) + 0.085f * mb;
+    l.least = use_wide ? 2.13f + (float)wide * (2.13f + (zp ? 1.232f : 1.092f) * (float)k128) + 0.054f * mb
+                       : 1.02f + (float)narrow * (2.85f + (zp ? 0.757f : 0.667f) * (float)k128) + 0.085f * mb;
   }
-  return ks_bw_best({m, n, k128, mb, M > 64, least}, sub, bits == 8, zp, ks_indices<kKsBwTiles>());
+  return ks_bw_best(l, sub, bits == 8, zp, ks_indices<kKsBwTiles>());
 }
 
 int qmm_wo_ksplit_bw_run(int tile, const WoBwArgs& a, int bits, int x_dt, hipStream_t stream) {
