@@ -228,7 +228,9 @@ int xla_amd_qmm_weight_only_gemm(const void* x, const void* w_tiled, const void*
  * weights, K % 128 == 0, 3 K <= 2^23; scale / zp of any floating dtype.
  * `workspace`: xla_amd_qmm_weight_only_gemm_f32_workspace_bytes(M, N, K) bytes
  * of device memory (the three parts: 6 M K), 16-byte aligned, free again when
- * the call's work has completed.
+ * the call's work has completed; it may be NULL when that size is 0.
+ * Where the tiles of the K split over waves are the faster ones (see above; size
+ * 0), x is multiplied as it is, in f32 products.
  */
 size_t xla_amd_qmm_weight_only_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int xla_amd_qmm_weight_only_gemm_f32(const float* x, const void* w_tiled, const void* scale, const void* zp,

@@ -72,3 +72,8 @@ def blockwise(m, n, k, c, bits, zp, x_dt=1):
 def skinny(m, n, k, c, bits, zp, x_dt=1):
   return ("xla_amd_qmm_weight_only_skinny", "ppppp" + "qqqq" + "iiiiiii" + "p",
           [PTR, PTR, PTR, PTR if zp else 0, PTR, m, n, k, c, bits, *[x_dt] * 6, 0])
+
+
+def gemm_f32(m, n, k, zp=False, workspace=PTR, workspace_bytes=1 << 40):
+  return ("xla_amd_qmm_weight_only_gemm_f32", "pppppp" + "z" + "qqq" + "iip",
+          [PTR, PTR, PTR, PTR if zp else 0, PTR, workspace, workspace_bytes, m, n, k, 0, 0, 0])

@@ -169,3 +169,23 @@ def test_arguments_of_the_k_split_kernels():
   assert len(kernels) > 50
   for k in kernels:
     assert k["kernarg_bytes"] <= 120, (k["kernel"], k["kernarg_bytes"])
+
+
+def test_f32_rows_ask_for_no_workspace_they_do_not_use(tmp_path):
+  """The size asked for is what the launch writes: nothing where x is multiplied as it is (and then none is needed), the
+  three bf16 parts of x otherwise."""
+  lib = _lib.load()
+  as_it_is = [(128, 64, 128), (512, 1024, 4096), (300, 520, 640), (1, 64, 128), (128, 4096, 4096)]
+  in_parts = [(2048, 4096, 4096), (256, 8192, 256), (512, 4096, 128), (1000, 14336, 4096)]
+  sizes = [lib.xla_amd_qmm_weight_only_gemm_f32_workspace_bytes(*s) for s in as_it_is + in_parts]
+  assert sizes == [0] * len(as_it_is) + [6 * m * k for m, _, k in in_parts]
+  calls = [rec.gemm_f32(*s, workspace=0, workspace_bytes=0) for s in as_it_is]
+  calls += [f(*s) for s in in_parts for f in (rec.gemm_f32, lambda *s: rec.gemm_f32(*s, workspace_bytes=6 * s[0] * s[2] - 1),
+                                              lambda *s: rec.gemm_f32(*s, workspace=0))]
+  got = rec.record(calls, str(tmp_path))
+  for s, (rc, text, launches) in zip(as_it_is, got):
+    assert rc == 0 and len(launches) == 1 and "qmm_wo_ksplit_kernel" in launches[0].name, (s, text)
+  for s, (rc, text, launches), *short in zip(in_parts, *(got[len(as_it_is) + i::3] for i in range(3))):
+    assert rc == 0 and ["qmm_split3_kernel" in l.name for l in launches] == [True, False], (s, text, launches)
+    for rc, text, launches in short:
+      assert rc != 0 and not launches and "workspace" in text, s

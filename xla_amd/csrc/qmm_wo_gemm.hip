@@ -870,6 +870,7 @@ __global__ void __launch_bounds__(256) qmm_split3_kernel(const float* x, uint16_
 
 extern "C" size_t xla_amd_qmm_weight_only_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0) return 0;
+  if (qmm_wo_ksplit_f32_tile(M, N, K) >= 0) return 0;  // (x as it is)
   return (size_t)M * (size_t)K * 3 * sizeof(uint16_t);
 }
 
@@ -885,13 +886,13 @@ extern "C" int xla_amd_qmm_weight_only_gemm_f32(const float* x, const void* w_ti
   if ((((uintptr_t)x | (uintptr_t)w_tiled | (uintptr_t)out | (uintptr_t)workspace) & 15))
     return qmm_fail(XLA_AMD_QMM_EUNSUPPORTED, "weight_only_gemm_f32: x, w, out and workspace must be 16-byte aligned");
   if (M == 0) return XLA_AMD_QMM_OK;
-  const size_t need = xla_amd_qmm_weight_only_gemm_f32_workspace_bytes(M, N, K);
-  if (!workspace || workspace_bytes < need)
-    return qmm_fail(XLA_AMD_QMM_EINVAL, "weight_only_gemm_f32: workspace of %zu bytes, need %zu", workspace ? workspace_bytes : (size_t)0, need);
   hipStream_t s = (hipStream_t)stream;
   const int ks_tile = qmm_wo_ksplit_f32_tile(M, N, K);
   if (ks_tile >= 0)
     return qmm_wo_ksplit_run(ks_tile, x, w_tiled, scale, zp, out, M, N, K, XLA_AMD_DT_F32, scale_dt, zp_dt, XLA_AMD_DT_F32, XLA_AMD_DT_F32, XLA_AMD_DT_F32, s);
+  const size_t need = xla_amd_qmm_weight_only_gemm_f32_workspace_bytes(M, N, K);
+  if (!workspace || workspace_bytes < need)
+    return qmm_fail(XLA_AMD_QMM_EINVAL, "weight_only_gemm_f32: workspace of %zu bytes, need %zu", workspace ? workspace_bytes : (size_t)0, need);
   const int64_t quads = M * (K / 4);
   hipLaunchKernelGGL(qmm_split3_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, x, (uint16_t*)workspace, quads, (int)K);
   int rc = QMM_CHECK_LAUNCH("weight_only_gemm_f32 split launch");

@@ -195,9 +195,10 @@ std::optional<Tensor> weight_only(const Tensor& x_in, const Tensor& tiled, const
   if (kern == XLA_AMD_KERNEL_WEIGHT_ONLY_GEMM && x_dt == XLA_AMD_DT_F32) {
     count(kWoGemm);
     const size_t bytes = xla_amd_qmm_weight_only_gemm_f32_workspace_bytes(m, n, k);
-    Tensor ws = workspace(x, bytes);
+    const Tensor ws = bytes ? workspace(x, bytes) : Tensor();
     check(xla_amd_qmm_weight_only_gemm_f32((const float*)x.data_ptr(), tiled.data_ptr(), scale.data_ptr(), ptr(zp),
-                                           (float*)out.data_ptr(), ws.data_ptr(), bytes, m, n, k, s_dt, zp_dt, stream),
+                                           (float*)out.data_ptr(), bytes ? ws.data_ptr() : nullptr, bytes, m, n, k, s_dt,
+                                           zp_dt, stream),
           "weight_only_gemm_f32");
   } else if (kern == XLA_AMD_KERNEL_WEIGHT_ONLY_GEMM) {
     count(kWoGemm);
