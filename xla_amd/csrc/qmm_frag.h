@@ -45,24 +45,33 @@ __device__ __forceinline__ uint32_t cvt_w2(uint32_t d, HiC) {
   else return pack_f16(lo, hi);
 }
 
-// 8 packed int4 weights (one dword, nibble j = column P[j], biased by 8) -> 8
-// elements (1 + u/16) of the x dtype, u = w + 8 in 0..15.  The caller undoes
-// the affine map with the exact x sum: sum w*x = 16*(sum a*x - 1.5*sum x).
+// An int4 weight w becomes an element of the x dtype by setting mantissa bits alone, u = w + 8 in 0..15: 1 + u/16 in bf16,
+// 16 + u in f16.  The caller undoes the affine map with the exact x sum:
+//   sum w x = kInt4Factor (sum a x - kInt4Offset sum x)
+// In bf16 the factor may wait until behind the rounding of a dot product, a power of two commutes with it (down to 2^-126).
+// Not so in f16: a sixteenth of a dot product below 2^-10 is subnormal and would lose up to four of its bits, and one of
+// more than 65504 would not overflow.  (bf16 keeps 1 + u/16: sums of a x sixteen times as large would overflow at
+// x = 2^121.)
+template <int XT> constexpr float kInt4Factor = XT == XLA_AMD_DT_BF16 ? 16.0f : 1.0f;
+template <int XT> constexpr float kInt4Offset = XT == XLA_AMD_DT_BF16 ? 1.5f : 24.0f;
+template <int XT> constexpr uint32_t kInt4Bits = XT == XLA_AMD_DT_BF16 ? 0x3F803F80u : 0x4C004C00u;  // two elements of u = 0 ...
+template <int XT> constexpr uint32_t kInt4Mask = XT == XLA_AMD_DT_BF16 ? 0x00780078u : 0x03C003C0u;  // ... and the bits u sets
+
+// 8 packed int4 weights (one dword, nibble j = column P[j], biased by 8) -> 8 elements.
 template <int XT>
 __device__ __forceinline__ i32x4 cvt_w4(uint32_t d) {
   i32x4 o;
+  constexpr uint32_t mask = kInt4Mask<XT>, zero = kInt4Bits<XT>;
   if constexpr (XT == XLA_AMD_DT_BF16) {
-    const uint32_t mask = 0x00780078u, one = 0x3F803F80u;  // mantissa bits 3..6 of bf16
-    o[0] = ((d << 3) & mask) | one;
-    o[1] = ((d >> 1) & mask) | one;
-    o[2] = ((d >> 5) & mask) | one;
-    o[3] = ((d >> 9) & mask) | one;
+    o[0] = ((d << 3) & mask) | zero;
+    o[1] = ((d >> 1) & mask) | zero;
+    o[2] = ((d >> 5) & mask) | zero;
+    o[3] = ((d >> 9) & mask) | zero;
   } else {
-    const uint32_t mask = 0x03C003C0u, one = 0x3C003C00u;  // mantissa bits 6..9 of f16
-    o[0] = ((d << 6) & mask) | one;
-    o[1] = ((d << 2) & mask) | one;
-    o[2] = ((d >> 2) & mask) | one;
-    o[3] = ((d >> 6) & mask) | one;
+    o[0] = ((d << 6) & mask) | zero;
+    o[1] = ((d << 2) & mask) | zero;
+    o[2] = ((d >> 2) & mask) | zero;
+    o[3] = ((d >> 6) & mask) | zero;
   }
   return o;
 }

@@ -384,9 +384,9 @@ qmm_skinny_kernel(SkinnyArgs a) {
     zacc[mt] = f32x4{0, 0, 0, 0};
   });
 
-  // Undo the int4 affine map (MFMA path only): dot = 16 * (acc - 1.5 * xsum).
+  // Undo the int4 affine map (MFMA path only).
   auto true_dot = [&](float accv, float xsv) __attribute__((always_inline)) -> float {
-    if constexpr (BITS == 4 && kMfma) return 16.0f * (accv - 1.5f * xsv);
+    if constexpr (BITS == 4 && kMfma) return kInt4Factor<XT> * (accv - kInt4Offset<XT> * xsv);
     return accv;
   };
 
@@ -445,8 +445,8 @@ qmm_skinny_kernel(SkinnyArgs a) {
         const float xsv = NEEDXS ? xs[mt][0] : 0.f;
         float p;
         if constexpr (RED != kRedRaw && BITS == 4 && kMfma) {
-          // the int4 map's factor 16 is applied once, to the sum over the blocks (a power of two commutes with the rounding)
-          p = qmm_round_dt(fmaf(-1.5f, xsv, acc[mt][v] + accb[mt][v]), dot_dt);
+          // (the int4 map's factor is applied once, to the sum over the blocks)
+          p = qmm_round_dt(fmaf(-kInt4Offset<XT>, xsv, acc[mt][v] + accb[mt][v]), dot_dt);
         } else {
           p = qmm_round_dt(true_dot(acc[mt][v] + accb[mt][v], xsv), dot_dt);
         }
@@ -719,7 +719,7 @@ qmm_skinny_kernel(SkinnyArgs a) {
     const int m = 16 * mt + r;
     const int n = n_wave + 4 * g;
     if (m < M && n + 3 >= ch_lo && n < ch_hi) {
-      constexpr float kBlockFactor = (RED != kRedRaw && BITS == 4 && kMfma) ? 16.0f : 1.0f;  // see block_epilogue
+      constexpr float kBlockFactor = (RED != kRedRaw && BITS == 4 && kMfma) ? kInt4Factor<XT> : 1.0f;  // see block_epilogue
       if constexpr (RED != kRedRaw) {
         if (a.slices > 1) {
           // one K slice of several (whole quantization blocks): the sums over this slice's blocks go to the workspace,

@@ -17,9 +17,8 @@
 // the per-channel case as one block):
 //   per block s:  p = round_x(sum_c w x);  out_acc += scale[s,n] * p;  z_acc += round_x(sum_c x) * zp[s,n]
 //   out = round_x(out_acc);  with a zero point  out = round_x(out - round_x(z_acc)).
-// int4 weights are expanded to 1 + u/16 (u = w + 8) and the affine map is undone with the exact
-// block sum of x, sum w x = 16 (sum a x - 1.5 sum x); the factor 16 is applied once per output (a
-// power of two commutes with the rounding).
+// int4 weights are expanded by an affine map (qmm_frag.h) that is undone with the exact block sum of x; its factor is
+// applied once per output.
 #include "qmm_common.h"
 #include "qmm_frag.h"
 #include "qmm_wo_bw.h"
@@ -187,7 +186,7 @@ qmm_wo_bw_gemm_kernel(WoBwArgs a) {
         qmm_static_for<MT>([&](auto mc) {
           constexpr int mt = mc;
           float d = acc[gi][mt][v];
-          if constexpr (BITS == 4) d = fmaf(-1.5f, xs[mt][0], d);  // (times 16, applied at the end)
+          if constexpr (BITS == 4) d = fmaf(-kInt4Offset<XT>, xs[mt][0], d);  // (times the factor, applied at the end)
           const float p = qmm_round_dt(d, XT);
           sacc[gi][mt][v] = fmaf(sc, p, sacc[gi][mt][v]);
           if constexpr (HASZP) zacc[gi][mt][v] = fmaf(xs_r[mt], zv, zacc[gi][mt][v]);
@@ -237,7 +236,7 @@ qmm_wo_bw_gemm_kernel(WoBwArgs a) {
 
   // ---- results: four consecutive channels of one row per lane ----
   auto store_results = [&](const BwItem& done) __attribute__((always_inline)) {
-  constexpr float kFactor = BITS == 4 ? 16.0f : 1.0f;
+  constexpr float kFactor = BITS == 4 ? kInt4Factor<XT> : 1.0f;
   qmm_static_for<MT>([&](auto mc) {
     constexpr int mt = mc;
     const int m = done.m0 + 16 * mt + r;
@@ -286,9 +285,9 @@ qmm_wo_bw_gemm_kernel(WoBwArgs a) {
     constexpr int gi = pr / (4 * (MT / 2)), v = (pr / (MT / 2)) % 4, mt = 2 * (pr % (MT / 2));
     if constexpr (ph == 0) {
       float d0 = acc2[Q][gi][mt][v], d1 = acc2[Q][gi][mt + 1][v];
-      if constexpr (BITS == 4) {  // (times 16, applied at the end)
-        d0 = fmaf(-1.5f, xs2[Q][mt][0], d0);
-        d1 = fmaf(-1.5f, xs2[Q][mt + 1][0], d1);
+      if constexpr (BITS == 4) {  // (times the factor, applied at the end)
+        d0 = fmaf(-kInt4Offset<XT>, xs2[Q][mt][0], d0);
+        d1 = fmaf(-kInt4Offset<XT>, xs2[Q][mt + 1][0], d1);
       }
       wo_bw_round2<XT>(d0, d1, p0, p1);
     }
@@ -311,11 +310,10 @@ qmm_wo_bw_gemm_kernel(WoBwArgs a) {
   };
   // Constants of the int4 expansion and the fragment of ones kept in registers the compiler cannot see through: it
   // would otherwise build the ones again for every j (two moves per MFMA against them), and with both constants of
-  // (x & mask) | one as literals it cannot use the single instruction for it.
+  // (x & mask) | zero as literals it cannot use the single instruction for it.
   i32x4 ones = ones_frag<XT>();
-  uint32_t k_one = XT == XLA_AMD_DT_BF16 ? 0x3F803F80u : 0x3C003C00u;
-  uint32_t k_mask = XT == XLA_AMD_DT_BF16 ? 0x00780078u : 0x03C003C0u;
-  asm volatile("" : "+v"(ones), "+v"(k_one), "+s"(k_mask));
+  uint32_t k_zero = kInt4Bits<XT>, k_mask = kInt4Mask<XT>;
+  asm volatile("" : "+v"(ones), "+v"(k_zero), "+s"(k_mask));
   // element q (two columns) of the fragment (j, gi) of the step's weights
   auto frag_q = [&](auto jc, auto gic, auto qc) __attribute__((always_inline)) {
     constexpr int j = jc, gi = gic, q = qc;
@@ -325,7 +323,7 @@ qmm_wo_bw_gemm_kernel(WoBwArgs a) {
       const uint32_t d = (uint32_t)wcur[gi][0][j];
       constexpr int sh = XT == XLA_AMD_DT_BF16 ? 4 * q - 3 : 4 * q - 6;  // right shift (negative: left)
       const uint32_t t = sh < 0 ? d << (sh < 0 ? -sh : 0) : d >> (sh < 0 ? 0 : sh);
-      return (int)((t & k_mask) | k_one);
+      return (int)((t & k_mask) | k_zero);
     }
   };
   // One step = one block into set P, out of LDS tile `tile`, with the rounding sequence of the block in set 1 - P

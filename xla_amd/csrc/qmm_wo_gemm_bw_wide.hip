@@ -9,8 +9,8 @@
 // what counts is how few instructions a step has:
 //  * the sums of x per step come from the copying waves, once per row (four MFMAs against ones for their 16 rows)
 //    instead of once per row and computing wave, and reach the computing waves as the MFMAs' initial accumulators
-//    (-1.5 sum x, four times side by side: a lane reads its accumulator quad), so that undoing the affine map of int4
-//    weights (1 + u/16, u = w + 8: sum w x = 16 (sum a x - 1.5 sum x)) costs no vector instruction;
+//    (-kInt4Offset sum x, four times side by side: a lane reads its accumulator quad), so that undoing the affine map of
+//    int4 weights (qmm_frag.h) costs no vector instruction;
 //  * the zero points' term is a matrix product over the blocks: the copying waves leave round_x(sum x) of 16 blocks
 //    in LDS, next to the zero points of the 16 blocks, and the computing waves add them with one MFMA per result tile.
 // The second wave per SIMD covers the waits of the first, and twice the channels per workgroup halve the copies of x.
@@ -41,7 +41,7 @@ static_assert(BM == 16 * kCopyWaves, "a copying wave copies and sums the 16 rows
 constexpr int MT = BM / 16;              // 16-row tiles: every computing wave owns all rows of its channels
 constexpr int BN = 16 * NG * kComputeWaves;  // 256 channels per workgroup
 constexpr int kEntry = BN * 2;           // one entry: the workgroup's channels, 2-byte values
-// LDS: scales of every resident step; -1.5 sum x of every resident step and row, four times; zero points and rounded
+// LDS: scales of every resident step; -kInt4Offset sum x of every resident step and row, four times; zero points and rounded
 // sums of x of two groups of 16 blocks; x
 constexpr int kXsq = 2 * CS * kEntry;
 constexpr int kZent = kXsq + 2 * CS * BM * 16;
@@ -137,7 +137,7 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
           });
           const float s = xs[0];  // (the same in every lane of a row)
           if constexpr (BITS == 4) {
-            const float q = -1.5f * s;
+            const float q = -kInt4Offset<XT> * s;
             if (g == 0) *(f32x4*)(smem + kXsq + ((slot_i * CS + t) * BM + 16 * cw + r) * 16) = f32x4{q, q, q, q};
           }
           if constexpr (HASZP) {
@@ -263,10 +263,9 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
     });
   };
   // Constants of the int4 expansion kept in registers the compiler cannot see through: with both constants of
-  // (x & mask) | one as literals it cannot use the single instruction for it.
-  uint32_t k_one = XT == XLA_AMD_DT_BF16 ? 0x3F803F80u : 0x3C003C00u;
-  uint32_t k_mask = XT == XLA_AMD_DT_BF16 ? 0x00780078u : 0x03C003C0u;
-  asm volatile("" : "+v"(k_one), "+s"(k_mask));
+  // (x & mask) | zero as literals it cannot use the single instruction for it.
+  uint32_t k_zero = kInt4Bits<XT>, k_mask = kInt4Mask<XT>;
+  asm volatile("" : "+v"(k_zero), "+s"(k_mask));
   // dword q (two columns) of the fragment (j, gi) of the weights in slot P (see cvt_w8 and cvt_w4)
   auto frag_q = [&](auto pc, auto jc, auto gic, auto qc) __attribute__((always_inline)) {
     constexpr int P = pc, j = jc, gi = gic, q = qc;
@@ -276,7 +275,7 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
       const uint32_t d = (uint32_t)wreg[P][gi][0][j];
       constexpr int sh = XT == XLA_AMD_DT_BF16 ? 4 * q - 3 : 4 * q - 6;  // right shift (negative: left)
       const uint32_t t = sh < 0 ? d << (sh < 0 ? -sh : 0) : d >> (sh < 0 ? 0 : sh);
-      return (int)((t & k_mask) | k_one);
+      return (int)((t & k_mask) | k_zero);
     }
   };
   // The weight fragments of one j (columns 32 g + 8 j .. + 7 of the step) in use and those of the next j, which are
@@ -345,7 +344,7 @@ qmm_wo_bw_wide_kernel(WoBwArgs a) {
     int l = lane;
     asm volatile("" : "+v"(l));  // (as in add_zero_points)
     const int r = l & 15, g = l >> 4;
-    constexpr float kFactor = BITS == 4 ? 16.0f : 1.0f;
+    constexpr float kFactor = BITS == 4 ? kInt4Factor<XT> : 1.0f;
     qmm_static_for<MT>([&](auto mc) {
       constexpr int mt = mc;
       const int m = done.m0 + 16 * mt + r;

@@ -14,8 +14,7 @@
 //
 // Arithmetic, one dtype (x's) throughout:
 //   p_b = round(sum_block x w); out = round(sum_b scale_b p_b); zero point: out = round(out - round(sum_b round(sum_block x) zp_b)).
-// int4 weights are expanded to 1 + u/16, u = w + 8: sum w x = 16 (sum a x - 1.5 sum x), the factor 16 applied at the end
-// (a power of two commutes with the rounding).
+// int4 weights are expanded by an affine map (qmm_frag.h), its factor applied at the end.
 //
 // This file is compiled per activation dtype and bits (-DQMM_WO_XT=1|2 for bf16 | f16, -DQMM_KS_BITS=4|8).
 #include "qmm_wo_bw.h"
@@ -154,7 +153,7 @@ qmm_wo_bw_gemm_kernel_ksplit(WoBwArgs a, KsTiles t) {
                 }
                 qmm_static_for<MT>([&](auto mc) {
                   constexpr int mt = mc;
-                  const float d = BITS == 4 ? fmaf(-1.5f, xs[mt][0], acc[gi][mt][v]) : acc[gi][mt][v];
+                  const float d = BITS == 4 ? fmaf(-kInt4Offset<XT>, xs[mt][0], acc[gi][mt][v]) : acc[gi][mt][v];
                   sacc[gi][mt][v] = fmaf(sc, qmm_round_dt(d, XT), sacc[gi][mt][v]);
                   if constexpr (HASZP) zacc[gi][mt][v] = fmaf(qmm_round_dt(xs[mt][0], XT), zv, zacc[gi][mt][v]);
                 });
@@ -209,7 +208,7 @@ qmm_wo_bw_gemm_kernel_ksplit(WoBwArgs a, KsTiles t) {
     }
   }
   qmm_bare_barrier();
-  constexpr float kFactor = BITS == 4 ? 16.0f : 1.0f;
+  constexpr float kFactor = BITS == 4 ? kInt4Factor<XT> : 1.0f;
   float o[kPer][4];
   qmm_static_for<kPer>([&](auto ic) {
     const int q = (int)ic * kThreads + (int)threadIdx.x;
@@ -223,7 +222,7 @@ qmm_wo_bw_gemm_kernel_ksplit(WoBwArgs a, KsTiles t) {
         qmm_static_for<4>([&](auto vc) {
           constexpr int v = vc;
           const int ch = min(n + v, N - 1);
-          const float dot = kFactor * (BITS == 4 ? fmaf(-1.5f, xsum, sum[v]) : sum[v]);
+          const float dot = kFactor * (BITS == 4 ? fmaf(-kInt4Offset<XT>, xsum, sum[v]) : sum[v]);
           float t = qmm_round_dt(qmm_load(a.scale, ch, XT) * qmm_round_dt(dot, XT), XT);
           if constexpr (HASZP) t = qmm_round_dt(t - qmm_round_dt(qmm_round_dt(xsum, XT) * qmm_load(a.zp, ch, XT), XT), XT);
           o[(int)ic][v] = t;
