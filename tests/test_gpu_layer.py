@@ -271,14 +271,14 @@ def test_graph_capture_needs_a_prepared_weight(ops):
 
 
 def test_graph_replays_of_the_routes_with_several_kernels(ops):
-  """One HIP graph over the routes that launch more than one kernel or use a workspace (K slices of per-channel and of
-  blockwise weights with their second kernel, the weight-only GEMM with a K split, the W8A8 operator's quantizer + GEMM):
-  every replay, with new activations copied in and eager work in between, gives the eager result."""
+  """One HIP graph over weight-only launches of 24 and 80 rows (K split over waves) and the W8A8 operator's quantizer +
+  GEMM: every replay, with new activations copied in and eager work in between, gives the eager result.  (K slices and
+  finishing kernels: test_graph_replays_of_workspaces.)"""
   op = torch.ops.xla.quantized_matmul
   m = 24
-  x1, w1, s1, _ = cases.per_channel_int8(m, 512, 8192, torch.bfloat16, torch.bfloat16, seed=61)      # K slices
-  x2, w2, s2, z2, _ = cases.blockwise(m, 256, 8192, 128, 4, torch.bfloat16, symmetric=False, seed=62)  # blockwise K slices
-  x3, w3, s3, _ = cases.per_channel_int8(80, 384, 2048, torch.bfloat16, torch.bfloat16, seed=63)     # tiled GEMM, K split
+  x1, w1, s1, _ = cases.per_channel_int8(m, 512, 8192, torch.bfloat16, torch.bfloat16, seed=61)
+  x2, w2, s2, z2, _ = cases.blockwise(m, 256, 8192, 128, 4, torch.bfloat16, symmetric=False, seed=62)
+  x3, w3, s3, _ = cases.per_channel_int8(80, 384, 2048, torch.bfloat16, torch.bfloat16, seed=63)
   x4 = cases.outlier_activations(96, 1024, torch.bfloat16, seed=64)                                  # W8A8
   _, w4, s4, _ = cases.per_channel_int8(1, 320, 1024, torch.bfloat16, torch.float32, seed=65)
   dev_ = lambda *ts: [t.cuda() for t in ts]
@@ -311,8 +311,52 @@ def test_graph_replays_of_the_routes_with_several_kernels(ops):
     torch.cuda.synchronize()
     for i, (a, b) in enumerate(zip(outs, eager)):
       assert torch.equal(a, b), f"replay {rep}, route {i}"
-  check(outs[0], oracle.quantized_matmul(x1d.cpu(), w1, s1), "K slices after the replays")
-  check(outs[1], oracle.quantized_matmul(x2d.cpu(), w2, s2, z2, block_size=128, int4_weight=True), "blockwise K slices after the replays")
+  check(outs[0], oracle.quantized_matmul(x1d.cpu(), w1, s1), "per-channel after the replays")
+  check(outs[1], oracle.quantized_matmul(x2d.cpu(), w2, s2, z2, block_size=128, int4_weight=True), "blockwise after the replays")
+
+
+# (m, n, k, block): two kernels and a workspace each (tests/test_launches.py pins that): K slices of per-channel and of
+# blockwise int4 weights, the tiled GEMM's K split with 64- and 128-row tiles, f32 rows in three bf16 parts
+GRAPH_ROUTES = [(24, 512, 14336, -1, "bf16"), (12, 256, 8192, 128, "bf16"), (48, 200, 16384, -1, "bf16"), (65, 333, 16384, -1, "bf16"),
+                (512, 4096, 128, -1, "f32")]
+
+
+def test_graph_replays_of_workspaces(ops):
+  """One HIP graph over the routes that leave partial results in a workspace for a second kernel: every replay, with new
+  activations copied in and eager work in between, gives the eager result."""
+  op = torch.ops.xla.quantized_matmul
+  calls, gen = [], cases.gen(71)
+  for m, n, k, c, xdt in GRAPH_ROUTES:
+    xdt = {"bf16": torch.bfloat16, "f32": torch.float32}[xdt]
+    if c == -1:
+      x, w, s, _ = cases.per_channel_int8(m, n, k, xdt, xdt, seed=m)
+      z = None
+    else:
+      x, w, s, z, _ = cases.blockwise(m, n, k, c, 4, xdt, symmetric=False, seed=m)
+    calls.append((x.cuda(), w.cuda(), s.cuda(), None if z is None else z.cuda(), c, c != -1))
+    ops.prepare_weight(calls[-1][1], block_size=c, int4_weight=c != -1, x_dtype=xdt)
+
+  def run():
+    return [op(*c) for c in calls]
+
+  before = ops.counters["wo_gemm"]
+  run()
+  assert ops.counters["wo_gemm"] == before + len(calls)
+  torch.cuda.synchronize()
+  g = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(g):
+    outs = run()
+  for rep in range(3):
+    for xd, *_ in calls:
+      xd.copy_((torch.randn(xd.shape, generator=gen) * (1 + rep)).to(xd.dtype))
+    g.replay()
+    torch.cuda.synchronize()
+    eager = run()
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(outs, eager)):
+      assert torch.equal(a, b), f"replay {rep}, route {i}"
+  for out, (x, w, s, z, c, int4) in zip(outs, calls):
+    check(out, oracle.quantized_matmul(x.cpu(), w.cpu(), s.cpu(), None if z is None else z.cpu(), block_size=c, int4_weight=int4), "after the replays")
 
 
 def test_quantizer_nan_row(ops):

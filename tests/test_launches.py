@@ -189,3 +189,52 @@ def test_f32_rows_ask_for_no_workspace_they_do_not_use(tmp_path):
     assert rc == 0 and ["qmm_split3_kernel" in l.name for l in launches] == [True, False], (s, text, launches)
     for rc, text, launches in short:
       assert rc != 0 and not launches and "workspace" in text, s
+
+
+def _with_f32_scale(call):
+  name, sig, args = call
+  return (name, sig, args[:13] + [0, 0, args[15], 0, 0] + args[-1:])  # scale, zero point, result and store
+
+
+def test_tiled_and_sliced_tests_run_those_kernels(tmp_path):
+  """The sizes tests/test_gpu_wo_gemm.py names after a kernel run that kernel (the operator's counters count entry points,
+  behind which the K split over waves takes most launches of 17 - 1000 rows)."""
+  from tests.test_gpu_wo_gemm import BW_SLICED, F32_IN_PARTS, NARROW, SLICED, TILED
+  calls, want = [], []
+  for x_dt in (1, 2):
+    for zp in (False, True):
+      for m, n, k, mt, kernels in TILED:
+        one = rec.blockwise(m, n, k, k, 8, zp, x_dt)
+        calls += [one, _with_f32_scale(one)]
+        want += [["qmm_wo_gemm_kernelILi%dELi%dE" % (x_dt, mt), "qmm_wo_gemm_finish_kernel"][:kernels]] * 2
+      for m, n, k in SLICED:
+        one = rec.blockwise(m, n, k, k, 8, zp, x_dt)
+        calls += [one, _with_f32_scale(one)]
+        want += [["qmm_skinny_kernelILi%dELi8ELi%dE" % (x_dt, 1 if m <= 16 else 2), "qmm_wo_gemm_finish_kernel"]] * 2
+    for m, n, k, c, bits, zp in BW_SLICED:
+      calls.append(rec.blockwise(m, n, k, c, bits, zp, x_dt))
+      want.append(["qmm_skinny_kernelILi%dELi%dELi%dE" % (x_dt, bits, 1 if m <= 16 else 2), "qmm_wo_bw_finish_kernel"])
+    for m, n, k, c, bits, zp in NARROW:
+      calls.append(rec.blockwise(m, n, k, k if c == -1 else c, bits, zp, x_dt))
+      want.append(["qmm_wo_bw_gemm_kernelILi%dELi%dELb%dELb%dE" % (x_dt, bits, zp, c == 128 and not (bits == 8 and zp))])
+  for zp in (False, True):
+    for s in F32_IN_PARTS:
+      calls.append(rec.gemm_f32(*s, zp=zp))
+      want.append(["qmm_split3_kernel", "qmm_wo_gemm_kernelILi1ELi8E"])
+  seen = set()
+  for call, names, (rc, text, launches) in zip(calls, want, rec.record(calls, str(tmp_path))):
+    assert rc == 0 and len(launches) == len(names) and all(n in l.name for n, l in zip(names, launches)), (call[2], names, text, launches)
+    seen.update(l.name for l in launches)
+  # every form of the tiled kernels: 16 of the 64-row tile, 10 of the 128-row one, 14 of the blockwise one
+  assert [sum(s in n for n in seen) for s in ("qmm_wo_gemm_kernelILi1ELi4E", "qmm_wo_gemm_kernelILi2ELi4E", "qmm_wo_gemm_kernelILi1ELi8E",
+                                              "qmm_wo_gemm_kernelILi2ELi8E", "qmm_wo_bw_gemm_kernelI")] == [8, 8, 5, 5, 14]
+
+
+def test_graph_of_workspaces_runs_two_kernels_each(tmp_path):
+  from tests.test_gpu_layer import GRAPH_ROUTES
+  calls = [rec.gemm_f32(m, n, k) if xdt == "f32" else rec.blockwise(m, n, k, k if c == -1 else c, 8 if c == -1 else 4, c != -1)
+           for m, n, k, c, xdt in GRAPH_ROUTES]
+  second = ["qmm_wo_gemm_finish_kernel", "qmm_wo_bw_finish_kernel", "qmm_wo_gemm_finish_kernel", "qmm_wo_gemm_finish_kernel",
+            "qmm_wo_gemm_kernel"]
+  for name, (rc, text, launches) in zip(second, rec.record(calls, str(tmp_path))):
+    assert rc == 0 and len(launches) == 2 and name in launches[1].name, (text, launches)
