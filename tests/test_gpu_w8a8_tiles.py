@@ -56,6 +56,12 @@ def test_64x128_asked_for(ops, m, n, k):
   _check(ops, m, n, k, block_m=64, block_n=128)
 
 
+# 128 x 128 tiles: three stages with one tile per compute unit at most, two with more
+@pytest.mark.parametrize("m,n,k", [(128, 128, 128), (129, 258, 272), (300, 200, 1040), (2100, 2100, 400)])
+def test_128x128_asked_for(ops, m, n, k):
+  _check(ops, m, n, k, block_m=128, block_n=128)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_quantizer_thread_counts(ops, dtype):
   for k in (2048, 2056, 4096, 4104, 8192, 8200, 16384, 16392):

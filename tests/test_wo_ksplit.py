@@ -132,7 +132,7 @@ def test_tiles_of_the_shapes(tmp_path):
 def test_against_the_oracle(m, n, k, bm, bn, xdt):
   import xla_amd.experimental.custom_kernel  # noqa: F401
   op = torch.ops.xla.quantized_matmul
-  for zp, sdt in ((False, xdt), (True, xdt), (True, torch.float32)):
+  for zp, sdt in ((False, torch.float32), (False, xdt), (True, xdt), (True, torch.float32)):
     x, w, s, _ = cases.per_channel_int8(m, n, k, xdt, sdt, seed=m + n)
     z = (torch.randn(n, generator=cases.gen(5)) * 0.01).to(sdt) if zp else None
     exp = oracle.quantized_matmul(x, w, s, z)
@@ -154,7 +154,7 @@ def test_against_the_oracle(m, n, k, bm, bn, xdt):
 def test_f32_against_f64(m, n, k, bm, bn):
   import xla_amd.experimental.custom_kernel  # noqa: F401
   op = torch.ops.xla.quantized_matmul
-  for zp, sdt in ((False, torch.float32), (True, torch.float32), (True, torch.bfloat16)):
+  for zp, sdt in ((False, torch.bfloat16), (False, torch.float32), (True, torch.float32), (True, torch.bfloat16)):
     x, w, s, _ = cases.per_channel_int8(m, n, k, torch.float32, sdt, seed=m + n)
     z = (torch.randn(n, generator=cases.gen(5)) * 0.01).to(sdt) if zp else None
     exp = (x.double() @ w.double().T) * s.double()
@@ -172,6 +172,30 @@ def test_f32_against_f64(m, n, k, bm, bn):
   bad = op(x.cuda(), wd, sd, zd).cpu()
   assert torch.equal(bad[:row], out[:row])
   assert not torch.isfinite(bad[row]).any()
+
+
+# past the K of this kernel the streaming kernel runs, with one and two x tiles and K split over four waves
+LONG_ROWS = [(8, 61, 66048, torch.float32), (20, 61, 66048, torch.bfloat16), (20, 61, 66048, torch.float16)]
+
+
+def test_long_rows_keep_the_streaming_kernel(tmp_path):
+  dts = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
+  calls = [rec.skinny(m, n, k, k, 8, zp, dts[xdt]) for m, n, k, xdt in LONG_ROWS for zp in (False, True)]
+  for call, (rc, text, launches) in zip(calls, rec.record(calls, str(tmp_path))):
+    assert rc == 0 and len(launches) == 1, text
+    assert re.search(r"qmm_skinny_kernelILi\dELi8ELi%dELi4ELi1E" % (2 if call[2][5] > 16 else 1), launches[0].name), launches
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,xdt", LONG_ROWS)
+def test_long_rows(m, n, k, xdt):
+  import xla_amd.experimental.custom_kernel  # noqa: F401
+  for zp, sdt in ((False, xdt), (True, xdt), (False, torch.float32), (True, torch.float32)):
+    x, w, s, _ = cases.per_channel_int8(m, n, k, xdt, sdt, seed=m)
+    z = (torch.randn(n, generator=cases.gen(5)) * 0.01).to(sdt) if zp else None
+    exp = oracle.quantized_matmul(x, w, s, z)
+    out = torch.ops.xla.quantized_matmul(x.cuda(), w.cuda(), s.cuda(), None if z is None else z.cuda()).cpu()
+    assert out.dtype == exp.dtype and cases.within_tolerance(out, exp) and cases.rel_l2(out, exp) < 1e-3, (zp, sdt)
 
 
 @pytest.mark.gpu
