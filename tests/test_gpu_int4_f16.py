@@ -9,7 +9,7 @@ from tests import launch_recorder as rec
 SHAPES = [
     (1, 64, 512, 128, True, "qmm_skinny_kernel"), (16, 256, 4096, 128, True, "qmm_skinny_kernel"),
     (12, 256, 8192, 128, False, "qmm_skinny_kernel"), (40, 132, 640, 128, True, "qmm_wo_bw_gemm_kernel_ksplit"),
-    (260, 3000, 384, 128, True, "qmm_wo_bw_gemm_kernelI"), (260, 3000, 512, 256, False, "qmm_wo_bw_gemm_kernelI"),
+    (260, 3000, 384, 128, True, "qmm_wo_bw_gemm_kernelI"), (300, 4096, 512, 256, False, "qmm_wo_bw_gemm_kernelI"),
     (130, 3000, 128, 128, False, "qmm_wo_bw_gemm_kernelI"), (1030, 2052, 256, 128, True, "qmm_wo_bw_wide_kernel"),
 ]
 

@@ -69,6 +69,33 @@ def test_tiles_of_the_blockwise_shapes(tmp_path):
     assert rc == 0 and launches and not any("ksplit" in l.name for l in launches), text
 
 
+def test_blockwise_launches_left_to_the_older_kernels(tmp_path):
+  """Blockwise launches that are shorter in K slices of the streaming kernel, in one pass of it, or in the tiles of the GEMM,
+  beside ones of the same kinds that are not."""
+  want = [
+      # K slices: 17 - 32 rows, few channels, a long K in long blocks
+      ((27, 620, 13312, 512, 8, False), "qmm_skinny_kernel"), ((17, 256, 16384, 256, 8, False), "qmm_skinny_kernel"),
+      ((24, 1536, 10240, 1024, 8, False), "qmm_skinny_kernel"), ((18, 4168, 11264, 512, 4, False), "qmm_skinny_kernel"),
+      ((32, 512, 4096, 128, 4, False), "ksplit"), ((24, 512, 14336, -1, 4, True), "ksplit"), ((32, 4096, 4096, 128, 4, True), "ksplit"),
+      # two long blocks
+      ((18, 4892, 1024, 512, 4, True), "qmm_skinny_kernel"), ((20, 1024, 2048, 1024, 8, False), "qmm_skinny_kernel"),
+      ((18, 4892, 1024, 128, 4, True), "ksplit"), ((20, 1024, 4096, 1024, 8, False), "ksplit"),
+      # tiles of the GEMM
+      ((314, 8176, 12800, 128, 4, False), "qmm_wo_bw_wide_kernel"), ((603, 4308, 13824, 128, 4, False), "qmm_wo_bw_wide_kernel"),
+      ((629, 3224, 7936, 128, 4, True), "qmm_wo_bw_wide_kernel"), ((633, 4224, 10240, 512, 8, False), "qmm_wo_bw_wide_kernel"),
+      ((128, 4096, 4096, 128, 4, True), "ksplit"), ((300, 2048, 8192, 256, 4, False), "ksplit"), ((100, 4096, 8192, 128, 8, False), "ksplit"),
+  ]
+  calls = [(rec.skinny if m <= 32 and k < 4096 else rec.blockwise)(m, n, k, k if c == -1 else c, bits, zp, dt)
+           for (m, n, k, c, bits, zp), _ in want for dt in (1, 2)]
+  for (shape, kernel), got in zip([w for w in want for _ in (1, 2)], rec.record(calls, str(tmp_path))):
+    rc, text, launches = got
+    assert rc == 0 and kernel in launches[0].name, (shape, text, launches)
+  # without the workspace that the slices need, the split takes them
+  name, sig, args = rec.blockwise(27, 620, 13312, 512, 8, False)
+  ((rc, text, launches),) = rec.record([(name, sig, args[:5] + [0, 0] + args[7:])], str(tmp_path))
+  assert rc == 0 and "ksplit" in launches[0].name, text
+
+
 def test_tiles_of_the_f32_shapes(tmp_path):
   calls = [rec.skinny(m, n, k, k, 8, zp, 0) for m, n, k, _, _ in F32_SHAPES for zp in (False, True)]
   seen = set()

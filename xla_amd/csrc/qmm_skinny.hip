@@ -955,7 +955,7 @@ extern "C" int xla_amd_qmm_weight_only_skinny(const void* x, const void* w_tiled
   // the same for blockwise and int4 weights against 17 - 64 rows of 2-byte x, every dtype x's
   if ((C != K || bits == 4) && M <= 64 && x_dt != XLA_AMD_DT_F32 && scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt &&
       store_dt == x_dt && (((uintptr_t)scale | (uintptr_t)zp) & 3) == 0) {
-    const int tile = qmm_wo_ksplit_bw_tile(M, N, K, C, bits, zp != nullptr);
+    const int tile = qmm_wo_ksplit_bw_tile(M, N, K, C, bits, zp != nullptr, x_dt == XLA_AMD_DT_F16, 1, (int)K);
     if (tile >= 0) {
       const WoBwArgs b{x, (const uint8_t*)w_tiled, scale, zp, out, (int)M, (int)N, (int)K, (int)C};
       return qmm_wo_ksplit_bw_run(tile, b, bits, x_dt, (hipStream_t)stream);

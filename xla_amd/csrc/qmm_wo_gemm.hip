@@ -792,43 +792,88 @@ int qmm_wo_ksplit_run(int tile, const void* x, const void* w_tiled, const void* 
 
 namespace {
 
+// ... of the blockwise kernel: the launch's shape with the tile picked so far, too.
+struct KsBwLaunch : KsLaunch {
+  uint32_t tiles = 0, rounds = 0, blocks = 0;  // blocks: of quantization per wave (tiles of 128 columns, per channel)
+};
 template <size_t i>
-inline void ks_bw_offer(KsLaunch& l, uint32_t sub, bool int8, bool zp) {
+inline void ks_bw_offer(KsBwLaunch& l, uint32_t sub, bool int8, bool zp) {
   constexpr KsBwTile t = kKsBwTiles[i];
   if (zp && !t.with_zp) return;
   const uint32_t tm = (l.m + t.bm - 1) / t.bm, tn = (l.n + t.bn - 1) / t.bn;
   if ((uint64_t)tm * tn > l.most_tiles) return;
-  const uint32_t all = tm * tn, blocks = sub == 1 ? l.k128 : l.k128 / sub;
-  const float rounds = (float)((all + 255) / 256), steps = (float)((blocks + t.kw - 1) / t.kw * sub);
-  l.offer((int)i, t.fixed + t.round * rounds + (t.step + (zp ? t.zp : 0.f) + (int8 ? t.int8 : 0.f)) * rounds * steps +
+  const uint32_t all = tm * tn, rounds = (all + 255) / 256, blocks = ((sub == 1 ? l.k128 : l.k128 / sub) + t.kw - 1) / t.kw;
+  const float r = (float)rounds, steps = (float)(blocks * sub);
+  l.offer((int)i, t.fixed + t.round * r + (t.step + (zp ? t.zp : 0.f) + (int8 ? t.int8 : 0.f)) * r * steps +
                       t.load * (float)all / 256 * steps + t.weight * l.weight);
+  if (l.best == (int)i) { l.tiles = all; l.rounds = rounds; l.blocks = blocks; }
 }
 template <size_t... i>
-inline int ks_bw_best(KsLaunch& l, uint32_t sub, bool int8, bool zp, std::index_sequence<i...>) {
+inline int ks_bw_best(KsBwLaunch& l, uint32_t sub, bool int8, bool zp, std::index_sequence<i...>) {
   (ks_bw_offer<i>(l, sub, int8, zp), ...);
   return l.best;
+}
+
+// Time of a launch of the tiled blockwise GEMM, us: 64 x 128 tiles, or 64 x 256 ones (wide_tiles); fitted to 11477 and
+// 1421 launches of 65 - 1000 rows (root mean square error 3.4 and 4.6 %).
+float bw_gemm_us(uint32_t m, uint32_t n, uint32_t k128, uint32_t blocks, uint32_t C, int bits, bool zp, bool f16) {
+  const uint32_t tm = (m + 63) / 64, narrow = tm * ((n + 127) / 128), wide = tm * ((n + 255) / 256);
+  const uint32_t rn = (narrow + 255) / 256, rw = (wide + 255) / 256;
+  const bool int8 = bits == 8;
+  if ((!zp || (!int8 && C == 128)) && rw * (zp ? 145u : int8 ? 165u : 155u) < rn * 100u) {
+    const float step = 0.552f + (f16 && C == 128 ? -0.090f : 0.f) + (zp ? 0.056f : 0.f) + (int8 ? 0.092f : 0.f);
+    return 3.498f + (float)rw * (2.649f + step * (float)k128 + 0.165f * (float)blocks) + 0.458f * (float)wide / 256 * (float)k128;
+  }
+  // (blocks of 128 columns are rounded during the next one's MFMAs, but for int8 with a zero point)
+  const float step = 0.592f + (f16 ? -0.035f : 0.f) + (zp ? 0.017f : 0.f) + (int8 ? -0.044f : 0.f) + (C == 128 && !(int8 && zp) ? -0.171f : 0.f);
+  return 2.638f + (float)rn * (1.575f + step * (float)k128 + (0.228f + (zp ? 0.062f : 0.f)) * (float)blocks) + 0.118f * (float)narrow / 256 * (float)k128;
+}
+
+// Time of the streaming kernel over K slices for 17 - 32 rows, and of the kernel that adds them, us: fitted to 6404 launches
+// (root mean square error 6 %).  A slice's steps of 512 columns (int4: 1024) are split over the waves (launch_split).
+float bw_slices_us(int64_t M, int64_t N, int64_t C, int bits, bool zp, bool perch, int slices, int k_per_slice) {
+  const int step = bits == 4 ? 1024 : 512, steps = (k_per_slice + step - 1) / step;
+  const int64_t groups = (N + 15) / 16;
+  int waves = 1;
+  if (perch || step % C == 0) {
+    if ((groups + 1) / 2 * slices <= 256 && steps >= 2) waves = 2;
+    if (groups * slices <= 256 && steps >= 4) waves = 4;
+  }
+  const float serial = (float)((steps + waves - 1) / waves), blocks = perch ? 0.f : (float)k_per_slice / (float)(C * waves);
+  const float sums = 4e-6f * (float)slices * (float)M * (float)N * (zp && !perch ? 2 : 1);
+  return 6.12f + serial * (0.966f + (bits == 4 ? 1.157f : 0.f) + (perch ? 0.058f : 0.f) + (zp ? 0.265f : 0.f) + (perch && zp ? 0.429f : 0.f)) +
+         1.046f * sums + blocks * (0.103f + (zp ? 0.035f : 0.f)) + (waves > 1 ? 1.53f : 0.f);
 }
 
 }  // namespace
 
 // Up to 16 rows the streaming kernel is as fast (0.8 - 1.2 of its time here).  17 - 32 rows: against up to 8192 channels
-// (0.57 - 0.91 of the streaming kernel's time; 11008 and 14336 channels 0.8 - 1.2).  33 - 64 rows, two passes of the
-// streaming kernel: against up to 16384 channels (0.34 - 0.71).  More: the shorter of the two estimates, the other being
-// the tiled GEMM's with its two tiles, fitted to 129 launches (root mean square error 4 - 6 %).
-int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, bool zp) {
+// (0.57 - 0.95 of the streaming kernel's time; 11008 and 14336 channels 0.8 - 1.2), except with two blocks of 512 columns or
+// more, which leave most waves without one (1.0 - 1.37); where the streaming kernel runs K slices, the shorter of the two
+// estimates (27 x 620 x 13312 in blocks of 512 takes 9.1 us in slices and would take 16.2; per channel by a tenth more, the
+// estimates here are that much too long).  33 - 64 rows, two passes of the streaming kernel: against up to 16384 channels
+// (0.34 - 0.9).  More: the shorter of the two estimates, by 4 % (314 x 8176 x 12800 int4 in blocks of 128 takes 92 us in
+// 64 x 256 tiles and would take 132).  Over 12900 launches of 65 - 1000 rows, weights out of HBM, that is on average 0.4 %
+// off the better kernel, and one in 900 takes over 1.05 of the tiled GEMM's time; over 1754 of 17 - 32 rows against sliced
+// weights 0.6 %.
+int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, bool zp, bool f16, int k_slices, int k_per_slice) {
   if (M <= 16 || M > (1 << 14) || N > (1 << 20) || N % 4 != 0 || K > 65536 || K % 128 != 0 || C % 128 != 0) return -1;
   if (bits == 8 && C == K) return -1;
   if (N > (M <= 32 ? 8192 : 16384) && M <= 64) return -1;
+  if (M <= 32 && C >= 512 && C < K && K / C <= 2) return -1;
   const uint32_t m = (uint32_t)M, n = (uint32_t)N, k128 = (uint32_t)K / 128, sub = C == K ? 1 : (uint32_t)C / 128;
-  const float mb = 1e-6f * (float)N * (float)K * (float)bits / 8;
-  KsLaunch l{m, n, k128, mb, 1024, kNoLimit};
-  if (M > 64) {
-    const uint32_t tm = (m + 63) / 64, narrow = (tm * ((n + 127) / 128) + 255) / 256, wide = (tm * ((n + 255) / 256) + 255) / 256;
-    const bool use_wide = (!zp || (bits == 4 && C == 128)) && wide * (zp ? 145u : bits == 4 ? 155u : 165u) < narrow * 100u;  // (wide_tiles)
-    l.least = use_wide ? 2.13f + (float)wide * (2.13f + (zp ? 1.232f : 1.092f) * (float)k128) + 0.054f * mb
-                       : 1.02f + (float)narrow * (2.85f + (zp ? 0.757f : 0.667f) * (float)k128) + 0.085f * mb;
-  }
-  return ks_bw_best(l, sub, bits == 8, zp, ks_indices<kKsBwTiles>());
+  const bool perch = C == K;
+  KsBwLaunch l{{m, n, k128, 1e-6f * (float)N * (float)K * (float)bits / 8, 1024, kNoLimit}};
+  const int tile = ks_bw_best(l, sub, bits == 8, zp, ks_indices<kKsBwTiles>());
+  if (tile < 0 || (M <= 64 && k_slices <= 1)) return tile;
+  const auto& t = kKsBwTiles[tile].time;
+  const float rounds = (float)l.rounds, steps = (float)(l.blocks * sub);
+  const float us = t.fixed + t.round * rounds + (t.step + (bits == 8 ? t.int8 : 0.f) + (perch ? t.perch : 0.f)) * rounds * steps +
+                   t.load * (float)l.tiles / 256 * steps + (perch ? 0.f : (t.block + (zp ? t.zp : 0.f)) * rounds * (float)l.blocks) +
+                   t.weight * l.weight;
+  const uint32_t blocks = perch ? 0 : k128 / sub;
+  if (M > 64) return 1.04f * us < bw_gemm_us(m, n, k128, blocks, (uint32_t)C, bits, zp, f16) ? tile : -1;
+  return (perch ? 0.9f : 1.f) * us < bw_slices_us(M, N, C, bits, zp, perch, k_slices, k_per_slice) ? tile : -1;
 }
 
 int qmm_wo_ksplit_bw_run(int tile, const WoBwArgs& a, int bits, int x_dt, hipStream_t stream) {
@@ -965,20 +1010,23 @@ extern "C" int xla_amd_qmm_weight_only_gemm(const void* x, const void* w_tiled, 
   // (blockwise weights in the weight-streaming kernel: every dtype but the stored one is x's, at least 8 scales)
   const bool bw_ok = !blockwise || (scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt && (K / C) * N >= 8 &&
                                     (((uintptr_t)scale | (uintptr_t)zp) & 3) == 0);
+  // few rows: the weight-streaming kernel over K slices, when that is what its plan says and the workspace is there
+  int per = (int)K, slices = 1;
+  if (M <= 32 && bw_ok) {
+    slices = qmm_skinny_k_slices(M, N, K, C, bits, &per);
+    const size_t need = slice_workspace_floats(slices, M, N, blockwise) * sizeof(float);
+    if (!(workspace && workspace_bytes >= need && (((uintptr_t)workspace) & 15) == 0)) slices = 1;
+  }
   if ((blockwise || bits == 4) && scale_dt == x_dt && (!zp || zp_dt == x_dt) && dot_dt == x_dt && store_dt == x_dt &&
       ((((uintptr_t)scale | (uintptr_t)zp) & 3) | ((uintptr_t)out & 7)) == 0) {
-    const int tile = qmm_wo_ksplit_bw_tile(M, N, K, C, bits, zp != nullptr);
+    const int tile = qmm_wo_ksplit_bw_tile(M, N, K, C, bits, zp != nullptr, x_dt == XLA_AMD_DT_F16, slices, per);
     if (tile >= 0) {
       const WoBwArgs b{x, (const uint8_t*)w_tiled, scale, zp, out, (int)M, (int)N, (int)K, (int)C};
       return qmm_wo_ksplit_bw_run(tile, b, bits, x_dt, (hipStream_t)stream);
     }
   }
-  if (M <= 32 && bw_ok) {
-    // few rows: the weight-streaming kernel over K slices, when that is what its plan says and the workspace is there
-    int per;
-    const int slices = qmm_skinny_k_slices(M, N, K, C, bits, &per);
-    const size_t need = slice_workspace_floats(slices, M, N, blockwise) * sizeof(float);
-    if (slices > 1 && workspace && workspace_bytes >= need && (((uintptr_t)workspace) & 15) == 0) {
+  {
+    if (slices > 1) {
       SkinnyArgs k;
       k.x = x; k.w = (const uint8_t*)w_tiled; k.scale = scale; k.zp = zp; k.out = out;
       k.M = (int)M; k.N = (int)N; k.K = (int)K; k.C = (int)C;
