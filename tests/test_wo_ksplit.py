@@ -96,6 +96,17 @@ def test_blockwise_launches_left_to_the_older_kernels(tmp_path):
   assert rc == 0 and "ksplit" in launches[0].name, text
 
 
+def test_many_rows_against_few_channels(tmp_path):
+  """More rows than the estimates were fitted to: the reads of x decide."""
+  want = [((5650, 317, 7936, -1, 8, False), "qmm_wo_gemm_kernel"), ((2557, 949, 13952, -1, 8, False), "qmm_wo_gemm_kernel"),
+          ((2048, 1000, 640, -1, 8, True), "ksplit"), ((1500, 600, 4096, -1, 8, False), "ksplit"),
+          ((3956, 196, 3200, -1, 4, True), "qmm_wo_bw_gemm_kernelI"), ((6234, 156, 3584, 512, 4, True), "qmm_wo_bw_gemm_kernelI"),
+          ((1927, 492, 1408, 128, 8, True), "qmm_wo_bw_gemm_kernelI"), ((1200, 512, 4096, 128, 4, True), "ksplit")]
+  calls = [rec.blockwise(m, n, k, k if c == -1 else c, bits, zp, dt) for (m, n, k, c, bits, zp), _ in want for dt in (1, 2)]
+  for (shape, kernel), (rc, text, launches) in zip([w for w in want for _ in (1, 2)], rec.record(calls, str(tmp_path))):
+    assert rc == 0 and kernel in launches[0].name, (shape, text, launches)
+
+
 def test_tiles_of_the_f32_shapes(tmp_path):
   calls = [rec.skinny(m, n, k, k, 8, zp, 0) for m, n, k, _, _ in F32_SHAPES for zp in (False, True)]
   seen = set()

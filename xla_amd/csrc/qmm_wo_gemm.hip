@@ -719,6 +719,12 @@ inline int ks_best(KsLaunch& l, std::index_sequence<i...>) {
   (ks_offer<tiles, i>(l), ...);
   return l.best;
 }
+// 10^6 bytes of 2-byte x as often as they are read out of HBM: once for each XCD, as far as there are columns of tiles (see
+// ks_tile_of).  Up to the 1000 rows that the estimates were fitted to it is a small part of their other terms.
+inline float ks_x_reads(int64_t M, int64_t N, int64_t K, uint32_t bn) {
+  const int64_t columns = (N + bn - 1) / bn;
+  return 2e-6f * (float)M * (float)K * (float)(columns < 8 ? columns : 8);
+}
 template <const auto& tiles> constexpr auto ks_indices() { return std::make_index_sequence<sizeof(tiles) / sizeof(tiles[0])>(); }
 
 }  // namespace
@@ -727,7 +733,8 @@ template <const auto& tiles> constexpr auto ks_indices() { return std::make_inde
 // streaming kernel's time; wider outputs 0.99 - 1.06), except where that runs K slices of a long K (4096 x 14336: 1.01
 // - 1.03, 512 x 14336: 1.1).  More rows: the shorter of the two estimates.  Over 297 measured shapes that is on
 // average 0.4 % off the better of the two, and 0.68 of the time of the tiled GEMM with its K slices; the worst choice
-// took 5 % longer than the tiled GEMM.
+// took 5 % longer than the tiled GEMM.  More than 1000 rows: with the reads of x added (582 launches of 1000 - 8192 rows against
+// 64 - 4096 channels: 0.64 of the tiled GEMM's time, none longer by 5 %; without them up to 1.39).
 int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
   if (M <= 16 || K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14)) return -1;
   if (M <= 32) {
@@ -735,12 +742,14 @@ int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
     if (N > 8192 || (K > 8192 && qmm_skinny_k_slices(M, N, K, K, 8, &per) > 1)) return -1;
   }
   KsLaunch l{(uint32_t)M, (uint32_t)N, (uint32_t)K / 128, 1e-6f * (float)N * (float)K, 1024, kNoLimit};
-  if (M > 32) {
-    const Plan p = make_plan(M, N, K, false);
-    if (p.mt == 4 && p.ng == 4) return -1;  // more than 49152 channels: the tiled GEMM's rounds are full
-    l.least = (float)plan_us(p, M, N, K);
-  }
-  return ks_best<kKsTiles>(l, ks_indices<kKsTiles>());
+  if (M <= 32) return ks_best<kKsTiles>(l, ks_indices<kKsTiles>());
+  const Plan p = make_plan(M, N, K, false);
+  if (p.mt == 4 && p.ng == 4) return -1;  // more than 49152 channels (the tiled GEMM's rounds are full), or 128 and fewer
+  const float tiled = (float)plan_us(p, M, N, K);
+  l.least = tiled;
+  const int tile = ks_best<kKsTiles>(l, ks_indices<kKsTiles>());
+  if (tile >= 0 && M > 1000 && 1.05f * (1.03f * l.least + 0.031f * ks_x_reads(M, N, K, kKsTiles[tile].bn)) > tiled) return -1;
+  return tile;
 }
 
 // Up to 16 rows, one pass of the streaming kernel: against up to 8192 channels (0.66 - 0.97 of its time; 0.88 - 1.23 at 11700
@@ -854,7 +863,8 @@ float bw_slices_us(int64_t M, int64_t N, int64_t C, int bits, bool zp, bool perc
 // estimates here are that much too long).  33 - 64 rows, two passes of the streaming kernel: against up to 16384 channels
 // (0.34 - 0.9).  More: the shorter of the two estimates, by 4 % (314 x 8176 x 12800 int4 in blocks of 128 takes 92 us in
 // 64 x 256 tiles and would take 132).  Over 12900 launches of 65 - 1000 rows, weights out of HBM, that is on average 0.4 %
-// off the better kernel, and one in 900 takes over 1.05 of the tiled GEMM's time; over 1754 of 17 - 32 rows against sliced
+// off the better kernel, and one in 900 takes over 1.05 of the tiled GEMM's time (one in 300 of 19800 with 1000 - 8192 rows,
+// where the reads of x are added; without them up to 1.87); over 1754 of 17 - 32 rows against sliced
 // weights 0.6 %.
 int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, bool zp, bool f16, int k_slices, int k_per_slice) {
   if (M <= 16 || M > (1 << 14) || N > (1 << 20) || N % 4 != 0 || K > 65536 || K % 128 != 0 || C % 128 != 0) return -1;
@@ -868,10 +878,11 @@ int qmm_wo_ksplit_bw_tile(int64_t M, int64_t N, int64_t K, int64_t C, int bits, 
   if (tile < 0 || (M <= 64 && k_slices <= 1)) return tile;
   const auto& t = kKsBwTiles[tile].time;
   const float rounds = (float)l.rounds, steps = (float)(l.blocks * sub);
-  const float us = t.fixed + t.round * rounds + (t.step + (bits == 8 ? t.int8 : 0.f) + (perch ? t.perch : 0.f)) * rounds * steps +
+  float us = t.fixed + t.round * rounds + (t.step + (bits == 8 ? t.int8 : 0.f) + (perch ? t.perch : 0.f)) * rounds * steps +
                    t.load * (float)l.tiles / 256 * steps + (perch ? 0.f : (t.block + (zp ? t.zp : 0.f)) * rounds * (float)l.blocks) +
                    t.weight * l.weight;
   const uint32_t blocks = perch ? 0 : k128 / sub;
+  if (M > 1000) us = 1.02f * (0.925f * us + 0.0545f * ks_x_reads(M, N, K, kKsBwTiles[tile].bn));
   if (M > 64) return 1.04f * us < bw_gemm_us(m, n, k128, blocks, (uint32_t)C, bits, zp, f16) ? tile : -1;
   return (perch ? 0.9f : 1.f) * us < bw_slices_us(M, N, C, bits, zp, perch, k_slices, k_per_slice) ? tile : -1;
 }
