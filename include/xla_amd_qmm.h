@@ -170,14 +170,18 @@ int xla_amd_qmm_weight_only_skinny(const void* x, const void* w_tiled, const voi
                                    int dot_dt, int out_dt, int store_dt, void* stream);
 
 /*
- * Between the two kernels above and below lies a third (qmm_wo_ksplit.hip, per-channel int8 weights, bf16 or f16 x): a
- * tile of 16 - 64 rows x 16 - 128 channels per workgroup whose waves split K.  Both entry points run it where a
- * measured rule on M, N and K says so (more than 16 rows); it needs no workspace.
+ * Between the two kernels above and below lie two more, whose workgroups own a tile of 16 - 64 rows x 16 - 128 channels
+ * and split K over their waves: qmm_wo_ksplit.hip (per-channel int8 weights; bf16 or f16 x from 17 rows on, f32 x from
+ * one) and qmm_wo_ksplit_bw.hip (blockwise and int4 weights, N % 4 == 0, one 2-byte dtype throughout, from 17 rows
+ * on).  xla_amd_qmm_weight_only_skinny, _gemm and _gemm_f32 run them where a measured rule on the sizes says so, up to
+ * 16384 rows in at most 1024 tiles (f32 below 128 rows: 65535); they need no workspace.
  */
 
 /*
  * Bytes of workspace xla_amd_qmm_weight_only_gemm needs for a shape (0 when it
- * needs none, or for arguments it rejects).
+ * needs none, or for arguments it rejects): an upper bound over the dtypes and
+ * the zero point, which it is not told (blockwise and int4 weights against 17 -
+ * 32 rows may run without).
  */
 size_t xla_amd_qmm_weight_only_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t C, int bits);
 
@@ -194,10 +198,11 @@ size_t xla_amd_qmm_weight_only_gemm_workspace_bytes(int64_t M, int64_t N, int64_
  * cases return XLA_AMD_QMM_EUNSUPPORTED (the streaming kernel takes them).
  * Per-channel int8 weights (C == K, bits == 8): dtype arguments as for
  * xla_amd_qmm_weight_only_skinny.  Blockwise (C < K, C % 128 == 0) and int4
- * weights (bits == 4): a tile of 64 rows x 128 channels with the rounding points
+ * weights (bits == 4): a tile of 64 rows x 128 or 256 channels with the rounding points
  * of the blockwise statements (xla_quantized_matmul.py:115-133: every block's dot
  * product rounded to x's dtype before it is scaled); scale / zp [K/C, N]; they
- * need N % 4 == 0 and every dtype argument equal to x_dt, and use no workspace.
+ * need N % 4 == 0 and every dtype argument equal to x_dt, and use no workspace
+ * beyond 32 rows.
  * With at most 32 rows, few output channels and a long K (where
  * xla_amd_qmm_dispatch returns this kernel for such an M) the call runs the
  * streaming kernel over K slices instead, one slice of 64 channels per
@@ -218,7 +223,7 @@ int xla_amd_qmm_weight_only_gemm(const void* x, const void* w_tiled, const void*
 
 /*
  * The same for f32 activations (xla_amd_qmm_dispatch sends 128 rows or more
- * here; fewer take the streaming kernel, 16 rows per pass): out f32 [M,N] = F.linear(x, w) * scaler
+ * here; fewer take xla_amd_qmm_weight_only_skinny): out f32 [M,N] = F.linear(x, w) * scaler
  * (- rowsum(x) (x) zp), xla_quantized_matmul.py:113-114 with x of any floating
  * dtype, here f32.  x is split into three bf16 parts whose sum is x to the last
  * bit (hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid)) and the bf16

@@ -129,12 +129,13 @@ extern "C" int xla_amd_qmm_dispatch(int64_t M, int64_t N, int64_t K, int64_t C, 
     return XLA_AMD_KERNEL_W8A8_GENERIC;
   }
   if (C <= 0) C = K;
-  // many rows of 2-byte x against per-channel int8 weights: the tiled GEMM reads the weight once
-  // per 128 rows, the streaming kernel once per 32
+  // more rows of 2-byte x than the streaming kernel keeps, against per-channel int8 weights: the tiled GEMM, which reads
+  // the weight once per 128 rows, or behind its entry point the K split over waves
   if (C == K && bits == 8 && K % 128 == 0 && x_dt != XLA_AMD_DT_F32 && M > 32) return XLA_AMD_KERNEL_WEIGHT_ONLY_GEMM;
   // many rows of f32 x: the same GEMM over x split into three bf16 parts (xla_amd_qmm_weight_only_gemm_f32), three
-  // times the arithmetic, where the streaming kernel makes a pass over the weight for every 16 rows (from 128 rows
-  // on: 4096 x 4096 takes 103 us either way there, 14336 x 4096 118 against 250 us)
+  // times the arithmetic, or behind its entry point f32 products with K split over waves, whichever is estimated to be
+  // shorter; fewer rows do not gain from the parts (127 x 8192 x 4096 takes 76 us without; the parts take 11 and 78 per round
+  // of 128 x 128 tiles at that K)
   if (C == K && bits == 8 && K % 128 == 0 && 3 * K <= (1 << 23) && x_dt == XLA_AMD_DT_F32 && M >= 128) return XLA_AMD_KERNEL_WEIGHT_ONLY_GEMM;
   // few rows against few channels and a long K: the streaming kernel over K slices, behind the GEMM's entry point
   if ((bits == 8 || bits == 4) && x_dt != XLA_AMD_DT_F32 && K % C == 0) {
@@ -142,9 +143,9 @@ extern "C" int xla_amd_qmm_dispatch(int64_t M, int64_t N, int64_t K, int64_t C, 
     if (qmm_skinny_k_slices(M, N, K, C, bits, &per) > 1) return XLA_AMD_KERNEL_WEIGHT_ONLY_GEMM;
   }
   // many rows against blockwise or int4 weights: the tiled GEMM with per-block rounding points (the caller
-  // must also have scale / zero point / result of x's dtype; else it takes the streaming kernel, pass by pass).
-  // Up to 64 rows two passes of the streaming kernel are as fast or faster (a 64 x 128 tile per workgroup and
-  // no K split: 4096 channels are 32 workgroups).
+  // must also have scale / zero point / result of x's dtype; else it takes the streaming kernel, pass by pass), or the K
+  // split over waves.  Up to 64 rows that split stands behind the streaming kernel's entry point too, and where it is
+  // not the faster one two passes of the streaming kernel beat 64 x 128 tiles (4096 channels are 32 workgroups).
   if ((C != K || bits == 4) && (bits == 8 || bits == 4) && K % 128 == 0 && C % 128 == 0 && N % 4 == 0 &&
       x_dt != XLA_AMD_DT_F32 && M > 64)
     return XLA_AMD_KERNEL_WEIGHT_ONLY_GEMM;

@@ -146,7 +146,7 @@ constexpr KsTile kKsTiles[] = {
     {64, 64, 4, 1.40f, 0.962f, 0.344f, 2.313f, 0.031f}, {64, 96, 4, 1.65f, 1.148f, 0.466f, 2.839f, 0.047f},
     {64, 128, 4, 1.54f, 1.337f, 0.672f, 3.471f, 0.041f},
 };
-// ... and for f32 x: 1036 measurements of 300 shapes with 1 - 127 rows, rms error 2 - 8 %.
+// ... and for f32 x: 1036 measurements of 300 shapes with 1 - 127 rows, root mean square error 2 - 8 %.
 constexpr KsTile kKsTilesF32[] = {
     {16, 16, 8, 2.66f, 1.323f, 0.269f, 0.406f, 0.009f}, {16, 32, 8, 3.01f, 2.346f, 0.380f, 0.015f, 0.057f},
     {16, 64, 8, 2.16f, 4.711f, 0.129f, 1.077f, 0.078f}, {16, 16, 4, 2.93f, 0.935f, 0.138f, 0.000f, 0.000f},

@@ -731,9 +731,9 @@ template <const auto& tiles> constexpr auto ks_indices() { return std::make_inde
 
 // Up to 16 rows the streaming kernel is as fast.  17 - 32 rows: against up to 8192 channels (0.72 - 0.99 of the
 // streaming kernel's time; wider outputs 0.99 - 1.06), except where that runs K slices of a long K (4096 x 14336: 1.01
-// - 1.03, 512 x 14336: 1.1).  More rows: the shorter of the two estimates.  Over 297 measured shapes that is on
-// average 0.4 % off the better of the two, and 0.68 of the time of the tiled GEMM with its K slices; the worst choice
-// took 5 % longer than the tiled GEMM.  More than 1000 rows: with the reads of x added (582 launches of 1000 - 8192 rows against
+// - 1.03, 512 x 14336: 1.1).  More rows: the shorter of the two estimates; over the 297 shapes
+// they were fitted to that is on average 0.4 % off the better of the two, and over 2500 others of 17 - 1000 rows 1 % take more
+// than 1.04 of the kernels before, 1.1 at most.  More than 1000 rows: with the reads of x added (582 launches of 1000 - 8192 rows against
 // 64 - 4096 channels: 0.64 of the tiled GEMM's time, none longer by 5 %; without them up to 1.39).
 int qmm_wo_ksplit_tile(int64_t M, int64_t N, int64_t K) {
   if (M <= 16 || K % 128 != 0 || K > 65536 || N > (1 << 20) || M > (1 << 14)) return -1;

@@ -23,15 +23,15 @@ inline KsTiles ks_tiles(int M, int N, int bm, int bn) {
   return t;
 }
 
-// SUMS: arrays of partial sums per K group of waves; TAIL: other bytes of LDS.
-template <int XT, int MT, int NG, int KW, int CW, int SUMS, int TAIL> struct KsCfg {
+// TAIL: bytes of LDS beside the ring and, after it, the partial sums.
+template <int XT, int MT, int NG, int KW, int CW, int TAIL> struct KsCfg {
   static constexpr int NW = KW * CW;             // computing waves
   static constexpr int BM = 16 * MT, BN = 16 * NG * CW;
   static constexpr int ROW = XT == XLA_AMD_DT_F32 ? 512 : 256;  // bytes of one row of a tile (128 columns of x)
   static constexpr int TILE = BM * ROW;
   static constexpr int SLOT = KW * TILE;
   static constexpr int PITCH = BN + 4;           // floats per row of the partial sums (4 more: rows start on other banks)
-  static constexpr int kSums = KW * BM * (SUMS * PITCH + 1) * 4;  // partial sums, and partial row sums of x
+  static constexpr int kSums = KW * BM * (PITCH + 1) * 4;  // partial sums, and partial row sums of x
   static constexpr int kFit = (kLds - TAIL) / SLOT;
   static constexpr int R = kFit < 8 ? kFit : 8;  // slots of the ring
   static_assert(R >= 2, "the ring needs room to run ahead");
@@ -58,7 +58,7 @@ __device__ __forceinline__ bool ks_tile_of(const KsTiles& t, int M, int bn, int&
 // Copying wave cw: the x tiles of all slots, KW per slot (tile_of(slot, k): the k th), R - 1 slots ahead of the
 // computing waves, which it meets once per slot and once more when they have read the last one.  ahead() runs between
 // the first slots' copies and the rest, behind() before that last meeting.
-template <class Cfg, int MT, int KW, class TileOf, class Ahead, class Behind>
+template <class Cfg, int KW, class TileOf, class Ahead, class Behind>
 __device__ __forceinline__ void ks_copy_x(const void* x, int K, int m0, int rows, int steps, int cw, int lane, char* ring,
                                           TileOf&& tile_of, Ahead&& ahead_of_loop, Behind&& behind_loop) {
   typedef __attribute__((address_space(3))) void* lds_ptr_t;

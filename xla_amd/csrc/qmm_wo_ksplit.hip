@@ -15,10 +15,13 @@
 // R - 1 slots ahead by four copying waves (global -> LDS without registers; only live rows are copied); the workgroup
 // meets once per slot.  MFMA mapping and arithmetic are those of qmm_wo_gemm.hip.
 //
-// What bounds it: 4 us that do not depend on K (launch, first loads, the sums through LDS), then about 75 KB per us
-// and compute unit, x and weights together; at 64 x 48 per workgroup (100 x 6144 x 4096) the MFMAs alone would take
-// 0.87 of the 1.05 us a step of 512 columns takes.  Measured with weights out of HBM / out of the Infinity Cache, us:
-//   100 x 6144 x 4096      20.1 / 19.0  ->  14.3 / 12.1        32 x 4096 x 4096   9.9 / 9.1  ->  8.3 / 7.3
+// What bounds it: 4 us that do not depend on K (launch, first loads, the sums through LDS), then waiting: 60 - 75 KB per us
+// and compute unit arrive, x and weights together, where the copies of an LDS-tiled kernel reach 110 - 130 out of L2.  By
+// counters the waves wait for data or at the barrier of each slot in 61 % of their cycles (64 x 4096 x 4096, 32 x 32 tiles on
+// 256 compute units; the MFMAs are busy 11 % of the time, LDS conflicts cost 12 %), in 51 % for 100 x 6144 x 4096 with a zero
+// point (64 x 64 tiles, 192 workgroups; MFMAs 39 %, a third of them the row sums of x, which both waves along the channels
+// make).  Measured with weights out of HBM / out of the Infinity Cache, us:
+//   100 x 6144 x 4096      20.1 / 19.0  ->  14.0 / 12.1        32 x 4096 x 4096   9.9 / 9.1  ->  8.3 / 7.3
 //   64 x 4096 x 4096       15.3 / 13.4  ->   9.5 /  8.3        32 x 1024 x 4096   7.9 / 7.5  ->  5.9 / 5.3
 //   256 x 4096 x 4096      21.8 / 20.9  ->  15.1 / 12.9        48 x 3072 x 1536  11.0 / 9.6  ->  5.5 / 4.9
 // Tried and not kept: streaming loads of the weights (no gain out of HBM, 0.5 - 1 us lost out of the cache); a deeper
@@ -29,13 +32,17 @@
 // MFMAs, one column per lane and instruction: true f32 products, an eighth of the bf16 rate, so the matrix cores bound
 // all but the smallest launches (64 x 4096 x 4096: 22 us, 14 of them MFMAs).  The streaming kernel before it made a pass
 // over the weight per 16 rows and split K over two waves at most, 512 columns each: 8 x 1024 x 1024 6.6 -> 4.6 us, 32 x
-// 4096 x 4096 25.6 -> 14.4, 100 x 1024 x 1024 43 -> 6.5; over 300 shapes of 1 - 127 rows 0.49 of the time.
+// 4096 x 4096 25.6 -> 14.4, 100 x 1024 x 1024 43 -> 6.5; over 300 drawn launches of 1 - 127 rows 0.53 of the time (geometric
+// mean, as below).  f32 MFMAs are busy 66 % of the cycles at 64 x 4096 x 4096.
+//
+// Over 2500 drawn launches of 17 - 1000 rows of 2-byte x (N 512 - 14336, K 1024 - 14336, weights out of HBM), with the older
+// kernels where they are estimated to be faster, 0.61 of the time of the kernels before.
 //
 // This file is compiled per activation dtype and set of tiles (-DQMM_WO_XT=0|1|2 for f32 | bf16 | f16, -DQMM_KS_PART=0|1|2).
 #include "qmm_wo_ksplit.h"
 
 #if !defined(QMM_WO_XT) || !defined(QMM_KS_PART)
-#error "compile with -DQMM_WO_XT=<XLA_AMD_DT_BF16|XLA_AMD_DT_F16 value> -DQMM_KS_PART=<0|1|2>"
+#error "compile with -DQMM_WO_XT=<XLA_AMD_DT_F32|XLA_AMD_DT_BF16|XLA_AMD_DT_F16 value> -DQMM_KS_PART=<0|1|2>"
 #endif
 
 namespace {
@@ -46,7 +53,7 @@ template <int NG, int CW> constexpr int ks_tail() { return 2 * 16 * NG * CW * 4;
 template <int XT, int MT, int NG, int KW, int CW, int P, bool HASZP, bool UNI>
 __global__ void __launch_bounds__((KW * CW + kCopyWaves) * 64)
 qmm_wo_ksplit_kernel(KsArgs a) {
-  using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, ks_tail<NG, CW>()>;
+  using Cfg = KsCfg<XT, MT, NG, KW, CW, ks_tail<NG, CW>()>;
   constexpr bool kF32 = XT == XLA_AMD_DT_F32;
   constexpr int NW = Cfg::NW, BM = Cfg::BM, BN = Cfg::BN, TILE = Cfg::TILE, SLOT = Cfg::SLOT, R = Cfg::R;
   constexpr int kThreads = (NW + kCopyWaves) * 64;
@@ -70,7 +77,7 @@ qmm_wo_ksplit_kernel(KsArgs a) {
     // ---- copying waves: x, and the scales of the tile's channels, which are used at the very end ----
     const int cw = wave - NW;
     uint32_t s_raw = 0, z_raw = 0;
-    ks_copy_x<Cfg, MT, KW>(
+    ks_copy_x<Cfg, KW>(
         a.x, K, m0, rows, steps, cw, lane, ring, [&](int n, int k) { return min(n * KW + k, n_tiles - 1); },
         [&]() {
           if (cw * 64 + lane < BN) {
@@ -221,7 +228,7 @@ qmm_wo_ksplit_kernel(KsArgs a) {
 
 template <int XT, int MT, int NG, int KW, int CW, int P>
 int launch(KsArgs& a, hipStream_t stream) {
-  using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, ks_tail<NG, CW>()>;
+  using Cfg = KsCfg<XT, MT, NG, KW, CW, ks_tail<NG, CW>()>;
   a.t = ks_tiles(a.M, a.N, Cfg::BM, Cfg::BN);
   const dim3 grid(8u * (unsigned)a.t.per_xcd), block((Cfg::NW + kCopyWaves) * 64);
   const int steps = (a.K / 128 + KW - 1) / KW;

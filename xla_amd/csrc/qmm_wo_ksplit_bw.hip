@@ -8,8 +8,8 @@
 // The tiled GEMM splits no K (100 rows against 4096 channels are 64 workgroups), and up to 64 rows the streaming kernel
 // made a pass over the weight per 32.  Weights out of HBM / out of the Infinity Cache (geometric mean), us, int4 in blocks
 // of 128 with zero points against 4096 x 4096: 32 rows 14.6 -> 8.9, 64 rows 28.4 -> 10.8, 128 rows 28.2 -> 14.4, 256 rows
-// 28.5 -> 25; against 4096 x 14336 without: 64 rows 79 -> 27, 128 rows 82 -> 36.  Over 218 shapes of 17 - 1000 rows, with
-// the older kernels where they are estimated to be faster, 0.59 of the time.  What bounds it: fetching, as there, up to
+// 28.5 -> 25; against 4096 x 14336 without: 64 rows 79 -> 27, 128 rows 82 -> 36.  Over 2500 drawn launches of 17 -
+// 1000 rows, with the older kernels where they are estimated to be faster, 0.63 of the time (geometric mean).  What bounds it: fetching, as there, up to
 // 32 rows; beyond, the vector instructions of a block's end (four to six per result and block).
 //
 // Arithmetic, one dtype (x's) throughout:
@@ -29,7 +29,7 @@ namespace {
 template <int XT, int BITS, int MT, int NG, int KW, int CW, int P, bool HASZP, bool PERCH>
 __global__ void __launch_bounds__((KW * CW + kCopyWaves) * 64)
 qmm_wo_bw_gemm_kernel_ksplit(WoBwArgs a, KsTiles t) {
-  using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, 0>;
+  using Cfg = KsCfg<XT, MT, NG, KW, CW, 0>;
   constexpr int NW = Cfg::NW, BM = Cfg::BM, BN = Cfg::BN, TILE = Cfg::TILE, SLOT = Cfg::SLOT, R = Cfg::R;
   constexpr int kThreads = (NW + kCopyWaves) * 64;
   constexpr bool NEEDXS = HASZP || BITS == 4;
@@ -52,7 +52,7 @@ qmm_wo_bw_gemm_kernel_ksplit(WoBwArgs a, KsTiles t) {
   const int steps = (n_blocks + KW - 1) / KW * sub;
 
   if (__builtin_expect(wave >= NW, 0)) {
-    ks_copy_x<Cfg, MT, KW>(
+    ks_copy_x<Cfg, KW>(
         a.x, K, m0, rows, steps, wave - NW, lane, ring,
         [&](int n, int k) {
           const int u = sub == 1 ? n : n / sub;
@@ -254,7 +254,7 @@ qmm_wo_bw_gemm_kernel_ksplit(WoBwArgs a, KsTiles t) {
 // ZP: a tile for launches with a zero point too (96 more sums would not fit the registers of the largest one)
 template <int XT, int BITS, int MT, int NG, int KW, int CW, int P, bool ZP = true>
 int launch(const WoBwArgs& a, hipStream_t stream) {
-  using Cfg = KsCfg<XT, MT, NG, KW, CW, 1, 0>;
+  using Cfg = KsCfg<XT, MT, NG, KW, CW, 0>;
   const KsTiles t = ks_tiles(a.M, a.N, Cfg::BM, Cfg::BN);
   const dim3 grid(8u * (unsigned)t.per_xcd), block((Cfg::NW + kCopyWaves) * 64);
   const bool perch = a.C == a.K;
