@@ -1036,38 +1036,36 @@ extern "C" int xla_amd_qmm_weight_only_gemm(const void* x, const void* w_tiled, 
       return qmm_wo_ksplit_bw_run(tile, b, bits, x_dt, (hipStream_t)stream);
     }
   }
-  {
-    if (slices > 1) {
-      SkinnyArgs k;
-      k.x = x; k.w = (const uint8_t*)w_tiled; k.scale = scale; k.zp = zp; k.out = out;
-      k.M = (int)M; k.N = (int)N; k.K = (int)K; k.C = (int)C;
-      k.G = xla_amd_qmm_tile_group(N, K, C, bits);
-      k.scale_dt = scale_dt; k.zp_dt = zp ? zp_dt : x_dt; k.out_dt = out_dt; k.dot_dt = dot_dt; k.store_dt = store_dt;
-      k.k_per_slice = per; k.slices = slices;
-      k.part = (float*)workspace;
-      const size_t mn = (size_t)slices * (size_t)M * (size_t)N;
-      k.part_xs = blockwise ? nullptr : k.part + mn;
-      k.part_z = blockwise && zp ? k.part + mn : nullptr;
-      int rc = x_dt == XLA_AMD_DT_BF16 ? qmm_skinny_launch_bf16(k, bits, zp != nullptr, (hipStream_t)stream)
-                                       : qmm_skinny_launch_f16(k, bits, zp != nullptr, (hipStream_t)stream);
-      if (rc != XLA_AMD_QMM_OK) return rc;
-      if (blockwise) {
-        const int64_t threads = M * (N / 4);
-        hipLaunchKernelGGL(qmm_wo_bw_finish_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                           (hipStream_t)stream, k.part, k.part_z, out, (int)M, (int)N, slices, out_dt,
-                           qmm_promote(x_dt, k.zp_dt), store_dt);
-        return QMM_CHECK_LAUNCH("weight_only_gemm blockwise finish launch");
-      }
-      WoGemmArgs f;
-      f.x = x; f.w = (const uint8_t*)w_tiled; f.scale = scale; f.zp = zp; f.out = out;
-      f.part = k.part; f.part_xs = k.part_xs;
-      f.M = (int)M; f.N = (int)N; f.K = (int)K; f.G = k.G; f.k_per_split = per; f.split = slices;
-      f.scale_dt = scale_dt; f.zp_dt = zp ? zp_dt : x_dt; f.dot_dt = dot_dt; f.out_dt = out_dt; f.store_dt = store_dt;
-      const int64_t threads = M * ((N + 3) / 4);
-      hipLaunchKernelGGL(qmm_wo_gemm_finish_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                         (hipStream_t)stream, f, x_dt);
-      return QMM_CHECK_LAUNCH("weight_only_gemm finish launch");
+  if (slices > 1) {
+    SkinnyArgs k;
+    k.x = x; k.w = (const uint8_t*)w_tiled; k.scale = scale; k.zp = zp; k.out = out;
+    k.M = (int)M; k.N = (int)N; k.K = (int)K; k.C = (int)C;
+    k.G = xla_amd_qmm_tile_group(N, K, C, bits);
+    k.scale_dt = scale_dt; k.zp_dt = zp ? zp_dt : x_dt; k.out_dt = out_dt; k.dot_dt = dot_dt; k.store_dt = store_dt;
+    k.k_per_slice = per; k.slices = slices;
+    k.part = (float*)workspace;
+    const size_t mn = (size_t)slices * (size_t)M * (size_t)N;
+    k.part_xs = blockwise ? nullptr : k.part + mn;
+    k.part_z = blockwise && zp ? k.part + mn : nullptr;
+    int rc = x_dt == XLA_AMD_DT_BF16 ? qmm_skinny_launch_bf16(k, bits, zp != nullptr, (hipStream_t)stream)
+                                     : qmm_skinny_launch_f16(k, bits, zp != nullptr, (hipStream_t)stream);
+    if (rc != XLA_AMD_QMM_OK) return rc;
+    if (blockwise) {
+      const int64_t threads = M * (N / 4);
+      hipLaunchKernelGGL(qmm_wo_bw_finish_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                         (hipStream_t)stream, k.part, k.part_z, out, (int)M, (int)N, slices, out_dt,
+                         qmm_promote(x_dt, k.zp_dt), store_dt);
+      return QMM_CHECK_LAUNCH("weight_only_gemm blockwise finish launch");
     }
+    WoGemmArgs f;
+    f.x = x; f.w = (const uint8_t*)w_tiled; f.scale = scale; f.zp = zp; f.out = out;
+    f.part = k.part; f.part_xs = k.part_xs;
+    f.M = (int)M; f.N = (int)N; f.K = (int)K; f.G = k.G; f.k_per_split = per; f.split = slices;
+    f.scale_dt = scale_dt; f.zp_dt = zp ? zp_dt : x_dt; f.dot_dt = dot_dt; f.out_dt = out_dt; f.store_dt = store_dt;
+    const int64_t threads = M * ((N + 3) / 4);
+    hipLaunchKernelGGL(qmm_wo_gemm_finish_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, f, x_dt);
+    return QMM_CHECK_LAUNCH("weight_only_gemm finish launch");
   }
   if (C != K || bits != 8) {
     // blockwise and int4 weights: the tiled GEMM with per-block rounding points (every dtype x's)
